@@ -1478,7 +1478,9 @@ int rf_run(rhg_context_t *c, const rhg_columns_t *cols, int32_t device_ptrs,
   int64_t chunk = (int64_t) (avail / 2 / per_col);
   if (chunk < 1) return fail(RHG_ENOMEM, "device memory too small for one response-function column");
   if (chunk > ncol_all) chunk = ncol_all;
-  if (chunk > 64) chunk = chunk / 64 * 64;
+  // whole blocks of 64 columns where the batch is split; a batch that fits is
+  // one chunk (90 columns of the 400-line list as 64 + 26: 343 ms, as 90: 178 ms)
+  if (chunk < ncol_all && chunk > 64) chunk = chunk / 64 * 64;
   // PYRH_AMD_RF_CHUNK caps the chunk (tests of the chunked path)
   if (const char *cap = getenv("PYRH_AMD_RF_CHUNK")) {
     const long v = strtol(cap, nullptr, 10);
@@ -1862,7 +1864,10 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
   HIPCHECK(hipMemGetInfo(&freeb, &totb));
   const size_t budget = freeb / 4 * 3;
   int chunk = (int) std::min<size_t>((size_t) ncol_all, budget / per_col);
-  if (chunk > 64) chunk = chunk / 64 * 64;
+  // whole blocks of 64 columns where the batch is split; a batch that fits is
+  // one chunk whatever its size (1500 columns of the Ca II atom as 1472 + 28
+  // ran a second solve for the 28: 694 ms, in one chunk 521 ms)
+  if (chunk < ncol_all && chunk > 64) chunk = chunk / 64 * 64;
   if (chunk < 1) return fail(RHG_ENOMEM, "device memory too small for one NLTE column");
 
   NlteTimer tm_all, tm_k;
