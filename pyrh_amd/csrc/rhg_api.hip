@@ -107,7 +107,7 @@ struct rhg_context {
   DevBuf atmos, ndep, state, moving, cchi, ceta, stokes, chiref, census, census_sum;
   // response functions: perturbed inputs/states, tangents, tape, adjoints
   DevBuf rf_atm[2], rf_state[2], rf_cont[4], rf_chiref[2], rf_moving, rf_ndep, rf_dstate,
-      rf_dcont[2], rf_dchiref, rf_car, rf_aP, rf_aZ, rf_aB, rf_out;
+      rf_dcont[2], rf_dchiref, rf_pts, rf_car, rf_aP, rf_aZ, rf_aB, rf_out;
   // log gf response functions: inward intensities, output, parameter lines
   DevBuf at_iin, at_out, at_par;
   // NLTE: the active atom (packed arrays and its DevNlte), the batch arrays
@@ -1395,26 +1395,40 @@ int rf_chunk(rhg_context_t *c, const double *d_atm, const int32_t *d_ndep, int n
     dim3 grd((unsigned) rhg::xcd_grid(ncb, npol));
     double *car = (double *) c->rf_car.p;
     R *aP = (R *) c->rf_aP.p, *aZ = (R *) c->rf_aZ.p, *aB = (R *) c->rf_aB.p;
-    hipLaunchKernelGGL(rhg::k_rf_forward<R>, grd, blk, 0, c->stream, c->d_model, d_ndep, moving, ncol,
-                       Nmax, state, c->d_out_ls, c->d_io_pol, npol, nout, cchi, ceta, mu, d_out,
-                       car);
+    double *pts = (double *) c->rf_pts.p;
+    // The points and the chain are independent over depth: their depths are
+    // split over workgroups until about 16 waves per SIMD are queued (1024
+    // SIMDs), so that few rays fill the chip and ragged columns even out.
+    const int64_t rays = (int64_t) ncb * npol;
+    const int nsplit = (int) std::min<int64_t>(Nmax, std::max<int64_t>(1, 16384 / rays));
+    const int kd = (Nmax + nsplit - 1) / nsplit;
+    const dim3 grdk(grd.x, (unsigned) ((Nmax + kd - 1) / kd));
+#define RHG_LAUNCH_PTS(LT)                                                                       \
+  hipLaunchKernelGGL((rhg::k_rf_points<R, LT>), grdk, blk, LT ? (unsigned) c->tab_bytes : 0u,    \
+                     c->stream, c->d_model, d_ndep, moving, ncol, Nmax, state, c->d_out_ls,      \
+                     c->d_io_pol, npol, cchi, ceta, mu, kd, pts, c->tab_maxl, c->tab_maxc)
+    if (c->tab_bytes > 0 && c->tune_line_table) RHG_LAUNCH_PTS(true);
+    else RHG_LAUNCH_PTS(false);
+#undef RHG_LAUNCH_PTS
+    HIPCHECK(hipGetLastError());
+    hipLaunchKernelGGL((rhg::k_rf_forward<sizeof(R) == 4>), grd, blk, 0, c->stream, c->d_model, d_ndep,
+                       ncol, Nmax, state, c->d_out_ls, c->d_io_pol, npol, nout,
+                       (const double *) pts, mu, d_out, car);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipEventRecord(c->ev[3], c->stream));
-    hipLaunchKernelGGL(rhg::k_rf_reverse<R>, grd, blk, 0, c->stream, c->d_model, d_ndep, moving, ncol,
-                       Nmax, state, c->d_out_ls, c->d_io_pol, npol, cchi, ceta, mu, car, aP, aZ,
-                       aB);
+    hipLaunchKernelGGL(rhg::k_rf_reverse<R>, grd, blk, 0, c->stream, c->d_model, d_ndep, ncol,
+                       Nmax, state, c->d_out_ls, c->d_io_pol, npol, (const double *) pts, mu,
+                       (const double *) car, aP, aZ, aB);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipEventRecord(c->ev[4], c->stream));
-    if (pl.npar <= 3)
-      hipLaunchKernelGGL((rhg::k_rf_chain<R, 3>), grd, blk, 0, c->stream, c->d_model, d_ndep, moving,
-                         ncol, Nmax, state, dstate, chiref, (const double *) c->rf_dchiref.p, cchi,
-                         ceta, (const R *) c->rf_dcont[0].p, (const R *) c->rf_dcont[1].p,
-                         c->d_out_ls, c->d_io_pol, npol, nout, mu, scale, pl, aP, aZ, aB, d_rf, ldr);
-    else
-      hipLaunchKernelGGL((rhg::k_rf_chain<R, 6>), grd, blk, 0, c->stream, c->d_model, d_ndep, moving,
-                         ncol, Nmax, state, dstate, chiref, (const double *) c->rf_dchiref.p, cchi,
-                         ceta, (const R *) c->rf_dcont[0].p, (const R *) c->rf_dcont[1].p,
-                         c->d_out_ls, c->d_io_pol, npol, nout, mu, scale, pl, aP, aZ, aB, d_rf, ldr);
+#define RHG_LAUNCH_CHAIN(NP)                                                                     \
+  hipLaunchKernelGGL((rhg::k_rf_chain<R, NP>), grdk, blk, 0, c->stream, c->d_model, d_ndep, moving, \
+                     ncol, Nmax, state, dstate, chiref, (const double *) c->rf_dchiref.p, cchi,  \
+                     ceta, (const R *) c->rf_dcont[0].p, (const R *) c->rf_dcont[1].p,           \
+                     c->d_out_ls, c->d_io_pol, npol, nout, mu, scale, pl, aP, aZ, aB, d_rf, ldr, kd)
+    if (pl.npar <= 3) RHG_LAUNCH_CHAIN(3);
+    else RHG_LAUNCH_CHAIN(6);
+#undef RHG_LAUNCH_CHAIN
     HIPCHECK(hipGetLastError());
   } else {
     HIPCHECK(hipEventRecord(c->ev[3], c->stream));
@@ -1439,7 +1453,7 @@ int rf_chunk(rhg_context_t *c, const double *d_atm, const int32_t *d_ndep, int n
 
 // The response functions of a batch, in column chunks whose work buffers
 // (column state, continuum, tangents, the forward sweep's carried state and
-// the point adjoints: about npol * Nmax * 300 bytes per column) fit in half
+// the points, the point adjoints: about npol * Nmax * 360 bytes per column) fit in half
 // of the device memory available; the outputs are the whole batch's.
 template <typename R>
 int rf_run(rhg_context_t *c, const rhg_columns_t *cols, int32_t device_ptrs,
@@ -1456,13 +1470,13 @@ int rf_run(rhg_context_t *c, const rhg_columns_t *cols, int32_t device_ptrs,
       (size_t) Nmax * ((size_t) nfield * 8 + 2 * nout * rsz + 8 + ncopy * 9 * 8 +
                        ncopy * (size_t) nfield * 8 + 4 * (size_t) nout * 8 + 2 * 8 +
                        RHG_RF_NPARAM * (size_t) nfield * 8 + 2 * nout * rsz + 8 +
-                       npl * rhg::RF_NCARRY * 8 + npl * 4 * 8 * rsz + npl * 4 * rsz) +
+                       npl * 8 * 8 + npl * rhg::RF_NCARRY * 8 + npl * 4 * 8 * rsz + npl * 4 * rsz) +
       npl * 8 * rsz + (1 + 2 * ncopy) * sizeof(int32_t);
   DevBuf *work[] = {&c->state, &c->moving, &c->cchi, &c->ceta, &c->chiref, &c->rf_atm[0],
                     &c->rf_atm[1], &c->rf_state[0], &c->rf_state[1], &c->rf_cont[0],
                     &c->rf_cont[1], &c->rf_cont[2], &c->rf_cont[3], &c->rf_chiref[0],
                     &c->rf_chiref[1], &c->rf_moving, &c->rf_ndep, &c->rf_dstate, &c->rf_dcont[0],
-                    &c->rf_dcont[1], &c->rf_dchiref, &c->rf_car, &c->rf_aP, &c->rf_aZ, &c->rf_aB};
+                    &c->rf_dcont[1], &c->rf_dchiref, &c->rf_pts, &c->rf_car, &c->rf_aP, &c->rf_aZ, &c->rf_aB};
   size_t held = 0;
   for (DevBuf *b : work) held += b->bytes;
   size_t freeb = 0, totb = 0;
@@ -1491,6 +1505,7 @@ int rf_run(rhg_context_t *c, const rhg_columns_t *cols, int32_t device_ptrs,
   const size_t st_b = (size_t) npts * nfield * sizeof(double);
   const size_t cc_b = (size_t) npts * nout * rsz;
   const size_t cc64_b = (size_t) npts * nout * sizeof(double);
+  const size_t pts_b = npl * Nmax * 8 * chunk * sizeof(double);
   const size_t car_b = npl * Nmax * rhg::RF_NCARRY * chunk * sizeof(double);
   const size_t aP_b = npl * 4 * Nmax * 8 * chunk * rsz;
   const size_t aZ_b = npl * 4 * Nmax * chunk * rsz;
@@ -1507,7 +1522,7 @@ int rf_run(rhg_context_t *c, const rhg_columns_t *cols, int32_t device_ptrs,
       c->rf_ndep.ensure(ncopy * chunk * sizeof(int32_t)) ||
       c->rf_dstate.ensure(st_b * RHG_RF_NPARAM) || c->rf_dcont[0].ensure(cc_b) ||
       c->rf_dcont[1].ensure(cc_b) || c->rf_dchiref.ensure((size_t) npts * sizeof(double)) ||
-      c->rf_car.ensure(car_b) || c->rf_aP.ensure(aP_b) ||
+      c->rf_pts.ensure(pts_b) || c->rf_car.ensure(car_b) || c->rf_aP.ensure(aP_b) ||
       c->rf_aZ.ensure(aZ_b) || c->rf_aB.ensure(aB_b))
     return fail(RHG_ENOMEM, "device allocation for the response functions failed");
   const double *d_atm = (const double *) cols->atmos;

@@ -508,16 +508,23 @@ __global__ void k_rf_rep_ndep(const int32_t *ndep, int ncol, int32_t *out);
 template <typename O>
 __global__ void k_rf_diff(const double *S, int64_t W, int64_t off_p, int64_t off_m, int ncol,
                           int64_t nrows, double scale, O *out);
+template <typename R, bool LT>
+__global__ void k_rf_points(const DevModel *M, const int32_t *ndep, const int32_t *moving, int ncol,
+                            int Nmax, const double *state, const int32_t *out_ls,
+                            const int32_t *io_list, int nlist, const R *cchi, const R *ceta,
+                            double mu, int kd, double *pts, int tab_maxl, int tab_maxc);
+// FP64 in both forms; FORM 0 keeps the reference's operation order, FORM 1 is
+// compiled with FMA contraction
+template <int FORM>
+__global__ void k_rf_forward(const DevModel *M, const int32_t *ndep, int ncol, int Nmax,
+                             const double *state, const int32_t *out_ls, const int32_t *io_list,
+                             int nlist, int nout, const double *pts, double mu, double *stokes,
+                             double *car);
 template <typename R>
-__global__ void k_rf_forward(const DevModel *M, const int32_t *ndep, const int32_t *moving, int ncol,
-                             int Nmax, const double *state, const int32_t *out_ls,
-                             const int32_t *io_list, int nlist, int nout, const R *cchi,
-                             const R *ceta, double mu, double *stokes, double *car);
-template <typename R>
-__global__ void k_rf_reverse(const DevModel *M, const int32_t *ndep, const int32_t *moving, int ncol,
-                             int Nmax, const double *state, const int32_t *out_ls,
-                             const int32_t *io_list, int nlist, const R *cchi, const R *ceta,
-                             double mu, const double *car, R *aP, R *aZ, R *aB);
+__global__ void k_rf_reverse(const DevModel *M, const int32_t *ndep, int ncol, int Nmax,
+                             const double *state, const int32_t *out_ls, const int32_t *io_list,
+                             int nlist, const double *pts, double mu, const double *car, R *aP,
+                             R *aZ, R *aB);
 // the response-function parameters of one call (rhg_rf_param order)
 struct RfParamList {
   int32_t npar;
@@ -529,7 +536,7 @@ __global__ void k_rf_chain(const DevModel *M, const int32_t *ndep, const int32_t
                            const double *dchiref, const R *cchi, const R *ceta, const R *dcchi,
                            const R *dceta, const int32_t *out_ls, const int32_t *io_list, int nlist,
                            int nout, double mu, int atm_scale, RfParamList pl, const R *aP,
-                           const R *aZ, const R *aB, R *rf, int64_t ldr);
+                           const R *aZ, const R *aB, R *rf, int64_t ldr, int kd);
 __global__ void k_census(const DevModel *M, const int32_t *ndep, const int32_t *moving, int ncol,
                          int Nmax, const double *state, int nfield, const int32_t *out_ls,
                          int nout, double mu, int32_t *census);

@@ -8,17 +8,18 @@
 //     depth perturbed at once gives d(field)/d p(k) at all depths
 //     (k_rf_perturb + k_state twice, FP64); the same for the continuum and
 //     for chi at the reference wavelength.
-//  2. k_rf_forward: the synthesis of k_formal_stokes that also keeps, per
-//     ray, the 13 carried scalars of the recursion entering each depth step
+//  2. k_rf_points: the points (opacity, source functions, reduced
+//     propagation matrix) of every ray and depth, in parallel over depths;
+//     k_rf_forward: the recursion of k_formal_stokes on them, which also
+//     keeps, per ray, the 13 carried scalars entering each depth step
 //     (Stokes vector, derivatives of S and q, optical-depth interval, chi
-//     derivative); not the points.
+//     derivative).
 //  3. k_rf_reverse: one reverse depth sweep per ray for the four outputs
 //     I, Q, U, V at once, with the hand-written vector-Jacobian product of
-//     each step (delo_step_vjp, rhg_adjoint.hpp).  The points (opacity,
-//     source functions, reduced propagation matrix) are formed again as the
-//     sweep reaches them.  Each point's adjoint is stored once, when the
-//     last step reading it is done, with those of the path lengths |dz| and
-//     of the lower boundary's Planck values.
+//     each step (delo_step_vjp, rhg_adjoint.hpp), reading the same points.
+//     Each point's adjoint is stored once, when the last step reading it is
+//     done, with those of the path lengths |dz| and of the lower boundary's
+//     Planck values.
 //  4. k_rf_chain: per (ray, depth), the point's derivative along each
 //     parameter's state tangent (form_point on dual numbers: line opacity,
 //     Zeeman-split Voigt/Faraday-Voigt profiles, continuum), contracted with
@@ -65,9 +66,8 @@ __device__ __forceinline__ T point_get(const Point<T> &p, int m) {
 
 // carry[((t * Nmax + k) * NCARRY_STEP + c) * ncol + column] (t = entry of the
 // wavelength list): the carried state entering the step at depth k
-// (k = 1 .. N-2); k = 0 holds the state entering the last interval.  The
-// points (opacity, source functions, K') are not stored: the reverse sweep
-// forms them again.
+// (k = 1 .. N-2); k = 0 holds the state entering the last interval.
+// pts[((t * Nmax + k) * 8 + m) * ncol + column]: the points (point_get order).
 #define RF_SETUP()                                                                       \
   const DevModel &M = *Mp;                                                               \
   int cb, t;                                                                             \
@@ -77,40 +77,90 @@ __device__ __forceinline__ T point_get(const Point<T> &p, int m) {
   const int io = io_list[t];                                                             \
   const int N = ndep[ic];                                                                \
   const int ls = out_ls[io];                                                             \
-  const int moving = moving_arr[ic];                                                     \
   const int64_t fs = (int64_t) Nmax * ncol;                                              \
   const double *st0 = state + ic;                                                        \
   const double *dzc = st0 + (int64_t) RHG_CF_DZ * fs;                                    \
   const double *Tc = st0 + (int64_t) RHG_CF_T * fs;                                      \
   const double *lc = M.lamconst + (int64_t) ls * RHG_LC_NCONST;                          \
-  (void) lc; (void) Tc; (void) moving;
+  (void) lc; (void) Tc; (void) dzc;
 #define DZ(kk) dzc[(int64_t) (kk) * ncol]
 #define CAR(kk, c) car[((((int64_t) t * Nmax + (kk)) * NCARRY_STEP + (c)) * ncol) + ic]
-// the point at depth jj: FP64, with the Voigt functions in R
+// the point at depth jj
 #define RF_POINT(jj, P)                                                                  \
-  form_point_v<R>(M, ls, has_line, st0 + (int64_t) (jj) * ncol, fs, mu_d, moving,        \
-                  cc[(int64_t) (jj) * ncol], ce[(int64_t) (jj) * ncol], P)
+  do {                                                                                   \
+    const double *pp_ = pts + ((int64_t) t * Nmax + (jj)) * 8 * ncol + ic;               \
+    P.chi = pp_[0];                                                                      \
+    _Pragma("unroll") for (int n_ = 0; n_ < 4; n_++) P.S[n_] = pp_[(1 + n_) * (int64_t) ncol]; \
+    _Pragma("unroll") for (int n_ = 0; n_ < 3; n_++) P.q[n_] = pp_[(5 + n_) * (int64_t) ncol]; \
+  } while (0)
 
-template <typename R>
+// The points of depths blockIdx.y * kd .. + kd - 1 of every ray: FP64, with
+// the Voigt functions in R, the wavelength's line list staged in LDS (LT) or
+// read from the model.  A ray's sweeps are a serial chain over depth and a
+// small batch has few rays, so forming the points inside the sweeps (twice,
+// and again in every wave's chain) left the chip idle: the points are formed
+// here with every depth at once and read back, 64 bytes each.
+//   90 columns of 64-256 depths, 350 wavelengths of the 400-line list, FP64:
+//   forward 23.0 -> 2.3 + 9.9 for the points, reverse 75.8 -> 25.3 ms; the
+//   512-column 112-wavelength batch (FP32 form) 0.85 -> 0.20 + 0.25 and
+//   1.87 -> 1.17 ms
+template <typename R, bool LT>
 __global__ void __launch_bounds__(64)
-k_rf_forward(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
-             const int32_t *__restrict__ moving_arr, int ncol, int Nmax,
-             const double *__restrict__ state, const int32_t *__restrict__ out_ls,
-             const int32_t *__restrict__ io_list, int nlist, int nout,
-             const R *__restrict__ cchi, const R *__restrict__ ceta, double mu_d,
-             double *__restrict__ stokes, double *__restrict__ car) {
+k_rf_points(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
+            const int32_t *__restrict__ moving_arr, int ncol, int Nmax,
+            const double *__restrict__ state, const int32_t *__restrict__ out_ls,
+            const int32_t *__restrict__ io_list, int nlist, const R *__restrict__ cchi,
+            const R *__restrict__ ceta, double mu_d, int kd, double *__restrict__ pts,
+            int tab_maxl, int tab_maxc) {
+  int cb0, t0;
+  xcd_tile(blockIdx.x, nlist, cb0, t0);
+  if (cb0 * 64 >= ncol) return;
+  auto tab = [&]() {
+    const int ls0 = out_ls[io_list[t0]];
+    if constexpr (LT) {
+      extern __shared__ __align__(8) char lds_tab[];
+      return stage_lines(*Mp, ls0, lds_tab, tab_maxl, tab_maxc);
+    } else {
+      const int p0 = Mp->lam_line_ptr[ls0];
+      return LineTabG(*Mp, p0, Mp->lam_line_ptr[ls0 + 1] - p0);
+    }
+  }();
   RF_SETUP();
+  const int moving = moving_arr[ic];
   const R *cc = cchi + (int64_t) io * Nmax * ncol + ic;
   const R *ce = ceta + (int64_t) io * Nmax * ncol + ic;
   const int has_line = ldc(M.lam_line_ptr)[ls + 1] > ldc(M.lam_line_ptr)[ls];
+  const int k0 = (int) blockIdx.y * kd, k1 = N < k0 + kd ? N : k0 + kd;
+  for (int k = k0; k < k1; k++) {
+    Point<double> P;
+    form_point_vt<R, R, false>(tab, M.ncont, has_line, st0 + (int64_t) k * ncol, fs, mu_d, moving,
+                               cc[(int64_t) k * ncol], ce[(int64_t) k * ncol], P);
+    double *pp = pts + ((int64_t) t * Nmax + k) * 8 * ncol + ic;
+#pragma unroll
+    for (int m = 0; m < 8; m++) pp[m * (int64_t) ncol] = point_get(P, m);
+  }
+}
+
+template <int FORM>
+__global__ void __launch_bounds__(64)
+k_rf_forward(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
+             int ncol, int Nmax,
+             const double *__restrict__ state, const int32_t *__restrict__ out_ls,
+             const int32_t *__restrict__ io_list, int nlist, int nout,
+             const double *__restrict__ pts, double mu_d,
+             double *__restrict__ stokes, double *__restrict__ car) {
+  RF_SETUP();
   const double imu = 1.0 / mu_d;
   const double B2a = planck(Tc[(int64_t) (N - 2) * ncol], lc[RHG_LC_HC_KLA], lc[RHG_LC_TWOHNU3_C2]);
   const double B2b = planck(Tc[(int64_t) (N - 1) * ncol], lc[RHG_LC_HC_KLA], lc[RHG_LC_TWOHNU3_C2]);
   DeloState<double> s;
-  Point<double> Pn;
+  Point<double> Pn, Pa;
+  RF_POINT(N - 1, Pa);
   double cv[NCARRY_STEP];
   for (int j = N - 1; j >= -1; j--) {
-    if (j >= 0) RF_POINT(j, Pn);
+    // the next point's loads are in flight while this step runs
+    Pn = Pa;
+    if (j > 0) RF_POINT(j - 1, Pa);
     if (j == N - 1) {
       s.Pu = Pn;
     } else if (j == N - 2) {
@@ -176,8 +226,8 @@ struct PbarRing {
 
 // One reverse sweep per (column, wavelength) for the four outputs at once:
 // the last interval, each depth step and the prologue by their hand-written
-// vector-Jacobian products (rhg_adjoint.hpp).  The points are formed again,
-// one per step (the point k+1 entering the window of step k); the carried
+// vector-Jacobian products (rhg_adjoint.hpp), on k_rf_points's points (one
+// read per step, the point k+1 entering the window of step k); the carried
 // state entering each step comes from the forward pass.  A point's adjoint
 // is complete after the step at which it is the second point downwind
 // (k = j + 2) and is stored then, once; a path length's after the step
@@ -185,16 +235,13 @@ struct PbarRing {
 template <typename R>
 __global__ void __launch_bounds__(64)
 k_rf_reverse(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
-             const int32_t *__restrict__ moving_arr, int ncol, int Nmax,
+             int ncol, int Nmax,
              const double *__restrict__ state, const int32_t *__restrict__ out_ls,
-             const int32_t *__restrict__ io_list, int nlist, const R *__restrict__ cchi,
-             const R *__restrict__ ceta, double mu_d, const double *__restrict__ car,
+             const int32_t *__restrict__ io_list, int nlist, const double *__restrict__ pts,
+             double mu_d, const double *__restrict__ car,
              R *__restrict__ aP, R *__restrict__ aZ, R *__restrict__ aB) {
   __shared__ R ring_lds[4 * 4 * 8 * 64];
   RF_SETUP();
-  const R *cc = cchi + (int64_t) io * Nmax * ncol + ic;
-  const R *ce = ceta + (int64_t) io * Nmax * ncol + ic;
-  const int has_line = ldc(M.lam_line_ptr)[ls + 1] > ldc(M.lam_line_ptr)[ls];
   const double imu = 1.0 / mu_d;
   PbarRing<R> ring{ring_lds, (int) threadIdx.x, 1};
   for (int d = 0; d < 4; d++)
@@ -305,7 +352,9 @@ k_rf_reverse(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
 // requested parameter pl.p[i] (i < npar <= NP); chiref and dchiref are
 // [column][depth] (as k_geometry writes chi_ref).  One pass of form_point on
 // NP-tangent dual numbers per depth gives d(point)/dp for every requested
-// parameter (the Humlicek functions by their complex derivative).
+// parameter (the Humlicek functions by their complex derivative).  The
+// depths are independent: workgroup (ray block, y) takes depths y * kd ..
+// + kd - 1.
 // The FP32 form's three-tangent chain is held to two waves per SIMD (it
 // needs 292 registers at one; two cost 36 spilled to scratch and run 1024
 // columns of 64-256 depths under 400 Zeeman lines 1.6x faster); the others
@@ -320,8 +369,10 @@ k_rf_chain(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
            const R *__restrict__ dcchi, const R *__restrict__ dceta,
            const int32_t *__restrict__ out_ls, const int32_t *__restrict__ io_list, int nlist,
            int nout, double mu_d, int atm_scale, RfParamList pl, const R *__restrict__ aP,
-           const R *__restrict__ aZ, const R *__restrict__ aB, R *__restrict__ rf, int64_t ldr) {
+           const R *__restrict__ aZ, const R *__restrict__ aB, R *__restrict__ rf, int64_t ldr,
+           int kd) {
   RF_SETUP();
+  const int moving = moving_arr[ic];
   using D = DualN<double, NP>;
   using DV = DualN<R, NP>;
   const int has_line = ldc(M.lam_line_ptr)[ls + 1] > ldc(M.lam_line_ptr)[ls];
@@ -332,7 +383,8 @@ k_rf_chain(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
 #pragma unroll
   for (int i = 0; i < NP; i++)
     if (i < pl.npar && pl.p[i] == RHG_RF_T) iT = i;
-  for (int k = 0; k < N; k++) {
+  const int k0 = (int) blockIdx.y * kd, k1 = N < k0 + kd ? N : k0 + kd;
+  for (int k = k0; k < k1; k++) {
     const double *stk = st0 + (int64_t) k * ncol;
     const int64_t ck = ((int64_t) io * Nmax + k) * ncol + ic;
     const double *dst[NP];
@@ -422,27 +474,28 @@ k_rf_chain(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
 #undef AB
 
 #define RHG_RF_INST(R)                                                                          \
-  template __global__ void k_rf_forward<R>(const DevModel *, const int32_t *, const int32_t *,  \
+  template __global__ void k_rf_points<R, false>(                                               \
+      const DevModel *, const int32_t *, const int32_t *, int, int, const double *,             \
+      const int32_t *, const int32_t *, int, const R *, const R *, double, int, double *, int, int); \
+  template __global__ void k_rf_points<R, true>(                                                \
+      const DevModel *, const int32_t *, const int32_t *, int, int, const double *,             \
+      const int32_t *, const int32_t *, int, const R *, const R *, double, int, double *, int, int); \
+  template __global__ void k_rf_forward<sizeof(R) == 4>(                                        \
+      const DevModel *, const int32_t *, int, int, const double *, const int32_t *,             \
+      const int32_t *, int, int, const double *, double, double *, double *);                   \
+  template __global__ void k_rf_reverse<R>(const DevModel *, const int32_t *,                  \
                                            int, int, const double *, const int32_t *,          \
-                                           const int32_t *, int, int, const R *, const R *,    \
-                                           double, double *, double *);                        \
-  template __global__ void k_rf_reverse<R>(const DevModel *, const int32_t *, const int32_t *,  \
-                                           int, int, const double *, const int32_t *,          \
-                                           const int32_t *, int, const R *, const R *, double, \
+                                           const int32_t *, int, const double *, double,       \
                                            const double *, R *, R *, R *);                     \
-  template __global__ void k_rf_chain<R, 3>(const DevModel *, const int32_t *, const int32_t *, \
-                                            int, int, const double *, const double *,          \
-                                            const double *, const double *, const R *,         \
-                                            const R *, const R *, const R *, const int32_t *,  \
-                                            const int32_t *, int, int, double, int,            \
-                                            RfParamList, const R *, const R *, const R *, R *, \
-                                            int64_t);                                          \
-  template __global__ void k_rf_chain<R, 6>(const DevModel *, const int32_t *, const int32_t *, \
-                                            int, int, const double *, const double *,          \
-                                            const double *, const double *, const R *,         \
-                                            const R *, const R *, const R *, const int32_t *,  \
-                                            const int32_t *, int, int, double, int,            \
-                                            RfParamList, const R *, const R *, const R *, R *, \
-                                            int64_t);
+  RHG_RF_CHAIN(R, 3)                                                                            \
+  RHG_RF_CHAIN(R, 6)
+#define RHG_RF_CHAIN(R, NP)                                                                     \
+  template __global__ void k_rf_chain<R, NP>(const DevModel *, const int32_t *, const int32_t *, \
+                                             int, int, const double *, const double *,          \
+                                             const double *, const double *, const R *,         \
+                                             const R *, const R *, const R *, const int32_t *,  \
+                                             const int32_t *, int, int, double, int,            \
+                                             RfParamList, const R *, const R *, const R *, R *, \
+                                             int64_t, int);
 
 }  // namespace rhg
