@@ -1407,8 +1407,8 @@ int rf_chunk(rhg_context_t *c, const double *d_atm, const int32_t *d_ndep, int n
   hipLaunchKernelGGL((rhg::k_rf_points<R, LT>), grdk, blk, LT ? (unsigned) c->tab_bytes : 0u,    \
                      c->stream, c->d_model, d_ndep, moving, ncol, Nmax, state, c->d_out_ls,      \
                      c->d_io_pol, npol, cchi, ceta, mu, kd, pts, c->tab_maxl, c->tab_maxc)
-    if (c->tab_bytes > 0 && c->tune_line_table) RHG_LAUNCH_PTS(true);
-    else RHG_LAUNCH_PTS(false);
+    const bool lt = c->tab_bytes > 0 && c->tune_line_table;
+    if (lt) RHG_LAUNCH_PTS(true); else RHG_LAUNCH_PTS(false);
 #undef RHG_LAUNCH_PTS
     HIPCHECK(hipGetLastError());
     hipLaunchKernelGGL((rhg::k_rf_forward<sizeof(R) == 4>), grd, blk, 0, c->stream, c->d_model, d_ndep,
@@ -1421,13 +1421,14 @@ int rf_chunk(rhg_context_t *c, const double *d_atm, const int32_t *d_ndep, int n
                        (const double *) car, aP, aZ, aB);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipEventRecord(c->ev[4], c->stream));
-#define RHG_LAUNCH_CHAIN(NP)                                                                     \
-  hipLaunchKernelGGL((rhg::k_rf_chain<R, NP>), grdk, blk, 0, c->stream, c->d_model, d_ndep, moving, \
-                     ncol, Nmax, state, dstate, chiref, (const double *) c->rf_dchiref.p, cchi,  \
-                     ceta, (const R *) c->rf_dcont[0].p, (const R *) c->rf_dcont[1].p,           \
-                     c->d_out_ls, c->d_io_pol, npol, nout, mu, scale, pl, aP, aZ, aB, d_rf, ldr, kd)
-    if (pl.npar <= 3) RHG_LAUNCH_CHAIN(3);
-    else RHG_LAUNCH_CHAIN(6);
+#define RHG_LAUNCH_CHAIN(LT)                                                                     \
+  hipLaunchKernelGGL((rhg::k_rf_chain<R, LT>), grdk, blk, LT ? (unsigned) c->tab_bytes : 0u,     \
+                     c->stream, c->d_model, d_ndep, moving, ncol, Nmax, state, dstate, chiref,   \
+                     (const double *) c->rf_dchiref.p, (const double *) pts,                     \
+                     (const R *) c->rf_dcont[0].p, (const R *) c->rf_dcont[1].p,                 \
+                     c->d_out_ls, c->d_io_pol, npol, nout, mu, scale, pl, aP, aZ, aB, d_rf, ldr, kd, \
+                     c->tab_maxl, c->tab_maxc)
+    if (lt) RHG_LAUNCH_CHAIN(true); else RHG_LAUNCH_CHAIN(false);
 #undef RHG_LAUNCH_CHAIN
     HIPCHECK(hipGetLastError());
   } else {

@@ -177,124 +177,7 @@ __device__ __forceinline__ void w3d(double dtau, double *w, double *dw) {
 }
 
 
-// ---------------------------------------------------------------------------
-// Multi-tangent dual numbers: a value and NP directional derivatives, for
-// the response functions' chain to the atmosphere parameters (one pass
-// carries every parameter's tangent; the value is computed once).
-template <typename R, int NP>
-struct DualN {
-  R v, d[NP];
-  DualN() = default;
-  template <typename S, typename = std::enable_if_t<std::is_arithmetic<S>::value>>
-  __device__ __forceinline__ DualN(S val) : v(R(val)) {
-#pragma unroll
-    for (int i = 0; i < NP; i++) d[i] = R(0);
-  }
-  template <typename S, typename = std::enable_if_t<!std::is_same<S, R>::value>>
-  __device__ __forceinline__ explicit DualN(const DualN<S, NP> &o) : v(R(o.v)) {
-#pragma unroll
-    for (int i = 0; i < NP; i++) d[i] = R(o.d[i]);
-  }
-  friend __device__ __forceinline__ DualN operator+(const DualN &a, const DualN &b) {
-    DualN r;
-    r.v = a.v + b.v;
-#pragma unroll
-    for (int i = 0; i < NP; i++) r.d[i] = a.d[i] + b.d[i];
-    return r;
-  }
-  friend __device__ __forceinline__ DualN operator-(const DualN &a, const DualN &b) {
-    DualN r;
-    r.v = a.v - b.v;
-#pragma unroll
-    for (int i = 0; i < NP; i++) r.d[i] = a.d[i] - b.d[i];
-    return r;
-  }
-  friend __device__ __forceinline__ DualN operator*(const DualN &a, const DualN &b) {
-    DualN r;
-    r.v = a.v * b.v;
-#pragma unroll
-    for (int i = 0; i < NP; i++) r.d[i] = a.d[i] * b.v + a.v * b.d[i];
-    return r;
-  }
-  friend __device__ __forceinline__ DualN operator/(const DualN &a, const DualN &b) {
-    DualN r;
-    const R ib = R(1) / b.v;
-    r.v = a.v * ib;
-#pragma unroll
-    for (int i = 0; i < NP; i++) r.d[i] = (a.d[i] - r.v * b.d[i]) * ib;
-    return r;
-  }
-  friend __device__ __forceinline__ DualN operator-(const DualN &a) {
-    DualN r;
-    r.v = -a.v;
-#pragma unroll
-    for (int i = 0; i < NP; i++) r.d[i] = -a.d[i];
-    return r;
-  }
-  __device__ __forceinline__ DualN &operator+=(const DualN &b) { *this = *this + b; return *this; }
-  __device__ __forceinline__ DualN &operator-=(const DualN &b) { *this = *this - b; return *this; }
-  __device__ __forceinline__ DualN &operator*=(const DualN &b) { *this = *this * b; return *this; }
-  friend __device__ __forceinline__ bool operator>(const DualN &a, const DualN &b) { return a.v > b.v; }
-  friend __device__ __forceinline__ bool operator<(const DualN &a, const DualN &b) { return a.v < b.v; }
-  friend __device__ __forceinline__ bool operator>=(const DualN &a, const DualN &b) { return a.v >= b.v; }
-  friend __device__ __forceinline__ bool operator<=(const DualN &a, const DualN &b) { return a.v <= b.v; }
-  friend __device__ __forceinline__ bool operator==(const DualN &a, const DualN &b) { return a.v == b.v; }
-  friend __device__ __forceinline__ bool operator!=(const DualN &a, const DualN &b) { return a.v != b.v; }
-};
-
-template <typename R, int NP>
-__device__ __forceinline__ R val(const DualN<R, NP> &x) { return x.v; }
-
-// f(x) with f(x.v) = fv and f'(x.v) = fd
-template <typename R, int NP>
-__device__ __forceinline__ DualN<R, NP> dn_apply(const DualN<R, NP> &x, R fv, R fd) {
-  DualN<R, NP> r;
-  r.v = fv;
-#pragma unroll
-  for (int i = 0; i < NP; i++) r.d[i] = fd * x.d[i];
-  return r;
-}
-template <typename R, int NP>
-__device__ __forceinline__ DualN<R, NP> fabs(const DualN<R, NP> &x) {
-  return dn_apply(x, x.v < R(0) ? -x.v : x.v, x.v < R(0) ? R(-1) : R(1));
-}
-template <typename R, int NP>
-__device__ __forceinline__ DualN<R, NP> rexp(const DualN<R, NP> &x) {
-  const R e = rexp(x.v);
-  return dn_apply(x, e, e);
-}
-template <typename R, int NP>
-__device__ __forceinline__ DualN<R, NP> rrcp(const DualN<R, NP> &x) {
-  const R r = rrcp(x.v);
-  return dn_apply(x, r, -r * r);
-}
-template <typename R, int NP>
-__device__ __forceinline__ DualN<R, NP> rdiv(const DualN<R, NP> &a, const DualN<R, NP> &b) {
-  return a * rrcp(b);
-}
-
-// Armstrong's function with its partials in a and v (as for Dual)
-template <typename R, int NP>
-__device__ __forceinline__ DualN<R, NP> voigt_armstrong_t(const DualN<R, NP> &a,
-                                                          const DualN<R, NP> &v) {
-  const double av = (double) a.v, vv = (double) v.v, h = 1.0e-6;
-  const double H = voigt_armstrong(av, vv);
-  const double da = (voigt_armstrong(av + h, vv) - voigt_armstrong(av > h ? av - h : av, vv)) /
-                    (av > h ? 2.0 * h : h);
-  const double dv = (voigt_armstrong(av, vv + h) - voigt_armstrong(av, vv - h)) / (2.0 * h);
-  DualN<R, NP> r;
-  r.v = (R) H;
-#pragma unroll
-  for (int i = 0; i < NP; i++) r.d[i] = (R) (da * (double) a.d[i] + dv * (double) v.d[i]);
-  return r;
-}
-
-// The Humlicek functions of the line profiles.  A plain or dual argument
-// evaluates voigt_humlicek() in that type.  For NP tangents: w = H + iF is
-// an analytic function of z = a - iv inside each region (rational, region
-// IV with exp(z^2)), so one evaluation on a dual number seeded in a gives
-// w' = dw/dz = (H_a, F_a), and dH = H_a da + F_a dv, dF = F_a da - H_a dv
-// (Cauchy-Riemann) for every tangent.
+// The Humlicek functions of the line profiles, in T.
 // `region` is Humlicek's region of the argument (humlicek_region).
 template <typename T>
 struct VoigtEval {
@@ -302,25 +185,84 @@ struct VoigtEval {
     return voigt_humlicek_r<T>(a, v, region, F);
   }
 };
-template <typename R, int NP>
-struct VoigtEval<DualN<R, NP>> {
-  static __device__ __forceinline__ DualN<R, NP> eval(const DualN<R, NP> &a,
-                                                      const DualN<R, NP> &v, int region,
-                                                      DualN<R, NP> *F) {
-    Dual<R> Fd;
-    const Dual<R> Hd =
-        voigt_humlicek_r<Dual<R>>(Dual<R>(a.v, R(1)), Dual<R>(v.v, R(0)), region, &Fd);
-    const R Ha = Hd.d, Fa = Fd.d;
-    DualN<R, NP> H;
-    H.v = Hd.v;
-    F->v = Fd.v;
+
+// H and its partial derivatives in a and v.  w = H + iF is an analytic
+// function of z = a - iv inside each region (a quotient N/D, region IV with
+// exp(z^2)), so w' = (N' - w D') / D in closed form gives H_a = Re w' and
+// H_v = Im w' (Cauchy-Riemann).  A dual-number evaluation of the same
+// quotients costs three times the plain function; this about twice.
+template <typename R>
+__device__ __forceinline__ R voigt_humlicek_d(R a, R v, int region, R *Ha, R *Hv) {
+  const cpx<R> z = {a, -v};
+  cpx<R> n, d, dn, dd, e = {R(0), R(0)};
+  if (region == 0) {
+    n = {R(0.5641896) * z.r, R(0.5641896) * z.i};
+    d = cmul(z, z);
+    d.r = d.r + R(0.5);
+    dn = {R(0.5641896), R(0)};
+    dd = {R(2) * z.r, R(2) * z.i};
+  } else if (region == 1) {
+    const cpx<R> u = cmul(z, z);
+    cpx<R> t = {R(0.5641896) * u.r + R(1.410474), R(0.5641896) * u.i};
+    n = cmul(z, t);
+    dn = {R(3.0 * 0.5641896) * u.r + R(1.410474), R(3.0 * 0.5641896) * u.i};
+    d = cmul(u, {u.r + R(3), u.i});
+    d.r = d.r + R(0.75);
+    dd = cmul(z, {R(4) * u.r + R(6), R(4) * u.i});
+  } else if (region == 2) {
+    const R a3[5] = {R(0.5642236), R(3.778987), R(11.96482), R(20.20933), R(16.4955)};
+    const R b3[5] = {R(6.699398), R(21.69274), R(39.27121), R(38.82363), R(16.4955)};
+    n = {a3[0], R(0)};
+    d = {z.r + b3[0], z.i};
+    dn = {R(0), R(0)};
+    dd = {R(1), R(0)};
 #pragma unroll
-    for (int i = 0; i < NP; i++) {
-      H.d[i] = Ha * a.d[i] + Fa * v.d[i];
-      F->d[i] = Fa * a.d[i] - Ha * v.d[i];
+    for (int k = 1; k < 5; k++) {
+      dn = cmul(dn, z); dn.r = dn.r + n.r; dn.i = dn.i + n.i;
+      dd = cmul(dd, z); dd.r = dd.r + d.r; dd.i = dd.i + d.i;
+      n = cmul(n, z); n.r = n.r + a3[k];
+      d = cmul(d, z); d.r = d.r + b3[k];
     }
-    return H;
+  } else {
+    const R a4[7] = {R(0.56419), R(1.320522), R(35.7668), R(219.031), R(1540.787), R(3321.99),
+                     R(36183.31)};
+    const R b4[7] = {R(1.841439), R(61.57037), R(364.2191), R(2186.181), R(9022.228), R(24322.84),
+                     R(32066.6)};
+    const cpx<R> zz = cmul(z, z), u = {-zz.r, -zz.i};
+    cpx<R> p = {a4[0], R(0)}, pu = {R(0), R(0)}, du = {R(1), R(0)};
+    d = {u.r + b4[0], u.i};
+#pragma unroll
+    for (int k = 1; k < 7; k++) {
+      pu = cmul(u, pu); pu.r = pu.r + p.r; pu.i = pu.i + p.i;
+      du = cmul(u, du); du.r = du.r + d.r; du.i = du.i + d.i;
+      p = cmul(u, p); p.r = p.r + a4[k];
+      d = cmul(u, d); d.r = d.r + b4[k];
+    }
+    const R ex = rexp(zz.r);
+    R sn, cs;
+    rsincos(zz.i, &sn, &cs);
+    e = {ex * cs, ex * sn};
+    n = cmul(z, p);
+    // d/dz = -2z d/du: n' = p - 2 z^2 p_u = p + 2 u p_u, d' = -2 z d_u
+    const cpx<R> upu = cmul(u, pu);
+    dn = {p.r + R(2) * upu.r, p.i + R(2) * upu.i};
+    dd = cmul({R(-2) * z.r, R(-2) * z.i}, du);
   }
-};
+  const R id = rrcp(d.r * d.r + d.i * d.i);
+  auto over_d = [&](cpx<R> x) {
+    return cpx<R>{(x.r * d.r + x.i * d.i) * id, (x.i * d.r - x.r * d.i) * id};
+  };
+  const cpx<R> w = over_d(n), wd = cmul(w, dd);
+  const cpx<R> dw = over_d({dn.r - wd.r, dn.i - wd.i});
+  if (region == 3) {
+    const cpx<R> ze = cmul(z, e);
+    *Ha = R(2) * ze.r - dw.r;
+    *Hv = R(2) * ze.i - dw.i;
+    return e.r - w.r;
+  }
+  *Ha = dw.r;
+  *Hv = dw.i;
+  return w.r;
+}
 
 }  // namespace rhg

@@ -305,7 +305,7 @@ __device__ __forceinline__ T line_profile_t(const Tab &tab, int i, int lb, const
       const T cosg = F(RHG_CF_COSG);
       const T sin2_gamma = T(1.0) - cosg * cosg;
       const T vB = T(tab.larmor(i)) * F(RHG_CF_B) * ivb;
-      T phi_sm = T(0), phi_pi = T(0), phi_sp = T(0), H, Fv;
+      T phi_sm = T(0), phi_pi = T(0), phi_sp = T(0);
       T psi_sm = T(0), psi_pi = T(0), psi_sp = T(0);
       const int c0 = tab.c0(i), c1 = tab.c1(i);
       if constexpr (Tab::grouped) {
@@ -335,8 +335,9 @@ __device__ __forceinline__ T line_profile_t(const Tab &tab, int i, int lb, const
           TV Fw;
           const T u = v - T(tab.shift(nz)) * vB;
           const int reg = humlicek_region(val(adamp), val(u));
-          H = (T) VoigtEval<TV>::eval((TV) adamp, (TV) u, reg, &Fw);
-          Fv = (T) Fw;
+          const T H = (T) VoigtEval<TV>::eval((TV) adamp, (TV) u, reg, &Fw);
+          const T Fv = (T) Fw;
+          (void) Fv;
           const int q = tab.q(nz);
           const T sg = T(tab.strength(nz));
           acc_prod(q == -1 ? phi_sm : (q == 0 ? phi_pi : phi_sp), sg, H);
@@ -530,13 +531,13 @@ struct RfParamList {
   int32_t npar;
   int32_t p[RHG_RF_NPARAM];
 };
-template <typename R, int NP>
+template <typename R, bool LT>
 __global__ void k_rf_chain(const DevModel *M, const int32_t *ndep, const int32_t *moving, int ncol,
                            int Nmax, const double *state, const double *dstate, const double *chiref,
-                           const double *dchiref, const R *cchi, const R *ceta, const R *dcchi,
-                           const R *dceta, const int32_t *out_ls, const int32_t *io_list, int nlist,
-                           int nout, double mu, int atm_scale, RfParamList pl, const R *aP,
-                           const R *aZ, const R *aB, R *rf, int64_t ldr, int kd);
+                           const double *dchiref, const double *pts, const R *dcchi, const R *dceta,
+                           const int32_t *out_ls, const int32_t *io_list, int nlist, int nout,
+                           double mu, int atm_scale, RfParamList pl, const R *aP, const R *aZ,
+                           const R *aB, R *rf, int64_t ldr, int kd, int tab_maxl, int tab_maxc);
 __global__ void k_census(const DevModel *M, const int32_t *ndep, const int32_t *moving, int ncol,
                          int Nmax, const double *state, int nfield, const int32_t *out_ls,
                          int nout, double mu, int32_t *census);

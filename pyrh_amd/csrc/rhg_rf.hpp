@@ -20,10 +20,10 @@
 //     Each point's adjoint is stored once, when the last step reading it is
 //     done, with those of the path lengths |dz| and of the lower boundary's
 //     Planck values.
-//  4. k_rf_chain: per (ray, depth), the point's derivative along each
-//     parameter's state tangent (form_point on dual numbers: line opacity,
-//     Zeeman-split Voigt/Faraday-Voigt profiles, continuum), contracted with
-//     the point adjoints, plus the path-length terms (tau500 scale: dz(j)
+//  4. k_rf_chain: per (ray, depth), the point adjoints pulled back through
+//     the point's formation (line opacity, Zeeman-split Voigt profiles,
+//     continuum) to the column state and contracted with each parameter's
+//     state tangent, plus the path-length terms (tau500 scale: dz(j)
 //     depends on chi_ref at j-1 and j) and the boundary terms.
 // The recursion, its adjoint and the points are FP64 in both forms; the FP32
 // form evaluates the Voigt functions (and their derivatives) in float.
@@ -83,6 +83,22 @@ __device__ __forceinline__ T point_get(const Point<T> &p, int m) {
   const double *Tc = st0 + (int64_t) RHG_CF_T * fs;                                      \
   const double *lc = M.lamconst + (int64_t) ls * RHG_LC_NCONST;                          \
   (void) lc; (void) Tc; (void) dzc;
+// the wavelength's line table (before RF_SETUP: every lane of the wavefront
+// takes part in staging it)
+#define RF_LINE_TABLE()                                                                  \
+  int cb0, t0;                                                                           \
+  xcd_tile(blockIdx.x, nlist, cb0, t0);                                                  \
+  if (cb0 * 64 >= ncol) return;                                                          \
+  auto tab = [&]() {                                                                     \
+    const int ls0 = out_ls[io_list[t0]];                                                 \
+    if constexpr (LT) {                                                                  \
+      extern __shared__ __align__(8) char lds_tab[];                                     \
+      return stage_lines(*Mp, ls0, lds_tab, tab_maxl, tab_maxc);                         \
+    } else {                                                                             \
+      const int p0 = ldc(Mp->lam_line_ptr)[ls0];                                         \
+      return LineTabG(*Mp, p0, ldc(Mp->lam_line_ptr)[ls0 + 1] - p0);                     \
+    }                                                                                    \
+  }()
 #define DZ(kk) dzc[(int64_t) (kk) * ncol]
 #define CAR(kk, c) car[((((int64_t) t * Nmax + (kk)) * NCARRY_STEP + (c)) * ncol) + ic]
 // the point at depth jj
@@ -112,19 +128,7 @@ k_rf_points(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
             const int32_t *__restrict__ io_list, int nlist, const R *__restrict__ cchi,
             const R *__restrict__ ceta, double mu_d, int kd, double *__restrict__ pts,
             int tab_maxl, int tab_maxc) {
-  int cb0, t0;
-  xcd_tile(blockIdx.x, nlist, cb0, t0);
-  if (cb0 * 64 >= ncol) return;
-  auto tab = [&]() {
-    const int ls0 = out_ls[io_list[t0]];
-    if constexpr (LT) {
-      extern __shared__ __align__(8) char lds_tab[];
-      return stage_lines(*Mp, ls0, lds_tab, tab_maxl, tab_maxc);
-    } else {
-      const int p0 = Mp->lam_line_ptr[ls0];
-      return LineTabG(*Mp, p0, Mp->lam_line_ptr[ls0 + 1] - p0);
-    }
-  }();
+  RF_LINE_TABLE();
   RF_SETUP();
   const int moving = moving_arr[ic];
   const R *cc = cchi + (int64_t) io * Nmax * ncol + ic;
@@ -349,80 +353,184 @@ k_rf_reverse(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
 // 4. chain to the atmosphere parameters
 
 // rf[((((i * Nmax + k) * 4 + o) * nout + io) * ldr + column] for the i-th
-// requested parameter pl.p[i] (i < npar <= NP); chiref and dchiref are
-// [column][depth] (as k_geometry writes chi_ref).  One pass of form_point on
-// NP-tangent dual numbers per depth gives d(point)/dp for every requested
-// parameter (the Humlicek functions by their complex derivative).  The
-// depths are independent: workgroup (ray block, y) takes depths y * kd ..
-// + kd - 1.
-// The FP32 form's three-tangent chain is held to two waves per SIMD (it
-// needs 292 registers at one; two cost 36 spilled to scratch and run 1024
-// columns of 64-256 depths under 400 Zeeman lines 1.6x faster); the others
-// keep one.
-template <typename R, int NP>
-__global__ void __launch_bounds__(64, (NP <= 3 && sizeof(R) == 4 ? 2 : 1))
+// requested parameter pl.p[i]; chiref and dchiref are [column][depth] (as
+// k_geometry writes chi_ref).  Per (ray, depth) the four outputs' point
+// adjoints are pulled back through the point's formation: to the opacities
+// and emissivities (reading the point itself from k_rf_points), per line to
+// chi_l, eta_l, the damping, the Doppler width, v_LOS, B and the angles, and
+// those are contracted with the parameters' state tangents.  What a parameter
+// moves is known: T the line constants, the continuum, the path lengths and
+// the boundary; v_mic the Doppler width and damping; v_LOS, B and the angles
+// their own fields (the tangents of all other fields are zero).
+//
+// The depths are independent: workgroup (ray block, y) takes depths y * kd ..
+// + kd - 1.  A Zeeman component costs one Voigt function with its derivative
+// and four sums whatever the number of parameters: u = v - shift vB, so a
+// Delta M group needs S(H), S(H_a), S(H_v), S(shift H_v) only.  (Evaluating
+// the point on dual numbers, one tangent per parameter, was bound by the
+// registers of those tangents: 1 wave per SIMD, 53.1 ms for 90 columns of
+// 64-256 depths x 350 wavelengths of the 400-line list, FP64, T, v_LOS and
+// B, and 2.49 ms for 512 columns x 112 wavelengths, FP32 form, all six.  This
+// form: 33.4 and 1.59 ms at two waves per SIMD.)
+template <typename R, bool LT>
+__global__ void __launch_bounds__(64, 2)
 k_rf_chain(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
            const int32_t *__restrict__ moving_arr, int ncol, int Nmax,
            const double *__restrict__ state, const double *__restrict__ dstate,
            const double *__restrict__ chiref, const double *__restrict__ dchiref,
-           const R *__restrict__ cchi, const R *__restrict__ ceta,
-           const R *__restrict__ dcchi, const R *__restrict__ dceta,
-           const int32_t *__restrict__ out_ls, const int32_t *__restrict__ io_list, int nlist,
-           int nout, double mu_d, int atm_scale, RfParamList pl, const R *__restrict__ aP,
-           const R *__restrict__ aZ, const R *__restrict__ aB, R *__restrict__ rf, int64_t ldr,
-           int kd) {
+           const double *__restrict__ pts, const R *__restrict__ dcchi,
+           const R *__restrict__ dceta, const int32_t *__restrict__ out_ls,
+           const int32_t *__restrict__ io_list, int nlist, int nout, double mu, int atm_scale,
+           RfParamList pl, const R *__restrict__ aP, const R *__restrict__ aZ,
+           const R *__restrict__ aB, R *__restrict__ rf, int64_t ldr, int kd, int tab_maxl,
+           int tab_maxc) {
+  RF_LINE_TABLE();
   RF_SETUP();
   const int moving = moving_arr[ic];
-  using D = DualN<double, NP>;
-  using DV = DualN<R, NP>;
-  const int has_line = ldc(M.lam_line_ptr)[ls + 1] > ldc(M.lam_line_ptr)[ls];
-  const D muD = D(mu_d);
-  const int64_t npts = (int64_t) Nmax * ncol;
-  const int64_t tan_stride = (int64_t) state_nfield(M.ncont, M.nline) * npts;
-  int iT = -1;
+  const int lb = line_field_base(M.ncont);
+  const int64_t tan_stride = (int64_t) state_nfield(M.ncont, M.nline) * fs;
+  bool wants[RHG_RF_NPARAM];
 #pragma unroll
-  for (int i = 0; i < NP; i++)
-    if (i < pl.npar && pl.p[i] == RHG_RF_T) iT = i;
+  for (int q = 0; q < RHG_RF_NPARAM; q++) {
+    wants[q] = false;
+#pragma unroll
+    for (int i = 0; i < RHG_RF_NPARAM; i++) wants[q] |= i < pl.npar && pl.p[i] == q;
+  }
+  const bool want_T = wants[RHG_RF_T], want_vm = wants[RHG_RF_VMIC];
   const int k0 = (int) blockIdx.y * kd, k1 = N < k0 + kd ? N : k0 + kd;
   for (int k = k0; k < k1; k++) {
     const double *stk = st0 + (int64_t) k * ncol;
-    const int64_t ck = ((int64_t) io * Nmax + k) * ncol + ic;
-    const double *dst[NP];
-#pragma unroll
-    for (int i = 0; i < NP; i++)
-      dst[i] = i < pl.npar ? dstate + pl.p[i] * tan_stride + (int64_t) k * ncol + ic : nullptr;
-    auto F = [stk, &dst, fs, &pl](int f) {
-      D x(stk[f * fs]);
-#pragma unroll
-      for (int i = 0; i < NP; i++) x.d[i] = i < pl.npar ? dst[i][f * fs] : 0.0;
-      return x;
-    };
-    D cch((double) cchi[ck]), cet((double) ceta[ck]);
-    if (iT >= 0) {
-#pragma unroll
-      for (int i = 0; i < NP; i++)
-        if (i == iT) { cch.d[i] = (double) dcchi[ck]; cet.d[i] = (double) dceta[ck]; }
-    }
-    Point<D> P;
-    form_point_f<D, DV>(M, ls, has_line, F, muD, moving, cch, cet, P);
-    double res[NP][4];
+    // tangent of field f along parameter q at this depth
+    auto tangent = [&](int q, int f) { return dstate[q * tan_stride + f * fs + (int64_t) k * ncol + ic]; };
+    Point<double> P;
+    RF_POINT(k, P);
+    // adjoints of chi_I,Q,U,V (ac) and eta_I,Q,U,V (ae): S_n = eta_n / chi_I,
+    // q_n = chi_n / chi_I
+    double ac[4][4], ae[4][4];
+    const double ichi = rrcp(P.chi);
 #pragma unroll
     for (int o = 0; o < 4; o++) {
-      double ap[8];
+      ac[o][0] = (double) AP(o, k, 0);
 #pragma unroll
-      for (int m = 0; m < 8; m++) ap[m] = (double) AP(o, k, m);
+      for (int n = 0; n < 4; n++) {
+        ae[o][n] = (double) AP(o, k, 1 + n) * ichi;
+        ac[o][0] -= ae[o][n] * P.S[n];
+      }
 #pragma unroll
-      for (int i = 0; i < NP; i++) {
-        double acc = ap[0] * P.chi.d[i];
-#pragma unroll
-        for (int n = 0; n < 4; n++) acc += ap[1 + n] * P.S[n].d[i];
-#pragma unroll
-        for (int n = 0; n < 3; n++) acc += ap[5 + n] * P.q[n].d[i];
-        res[i][o] = acc;
+      for (int n = 0; n < 3; n++) {
+        ac[o][1 + n] = (double) AP(o, k, 5 + n) * ichi;
+        ac[o][0] -= ac[o][1 + n] * P.q[n];
       }
     }
-    if (iT >= 0) {
-      double extra[4] = {0.0, 0.0, 0.0, 0.0};
+    const double vz = stk[RHG_CF_VLOS * fs], Bf = stk[RHG_CF_B * fs], cosg = stk[RHG_CF_COSG * fs],
+                 cos2x = stk[RHG_CF_COS2X * fs], sin2x = stk[RHG_CF_SIN2X * fs];
+    const double sin2 = 1.0 - cosg * cosg;
+    // adjoints of v_LOS, B, cos gamma, cos 2chi, sin 2chi; responses to T, v_mic
+    double a_vz[4], a_B[4], a_g[4], a_c[4], a_s[4], r_T[4], r_vm[4];
+#pragma unroll
+    for (int o = 0; o < 4; o++) a_vz[o] = a_B[o] = a_g[o] = a_c[o] = a_s[o] = r_T[o] = r_vm[o] = 0.0;
+    for (int i = 0; i < tab.n; i++) {
+      const int l = tab.line(i);
+      const double chi_l = stk[(lb + 4 * l) * fs], eta_l = stk[(lb + 4 * l + 1) * fs];
+      const double adamp = stk[(lb + 4 * l + 2) * fs], ivb = stk[(lb + 4 * l + 3) * fs];
+      double t_chi = 0.0, t_eta = 0.0, t_a = 0.0, t_ivb = 0.0, m_a = 0.0, m_ivb = 0.0;
+      if (want_T) {
+        t_chi = tangent(RHG_RF_T, lb + 4 * l);
+        t_eta = tangent(RHG_RF_T, lb + 4 * l + 1);
+        t_a = tangent(RHG_RF_T, lb + 4 * l + 2);
+        t_ivb = tangent(RHG_RF_T, lb + 4 * l + 3);
+      }
+      if (want_vm) {
+        m_a = tangent(RHG_RF_VMIC, lb + 4 * l + 2);
+        m_ivb = tangent(RHG_RF_VMIC, lb + 4 * l + 3);
+      }
+      double dv = tab.dv(i);
+      if (moving) dv += mu * vz;
+      const double v = dv * ivb, sv = ivb * INV_SQRTPI;
+      if (tab.damped(i) && tab.polar(i)) {
+        const double vB1 = tab.larmor(i) * ivb, vB = vB1 * Bf;
+        auto add = [&](int nz, double (&s)[4]) {
+          const double sh = tab.shift(nz), sg = tab.strength(nz), u = v - sh * vB;
+          R Ha, Hv;
+          const R H0 = voigt_humlicek_d<R>((R) adamp, (R) u, humlicek_region(adamp, u), &Ha, &Hv);
+          const double sHv = sg * (double) Hv;
+          s[0] += sg * (double) H0;
+          s[1] += sg * (double) Ha;
+          s[2] += sHv;
+          s[3] += sh * sHv;
+        };
+        double s[3][4] = {};
+        const int c0 = tab.c0(i), c1 = tab.c1(i);
+        if constexpr (LT) {
+          const int cpi = tab.cpi(i), csp = tab.csp(i);
+          for (int nz = c0; nz < cpi; nz++) add(nz, s[0]);
+          for (int nz = cpi; nz < csp; nz++) add(nz, s[1]);
+          for (int nz = csp; nz < c1; nz++) add(nz, s[2]);
+        } else {
+          for (int nz = c0; nz < c1; nz++) {
+            const int q = tab.q(nz);
+            if (q == -1) add(nz, s[0]);
+            else if (q == 0) add(nz, s[1]);
+            else add(nz, s[2]);
+          }
+        }
+        const double sigma = s[2][0] + s[0][0], diff = s[2][0] - s[0][0];
+        const double delta = 0.5 * s[1][0] - 0.25 * sigma;
+        const double f0 = (delta * sin2 + 0.5 * sigma) * sv, fq = delta * sin2 * sv,
+                     f3 = 0.5 * diff * cosg * sv;
+#pragma unroll
+        for (int o = 0; o < 4; o++) {
+          const double w_chi = ac[o][0] * f0 + (ac[o][1] * cos2x + ac[o][2] * sin2x) * fq + ac[o][3] * f3;
+          const double w_eta = ae[o][0] * f0 + (ae[o][1] * cos2x + ae[o][2] * sin2x) * fq + ae[o][3] * f3;
+          double w[4];
+#pragma unroll
+          for (int n = 0; n < 4; n++) w[n] = ac[o][n] * chi_l + ae[o][n] * eta_l;
+          // coefficients of delta sin^2 sv, sigma sv / 2 and diff cos g sv / 2
+          const double X = w[0] + w[1] * cos2x + w[2] * sin2x;
+          const double A_d = X * sin2 * sv, A_s = 0.5 * w[0] * sv, A_f = 0.5 * w[3] * cosg * sv;
+          const double W0 = A_s - A_f - 0.25 * A_d, W1 = 0.5 * A_d, W2 = A_s + A_f - 0.25 * A_d;
+          const double C_a = W0 * s[0][1] + W1 * s[1][1] + W2 * s[2][1];
+          const double C_v = W0 * s[0][2] + W1 * s[1][2] + W2 * s[2][2];
+          const double C_vB = -(W0 * s[0][3] + W1 * s[1][3] + W2 * s[2][3]);
+          const double C_sv = X * delta * sin2 + w[0] * 0.5 * sigma + w[3] * 0.5 * diff * cosg;
+          const double C_ivb = C_v * dv + C_vB * (tab.larmor(i) * Bf) + C_sv * INV_SQRTPI;
+          if (moving) a_vz[o] += C_v * mu * ivb;
+          a_B[o] += C_vB * vB1;
+          a_g[o] += (0.5 * w[3] * diff - 2.0 * cosg * X * delta) * sv;
+          a_c[o] += w[1] * fq;
+          a_s[o] += w[2] * fq;
+          r_T[o] += w_chi * t_chi + w_eta * t_eta + C_a * t_a + C_ivb * t_ivb;
+          r_vm[o] += C_a * m_a + C_ivb * m_ivb;
+        }
+      } else {
+        // an unpolarized profile: phi_I only
+        double H, Ha = 0.0, Hv;
+        if (tab.damped(i)) {
+          // Armstrong's function is analytic: central differences
+          const double h = 1.0e-6;
+          H = voigt_armstrong(adamp, v);
+          Ha = (voigt_armstrong(adamp + h, v) - voigt_armstrong(adamp > h ? adamp - h : adamp, v)) /
+               (adamp > h ? 2.0 * h : h);
+          Hv = (voigt_armstrong(adamp, v + h) - voigt_armstrong(adamp, v - h)) / (2.0 * h);
+        } else {
+          H = fabs(v) <= MAX_GAUSS_DOPPLER ? exp(-v * v) : 0.0;
+          Hv = -2.0 * v * H;
+        }
+#pragma unroll
+        for (int o = 0; o < 4; o++) {
+          const double w0 = (ac[o][0] * chi_l + ae[o][0] * eta_l) * sv, f0 = H * sv;
+          const double C_ivb = w0 * Hv * dv + w0 * H * rrcp(ivb);
+          if (moving) a_vz[o] += w0 * Hv * mu * ivb;
+          r_T[o] += (ac[o][0] * t_chi + ae[o][0] * t_eta) * f0 + w0 * Ha * t_a + C_ivb * t_ivb;
+          r_vm[o] += w0 * Ha * m_a + C_ivb * m_ivb;
+        }
+      }
+    }
+    if (want_T) {
+      const int64_t ck = ((int64_t) io * Nmax + k) * ncol + ic;
+      const double dcc = (double) dcchi[ck], dce = (double) dceta[ck];
+#pragma unroll
+      for (int o = 0; o < 4; o++) r_T[o] += ac[o][0] * dcc + ae[o][0] * dce;
       // path lengths on the tau500 scale: |dz(j)| = 2 (tau_j - tau_{j-1}) /
       // (chi_ref(j-1) + chi_ref(j)), j = k and k + 1
       if (atm_scale == 0) {
@@ -434,7 +542,7 @@ k_rf_chain(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
             const double den = chiref[(int64_t) ic * Nmax + j - 1] + chiref[(int64_t) ic * Nmax + j];
             const double dzdT = -DZ(j) / den * dchi;
 #pragma unroll
-            for (int o = 0; o < 4; o++) extra[o] += (double) AZ(o, j) * dzdT;
+            for (int o = 0; o < 4; o++) r_T[o] += (double) AZ(o, j) * dzdT;
           }
         }
       }
@@ -446,26 +554,46 @@ k_rf_chain(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
           const double e = exp(x), B = lc[RHG_LC_TWOHNU3_C2] / (e - 1.0);
           dB = B * x * e / (e - 1.0) / T;
         }
-        const double dTdp = dstate[RHG_RF_T * tan_stride + (int64_t) RHG_CF_T * fs + (int64_t) k * ncol + ic];
+        const double dTdp = tangent(RHG_RF_T, RHG_CF_T);
 #pragma unroll
-        for (int o = 0; o < 4; o++) extra[o] += (double) AB(o, k - (N - 2)) * (dB * dTdp);
+        for (int o = 0; o < 4; o++) r_T[o] += (double) AB(o, k - (N - 2)) * (dB * dTdp);
       }
-#pragma unroll
-      for (int i = 0; i < NP; i++)
-        if (i == iT)
-#pragma unroll
-          for (int o = 0; o < 4; o++) res[i][o] += extra[o];
     }
+    auto store = [&](int i, const double (&r)[4]) {
 #pragma unroll
-    for (int i = 0; i < NP; i++)
-      if (i < pl.npar)
+      for (int o = 0; o < 4; o++)
+        rf[((((int64_t) i * Nmax + k) * 4 + o) * nout + io) * ldr + ic] = (R) r[o];
+    };
+    for (int i = 0; i < pl.npar; i++) {
+      const int q = pl.p[i];
+      double r[4];
+      if (q == RHG_RF_T) {
+        store(i, r_T);
+      } else if (q == RHG_RF_VMIC) {
+        store(i, r_vm);
+      } else if (q == RHG_RF_VLOS) {
+        const double t = tangent(q, RHG_CF_VLOS);
 #pragma unroll
-        for (int o = 0; o < 4; o++)
-          rf[((((int64_t) i * Nmax + k) * 4 + o) * nout + io) * ldr + ic] = (R) res[i][o];
+        for (int o = 0; o < 4; o++) r[o] = a_vz[o] * t;
+        store(i, r);
+      } else if (q == RHG_RF_B) {
+        const double t = tangent(q, RHG_CF_B);
+#pragma unroll
+        for (int o = 0; o < 4; o++) r[o] = a_B[o] * t;
+        store(i, r);
+      } else {
+        const double tg = tangent(q, RHG_CF_COSG), tc = tangent(q, RHG_CF_COS2X),
+                     ts = tangent(q, RHG_CF_SIN2X);
+#pragma unroll
+        for (int o = 0; o < 4; o++) r[o] = a_g[o] * tg + a_c[o] * tc + a_s[o] * ts;
+        store(i, r);
+      }
+    }
   }
 }
 
 #undef RF_SETUP
+#undef RF_LINE_TABLE
 #undef RF_POINT
 #undef DZ
 #undef CAR
@@ -487,15 +615,15 @@ k_rf_chain(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
                                            int, int, const double *, const int32_t *,          \
                                            const int32_t *, int, const double *, double,       \
                                            const double *, R *, R *, R *);                     \
-  RHG_RF_CHAIN(R, 3)                                                                            \
-  RHG_RF_CHAIN(R, 6)
-#define RHG_RF_CHAIN(R, NP)                                                                     \
-  template __global__ void k_rf_chain<R, NP>(const DevModel *, const int32_t *, const int32_t *, \
+  RHG_RF_CHAIN(R, false)                                                                        \
+  RHG_RF_CHAIN(R, true)
+#define RHG_RF_CHAIN(R, LT)                                                                     \
+  template __global__ void k_rf_chain<R, LT>(const DevModel *, const int32_t *, const int32_t *, \
                                              int, int, const double *, const double *,          \
-                                             const double *, const double *, const R *,         \
-                                             const R *, const R *, const R *, const int32_t *,  \
+                                             const double *, const double *, const double *,    \
+                                             const R *, const R *, const int32_t *,             \
                                              const int32_t *, int, int, double, int,            \
                                              RfParamList, const R *, const R *, const R *, R *, \
-                                             int64_t, int);
+                                             int64_t, int, int, int);
 
 }  // namespace rhg
