@@ -63,6 +63,9 @@ static __device__ __align__(256) unsigned char scratch[RHG_NOALLOC_SCRATCH_BYTES
 namespace {
 
 constexpr int kMaxDevices = 64;
+// the hydrostatic builder's records held at a time: 16384 columns of 82
+// depths and 99 elements
+constexpr size_t kHseRecBytes = (size_t) 4 << 30;
 // LDS for a staged line list, at most: 16 KB keeps 8 one-wavefront
 // workgroups per CU (the register limit of the polarized kernels)
 constexpr size_t kLineTabMaxBytes = 16384;
@@ -82,6 +85,16 @@ int noalloc_scratch_init(int device) {
 }
 
 }  // namespace
+
+// The element tables of the last rhg_hse_t, and what hse_tables derives from
+// them: the record's slots and the segments of k_hse_tables (rhg_hse.hpp).
+struct HseHost {
+  std::vector<int32_t> nstage, ptr;
+  std::vector<double> logpf, ionpot, abund;
+  int he_group = -1, nrec = 0, nseg = 0, nseg_height = 0;
+  size_t off[10]{};   // byte offsets of the device arrays in hs_el
+  bool uploaded = false;
+};
 
 struct rhg_context {
   int device = 0;
@@ -132,8 +145,10 @@ struct rhg_context {
   DevBuf gr_pol, gr_pol_ptr, gr_scal, gr_scal_ptr, gr_tile, gr_mask, gr_blk, gr_col;
   double nlte_ms[RHG_NLTE_NTIMING]{};
   // hydrostatic equilibrium: element tables, inputs, outputs, timing
-  DevBuf hs_nstage, hs_ptr, hs_logpf, hs_ionpot, hs_abund, hs_in, hs_ndep, hs_out, hs_niter,
-      hs_scr;
+  // (hs_el holds HseHost's tables on the device, uploaded when they differ
+  // from the last call's), per-depth records of the batch
+  DevBuf hs_el, hs_in, hs_ndep, hs_out, hs_niter, hs_rec;
+  HseHost hs;
   float hse_ms = 0.0f;
   bool ref_has_line = false;   // a Kurucz line covers the reference wavelength
   int hse_lpc = 0;
@@ -2213,22 +2228,104 @@ static int hse_tables(rhg_context_t *c, const rhg_hse_t *h, rhg::DevHse &H) {
     if (h->el_pf_ptr[e] != npfel) return fail(RHG_EINVAL, "element tables are not packed");
     npfel += (int64_t) h->el_nstage[e] * dm.npf;
   }
-  if (c->hs_nstage.ensure(h->nel * sizeof(int32_t)) || c->hs_ptr.ensure(h->nel * sizeof(int32_t)) ||
-      c->hs_logpf.ensure(npfel * sizeof(double)) || c->hs_ionpot.ensure(npfel * sizeof(double)) ||
-      c->hs_abund.ensure(h->nel * sizeof(double)))
-    return fail(RHG_ENOMEM, "device allocation for the element tables failed");
-  HIPCHECK(hipSetDevice(c->device));
-  HIPCHECK(hipMemcpyAsync(c->hs_nstage.p, h->el_nstage, h->nel * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
-  HIPCHECK(hipMemcpyAsync(c->hs_ptr.p, h->el_pf_ptr, h->nel * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
-  HIPCHECK(hipMemcpyAsync(c->hs_logpf.p, h->el_logpf, npfel * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  HIPCHECK(hipMemcpyAsync(c->hs_ionpot.p, h->el_ionpot, npfel * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  HIPCHECK(hipMemcpyAsync(c->hs_abund.p, h->el_abund, h->nel * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  // the tables are uploaded when their content differs from the last call's
+  // (a potential is kept per stage: entry el_pf_ptr / npf + stage)
+  rhg::DevHse D{};
+  HseHost &k = c->hs;
+  const int he_group = (h->he_atom >= 0 && h->ray_He > 0.0) ? h->he_atom : -1;
+  const size_t nst = (size_t) (npfel / dm.npf);
+  std::vector<double> ionpot(nst);
+  for (int e = 0; e < h->nel; e++)
+    for (int j = 0; j < h->el_nstage[e]; j++)
+      ionpot[h->el_pf_ptr[e] / dm.npf + j] = h->el_ionpot[h->el_pf_ptr[e] + j];
+  auto same = [](const auto &v, const auto *p, size_t n) {
+    return v.size() == n && memcmp(v.data(), p, n * sizeof(*p)) == 0;
+  };
+  if (!k.uploaded || k.he_group != he_group || !same(k.nstage, h->el_nstage, h->nel) ||
+      !same(k.logpf, h->el_logpf, (size_t) npfel) || !same(k.ionpot, ionpot.data(), nst) ||
+      !same(k.abund, h->el_abund, h->nel)) {
+    k.uploaded = false;
+    k.he_group = he_group;
+    k.nstage.assign(h->el_nstage, h->el_nstage + h->nel);
+    k.ptr.assign(h->el_pf_ptr, h->el_pf_ptr + h->nel);
+    k.logpf.assign(h->el_logpf, h->el_logpf + npfel);
+    k.abund.assign(h->el_abund, h->el_abund + h->nel);
+    k.ionpot = ionpot;
+    // slots of the record: HSE_NMISC numbers, the level groups of every
+    // molecule nucleus and He, the molecules, the stage factors
+    const int ngrp = dm.nnuclei + 1, g0 = rhg::HSE_NMISC, m0 = g0 + ngrp * (rhg::HSE_NDZ + 1),
+              s0 = m0 + dm.nmol;
+    std::vector<int32_t> code, pf, seg;
+    std::vector<double> ip, ab;
+    std::vector<int> order(h->nel);
+    for (int e = 0; e < h->nel; e++) order[e] = e;
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int a, int b) { return h->el_nstage[a] > h->el_nstage[b]; });
+    for (int e : order) {
+      const int ns = h->el_nstage[e];
+      if (s0 + pf.size() > 0xffff) return fail(RHG_EUNSUPPORTED, "too many ionisation stages");
+      code.push_back((int32_t) ((s0 + pf.size()) << 4 | ns) | (e == 0 ? rhg::HSE_CODE_H : 0));
+      ab.push_back(h->el_abund[e]);
+      for (int j = 1; j < ns; j++) {
+        pf.push_back(h->el_pf_ptr[e] + (j - 1) * dm.npf);
+        ip.push_back(h->el_ionpot[h->el_pf_ptr[e] + j - 1]);
+      }
+    }
+    k.nrec = s0 + (int) pf.size();
+    auto add = [&](int kind, int first, int n, int slot) {
+      for (int v : {kind, first, n, slot}) seg.push_back(v);
+    };
+    add(rhg::HSE_SEG_MISC, 0, rhg::HSE_NMISC, 0);
+    for (int i = 0; i < (int) pf.size(); i += rhg::HSE_SEG)
+      add(rhg::HSE_SEG_STAGES, i, std::min(rhg::HSE_SEG, (int) pf.size() - i), s0 + i);
+    k.nseg_height = (int) seg.size() / 4;   // the height scale needs no opacity
+    for (int i = 0; i < ngrp; i++) {
+      const int ia = i < dm.nnuclei ? c->h_nucl_atom[i] : he_group;
+      if (ia >= 0) add(rhg::HSE_SEG_GROUPS, ia, rhg::HSE_NDZ + 1, g0 + i * (rhg::HSE_NDZ + 1));
+    }
+    for (int m = 0; m < dm.nmol; m += 2)
+      add(rhg::HSE_SEG_MOLECULES, m, std::min(2, dm.nmol - m), m0 + m);
+    k.nseg = (int) seg.size() / 4;
+    std::vector<char> buf;
+    int na = 0;
+    auto put = [&](const void *p, size_t bytes) {
+      k.off[na++] = buf.size();
+      buf.insert(buf.end(), (const char *) p, (const char *) p + bytes);
+      buf.resize((buf.size() + 15) & ~(size_t) 15);
+    };
+    put(k.nstage.data(), k.nstage.size() * sizeof(int32_t));
+    put(k.ptr.data(), k.ptr.size() * sizeof(int32_t));
+    put(k.logpf.data(), k.logpf.size() * sizeof(double));
+    put(k.ionpot.data(), k.ionpot.size() * sizeof(double));
+    put(k.abund.data(), k.abund.size() * sizeof(double));
+    put(seg.data(), seg.size() * sizeof(int32_t));
+    put(code.data(), code.size() * sizeof(int32_t));
+    put(pf.data(), pf.size() * sizeof(int32_t));
+    put(ip.data(), ip.size() * sizeof(double));
+    put(ab.data(), ab.size() * sizeof(double));
+    if (c->hs_el.ensure(buf.size() + 16))
+      return fail(RHG_ENOMEM, "device allocation for the element tables failed");
+    HIPCHECK(hipSetDevice(c->device));
+    // a synchronous copy on the stream's idle end: buf is on this call's stack
+    HIPCHECK(hipMemcpyAsync(c->hs_el.p, buf.data(), buf.size(), hipMemcpyHostToDevice, c->stream));
+    HIPCHECK(hipStreamSynchronize(c->stream));
+    k.uploaded = true;
+  }
+  const char *base = (const char *) c->hs_el.p;
+  H = D;
   H.nel = h->nel;
-  H.el_nstage = (const int32_t *) c->hs_nstage.p;
-  H.el_pf_ptr = (const int32_t *) c->hs_ptr.p;
-  H.el_logpf = (const double *) c->hs_logpf.p;
-  H.el_ionpot = (const double *) c->hs_ionpot.p;
-  H.el_abund = (const double *) c->hs_abund.p;
+  H.el_nstage = (const int32_t *) (base + k.off[0]);
+  H.el_pf_ptr = (const int32_t *) (base + k.off[1]);
+  H.el_logpf = (const double *) (base + k.off[2]);
+  H.el_ionpot = (const double *) (base + k.off[3]);
+  H.el_abund = (const double *) (base + k.off[4]);
+  H.seg = (const int32_t *) (base + k.off[5]);
+  H.el_code = (const int32_t *) (base + k.off[6]);
+  H.sl_pf = (const int32_t *) (base + k.off[7]);
+  H.sl_ip = (const double *) (base + k.off[8]);
+  H.el_ab = (const double *) (base + k.off[9]);
+  H.nrec = k.nrec;
+  H.np_dz = c->h_level_stage[c->h_atom_level_ptr[1] - 1] - c->h_level_stage[0];
   H.lam_index = h->lam_index;
   H.he_atom = h->he_atom;
   H.ray_H = h->ray_H;
@@ -2239,8 +2336,6 @@ static int hse_tables(rhg_context_t *c, const rhg_hse_t *h, rhg::DevHse &H) {
   H.scatt_fudge = h->scatt_fudge;
   H.nmax_iter = h->nmax_iter;
   H.iter_limit = h->iter_limit;
-  H.scr = nullptr;
-  H.nslot_stage = 0;
   return 0;
 }
 
@@ -2300,26 +2395,6 @@ int rhg_hse(rhg_context_t *c, const rhg_hse_t *h, int32_t ncol, int32_t Nmax, co
     d_pg = out + (size_t) 3 * ncol * Nmax;
     d_niter = niter_out ? (int32_t *) c->hs_niter.p : nullptr;
   }
-  // lanes per column: enough lane groups to give every SIMD of the chip two
-  // waves (256 CUs x 4 SIMDs x 64 lanes x 2, the occupancy k_hse is built
-  // for), at most 16
-  int lpc = 1;
-  while (lpc < 16 && (int64_t) ncol * lpc < 131072) lpc <<= 1;
-  if (const char *lanes_env = getenv("RHG_HSE_LANES")) {
-    const int v = atoi(lanes_env);
-    if (v == 1 || v == 2 || v == 4 || v == 8 || v == 16) lpc = v;
-  }
-  c->hse_lpc = lpc;
-  const int64_t nthr = (int64_t) ncol * lpc;
-  dim3 blk(rhg::HSE_BLOCK), grd((unsigned) ((nthr + rhg::HSE_BLOCK - 1) / rhg::HSE_BLOCK));
-  // stage-factor slots: the most stages (beyond the first) any group lane
-  // handles, its elements being sub, sub + lpc, ...
-  int nslot = 1;
-  for (int sub = 0; sub < lpc; sub++) {
-    int n = 0;
-    for (int e = sub; e < h->nel; e += lpc) n += h->el_nstage[e] - 1;
-    nslot = std::max(nslot, n);
-  }
   // the level groups: every molecule nucleus and He, ionisation differences
   // below HSE_NDZ
   for (int i = 0; i <= dm.nnuclei; i++) {
@@ -2331,25 +2406,57 @@ int rhg_hse(rhg_context_t *c, const rhg_hse_t *h, int32_t ncol, int32_t Nmax, co
         return fail(RHG_EUNSUPPORTED, "model atom with levels four or more ionisation stages "
                                       "above its ground level");
   }
-  const int64_t nlaunch = (int64_t) grd.x * rhg::HSE_BLOCK;
-  const int64_t nslot_all = nslot + (int64_t) (dm.nnuclei + 1) * (rhg::HSE_NDZ + 1);
-  if (c->hs_scr.ensure((size_t) nslot_all * nlaunch * sizeof(double)))
-    return fail(RHG_ENOMEM, "device allocation for the layer tables failed");
-  H.scr = (double *) c->hs_scr.p;
-  H.nslot_stage = nslot;
-  const size_t lds = (size_t) 3 * dm.nmol * rhg::HSE_BLOCK * sizeof(double);
+  // The records of all depths are formed before the chain runs, for as many
+  // columns at a time as HSE_REC_BYTES hold (or as can be allocated).
+  const size_t rec_col = (size_t) Nmax * H.nrec * sizeof(double);
+  int chunk = (int) std::min<size_t>(ncol, std::max<size_t>(kHseRecBytes / rec_col, 1));
+  while (c->hs_rec.ensure((size_t) chunk * rec_col)) {
+    if (chunk <= 64) return fail(RHG_ENOMEM, "device allocation for the layer tables failed");
+    chunk = (chunk + 1) / 2;
+  }
+  // Lanes per column.  More lanes shorten a column's chain (one column: 4.2
+  // ms with 8 lanes, 2.7 with 16, 2.5 with 32, 2.2 with 64) but repeat what
+  // the lanes compute alike, so they pay while the chip has a free SIMD for
+  // every wave (1024); 16384 columns take 12.4 ms with 8 lanes, whose eight
+  // records limit the workgroups per CU, 9.7 with 16, 13.4 with 32.
+  int lpc = 16;
+  while (lpc < 64 && (int64_t) chunk * lpc * 2 <= 65536) lpc <<= 1;
+  if (const char *lanes_env = getenv("RHG_HSE_LANES")) {
+    const int v = atoi(lanes_env);
+    if (v >= 1 && v <= 64 && !(v & (v - 1))) lpc = v;
+  }
+  c->hse_lpc = lpc;
+  H.lds_col = (H.nrec + dm.nmol) | 1;   // odd: the columns of a workgroup on different banks
+  H.lds_col0 = H.nel + (H.nel + 2 * dm.nmol + 1) / 2;
+  int cpb = std::min(8, rhg::HSE_BLOCK / lpc);
+  auto lds_bytes = [&](int n) { return ((size_t) H.lds_col0 + (size_t) n * H.lds_col) * sizeof(double); };
+  while (cpb > 1 && lds_bytes(cpb) > 65536) cpb--;
+  if (lds_bytes(cpb) > 65536) return fail(RHG_EUNSUPPORTED, "element tables too large for a workgroup");
+  const dim3 blk(rhg::HSE_BLOCK);
   HIPCHECK(hipEventRecord(c->ev[0], c->stream));
-  switch (dm.nnuclei) {
+  for (int c0 = 0; c0 < ncol; c0 += chunk) {
+    const int n = std::min(chunk, ncol - c0);
+    const int64_t o = (int64_t) c0 * Nmax, npts = (int64_t) n * Nmax;
+    double *rec = (double *) c->hs_rec.p;
+    hipLaunchKernelGGL(rhg::k_hse_tables,
+                       dim3((unsigned) ((npts + rhg::HSE_BLOCK - 1) / rhg::HSE_BLOCK),
+                            (unsigned) (atm_scale == 0 ? c->hs.nseg : c->hs.nseg_height)),
+                       blk, 0, c->stream, c->d_model, H, (int) npts, Nmax, d_ndep + c0, d_temp + o, rec);
+    HIPCHECK(hipGetLastError());
+    const dim3 grd((unsigned) ((n + cpb - 1) / cpb));
+    switch (dm.nnuclei) {
 #define RHG_LAUNCH_HSE(NN)                                                                          \
   case NN:                                                                                          \
-    hipLaunchKernelGGL(rhg::k_hse<NN>, grd, blk, lds, c->stream, c->d_model, H, lpc, ncol, Nmax,    \
-                       d_ndep, atm_scale, d_scale, d_temp, d_pgt, d_ne, d_nH, d_rho, d_pg, d_niter); \
+    hipLaunchKernelGGL(rhg::k_hse<NN>, grd, blk, lds_bytes(cpb), c->stream, c->d_model, H, lpc, cpb, n, \
+                       Nmax, d_ndep + c0, atm_scale, d_scale + o, d_temp + o, d_pgt + c0, rec,      \
+                       d_ne + o, d_nH + o, d_rho + o, d_pg + o, d_niter ? d_niter + o : nullptr);   \
     break;
-    RHG_LAUNCH_HSE(1) RHG_LAUNCH_HSE(2) RHG_LAUNCH_HSE(3) RHG_LAUNCH_HSE(4)
-    RHG_LAUNCH_HSE(5) RHG_LAUNCH_HSE(6) RHG_LAUNCH_HSE(7) RHG_LAUNCH_HSE(8)
+      RHG_LAUNCH_HSE(1) RHG_LAUNCH_HSE(2) RHG_LAUNCH_HSE(3) RHG_LAUNCH_HSE(4)
+      RHG_LAUNCH_HSE(5) RHG_LAUNCH_HSE(6) RHG_LAUNCH_HSE(7) RHG_LAUNCH_HSE(8)
 #undef RHG_LAUNCH_HSE
+    }
+    HIPCHECK(hipGetLastError());
   }
-  HIPCHECK(hipGetLastError());
   HIPCHECK(hipEventRecord(c->ev[1], c->stream));
   if (!device_ptrs) {
     HIPCHECK(hipMemcpyAsync(ne_out, d_ne, col_b, hipMemcpyDeviceToHost, c->stream));

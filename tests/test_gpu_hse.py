@@ -94,6 +94,28 @@ def test_hse_batch_matches_oracle(fix):
     np.testing.assert_array_equal(p2[0], ne[perm])
 
 
+@pytest.mark.parametrize("lanes", [2, 4, 8, 16, 32, 64])
+@pytest.mark.parametrize("scale", [0, 2])
+def test_hse_lane_groups(fix, lanes, scale, monkeypatch):
+    """Every lane-group width, on a column count that leaves the last
+    workgroup part empty, on both scales: the sums over elements and
+    molecules change order only (a few roundings, far below TOL)."""
+    import pyoracle
+    from pyrh_amd import workloads as W
+    e, hm = engine(fix, "single")
+    T = W.stokes_map(19, seed=W.SEED_BASE + 44)[:, 1]
+    nd = np.full(19, W.NDEP, np.int32)
+    nd[0], nd[9], nd[18] = 1, 2, 65
+    sc = np.broadcast_to(W.LOGTAU if scale == 0 else np.linspace(2000.0, -100.0, W.NDEP), T.shape)
+    monkeypatch.setenv("RHG_HSE_LANES", str(lanes))
+    out = e.hse(hm, sc, T, 0.1, scale, nd)
+    assert e.hse_timing()[1] == lanes
+    ref = pyoracle.hse(hm, sc, T, 0.1, scale, ndep=nd)
+    for a, b in zip(out[:4], (ref[0], ref[1], ref[2], ref[3])):
+        assert max(relerr(a[c, :nd[c]], b[c, :nd[c]]) for c in range(19)) < TOL
+    np.testing.assert_array_equal(out[4], ref[4])
+
+
 def test_hse_device_pointers(fix):
     import torch
     from pyrh_amd import workloads as W
