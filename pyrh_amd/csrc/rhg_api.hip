@@ -125,8 +125,8 @@ struct rhg_context {
   DevBuf at_iin, at_out, at_par;
   // NLTE: the active atom (packed arrays and its DevNlte), the batch arrays
   // of rhg::NlteBufs, active-column list, per-column reductions, output
-  DevBuf nl_atom, nl_dev, nl_nstar, nl_pops, nl_ntot, nl_vbroad, nl_nHe, nl_adamp, nl_wphi,
-      nl_Cmat, nl_Gam, nl_phi, nl_csca, nl_J, nl_jpar, nl_acc, nl_scr, nl_dJ, nl_hist, nl_act, nl_red,
+  DevBuf nl_atom, nl_dev, nl_geo, nl_nstar, nl_pops, nl_ntot, nl_vbroad, nl_nHe, nl_adamp, nl_wphi,
+      nl_Cmat, nl_phi, nl_bg, nl_J, nl_jpar, nl_acc, nl_dJ, nl_hist, nl_act, nl_red,
       nl_out, nl_iolist, nl_atm, nl_ndep, nl_st;
   // batches of uneven depth counts run sorted by depth count: the caller's
   // columns gathered into these, the outputs scattered back
@@ -1843,7 +1843,16 @@ int nlte_upload(rhg_context_t *c, const rhg_nlte_t *a, const NlteHost &h) {
 }
 
 struct NlteTimer {
-  hipEvent_t e[2]{};
+  std::vector<hipEvent_t> e;
+  // at least n events
+  int make(size_t n) {
+    while (e.size() < n) {
+      hipEvent_t x{};
+      if (hipEventCreate(&x) != hipSuccess) return -1;
+      e.push_back(x);
+    }
+    return 0;
+  }
   ~NlteTimer() {
     for (auto &x : e)
       if (x) (void) hipEventDestroy(x);
@@ -1851,6 +1860,20 @@ struct NlteTimer {
 };
 
 }  // namespace
+
+// run LAUNCH(L, P) with the lanes per ray direction L and the points per lane
+// P for Nmax depths (L P >= Nmax): two or three points per lane hide the
+// latency of a point's arithmetic, more spill
+#define RHG_RAY_POINTS(Nmax, LAUNCH)        \
+  do {                                      \
+    if ((Nmax) <= 64) LAUNCH(32, 2);        \
+    else if ((Nmax) <= 96) LAUNCH(32, 3);   \
+    else if ((Nmax) <= 128) LAUNCH(64, 2);  \
+    else if ((Nmax) <= 192) LAUNCH(64, 3);  \
+    else if ((Nmax) <= 256) LAUNCH(64, 4);  \
+    else LAUNCH(64, 8);                     \
+  } while (0)
+static_assert(64 * 8 >= RHG_MAX_DEPTH, "RHG_RAY_POINTS covers every depth count");
 
 extern "C" {
 
@@ -1882,15 +1905,14 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
 
   // device bytes per column; columns are solved in chunks that fit in 3/4
   // of the free device memory
+  const int Kp = rhg::nlte_pitch(Nmax);
   const size_t per_col =
-      (size_t) Nmax * sizeof(double) *
-          ((size_t) nfield + 5 * (size_t) nout + 2 * (size_t) nl + 3 + 2 * (size_t) a->nline +
-           2 * (size_t) nl * nl + (size_t) h.nphi * nrays * 2 + 2 * (size_t) h.nentry +
-           std::max((size_t) rhg::NLTE_NSLOT * (nlist - h.nbez),
-                    stokes_out ? (size_t) rhg::NLTE_NSLOT_EM * nlist : (size_t) 0) +
-           (size_t) NS * nl +
-           (size_t) nout) +
-      (size_t) nlist * sizeof(double) + 9 * (size_t) Nmax * sizeof(double) + 64;
+      (size_t) Nmax * sizeof(double) * ((size_t) nfield + 2 * (size_t) nout + 9) +
+      (size_t) Kp * sizeof(double) *
+          (5 * (size_t) nout + rhg::NG_N + 4 * (size_t) nl + 3 + 2 * (size_t) a->nline +
+           (size_t) nl * nl + (size_t) h.nphi * nrays * 2 + 2 * (size_t) h.nentry +
+           (size_t) NS * nl) +
+      ((size_t) nlist + 4 * (size_t) nout) * sizeof(double) + 64;
   size_t freeb = 0, totb = 0;
   HIPCHECK(hipMemGetInfo(&freeb, &totb));
   const size_t budget = freeb / 4 * 3;
@@ -1902,19 +1924,28 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
   if (chunk < 1) return fail(RHG_ENOMEM, "device memory too small for one NLTE column");
 
   NlteTimer tm_all, tm_k;
-  for (auto &x : tm_all.e) HIPCHECK(hipEventCreate(&x));
-  for (auto &x : tm_k.e) HIPCHECK(hipEventCreate(&x));
+  if (tm_all.make(2)) return fail(RHG_EDEVICE, "hipEventCreate");
   for (double &x : c->nlte_ms) x = 0.0;
   HIPCHECK(hipEventRecord(tm_all.e[0], c->stream));
   float ms = 0.0f;
-  // time one launch sequence on the stream into nlte_ms[slot]
+  // time one launch sequence on the stream into nlte_ms[slot]; the events
+  // are read at the next synchronisation of the stream (read_timers)
+  std::vector<int> pending;
   auto timed = [&](int slot, auto &&launch) -> int {
-    HIPCHECK(hipEventRecord(tm_k.e[0], c->stream));
+    const size_t i = 2 * pending.size();
+    if (tm_k.make(i + 2)) return fail(RHG_EDEVICE, "hipEventCreate");
+    HIPCHECK(hipEventRecord(tm_k.e[i], c->stream));
     if (int rc = launch()) return rc;
-    HIPCHECK(hipEventRecord(tm_k.e[1], c->stream));
-    HIPCHECK(hipEventSynchronize(tm_k.e[1]));
-    HIPCHECK(hipEventElapsedTime(&ms, tm_k.e[0], tm_k.e[1]));
-    c->nlte_ms[slot] += ms;
+    HIPCHECK(hipEventRecord(tm_k.e[i + 1], c->stream));
+    pending.push_back(slot);
+    return 0;
+  };
+  auto read_timers = [&]() -> int {
+    for (size_t i = 0; i < pending.size(); i++) {
+      HIPCHECK(hipEventElapsedTime(&ms, tm_k.e[2 * i], tm_k.e[2 * i + 1]));
+      c->nlte_ms[pending[i]] += ms;
+    }
+    pending.clear();
     return 0;
   };
 
@@ -1927,22 +1958,18 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
   for (int c0 = 0; c0 < ncol_all; c0 += chunk) {
     const int ncol = std::min(chunk, ncol_all - c0);
     const size_t pts = (size_t) ncol * Nmax * sizeof(double);
-    const int ncb_max = (ncol + 63) / 64;
+    const size_t row = (size_t) ncol * Kp * sizeof(double);   // of the depth-fastest arrays
     if (c->state.ensure(pts * nfield) || c->cchi.ensure(pts * nout) || c->ceta.ensure(pts * nout) ||
-        c->moving.ensure(ncol * sizeof(int32_t)) || c->nl_nstar.ensure(pts * nl) ||
-        c->nl_pops.ensure(pts * nl) || c->nl_ntot.ensure(pts) || c->nl_vbroad.ensure(pts) ||
-        c->nl_nHe.ensure(pts) || c->nl_adamp.ensure(pts * std::max(a->nline, 1)) ||
-        c->nl_wphi.ensure(pts * std::max(a->nline, 1)) || c->nl_Cmat.ensure(pts * nl * nl) ||
-        c->nl_Gam.ensure(pts * nl * nl) ||
-        c->nl_phi.ensure(pts * std::max(h.nphi, 1) * nrays * 2) || c->nl_csca.ensure(pts * nout) ||
-        c->nl_J.ensure(pts * nout * 2) || c->nl_acc.ensure(pts * h.nentry * 2) ||
-        c->nl_scr.ensure(std::max({(size_t) rhg::NLTE_NSLOT * (nlist - h.nbez),
-                                   stokes_out ? (size_t) rhg::NLTE_NSLOT_EM * nlist : (size_t) 0,
-                                   (size_t) 1}) *
-                         Nmax * ncb_max * 64 * sizeof(double)) ||
+        c->moving.ensure(ncol * sizeof(int32_t)) || c->nl_geo.ensure(row * rhg::NG_N) ||
+        c->nl_nstar.ensure(row * nl) || c->nl_pops.ensure(row * nl) || c->nl_ntot.ensure(row) ||
+        c->nl_vbroad.ensure(row) || c->nl_nHe.ensure(row) ||
+        c->nl_adamp.ensure(row * std::max(a->nline, 1)) ||
+        c->nl_wphi.ensure(row * std::max(a->nline, 1)) || c->nl_Cmat.ensure(row * nl * nl) ||
+        c->nl_phi.ensure(row * std::max(h.nphi, 1) * nrays * 2) || c->nl_bg.ensure(row * nout * 3) ||
+        c->nl_J.ensure(row * nout * 2) || c->nl_acc.ensure(row * h.nentry * 2) ||
         (stokes_out && !device_ptrs && c->nl_st.ensure((size_t) ncol * 4 * nout * sizeof(double))) ||
         c->nl_jpar.ensure(ncol * sizeof(int32_t)) ||
-        c->nl_dJ.ensure((size_t) nlist * ncol * sizeof(double)) || c->nl_hist.ensure(pts * NS * nl) ||
+        c->nl_dJ.ensure((size_t) nlist * ncol * sizeof(double)) || c->nl_hist.ensure(row * NS * nl) ||
         c->nl_act.ensure(ncol * sizeof(int32_t)) || c->nl_red.ensure(ncol * sizeof(double)) ||
         (!device_ptrs && (c->nl_atm.ensure(pts * 9) || c->nl_ndep.ensure(ncol * sizeof(int32_t)) ||
                           c->nl_out.ensure(pts * nl * (nstar_out ? 2 : 1)))))
@@ -1959,10 +1986,15 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
     rhg::NlteBufs B{};
     B.ncol = ncol;
     B.Nmax = Nmax;
+    B.Kp = Kp;
+    B.fs = (int64_t) ncol * Kp;
     B.nfield = nfield;
     B.nout = nout;
     B.ndep = d_ndep;
     B.state = (double *) c->state.p;
+    B.lte_chi = (const double *) c->cchi.p;
+    B.lte_eta = (const double *) c->ceta.p;
+    B.geo = (double *) c->nl_geo.p;
     B.nstar = (double *) c->nl_nstar.p;
     B.pops = (double *) c->nl_pops.p;
     B.ntot = (double *) c->nl_ntot.p;
@@ -1971,15 +2003,13 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
     B.adamp = (double *) c->nl_adamp.p;
     B.wphi = (double *) c->nl_wphi.p;
     B.Cmat = (double *) c->nl_Cmat.p;
-    B.Gam = (double *) c->nl_Gam.p;
     B.phi = (double *) c->nl_phi.p;
-    B.cchi = (double *) c->cchi.p;
-    B.ceta = (double *) c->ceta.p;
-    B.csca = (double *) c->nl_csca.p;
+    B.cchi = (double *) c->nl_bg.p;
+    B.ceta = B.cchi + B.fs * nout;
+    B.csca = B.ceta + B.fs * nout;
     B.J = (double *) c->nl_J.p;
     B.jpar = (int32_t *) c->nl_jpar.p;
     B.acc = (double *) c->nl_acc.p;
-    B.scr = (double *) c->nl_scr.p;
     B.dJ = (double *) c->nl_dJ.p;
     B.hist = (double *) c->nl_hist.p;
     int32_t *d_act = (int32_t *) c->nl_act.p;
@@ -2002,18 +2032,24 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
       hipLaunchKernelGGL((rhg::k_continuum<double, false>),
                          dim3((unsigned) ((npts + rhg::CONT_BLOCK - 1) / rhg::CONT_BLOCK)),
                          dim3(rhg::CONT_BLOCK), 0, c->stream, c->d_model, d_ndep, ncol, Nmax,
-                         B.state, nfield, c->d_out_ls, nout, B.cchi, B.ceta, (const int32_t *) nullptr, (const int32_t *) nullptr, (const int32_t *) nullptr, 0);
+                         B.state, nfield, c->d_out_ls, nout, (double *) c->cchi.p,
+                         (double *) c->ceta.p, (const int32_t *) nullptr, (const int32_t *) nullptr,
+                         (const int32_t *) nullptr, 0);
       HIPCHECK(hipGetLastError());
-      hipLaunchKernelGGL(rhg::k_nlte_bg, gpts, b64, 0, c->stream, c->d_model, d_at, B,
-                         c->d_out_ls);
+      hipLaunchKernelGGL(rhg::k_nlte_bg,
+                         dim3((unsigned) ((int64_t) ((ncol + 31) / 32) * ((Nmax + 31) / 32) *
+                                          (nout + rhg::NG_N))),
+                         dim3(256), 0, c->stream, c->d_model, d_at, B, c->d_out_ls);
       HIPCHECK(hipGetLastError());
       if (a->nline > 0) {
-        const int64_t np = npts * a->nline;
-        hipLaunchKernelGGL(rhg::k_nlte_profile, dim3((unsigned) ((np + 63) / 64)), b64, 0,
+        hipLaunchKernelGGL(rhg::k_nlte_profile, dim3((unsigned) ((npts + 63) / 64 * h.nphi)), b64, 0,
                            c->stream, c->d_model, d_at, B);
         HIPCHECK(hipGetLastError());
+        hipLaunchKernelGGL(rhg::k_nlte_wphi, dim3(gpts.x, (unsigned) a->nline), b64, 0, c->stream,
+                           d_at, B);
+        HIPCHECK(hipGetLastError());
       }
-      HIPCHECK(hipMemsetAsync(B.J, 0, pts * nout, c->stream));
+      HIPCHECK(hipMemsetAsync(B.J, 0, row * nout, c->stream));
       HIPCHECK(hipMemsetAsync(B.jpar, 0, ncol * sizeof(int32_t), c->stream));
       return 0;
     });
@@ -2027,18 +2063,32 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
                               c->stream));
       return 0;
     };
+    // columns a k_nlte_feautrier workgroup shares its lanes between: as many
+    // as 24 KB of LDS hold, fewer while they would leave SIMDs idle
+    auto fe_per = [&](int nact, int rays) {
+      int per = 12;
+      while (per > 1 && rhg::nlte_fe_lds(Nmax, per, rays) * sizeof(double) > 24576) per--;
+      while (per > 1 && (int64_t) nact * (nlist - h.nbez) / per < 1024) per--;
+      return per;
+    };
     auto rt = [&](int slot, int eval) -> int {
       const int nact = (int) act.size();
-      const int ncb = (nact + 63) / 64, nfe = nlist - h.nbez;
+      const int nfe = nlist - h.nbez;
       int r = timed(slot, [&]() -> int {
         if (h.nbez > 0) {
-          dim3 grd((unsigned) rhg::xcd_grid(ncb, h.nbez));
-#define RHG_LAUNCH_BEZ(MS)                                                                       \
-  hipLaunchKernelGGL((rhg::k_nlte_bezier<rhg::NLTE_RB, MS>), grd, b64, 0, c->stream, c->d_model, \
-                     d_at, B, d_act, nact, c->d_out_ls, d_iolist, h.nbez, 0, eval)
-          if (h.maxset_bez <= 2) RHG_LAUNCH_BEZ(2);
-          else if (h.maxset_bez <= 4) RHG_LAUNCH_BEZ(4);
-          else RHG_LAUNCH_BEZ(8);
+          const dim3 grd((unsigned) rhg::nlte_grid(nact, h.nbez));
+#define RHG_LAUNCH_BEZ(L, P, MS)                                                                 \
+  hipLaunchKernelGGL((rhg::k_nlte_bezier<L, P, MS>), grd, dim3(2 * L),                            \
+                     (size_t) Nmax * sizeof(double), c->stream, c->d_model, d_at, B, d_act, nact, \
+                     c->d_out_ls, d_iolist, h.nbez, 0, nlist, eval)
+#define RHG_LAUNCH_BEZ_P(L, P)                                                                   \
+  do {                                                                                           \
+    if (h.maxset_bez <= 2) RHG_LAUNCH_BEZ(L, P, 2);                                              \
+    else if (h.maxset_bez <= 4) RHG_LAUNCH_BEZ(L, P, 4);                                         \
+    else RHG_LAUNCH_BEZ(L, P, 8);                                                                \
+  } while (0)
+          RHG_RAY_POINTS(Nmax, RHG_LAUNCH_BEZ_P);
+#undef RHG_LAUNCH_BEZ_P
 #undef RHG_LAUNCH_BEZ
           HIPCHECK(hipGetLastError());
         }
@@ -2052,10 +2102,13 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
         if (nfe > 0) {
           // the member loops unrolled to the largest active set (one launch:
           // split by set size, the launches would not fill the GPU)
-          dim3 grd((unsigned) rhg::xcd_grid(ncb, nfe));
+          const int per = fe_per(nact, rhg::NLTE_FE_RAYS);
+          const dim3 grd((unsigned) rhg::nlte_grid((nact + per - 1) / per, nfe));
+          const size_t lds = rhg::nlte_fe_lds(Nmax, per, rhg::NLTE_FE_RAYS) * sizeof(double);
 #define RHG_LAUNCH_FE(MS)                                                                        \
-  hipLaunchKernelGGL((rhg::k_nlte_feautrier<MS>), grd, b64, 0, c->stream, c->d_model, d_at, B,   \
-                     d_act, nact, c->d_out_ls, d_iolist + h.nbez, nfe, h.nbez, eval)
+  hipLaunchKernelGGL((rhg::k_nlte_feautrier<MS, false>), grd, b64, lds, c->stream, c->d_model, d_at, \
+                     B, d_act, nact, per, c->d_out_ls, d_iolist + h.nbez, nfe, h.nbez, nlist, eval, \
+                     0.0, (double *) nullptr)
           if (h.maxset_fe <= 2) RHG_LAUNCH_FE(2);
           else if (h.maxset_fe <= 4) RHG_LAUNCH_FE(4);
           else if (h.maxset_fe <= 6) RHG_LAUNCH_FE(6);
@@ -2074,7 +2127,7 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
     auto fetch_red = [&]() -> int {
       HIPCHECK(hipMemcpyAsync(red.data(), d_red, ncol * sizeof(double), hipMemcpyDeviceToHost, c->stream));
       HIPCHECK(hipStreamSynchronize(c->stream));
-      return 0;
+      return read_timers();
     };
 
     // background scattering passes without the operator (each column stops
@@ -2084,7 +2137,7 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
       for (int it = 0; it < a->nmax_scatter && !act.empty(); it++) {
         if ((rc = rt(1, 0))) return rc;
         const int nact = (int) act.size();
-        hipLaunchKernelGGL(rhg::k_nlte_djmax, dim3((unsigned) ((nact + 63) / 64)), b64, 0, c->stream,
+        hipLaunchKernelGGL(rhg::k_nlte_djmax, dim3((unsigned) nact), b64, 0, c->stream,
                            B, d_act, nact, nlist, d_red);
         HIPCHECK(hipGetLastError());
         if ((rc = fetch_red())) return rc;
@@ -2102,28 +2155,29 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
     act.resize(ncol);
     for (int i = 0; i < ncol; i++) act[i] = i;
     if ((rc = upload_act())) return rc;
-    HIPCHECK(hipMemcpyAsync(B.hist, B.pops, pts * nl, hipMemcpyDeviceToDevice, c->stream));
+    HIPCHECK(hipMemcpyAsync(B.hist, B.pops, row * nl, hipMemcpyDeviceToDevice, c->stream));
     const int ndelay = std::max(a->ng_delay, a->ng_order + 2);
     for (int it = 1; it <= a->nmax_iter && !act.empty(); it++) {
       const int nact = (int) act.size();
       if ((rc = rt(2, 1))) return rc;
       rc = timed(3, [&]() -> int {
-        const int64_t n = (int64_t) nact * Nmax;
-        const dim3 g((unsigned) ((n + 63) / 64));
-        if (nl <= 4)
-          hipLaunchKernelGGL(rhg::k_nlte_stateq<4>, g, b64, 0, c->stream, d_at, B, d_act, nact, a->isum);
-        else if (nl <= 6)
-          hipLaunchKernelGGL(rhg::k_nlte_stateq<6>, g, b64, 0, c->stream, d_at, B, d_act, nact, a->isum);
-        else if (nl <= 8)
-          hipLaunchKernelGGL(rhg::k_nlte_stateq<8>, g, b64, 0, c->stream, d_at, B, d_act, nact, a->isum);
-        else
-          hipLaunchKernelGGL(rhg::k_nlte_stateq<16>, g, b64, 0, c->stream, d_at, B, d_act, nact, a->isum);
+#define RHG_LAUNCH_SE(NLP)                                                                        \
+  hipLaunchKernelGGL(rhg::k_nlte_stateq<NLP>,                                                       \
+                     dim3((unsigned) nact, (unsigned) ((Nmax - 1) / rhg::stateq_depths(NLP) + 1)),  \
+                     dim3(64 * rhg::stateq_waves(NLP)),                                             \
+                     (size_t) rhg::stateq_depths(NLP) * nl * nl * sizeof(double), c->stream, d_at,  \
+                     B, d_act, nact, a->isum)
+        if (nl <= 4) RHG_LAUNCH_SE(4);
+        else if (nl <= 6) RHG_LAUNCH_SE(6);
+        else if (nl <= 8) RHG_LAUNCH_SE(8);
+        else RHG_LAUNCH_SE(16);
+#undef RHG_LAUNCH_SE
         HIPCHECK(hipGetLastError());
         return 0;
       });
       if (rc) return rc;
       rc = timed(4, [&]() -> int {
-        hipLaunchKernelGGL(rhg::k_nlte_ng, dim3((unsigned) ((nact + 63) / 64)), b64, 0, c->stream, d_at,
+        hipLaunchKernelGGL(rhg::k_nlte_ng, dim3((unsigned) nact), dim3(rhg::NG_BLOCK), 0, c->stream, d_at,
                            B, d_act, nact, it, a->ng_order, ndelay, a->ng_period, d_red);
         HIPCHECK(hipGetLastError());
         return 0;
@@ -2150,7 +2204,7 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
       for (int it = 0; it < a->nmax_scatter && !act.empty(); it++) {
         if ((rc = rt(1, 0))) return rc;
         const int nact = (int) act.size();
-        hipLaunchKernelGGL(rhg::k_nlte_djmax, dim3((unsigned) ((nact + 63) / 64)), b64, 0, c->stream,
+        hipLaunchKernelGGL(rhg::k_nlte_djmax, dim3((unsigned) nact), b64, 0, c->stream,
                            B, d_act, nact, nlist, d_red);
         HIPCHECK(hipGetLastError());
         if ((rc = fetch_red())) return rc;
@@ -2161,10 +2215,25 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
         if (!act.empty() && (rc = upload_act())) return rc;
       }
       double *d_st = device_ptrs ? stokes_out + (size_t) c0 * 4 * nout : (double *) c->nl_st.p;
-      dim3 grd((unsigned) rhg::xcd_grid((ncol + 63) / 64, nlist));
-      hipLaunchKernelGGL(rhg::k_nlte_emergent, grd, b64, 0, c->stream, c->d_model, d_at, B,
-                         c->d_out_ls, d_iolist, nlist, cols->mu, d_st);
-      HIPCHECK(hipGetLastError());
+      const int nfe = nlist - h.nbez;
+      if (h.nbez > 0) {
+        const dim3 grd((unsigned) rhg::nlte_grid(ncol, h.nbez));
+#define RHG_LAUNCH_EM(L, P)                                                                      \
+  hipLaunchKernelGGL((rhg::k_nlte_emergent<L, P>), grd, b64, 0, c->stream, c->d_model, d_at, B,       \
+                     c->d_out_ls, d_iolist, h.nbez, cols->mu, d_st)
+        RHG_RAY_POINTS(Nmax, RHG_LAUNCH_EM);
+#undef RHG_LAUNCH_EM
+        HIPCHECK(hipGetLastError());
+      }
+      if (nfe > 0) {
+        const int per = fe_per(ncol, 1);
+        const dim3 grd((unsigned) rhg::nlte_grid((ncol + per - 1) / per, nfe));
+        hipLaunchKernelGGL((rhg::k_nlte_feautrier<2, true>), grd, b64,
+                           rhg::nlte_fe_lds(Nmax, per, 1) * sizeof(double), c->stream, c->d_model,
+                           d_at, B, (const int32_t *) nullptr, ncol, per, c->d_out_ls,
+                           d_iolist + h.nbez, nfe, h.nbez, nlist, 0, cols->mu, d_st);
+        HIPCHECK(hipGetLastError());
+      }
       if (!device_ptrs)
         HIPCHECK(hipMemcpyAsync(stokes_out + (size_t) c0 * 4 * nout, d_st,
                                 (size_t) ncol * 4 * nout * sizeof(double), hipMemcpyDeviceToHost,
@@ -2202,6 +2271,7 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
       memcpy(dpops_out + c0, dpops.data(), ncol * sizeof(double));
     }
     HIPCHECK(hipStreamSynchronize(c->stream));
+    if ((rc = read_timers())) return rc;
   }
   HIPCHECK(hipEventRecord(tm_all.e[1], c->stream));
   HIPCHECK(hipEventSynchronize(tm_all.e[1]));

@@ -2,14 +2,22 @@
 // iteration of rhf1d() (rh/iterate.c:48-143) as a sequence of batched
 // kernels over all columns at once.
 //
+// The iteration's arrays are depth-fastest and its kernels put a column's
+// depths on consecutive lanes.  One column is then hundreds of wavefronts
+// rather than one lane of each (the iteration of a single column used to be
+// as long as that of 1500), and the only serial chains left are a wavefront
+// scan (the short-characteristic recursion is affine in I) and the Feautrier
+// elimination.
+//
 // Set-up (once per batch, after k_state of the background model)
 //   k_nlte_pre      (column, depth): scattering opacity at the reference
 //                   wavelength (the depth scale), LTE populations, Doppler
 //                   widths, damping and the collision matrix.
-//   k_nlte_bg       (column, depth): scattering opacity at every wavelength,
-//                   added to the LTE continuum opacity.
-//   k_nlte_profile  (column, depth, line): absorption profiles for every
-//                   ray and direction, and their normalisation.
+//   k_nlte_bg       depth-fastest copies of the column state's fields and of
+//                   the LTE continuum, with the scattering opacity added.
+//   k_nlte_profile  (column, depth, line, wavelength): absorption profiles
+//                   for every ray and direction; k_nlte_wphi: their
+//                   normalisation.
 // Iteration (per pass, over the columns still iterating)
 //   k_nlte_bezier   (column, wavelength with a line): the rays of the
 //   k_nlte_feautrier (column, continuum-only wavelength)
@@ -36,28 +44,46 @@ __device__ __forceinline__ double planck_lam(double T, double lambda) {
   return (hc_Tkla <= MAX_EXPONENT) ? twohnu3_c2 / (exp(hc_Tkla) - 1.0) : 0.0;
 }
 
-// Fritsch & Butland centred derivative with the reference's divisions,
-// rh/bezier_aux.c:34-51
-// a / b as a times the hardware reciprocal estimate refined by two Newton
-// steps (relative error ~1e-16, not correctly rounded): the quotients of
-// the scalar Bezier rays, where the IEEE division sequence is a long
-// dependent chain per use
-__device__ __forceinline__ double ndiv(double a, double b) {
+// 1 / b and a / b by the hardware reciprocal estimate refined by two Newton
+// steps (relative error ~1e-16, not correctly rounded): the quotients of the
+// rays, where the IEEE division sequence is a long dependent chain per use
+__device__ __forceinline__ double nrcp(double b) {
   double r = __builtin_amdgcn_rcp(b);
   double e = fma(-b, r, 1.0);
   r = fma(r, e, r);
   e = fma(-b, r, 1.0);
-  return a * fma(r, e, r);
+  return fma(r, e, r);
+}
+__device__ __forceinline__ double ndiv(double a, double b) { return a * nrcp(b); }
+
+// Fritsch & Butland monotone derivative, rh/bezier_aux.c:34-51, from the
+// slopes of the two intervals and alpha = (1 + dn / (up + dn)) / 3
+__device__ __forceinline__ double monotone(double f_up, double f_dn, double alpha) {
+  const double p = f_up * f_dn;
+  return p > 0.0 ? p * nrcp(fma(alpha, f_dn, (1.0 - alpha) * f_up)) : 0.0;
 }
 
-__device__ __forceinline__ double cent_div(double dsup, double dsdn, double up, double c,
-                                           double dn) {
-  const double fim1 = ndiv(c - up, dsup), fi = ndiv(dn - c, dsdn);
-  if (fim1 * fi > 0) {
-    const double alpha = 0.333333333333333333333333 * (1.0 + ndiv(dsdn, dsdn + dsup));
-    return ndiv(fim1 * fi, (1.0 - alpha) * fim1 + alpha * fi);
-  }
-  return 0.0;
+// x of the lane `ctrl` names, or `old` where there is none
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ double dpp(double old, double x) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(x), CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(x), CTRL, ROWS, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+// x of the previous / the next lane (0 where there is none)
+template <int CTRL>
+__device__ __forceinline__ double shift(double x) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double from_prev(double x) { return shift<0x138>(x); }   // wave_shr:1
+__device__ __forceinline__ double from_next(double x) { return shift<0x130>(x); }   // wave_shl:1
+
+// LDS written by some lanes of the wavefront is read by others after this
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  __builtin_amdgcn_wave_barrier();
 }
 
 __device__ __forceinline__ double max0(double x) { return x > 0.0 ? x : 0.0; }
@@ -94,16 +120,16 @@ __global__ void k_nlte_pre(const DevModel *__restrict__ Mp, const DevNlte *__res
   const int64_t p = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
   const int ncol = B.ncol, Nmax = B.Nmax;
   if (p >= (int64_t) ncol * Nmax) return;
-  const int ic = (int) (p % ncol), k = (int) (p / ncol);
+  const int k = (int) (p % Nmax), ic = (int) (p / Nmax);
   if (k >= B.ndep[ic]) return;
-  const int64_t fs = (int64_t) Nmax * ncol;
+  const int64_t ss = (int64_t) Nmax * ncol, fs = B.fs;
   double *st = B.state + (int64_t) k * ncol + ic;
-  const double T = st[RHG_CF_T * fs], ne = st[RHG_CF_NE * fs], nHtot = st[RHG_CF_NHTOT * fs];
-  const double nH0 = st[RHG_CF_NH0 * fs], np = st[RHG_CF_NP * fs], nH2 = st[RHG_CF_NH2 * fs];
-  const double vturb = st[RHG_CF_VTURB * fs];
+  const double T = st[RHG_CF_T * ss], ne = st[RHG_CF_NE * ss], nHtot = st[RHG_CF_NHTOT * ss];
+  const double nH0 = st[RHG_CF_NH0 * ss], np = st[RHG_CF_NP * ss], nH2 = st[RHG_CF_NH2 * ss];
+  const double vturb = st[RHG_CF_VTURB * ss];
   const double c1 = (HPLANCK / (2.0 * PI * M_ELECTRON)) * (HPLANCK / KBOLTZMANN);
   const double cNe_T = 0.5 * ne * pow(c1 / T, 1.5);
-  const int64_t pk = (int64_t) k * ncol + ic;
+  const int64_t pk = (int64_t) ic * B.Kp + k;
 
   double nHe = 0.0;
   if (A.he_atom >= 0) {
@@ -118,7 +144,7 @@ __global__ void k_nlte_pre(const DevModel *__restrict__ Mp, const DevNlte *__res
     if (A.he_atom >= 0) sca += A.ray_He[lr] * nHe;
     sca += A.ray_H2[lr] * nH2;
     sca *= ldc(M.lamconst)[(int64_t) lr * RHG_LC_NCONST + RHG_LC_SCATT_FUDGE];
-    st[RHG_CF_HEIGHT * fs] += sca;
+    st[RHG_CF_HEIGHT * ss] += sca;
   }
 
   const int nl = A.nl, a = A.atom_index, l0 = ldc(M.atom_level_ptr)[a];
@@ -202,74 +228,120 @@ __global__ void k_nlte_pre(const DevModel *__restrict__ Mp, const DevNlte *__res
   }
 }
 
-// Scattering opacity (Thomson and Rayleigh on H, He and H2) at every output
-// wavelength: stored, and added to the LTE continuum opacity
-// (rh/background.c:342-465).
-__global__ void k_nlte_bg(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap,
-                          NlteBufs B, const int32_t *__restrict__ out_ls) {
+// Depth-fastest copies: row io < nout is the output wavelength's LTE
+// continuum with the scattering opacity (Thomson and Rayleigh on H, He and
+// H2, rh/background.c:342-465), its emissivity and the scattering opacity;
+// rows nout .. nout + NG_N - 1 are the column state's fields of NG_*.  One
+// 32 x 32 tile (columns x depths) of a row per workgroup of 256 threads,
+// turned in LDS, so that the column-fastest reads and the depth-fastest
+// writes are both in runs.
+__global__ void __launch_bounds__(256)
+k_nlte_bg(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap, NlteBufs B,
+          const int32_t *__restrict__ out_ls) {
   const DevNlte &A = *Ap;
-  const int64_t p = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-  const int ncol = B.ncol, Nmax = B.Nmax;
-  if (p >= (int64_t) ncol * Nmax) return;
-  const int ic = (int) (p % ncol), k = (int) (p / ncol);
-  if (k >= B.ndep[ic]) return;
-  const int64_t fs = (int64_t) Nmax * ncol;
-  const double *st = B.state + (int64_t) k * ncol + ic;
-  const double ne = st[RHG_CF_NE * fs], nH0 = st[RHG_CF_NH0 * fs], nH2 = st[RHG_CF_NH2 * fs];
-  const double nHe = B.nHe[(int64_t) k * ncol + ic];
   const DevModel &M = *Mp;
-  for (int io = 0; io < B.nout; io++) {
-    const int ls = out_ls[io];
-    double sca = ne * A.sigma_thomson;
-    sca += A.ray_H[ls] * nH0;
-    if (A.he_atom >= 0) sca += A.ray_He[ls] * nHe;
-    sca += A.ray_H2[ls] * nH2;
-    // the scattering fudge factor, rh/background.c:453-462
-    sca *= ldc(M.lamconst)[(int64_t) ls * RHG_LC_NCONST + RHG_LC_SCATT_FUDGE];
-    const int64_t q = (int64_t) io * fs + (int64_t) k * ncol + ic;
-    B.csca[q] = sca;
-    B.cchi[q] += sca;
+  const int ncol = B.ncol, Nmax = B.Nmax, nrow = B.nout + NG_N;
+  const int row = (int) (blockIdx.x % nrow), tile = (int) (blockIdx.x / nrow);
+  const int nkt = (Nmax + 31) / 32, c0 = tile / nkt * 32, k0 = tile % nkt * 32;
+  const int64_t ss = (int64_t) Nmax * ncol;
+  __shared__ double t[3][32][33];
+  const bool wave = row < B.nout;
+  const int ls = wave ? out_ls[row] : 0;
+  for (int i = threadIdx.x; i < 1024; i += 256) {
+    const int c = i % 32, k = i / 32, ic = c0 + c, kk = k0 + k;
+    if (ic >= ncol || kk >= Nmax || kk >= B.ndep[ic]) continue;
+    const double *st = B.state + (int64_t) kk * ncol + ic;
+    if (wave) {
+      double sca = st[RHG_CF_NE * ss] * A.sigma_thomson;
+      sca += A.ray_H[ls] * st[RHG_CF_NH0 * ss];
+      if (A.he_atom >= 0) sca += A.ray_He[ls] * B.nHe[(int64_t) ic * B.Kp + kk];
+      sca += A.ray_H2[ls] * st[RHG_CF_NH2 * ss];
+      // the scattering fudge factor, rh/background.c:453-462
+      sca *= ldc(M.lamconst)[(int64_t) ls * RHG_LC_NCONST + RHG_LC_SCATT_FUDGE];
+      const int64_t q = (int64_t) row * ss + (int64_t) kk * ncol + ic;
+      t[0][k][c] = B.lte_chi[q] + sca;
+      t[1][k][c] = B.lte_eta[q];
+      t[2][k][c] = sca;
+    } else {
+      const int f = row - B.nout;
+      t[0][k][c] = st[(f == NG_T ? RHG_CF_T : f == NG_VLOS ? RHG_CF_VLOS
+                       : f == NG_DZ ? RHG_CF_DZ : RHG_CF_HEIGHT) * ss];
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < 1024; i += 256) {
+    const int k = i % 32, c = i / 32, ic = c0 + c, kk = k0 + k;
+    if (ic >= ncol || kk >= Nmax || kk >= B.ndep[ic]) continue;
+    const int64_t pk = (int64_t) ic * B.Kp + kk;
+    if (wave) {
+      const int64_t q = (int64_t) row * B.fs + pk;
+      B.cchi[q] = t[0][k][c];
+      B.ceta[q] = t[1][k][c];
+      B.csca[q] = t[2][k][c];
+    } else {
+      B.geo[(int64_t) (row - B.nout) * B.fs + pk] = t[0][k][c];
+    }
   }
 }
 
 // Field-free absorption profiles of the atom's lines for every ray and
-// direction and their normalisation over the line's quadrature,
-// rh/profile.c:67-371 (Voigt function of Armstrong, rh/voigt.c:126-243).
+// direction, rh/profile.c:67-371 (Voigt function of Armstrong,
+// rh/voigt.c:126-243), one (column, depth) x (line, wavelength) per thread,
+// and into the rate accumulators (unused until the first iteration) the
+// wavelength's part of the normalisation integral.  Row
+// blockIdx.x % nphi of the lines' wavelengths is grid point la of line l.
 __global__ void k_nlte_profile(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap,
                                NlteBufs B) {
   const DevModel &M = *Mp;
   const DevNlte &A = *Ap;
-  const int64_t p = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-  const int ncol = B.ncol, Nmax = B.Nmax;
-  if (p >= (int64_t) ncol * Nmax * A.nline) return;
-  const int ic = (int) (p % ncol);
-  const int64_t q = p / ncol;
-  const int k = (int) (q % Nmax), l = (int) (q / Nmax);
+  const int ncol = B.ncol, Nmax = B.Nmax, row = (int) (blockIdx.x % A.nphi);
+  const int64_t p = (int64_t) (blockIdx.x / A.nphi) * blockDim.x + threadIdx.x;
+  if (p >= (int64_t) ncol * Nmax) return;
+  const int k = (int) (p % Nmax), ic = (int) (p / Nmax);
   if (k >= B.ndep[ic]) return;
-  const int64_t fs = (int64_t) Nmax * ncol, pk = (int64_t) k * ncol + ic;
-  const double vb = B.vbroad[pk], vz = B.state[RHG_CF_VLOS * fs + pk];
+  int l = 0;
+  while (l + 1 < A.nline && row >= A.ln_phi[l + 1]) l++;
+  const int la = row - A.ln_phi[l];
+  const int64_t fs = B.fs, pk = (int64_t) ic * B.Kp + k;
+  const double vb = B.vbroad[pk], vz = B.geo[NG_VLOS * fs + pk];
   const double adamp = B.adamp[(int64_t) l * fs + pk];
   const int t = A.ln_tr[l], nrays = A.nrays;
   const double lambda0 = A.ln_lambda0[l];
+  const int ls = A.tr_nblue[t] + la;
+  const double lamla = ldc(M.lamconst)[(int64_t) ls * RHG_LC_NCONST + RHG_LC_LAMBDA];
+  const double wl = A.tr_wlam[A.tr_ptr[t] + la];
+  const double v = (lamla - lambda0 - 0.0) * CLIGHT / (vb * lambda0);
   double wphi = 0.0;
-  for (int la = 0; la < A.tr_nlam[t]; la++) {
-    const int ls = A.tr_nblue[t] + la;
-    const double lamla = ldc(M.lamconst)[(int64_t) ls * RHG_LC_NCONST + RHG_LC_LAMBDA];
-    const double wl = A.tr_wlam[A.tr_ptr[t] + la];
-    const double v = (lamla - lambda0 - 0.0) * CLIGHT / (vb * lambda0);
-    for (int mu = 0; mu < nrays; mu++) {
-      const double wlamu = wl * 0.5 * A.wmu[mu];
-      const double vlos = A.muz[mu] * vz / vb;
-      for (int to_obs = 0; to_obs <= 1; to_obs++) {
-        const double sign = to_obs ? 1.0 : -1.0;
-        const double vk = v + sign * vlos;
-        const double ph = voigt_armstrong(adamp, vk) * 1.0 / (SQRTPI * vb);
-        B.phi[((((int64_t) (A.ln_phi[l] + la) * nrays + mu) * 2 + to_obs) * Nmax) * ncol + pk] = ph;
-        wphi += ph * wlamu;
-      }
+  for (int mu = 0; mu < nrays; mu++) {
+    const double wlamu = wl * 0.5 * A.wmu[mu];
+    const double vlos = A.muz[mu] * vz / vb;
+    for (int to_obs = 0; to_obs <= 1; to_obs++) {
+      const double sign = to_obs ? 1.0 : -1.0;
+      const double vk = v + sign * vlos;
+      const double ph = voigt_armstrong(adamp, vk) * 1.0 / (SQRTPI * vb);
+      B.phi[((int64_t) (row * nrays + mu) * 2 + to_obs) * fs + pk] = ph;
+      wphi += ph * wlamu;
     }
   }
-  B.wphi[(int64_t) l * fs + pk] = 1.0 / wphi;
+  B.acc[(int64_t) row * fs + pk] = wphi;
+}
+
+// 1 / the profile's integral over its quadrature, one (column, depth, line)
+// per thread
+__global__ void k_nlte_wphi(const DevNlte *__restrict__ Ap, NlteBufs B) {
+  const DevNlte &A = *Ap;
+  const int64_t p = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+  const int Nmax = B.Nmax, l = blockIdx.y;
+  if (p >= (int64_t) B.ncol * Nmax) return;
+  const int k = (int) (p % Nmax), ic = (int) (p / Nmax);
+  if (k >= B.ndep[ic]) return;
+  const int64_t pk = (int64_t) ic * B.Kp + k;
+  const int n = A.tr_nlam[A.ln_tr[l]];
+  const double *w = B.acc + (int64_t) A.ln_phi[l] * B.fs + pk;
+  double sum = 0.0;
+#pragma unroll 8
+  for (int la = 0; la < n; la++) sum += w[(int64_t) la * B.fs];
+  B.wphi[(int64_t) l * B.fs + pk] = 1.0 / sum;
 }
 
 // ---------------------------------------------------------------------------
@@ -291,27 +363,55 @@ struct SetInfo {
   int ncross[MS];
 };
 
-// per-depth member data
+// per-depth member data: populations' difference x = n_i - gij n_j, emission
+// e = tw gij n_j, gij and the quadrature weight
 template <int MS>
 struct SetDepth {
-  double ni[MS], nj[MS], gij[MS], wla[MS];
+  double x[MS], e[MS], gij[MS], wla[MS];
 };
 
-// accumulate the rate terms of ray r (intensity I, operator Psi / chi in
+// member data of the set at one depth (offset pk of a row, temperature T)
+template <int MS>
+__device__ __forceinline__ void set_depth(const NlteBufs &B, const SetInfo<MS> &si, int64_t pk,
+                                          double T, double lam, SetDepth<MS> &sd) {
+#pragma clang fp contract(fast)
+  const double hc_k = HC / (KBOLTZMANN * NM_TO_M);
+  const int64_t fs = B.fs;
+  const double bf = exp(-hc_k / (lam * T));
+#pragma unroll
+  for (int n = 0; n < MS; n++) {
+    sd.x[n] = sd.e[n] = sd.gij[n] = sd.wla[n] = 0.0;
+    if (n < si.n) {
+      const double ni = B.pops[(int64_t) si.ti[n] * fs + pk], nj = B.pops[(int64_t) si.tj[n] * fs + pk];
+      if (si.line[n] >= 0) {
+        sd.gij[n] = si.gline[n];
+        sd.wla[n] = si.wlam[n] * B.wphi[(int64_t) si.line[n] * fs + pk] * (1.0 / HC_4PI);
+      } else {
+        sd.gij[n] = B.nstar[(int64_t) si.ti[n] * fs + pk] / B.nstar[(int64_t) si.tj[n] * fs + pk] * bf;
+        sd.wla[n] = FOURPI / HPLANCK * (si.wlam[n] / lam);
+      }
+      sd.x[n] = ni - sd.gij[n] * nj;
+      sd.e[n] = si.tw[n] * sd.gij[n] * nj;
+    }
+  }
+}
+
+// accumulate the rate terms of one ray (intensity I, operator Psi / chi in
 // PsiC, direction weight wmu, absorption V of each member) into sIJ, sJI
 template <int MS>
 __device__ __forceinline__ void rate_terms(const SetInfo<MS> &si, const SetDepth<MS> &sd,
                                            const double (&V)[MS], double I, double PsiC,
                                            double wmu, double (&sIJ)[MS], double (&sJI)[MS]) {
+#pragma clang fp contract(fast)
   double eta = 0.0;
 #pragma unroll
   for (int n = 0; n < MS; n++)
-    if (n < si.n) eta += si.tw[n] * sd.gij[n] * V[n] * sd.nj[n];
-  const double Ieff = I - PsiC * eta;
+    if (n < si.n) eta += V[n] * sd.e[n];
+  const double Ieff = I - PsiC * eta, pw = PsiC * wmu;
   double chicc[MS], U[MS];
 #pragma unroll
   for (int n = 0; n < MS; n++) {
-    chicc[n] = V[n] * sd.wla[n] * (sd.ni[n] - sd.gij[n] * sd.nj[n]);
+    chicc[n] = V[n] * sd.wla[n] * sd.x[n];
     U[n] = si.tw[n] * sd.gij[n] * V[n];
   }
 #pragma unroll
@@ -325,13 +425,10 @@ __device__ __forceinline__ void rate_terms(const SetInfo<MS> &si, const SetDepth
         if ((si.m_ji[n] >> m) & 1u) Ui += U[m];
       }
       const double wlamu = V[n] * sd.wla[n] * wmu;
-      double gji = sJI[n], gij = sIJ[n];
-      gji += Ieff * wlamu;
-      gij += (si.tw[n] + Ieff) * sd.gij[n] * wlamu;
-      gij -= chi_up * PsiC * Uj * wmu;
-      for (int c = 0; c < si.ncross[n]; c++) gji += chi_dn * PsiC * Ui * wmu;
-      sJI[n] = gji;
-      sIJ[n] = gij;
+      sJI[n] += Ieff * wlamu;
+      sIJ[n] += (si.tw[n] + Ieff) * sd.gij[n] * wlamu;
+      sIJ[n] -= chi_up * Uj * pw;
+      for (int c = 0; c < si.ncross[n]; c++) sJI[n] += chi_dn * Ui * pw;
     }
   }
 }
@@ -390,695 +487,616 @@ __device__ __forceinline__ void set_info(const DevNlte &A, int ls, double lam, S
 }
 
 // ---------------------------------------------------------------------------
-// Wavelengths with an active line, one (column, wavelength) per thread:
-// the rays with the scalar cubic Bezier method and its diagonal operator
-// (rh/rhf1d/bezier_1D.c:306-541), both directions, the new mean intensity
-// and with eval_op the radiative rate terms (rh/rhf1d/formal.c:44-346,
-// rh/fillgamma.c:82-332).
-//
-// The RB rays of a direction are swept together, depth by depth: RB
-// independent recursions per thread.  The opacity and source function of
-// each ray are evaluated two depths ahead of the recursion into a window
-// in registers, so no per-depth array is kept.  At each depth the rays'
-// contributions to J and to each member's rate terms are summed in
-// registers and stored once per direction: the inward sweep writes them,
-// the outward sweep adds its own.  J is double-buffered per column
-// (jpar): the previous J enters the source function, the new one is built.
-//
-// Workgroups map to (64 columns of the active list, list wavelength) by
-// xcd_tile, so a block of columns' state and populations stay in one
-// XCD's L2 across the wavelengths.
-// With active sets of at most two members and RB = 3 rays per sweep the
-// kernel is held to two waves per SIMD (256 VGPRs, 22 spilled): measured
-// on a solve of 4096 columns of the Ca II atom, 10% faster than RB = 2 at
-// three waves (fewer sweeps re-read the background and update the rate
-// sums) and than RB = 3 or 5 at one.
-template <int RB, int MS>
-__global__ void __launch_bounds__(64, (MS <= 2 ? 2 : 1))
+// Short-characteristic rays with the scalar cubic Bezier method and its
+// diagonal operator (rh/rhf1d/bezier_1D.c:306-541).  L lanes per ray
+// direction (32: half a wavefront each, 64: a wavefront each; the first L
+// threads inward, the others outward), lane l holding the sweep's points
+// t = l P .. l P + P - 1 (depth t inward, N-1-t outward), so both directions
+// run the same code at the same time.  Everything but the intensity is local
+// to a point and its neighbours; the recursion I[t] = E[t] I[t-1] + b[t] is a
+// scan over the L lanes.
+
+// What the points fix for every ray: path |z[t] - z[t-1]|, its reciprocal and
+// the derivative's interval weight.
+template <int P>
+struct RayPath {
+  double dz[P], idz[P], al[P];
+};
+
+// one ray's intensity and operator at the points from the opacities C (with
+// reciprocals iC), source functions S, 1 / mu and the boundary's Planck
+// function (outward: B at the two deepest points)
+template <int L, int P>
+__device__ __forceinline__ void ray_sweep(const RayPath<P> &g, int t0, int N, bool outward,
+                                          double zmu, double B2_0, double B2_1,
+                                          const double (&C)[P], const double (&S)[P],
+                                          double (&I)[P], double (&Psi)[P]) {
+#pragma clang fp contract(fast)
+  double f[P], dchi[P], dtau[P], idt[P], sl[P], dS[P], E[P], b[P];
+  const double C_prev = from_prev(C[P - 1]), C_next = from_next(C[0]);
+  const double S_prev = from_prev(S[P - 1]);
+#pragma unroll
+  for (int s = 0; s < P; s++) f[s] = (C[s] - (s ? C[s > 0 ? s - 1 : 0] : C_prev)) * g.idz[s];
+  const double f_next = from_next(f[0]);
+#pragma unroll
+  for (int s = 0; s < P; s++) {
+    const int t = t0 + s;
+    const double fn = s < P - 1 ? f[s < P - 1 ? s + 1 : s] : f_next;
+    dchi[s] = monotone(f[s], fn, g.al[s]);
+    if (t == 0) dchi[s] = fn;
+    if (t == N - 1) dchi[s] = f[s];
+  }
+  const double dchi_prev = from_prev(dchi[P - 1]);
+#pragma unroll
+  for (int s = 0; s < P; s++) {
+    const double Cm = s ? C[s > 0 ? s - 1 : 0] : C_prev, dm = s ? dchi[s > 0 ? s - 1 : 0] : dchi_prev;
+    const double z3 = g.dz[s] * (1.0 / 3.0);
+    const double c1 = max0(C[s] - z3 * dchi[s]), c2 = max0(Cm + z3 * dm);
+    dtau[s] = g.dz[s] * zmu * (C[s] + Cm + c1 + c2) * 0.25;
+    idt[s] = nrcp(dtau[s]);
+    sl[s] = (S[s] - (s ? S[s > 0 ? s - 1 : 0] : S_prev)) * idt[s];
+  }
+  const double dtau_next = from_next(dtau[0]), sl_next = from_next(sl[0]);
+#pragma unroll
+  for (int s = 0; s < P; s++) {
+    const double tn = s < P - 1 ? dtau[s < P - 1 ? s + 1 : s] : dtau_next;
+    const double sn = s < P - 1 ? sl[s < P - 1 ? s + 1 : s] : sl_next;
+    // monotone() with alpha = (2 tn + dtau) / (3 (tn + dtau)), one reciprocal
+    const double ts = tn + dtau[s], p = sl[s] * sn;
+    dS[s] = p > 0.0 ? 3.0 * p * ts * nrcp((ts + dtau[s]) * sl[s] + (ts + tn) * sn) : 0.0;
+    if (t0 + s == 0) dS[s] = sn;
+  }
+  const double dS_prev = from_prev(dS[P - 1]);
+#pragma unroll
+  for (int s = 0; s < P; s++) {
+    const int t = t0 + s;
+    const double Cm = s ? C[s > 0 ? s - 1 : 0] : C_prev, Sm = s ? S[s > 0 ? s - 1 : 0] : S_prev;
+    const double dSm = s ? dS[s > 0 ? s - 1 : 0] : dS_prev;
+    // the last interval is linear, on its own (trapezoidal) path
+    const bool last = t == N - 1;
+    const double dt = last ? 0.5 * zmu * (C[s] + Cm) * g.dz[s] : dtau[s];
+    const double eps = exp(-dt), dt2 = dt * dt, dt3 = dt2 * dt;
+    double alpha, beta, gamma, theta, e;
+    if (dt >= 5.e-2) {   // bezier3_coeffs, rh/bezier_aux.c:333-359
+      const double i3 = idt[s] * idt[s] * idt[s];
+      e = eps;
+      alpha = (-6.0 + 6.0 * dt - 3.0 * dt2 + dt3 + 6.0 * eps) * i3;
+      beta = (6.0 + (-6.0 - dt * (6.0 + dt * (3.0 + dt))) * eps) * i3;
+      gamma = 3.0 * (6.0 + (-4.0 + dt) * dt - 2.0 * (3.0 + dt) * eps) * i3;
+      theta = 3.0 * (eps * (6.0 + dt2 + 4.0 * dt) + 2.0 * dt - 6.0) * i3;
+    } else {
+      const double dt4 = dt2 * dt2;
+      e = 1.0 - dt + 0.5 * dt2 - dt3 * (1.0 / 6.0) + dt4 * (1.0 / 24.0);
+      alpha = 0.25 * dt - 0.05 * dt2 + dt3 * (1.0 / 120.0) - dt4 * (1.0 / 840.0);
+      beta = 0.25 * dt - 0.20 * dt2 + dt3 * (1.0 / 12.0) - dt4 * (1.0 / 42.0);
+      gamma = 0.25 * dt - 0.10 * dt2 + dt3 * 0.025 - dt4 * (1.0 / 210.0);
+      theta = 0.25 * dt - 0.15 * dt2 + dt3 * 0.05 - dt4 * (1.0 / 84.0);
+    }
+    const double d3 = dt * (1.0 / 3.0);
+    E[s] = e;
+    b[s] = alpha * S[s] + beta * Sm + gamma * max0(S[s] - d3 * dS[s]) + theta * max0(Sm + d3 * dSm);
+    Psi[s] = alpha + gamma;
+    if (last) {
+      // w3, rh/w3.c:44-63
+      const bool thin = dt < 5.0E-4, thick = dt > 50.0;
+      const double w0 = thin ? dt * (1.0 - 0.5 * dt) : thick ? 1.0 : 1.0 - eps;
+      const double w1 = thin ? dt2 * (0.5 - dt / 3.0) : thick ? 1.0 : w0 - dt * eps;
+      const double w1t = ndiv(w1, dt);
+      E[s] = 1.0 - w0;
+      b[s] = w0 * S[s] - w1t * (S[s] - Sm);
+      Psi[s] = w0 - w1t;
+    }
+    if (t == 0) {
+      const double C1 = P > 1 ? C[P > 1 ? 1 : 0] : C_next;
+      const double d0 = 0.5 * zmu * (C[s] + C1) * g.dz[s];   // dz[0] holds the first interval
+      E[s] = 0.0;
+      b[s] = outward ? B2_1 - ndiv(B2_0 - B2_1, d0) : 0.0;
+      Psi[s] = 0.0;
+    }
+  }
+  // the lane's points composed, an inclusive scan over the lanes, then the
+  // points from the previous lane's intensity (E = 0 at t = 0, so the
+  // composed offset is the intensity itself)
+  double LE = E[0], Lb = b[0];
+#pragma unroll
+  for (int s = 1; s < P; s++) {
+    Lb = fma(E[s], Lb, b[s]);
+    LE *= E[s];
+  }
+#define RAY_SCAN(CTRL, ROWS)                                                              \
+  {                                                                                       \
+    const double pe = dpp<CTRL, ROWS>(1.0, LE), pb = dpp<CTRL, ROWS>(0.0, Lb);            \
+    Lb = fma(LE, pb, Lb);                                                                 \
+    LE *= pe;                                                                             \
+  }
+  RAY_SCAN(0x111, 0xf)   // row_shr:1
+  RAY_SCAN(0x112, 0xf)   // row_shr:2
+  RAY_SCAN(0x114, 0xf)   // row_shr:4
+  RAY_SCAN(0x118, 0xf)   // row_shr:8
+  RAY_SCAN(0x142, 0xa)   // row_bcast:15 into rows 1 and 3
+  if constexpr (L == 64) RAY_SCAN(0x143, 0xc)   // row_bcast:31 into rows 2 and 3
+#undef RAY_SCAN
+  double Iu = from_prev(Lb);
+#pragma unroll
+  for (int s = 0; s < P; s++) {
+    Iu = t0 + s == 0 ? b[s] : fma(E[s], Iu, b[s]);
+    I[s] = Iu;
+  }
+}
+
+// the lane's points: depths, paths and interval weights (points
+// past the last stand at the last depth and are never read)
+template <int P>
+__device__ __forceinline__ void ray_points(const NlteBufs &B, int64_t col, int t0, int N,
+                                           bool outward, int (&k)[P], RayPath<P> &g) {
+#pragma clang fp contract(fast)
+#pragma unroll
+  for (int s = 0; s < P; s++) {
+    const int t = t0 + s < N ? t0 + s : N - 1, tu = t > 0 ? t : 1;
+    k[s] = outward ? N - 1 - t : t;
+    // the interval between t - 1 and t (at t = 0: between 0 and 1)
+    g.dz[s] = B.geo[NG_DZ * B.fs + col + (outward ? N - tu : tu)];
+    g.idz[s] = nrcp(g.dz[s]);
+  }
+  const double dz_next = from_next(g.dz[0]);
+#pragma unroll
+  for (int s = 0; s < P; s++) {
+    const double dn = s < P - 1 ? g.dz[s < P - 1 ? s + 1 : s] : dz_next;
+    g.al[s] = 0.333333333333333333333333 * (1.0 + dn * nrcp(dn + g.dz[s]));
+  }
+}
+
+// Workgroup -> (slot of the active columns, entry of the wavelength list): the
+// wavelengths of a column on one XCD (xcd_tile), or, with fewer columns than
+// XCDs, over all of them.
+__device__ __forceinline__ bool nlte_tile(int nact, int nlist, int &slot, int &il) {
+  if (nact >= NXCD) {
+    xcd_tile(blockIdx.x, nlist, slot, il);
+    return slot < nact;
+  }
+  slot = (int) (blockIdx.x / nlist);
+  il = (int) (blockIdx.x % nlist);
+  return slot < nact;
+}
+
+// Wavelengths with an active line, one (column, wavelength) per workgroup of
+// 2 L threads:
+// the rays in both directions, the new mean intensity and with eval_op the
+// radiative rate terms (rh/rhf1d/formal.c:44-346, rh/fillgamma.c:82-332),
+// summed over the rays in registers; the outward lanes' sums are turned to
+// the inward lanes' depths through LDS at the end (N doubles).  J is
+// double-buffered per column (jpar): the previous J enters the source
+// function, the new one is built.
+// Measured on a pass over 465 such wavelengths: one column 26 us (5.3 ms with
+// a lane per column: all its wavefronts on one XCD, one lane of each), 1500
+// columns of 82 depths 9.9 ms (16.5): 3.76e9 vector instructions, 65% of the
+// SIMDs' cycles, the rest waits of the two wavefronts that the registers
+// allow.  P = 3 at 32 lanes per direction covers 82 depths with 85% of the
+// lanes.
+template <int L, int P, int MS>
+__global__ void __launch_bounds__(2 * L, (P <= 3 && MS <= 2 ? 2 : 1))
 k_nlte_bezier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap, NlteBufs B,
               const int32_t *__restrict__ act, int nact, const int32_t *__restrict__ out_ls,
-              const int32_t *__restrict__ io_list, int nlist, int il_off, int eval_op) {
+              const int32_t *__restrict__ io_list, int nlist, int il_off, int nlist_all,
+              int eval_op) {
+#pragma clang fp contract(fast)
+  extern __shared__ double turn[];
   const DevModel &M = *Mp;
   const DevNlte &A = *Ap;
-  const int ncb = (nact + 63) / 64;
-  int cb, il;
-  xcd_tile(blockIdx.x, nlist, cb, il);
-  if (cb >= ncb) return;
-  const int slot = cb * 64 + threadIdx.x;
-  if (slot >= nact) return;
+  int slot, il;
+  if (!nlte_tile(nact, nlist, slot, il)) return;
   const int ic = act[slot], io = io_list[il], ls = out_ls[io];
-  const int ncol = B.ncol, Nmax = B.Nmax, N = B.ndep[ic], nrays = A.nrays;
-  const int64_t fs = (int64_t) Nmax * ncol;
-#define STF(f, k) B.state[(int64_t) (f) * fs + (int64_t) (k) * ncol + ic]
-#define PK(k) ((int64_t) (k) * ncol + ic)
-  const int64_t wo = (int64_t) io * fs, jb = (int64_t) B.nout * fs;
+  const int N = B.ndep[ic], nrays = A.nrays;
+  const int64_t fs = B.fs, col = (int64_t) ic * B.Kp;
+  const int64_t wo = (int64_t) io * fs + col, jb = (int64_t) B.nout * fs;
   const int par = B.jpar[ic];
   const double *Jold = B.J + par * jb + wo;
   double *Jnew = B.J + (1 - par) * jb + wo;
-  const double *chic = B.cchi + wo, *etac = B.ceta + wo, *scac = B.csca + wo;
   const double lam = ldc(M.lamconst)[(int64_t) ls * RHG_LC_NCONST + RHG_LC_LAMBDA];
-  const double hc_k = HC / (KBOLTZMANN * NM_TO_M);
   SetInfo<MS> si;
   set_info<MS>(A, ls, lam, si);
-  const double B2_0 = planck_lam(STF(RHG_CF_T, N - 2), lam);
-  const double B2_1 = planck_lam(STF(RHG_CF_T, N - 1), lam);
-  double dJmax = 0.0;
-
-  // member data at depth k
-  auto depth = [&](int k, SetDepth<MS> &sd) {
-    const double T = STF(RHG_CF_T, k);
+  const bool outward = threadIdx.x >= L;
+  const int t0 = (int) (threadIdx.x & (L - 1)) * P;
+  const double *Tc = B.geo + NG_T * fs + col;
+  const double B2_0 = planck_lam(Tc[N - 2], lam), B2_1 = planck_lam(Tc[N - 1], lam);
+  int k[P];
+  RayPath<P> g;
+  ray_points<P>(B, col, t0, N, outward, k, g);
+  SetDepth<MS> sd[P];
+  double cc[P], s0[P], js[P], sIJ[P][MS], sJI[P][MS];
 #pragma unroll
-    for (int n = 0; n < MS; n++) {
-      sd.ni[n] = sd.nj[n] = sd.gij[n] = sd.wla[n] = 0.0;
-      if (n < si.n) {
-        sd.ni[n] = B.pops[(int64_t) si.ti[n] * fs + PK(k)];
-        sd.nj[n] = B.pops[(int64_t) si.tj[n] * fs + PK(k)];
-        if (si.line[n] >= 0) {
-          sd.gij[n] = si.gline[n];
-          sd.wla[n] = si.wlam[n] * B.wphi[(int64_t) si.line[n] * fs + PK(k)] / HC_4PI;
-        } else {
-          sd.gij[n] = B.nstar[(int64_t) si.ti[n] * fs + PK(k)] /
-                      B.nstar[(int64_t) si.tj[n] * fs + PK(k)] * exp(-hc_k / (lam * T));
-          sd.wla[n] = FOURPI / HPLANCK * (si.wlam[n] / lam);
+  for (int s = 0; s < P; s++) {
+    set_depth<MS>(B, si, col + k[s], Tc[k[s]], lam, sd[s]);
+    cc[s] = B.cchi[wo + k[s]];
+    s0[s] = fma(B.csca[wo + k[s]], Jold[k[s]], B.ceta[wo + k[s]]);
+    js[s] = 0.0;
+#pragma unroll
+    for (int n = 0; n < MS; n++) sIJ[s][n] = sJI[s][n] = 0.0;
+  }
+  const int dir = outward ? 1 : 0;
+  for (int mu = 0; mu < nrays; mu++) {
+    const double zmu = 1.0 / A.muz[mu], wmu = 0.5 * A.wmu[mu];
+    double V[P][MS], C[P], S[P], iC[P], I[P], Psi[P];
+#pragma unroll
+    for (int s = 0; s < P; s++) {
+      double chi = 0.0, eta = 0.0;
+#pragma unroll
+      for (int n = 0; n < MS; n++) {
+        V[s][n] = 0.0;
+        if (n < si.n) {
+          V[s][n] = si.line[n] >= 0
+                        ? si.cV[n] * B.phi[((int64_t) (si.prow[n] + mu) * 2 + dir) * fs + col + k[s]]
+                        : si.alpha[n];
+          chi += V[s][n] * sd[s].x[n];
+          eta += V[s][n] * sd[s].e[n];
         }
       }
+      C[s] = chi + cc[s];
+      iC[s] = nrcp(C[s]);
+      S[s] = (eta + s0[s]) * iC[s];
     }
-  };
-  // absorption per population of each member for ray mu, direction dir
-  auto absorb = [&](int k, int mu, int dir, double (&V)[MS]) {
+    ray_sweep<L, P>(g, t0, N, outward, zmu, B2_0, B2_1, C, S, I, Psi);
 #pragma unroll
-    for (int n = 0; n < MS; n++) {
-      V[n] = 0.0;
-      if (n < si.n) {
-        if (si.line[n] >= 0)
-          V[n] = si.cV[n] *
-                 B.phi[(((int64_t) (si.prow[n] + mu) * 2 + dir) * Nmax) * ncol + PK(k)];
-        else
-          V[n] = si.alpha[n];
-      }
-    }
-  };
-
-  for (int c0 = 0; c0 < nrays; c0 += RB) {
-    const int nrc = nrays - c0 < RB ? nrays - c0 : RB;
-    const bool last_chunk = c0 + RB >= nrays;
-    double zmu[RB], wmu[RB];
-#pragma unroll
-    for (int r = 0; r < RB; r++) {
-      zmu[r] = 1.0;
-      wmu[r] = 0.0;
-      if (r < nrc) {
-        zmu[r] = 1.0 / A.muz[c0 + r];
-        wmu[r] = 0.5 * A.wmu[c0 + r];
-      }
-    }
-    for (int dir = 0; dir <= 1; dir++) {
-      const bool first = (c0 == 0 && dir == 0);
-      // opacity and source function of the rays at depth k
-      auto opac = [&](int k, double (&C)[RB], double (&S)[RB]) {
-        SetDepth<MS> sd;
-        depth(k, sd);
-        const double cc = chic[PK(k)], ee = etac[PK(k)], ss = scac[PK(k)], jd = Jold[PK(k)];
-#pragma unroll
-        for (int r = 0; r < RB; r++) {
-          C[r] = 1.0;
-          S[r] = 0.0;
-          if (r < nrc) {
-            double V[MS];
-            absorb(k, c0 + r, dir, V);
-            double chi = 0.0, eta = 0.0;
-#pragma unroll
-            for (int n = 0; n < MS; n++) {
-              if (n < si.n) {
-                chi += V[n] * (sd.ni[n] - sd.gij[n] * sd.nj[n]);
-                eta += si.tw[n] * sd.gij[n] * V[n] * sd.nj[n];
-              }
-            }
-            C[r] = chi + cc;
-            double s = eta + ee;
-            s += ss * jd;
-            S[r] = ndiv(s, C[r]);
-          }
-        }
-      };
-      // J and rate terms of depth k
-      auto emit = [&](int k, const double (&I)[RB], const double (&Psi)[RB],
-                      const double (&C)[RB]) {
-        double js = 0.0;
-#pragma unroll
-        for (int r = 0; r < RB; r++)
-          if (r < nrc) js += wmu[r] * I[r];
-        double *jp = Jnew + PK(k);
-        const double jn = first ? js : *jp + js;
-        *jp = jn;
-        if (last_chunk && dir == 1) {
-          const double dJ = fabs(1.0 - Jold[PK(k)] / jn);
-          dJmax = dJmax > dJ ? dJmax : dJ;
-        }
-        if (!eval_op) return;
-        SetDepth<MS> sd;
-        depth(k, sd);
-        double sIJ[MS], sJI[MS];
-#pragma unroll
-        for (int n = 0; n < MS; n++) sIJ[n] = sJI[n] = 0.0;
-#pragma unroll
-        for (int r = 0; r < RB; r++) {
-          if (r < nrc) {
-            double V[MS];
-            absorb(k, c0 + r, dir, V);
-            rate_terms<MS>(si, sd, V, I[r], ndiv(Psi[r], C[r]), wmu[r], sIJ, sJI);
-          }
-        }
-#pragma unroll
-        for (int n = 0; n < MS; n++) {
-          if (n < si.n) {
-            double *aij = B.acc + ((int64_t) si.ent[n] * 2) * fs + PK(k);
-            double *aji = aij + fs;
-            *aij = first ? sIJ[n] : *aij + sIJ[n];
-            *aji = first ? sJI[n] : *aji + sJI[n];
-          }
-        }
-      };
-      // |z[a] - z[b]| for neighbouring depths
-      auto dzb = [&](int a, int b) { return STF(RHG_CF_DZ, a > b ? a : b); };
-      const int dk = dir ? -1 : 1, ks = dir ? N - 1 : 0, ke = dir ? 0 : N - 1;
-      double Cm[RB], C0[RB], Cp[RB], Cn[RB], Sm[RB], S0[RB], Sp[RB], Sn[RB];
-      double I_upw[RB], dchi_c[RB], dtau_uw[RB], dS_up[RB], I[RB], Psi[RB];
-      opac(ks, Cm, Sm);
-      opac(ks + dk, C0, S0);
-      opac(ks + 2 * dk, Cp, Sp);
-      {
-        const double dz0 = dzb(ks, ks + dk);
-#pragma unroll
-        for (int r = 0; r < RB; r++) {
-          const double dt = 0.5 * zmu[r] * (Cm[r] + C0[r]) * dz0;
-          I_upw[r] = dir ? B2_1 - (B2_0 - B2_1) / dt : 0.0;
-          Psi[r] = 0.0;
-        }
-        emit(ks, I_upw, Psi, Cm);
-        const int k = ks + dk;
-        const double dzu = dzb(k, k - dk), dzd = dzb(k + dk, k);
-#pragma unroll
-        for (int r = 0; r < RB; r++) {
-          const double dsup = dzu * zmu[r], dsdn = dzd * zmu[r];
-          const double dchi_up = ndiv(C0[r] - Cm[r], dsup);
-          dchi_c[r] = cent_div(dsup, dsdn, Cm[r], C0[r], Cp[r]);
-          const double c1 = max0(C0[r] - (dsup * (1.0 / 3.0)) * dchi_c[r]);
-          const double c2 = max0(Cm[r] + (dsup * (1.0 / 3.0)) * dchi_up);
-          dtau_uw[r] = dsup * (C0[r] + Cm[r] + c1 + c2) * 0.25;
-          dS_up[r] = ndiv(S0[r] - Sm[r], dtau_uw[r]);
-        }
-      }
-      for (int k = ks + dk; k != ke + dk; k += dk) {
-        if (k != ke) {
-          const double dzd = dzb(k + dk, k);
-          const bool far = abs(k - ke) > 1;
-          double dzd2 = 0.0;
-          if (far) {
-            opac(k + 2 * dk, Cn, Sn);
-            dzd2 = dzb(k + 2 * dk, k + dk);
-          } else {
-#pragma unroll
-            for (int r = 0; r < RB; r++) {
-              Cn[r] = 1.0;
-              Sn[r] = 0.0;
-            }
-          }
-#pragma unroll
-          for (int r = 0; r < RB; r++) {
-            const double dsdn = dzd * zmu[r];
-            const double dchi_dn = far ? cent_div(dsdn, dzd2 * zmu[r], C0[r], Cp[r], Cn[r])
-                                       : ndiv(Cp[r] - C0[r], dsdn);
-            double c1 = max0(C0[r] + (dsdn * (1.0 / 3.0)) * dchi_c[r]);
-            double c2 = max0(Cp[r] - (dsdn * (1.0 / 3.0)) * dchi_dn);
-            const double dtau_dw = dsdn * (C0[r] + Cp[r] + c1 + c2) * 0.25;
-            const double dt03 = dtau_uw[r] * (1.0 / 3.0);
-            double alpha, beta, gamma, theta, eps;
-            bezier3_coeffs(dtau_uw[r], alpha, beta, gamma, theta, eps);
-            const double dS_c = cent_div(dtau_uw[r], dtau_dw, Sm[r], S0[r], Sp[r]);
-            c1 = max0(S0[r] - dt03 * dS_c);
-            c2 = max0(Sm[r] + dt03 * dS_up[r]);
-            I[r] = I_upw[r] * eps + alpha * S0[r] + beta * Sm[r] + gamma * c1 + theta * c2;
-            Psi[r] = alpha + gamma;
-            I_upw[r] = I[r];
-            dchi_c[r] = dchi_dn;
-            dtau_uw[r] = dtau_dw;
-            dS_up[r] = dS_c;
-          }
-        } else {
-          const double dzu = dzb(k, k - dk);
-#pragma unroll
-          for (int r = 0; r < RB; r++) {
-            const double dt = 0.5 * zmu[r] * (C0[r] + Cm[r]) * dzu;
-            const double dS_uw = -(S0[r] - Sm[r]) / dt;
-            double w[3];
-            w3(dt, w);
-            I[r] = (1.0 - w[0]) * I_upw[r] + w[0] * S0[r] + w[1] * dS_uw;
-            Psi[r] = w[0] - w[1] / dt;
-          }
-        }
-        emit(k, I, Psi, C0);
-#pragma unroll
-        for (int r = 0; r < RB; r++) {
-          Cm[r] = C0[r];
-          C0[r] = Cp[r];
-          Cp[r] = Cn[r];
-          Sm[r] = S0[r];
-          S0[r] = Sp[r];
-          Sp[r] = Sn[r];
-        }
-      }
+    for (int s = 0; s < P; s++) {
+      js[s] += wmu * I[s];
+      if (eval_op) rate_terms<MS>(si, sd[s], V[s], I[s], Psi[s] * iC[s], wmu, sIJ[s], sJI[s]);
     }
   }
-  B.dJ[(int64_t) (il_off + il) * ncol + ic] = dJmax;
-#undef STF
-#undef PK
+  // the inward lanes add the outward lanes' sum at each of their depths
+  auto both = [&](int s, double x) -> double { return x + turn[k[s]]; };
+  auto put = [&](auto &&value) {
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < P; s++)
+      if (outward && t0 + s < N) turn[k[s]] = value(s);
+    __syncthreads();
+  };
+  put([&](int s) { return js[s]; });
+  double dJmax = 0.0;
+#pragma unroll
+  for (int s = 0; s < P; s++) {
+    if (!outward && t0 + s < N) {
+      const double jn = both(s, js[s]), dJ = fabs(1.0 - Jold[k[s]] / jn);
+      Jnew[k[s]] = jn;
+      dJmax = dJmax > dJ ? dJmax : dJ;
+    }
+  }
+  for (int o = L / 2; o >= 1; o >>= 1) {
+    const double x = __shfl_xor(dJmax, o);
+    dJmax = dJmax > x ? dJmax : x;
+  }
+  if (threadIdx.x == 0) B.dJ[(int64_t) ic * nlist_all + il_off + il] = dJmax;
+  if (!eval_op) return;
+#pragma unroll
+  for (int n = 0; n < MS; n++) {
+    if (n < si.n) {
+      double *aij = B.acc + ((int64_t) si.ent[n] * 2) * fs + col;
+      put([&](int s) { return sIJ[s][n]; });
+#pragma unroll
+      for (int s = 0; s < P; s++)
+        if (!outward && t0 + s < N) aij[k[s]] = both(s, sIJ[s][n]);
+      put([&](int s) { return sJI[s][n]; });
+#pragma unroll
+      for (int s = 0; s < P; s++)
+        if (!outward && t0 + s < N) aij[fs + k[s]] = both(s, sJI[s][n]);
+    }
+  }
 }
 
-#define RHG_INST_BEZ(MS)                                                                        \
-  template __global__ void k_nlte_bezier<NLTE_RB, MS>(const DevModel *, const DevNlte *, NlteBufs, \
-                                                      const int32_t *, int, const int32_t *,     \
-                                                      const int32_t *, int, int, int);
-RHG_INST_BEZ(2)
-RHG_INST_BEZ(4)
-RHG_INST_BEZ(8)
+#define RHG_INST_BEZ(L, P, MS)                                                                  \
+  template __global__ void k_nlte_bezier<L, P, MS>(const DevModel *, const DevNlte *, NlteBufs,  \
+                                                   const int32_t *, int, const int32_t *,        \
+                                                   const int32_t *, int, int, int, int);
+#define RHG_INST_BEZ_MS(L, P) RHG_INST_BEZ(L, P, 2) RHG_INST_BEZ(L, P, 4) RHG_INST_BEZ(L, P, 8)
+RHG_INST_BEZ_MS(32, 2)
+RHG_INST_BEZ_MS(32, 3)
+RHG_INST_BEZ_MS(64, 2)
+RHG_INST_BEZ_MS(64, 3)
+RHG_INST_BEZ_MS(64, 4)
+RHG_INST_BEZ_MS(64, 8)
+#undef RHG_INST_BEZ_MS
 #undef RHG_INST_BEZ
 
-// ---------------------------------------------------------------------------
-// Wavelengths with continua only, one (column, wavelength) per thread: one
-// opacity for all rays, and per ray the Feautrier solution with its
-// two-sided diagonal operator (rh/rhf1d/feautrier.c:56-202; P is the mean
-// of the two directions, weighted by the full ray weight).  The opacity,
-// source function and the elimination coefficients F and z of each ray
-// live in the thread's scratch rows; the back substitution runs the rays of
-// a chunk together and adds the rate terms of each depth as it reaches it.
-// MS is the largest active set among the wavelengths of io_list (the member
-// loops are unrolled to it).
-template <int MS>
-__global__ void __launch_bounds__(64)
-k_nlte_feautrier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap, NlteBufs B,
-                 const int32_t *__restrict__ act, int nact, const int32_t *__restrict__ out_ls,
-                 const int32_t *__restrict__ io_list, int nlist, int il_off, int eval_op) {
-  const DevModel &M = *Mp;
-  const DevNlte &A = *Ap;
-  const int ncb = (nact + 63) / 64;
-  int cb, il;
-  xcd_tile(blockIdx.x, nlist, cb, il);
-  if (cb >= ncb) return;
-  const int slot = cb * 64 + threadIdx.x;
-  if (slot >= nact) return;
-  const int ic = act[slot], io = io_list[il], ls = out_ls[io];
-  const int ncol = B.ncol, Nmax = B.Nmax, N = B.ndep[ic], nrays = A.nrays;
-  const int64_t fs = (int64_t) Nmax * ncol;
-  const int64_t nthr = (int64_t) nlist * ncb * 64;
-  double *scr = B.scr + (int64_t) il * ncb * 64 + slot;
-#define SCR(s, k) scr[((int64_t) (s) * Nmax + (k)) * nthr]
-#define STF(f, k) B.state[(int64_t) (f) * fs + (int64_t) (k) * ncol + ic]
-#define PK(k) ((int64_t) (k) * ncol + ic)
-  const int64_t wo = (int64_t) io * fs, jb = (int64_t) B.nout * fs;
-  const int par = B.jpar[ic];
-  const double *Jold = B.J + par * jb + wo;
-  double *Jnew = B.J + (1 - par) * jb + wo;
-  const double *chic = B.cchi + wo, *etac = B.ceta + wo, *scac = B.csca + wo;
-  const double lam = ldc(M.lamconst)[(int64_t) ls * RHG_LC_NCONST + RHG_LC_LAMBDA];
-  const double hc_k = HC / (KBOLTZMANN * NM_TO_M);
-  SetInfo<MS> si;
-  set_info<MS>(A, ls, lam, si);
-
-  auto depth = [&](int k, SetDepth<MS> &sd, double (&V)[MS]) {
-    const double T = STF(RHG_CF_T, k);
+// The member data of one depth at mu of the final ray: opacity and emission
+// of the active set (Armstrong profiles as the set-up's).
+__device__ __forceinline__ void emergent_set(const NlteBufs &B, const DevNlte &A,
+                                             const SetInfo<NLTE_MAXSET> &si, int64_t pk, double lam,
+                                             double mu, double &chi, double &eta) {
+  const int64_t fs = B.fs;
+  const double T = B.geo[NG_T * fs + pk], vb = B.vbroad[pk], vz = B.geo[NG_VLOS * fs + pk];
+  SetDepth<NLTE_MAXSET> sd;
+  set_depth<NLTE_MAXSET>(B, si, pk, T, lam, sd);
+  chi = eta = 0.0;
 #pragma unroll
-    for (int n = 0; n < MS; n++) {
-      sd.ni[n] = sd.nj[n] = sd.gij[n] = sd.wla[n] = V[n] = 0.0;
-      if (n < si.n) {
-        sd.ni[n] = B.pops[(int64_t) si.ti[n] * fs + PK(k)];
-        sd.nj[n] = B.pops[(int64_t) si.tj[n] * fs + PK(k)];
-        if (si.line[n] >= 0) {
-          // a line at a Feautrier wavelength (not produced by the set-up):
-          // its profile of the first ray
-          sd.gij[n] = si.gline[n];
-          sd.wla[n] = si.wlam[n] * B.wphi[(int64_t) si.line[n] * fs + PK(k)] / HC_4PI;
-          V[n] = si.cV[n] * B.phi[(((int64_t) si.prow[n] * 2) * Nmax) * ncol + PK(k)];
-        } else {
-          sd.gij[n] = B.nstar[(int64_t) si.ti[n] * fs + PK(k)] /
-                      B.nstar[(int64_t) si.tj[n] * fs + PK(k)] * exp(-hc_k / (lam * T));
-          sd.wla[n] = FOURPI / HPLANCK * (si.wlam[n] / lam);
-          V[n] = si.alpha[n];
-        }
+  for (int n = 0; n < NLTE_MAXSET; n++) {
+    if (n < si.n) {
+      double V = si.alpha[n];
+      if (si.line[n] >= 0) {
+        const int l = si.line[n];
+        const double lambda0 = A.ln_lambda0[l];
+        const double v = (lam - lambda0 - 0.0) * CLIGHT / (vb * lambda0);
+        const double vlos = mu * vz / vb;
+        V = si.cV[n] * (voigt_armstrong(B.adamp[(int64_t) l * fs + pk], v + 1.0 * vlos) * 1.0 /
+                        (SQRTPI * vb));
       }
+      chi += V * sd.x[n];
+      eta += V * sd.e[n];
     }
-  };
-
-  for (int k = 0; k < N; k++) {
-    SetDepth<MS> sd;
-    double V[MS];
-    depth(k, sd, V);
-    double chi = 0.0, eta = 0.0;
-#pragma unroll
-    for (int n = 0; n < MS; n++) {
-      if (n < si.n) {
-        chi += V[n] * (sd.ni[n] - sd.gij[n] * sd.nj[n]);
-        eta += si.tw[n] * sd.gij[n] * V[n] * sd.nj[n];
-      }
-    }
-    const double chi_t = chi + chic[PK(k)];
-    double S = eta + etac[PK(k)];
-    S += scac[PK(k)] * Jold[PK(k)];
-    SCR(NS_CHI, k) = chi_t;
-    SCR(NS_S, k) = S / chi_t;
   }
-  const double B2_0 = planck_lam(STF(RHG_CF_T, N - 2), lam);
-  const double B2_1 = planck_lam(STF(RHG_CF_T, N - 1), lam);
-#define CHI(k) SCR(NS_CHI, k)
-#define SRC(k) SCR(NS_S, k)
-#define HGT(k) STF(RHG_CF_HEIGHT, k)
-  // The rays in chunks of up to RF: each ray's forward elimination into its
-  // own F and z rows, then the back substitution of the chunk's rays
-  // together, so that each depth forms the member data once and updates J
-  // and the rate sums once per chunk.  The rays are summed in ray order, as
-  // one ray at a time would sum them.
-  constexpr int RF = NLTE_FE_RAYS;
-  for (int c0 = 0; c0 < nrays; c0 += RF) {
-    const int nrc = nrays - c0 < RF ? nrays - c0 : RF;
-    double wmu[RF], zmu[RF];
-#pragma unroll
-    for (int r = 0; r < RF; r++) {
-      wmu[r] = r < nrc ? A.wmu[c0 + r] : 0.0;
-      zmu[r] = r < nrc ? 0.5 / A.muz[c0 + r] : 1.0;
-    }
-    auto emit = [&](int k, const double (&P)[RF], const double (&Psi)[RF]) {
-      double *jp = Jnew + PK(k);
-      double j = c0 == 0 ? 0.0 : *jp;
-#pragma unroll
-      for (int r = 0; r < RF; r++)
-        if (r < nrc) j = (c0 + r == 0 ? 0.0 : j) + P[r] * wmu[r];
-      *jp = j;
-      if (!eval_op) return;
-      SetDepth<MS> sd;
-      double V[MS], aIJ[MS], aJI[MS];
-      depth(k, sd, V);
-#pragma unroll
-      for (int n = 0; n < MS; n++) {
-        aIJ[n] = aJI[n] = 0.0;
-        if (n < si.n && c0 > 0) {
-          const double *aij = B.acc + ((int64_t) si.ent[n] * 2) * fs + PK(k);
-          aIJ[n] = aij[0];
-          aJI[n] = aij[fs];
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < RF; r++) {
-        if (r < nrc) {
-          double sIJ[MS], sJI[MS];
-#pragma unroll
-          for (int n = 0; n < MS; n++) sIJ[n] = sJI[n] = 0.0;
-          rate_terms<MS>(si, sd, V, P[r], Psi[r] / CHI(k), wmu[r], sIJ, sJI);
-#pragma unroll
-          for (int n = 0; n < MS; n++) {
-            aIJ[n] = (c0 + r == 0 ? 0.0 : aIJ[n]) + sIJ[n];
-            aJI[n] = (c0 + r == 0 ? 0.0 : aJI[n]) + sJI[n];
-          }
-        }
-      }
-#pragma unroll
-      for (int n = 0; n < MS; n++) {
-        if (n < si.n) {
-          double *aij = B.acc + ((int64_t) si.ent[n] * 2) * fs + PK(k);
-          aij[0] = aIJ[n];
-          aij[fs] = aJI[n];
-        }
-      }
-    };
-    auto dtau = [&](int r, int k) {
-      return zmu[r] * (CHI(k) + CHI(k + 1)) * (HGT(k) - HGT(k + 1));
-    };
-    // forward elimination, rh/rhf1d/feautrier.c:56-202 (dark top,
-    // thermalised bottom, STANDARD order), ray r into rows NS_F + 2 r and
-    // NS_Z + 2 r
-    double F[RF], z[RF], dtm1[RF], abc0[RF], C1_0[RF];
-#pragma unroll
-    for (int r = 0; r < RF; r++) {
-      if (r < nrc) {
-        const double dt0 = dtau(r, 0);
-        abc0[r] = 1.0 + 2.0 * 1.0 / dt0;
-        C1_0[r] = 2.0 / (dt0 * dt0);
-        const double S0 = SRC(0) + 2.0 * 0.0 / ((1.0 + 0.0) * dt0);
-        F[r] = abc0[r] / C1_0[r];
-        z[r] = S0 / (abc0[r] + C1_0[r]);
-        SCR(NS_F + 2 * r, 0) = F[r];
-        SCR(NS_Z + 2 * r, 0) = z[r];
-        dtm1[r] = dt0;
-      }
-    }
-    for (int k = 1; k < N - 1; k++) {
-#pragma unroll
-      for (int r = 0; r < RF; r++) {
-        if (r < nrc) {
-          const double dtk = dtau(r, k);
-          const double dtau_mid = 0.5 * (dtk + dtm1[r]);
-          const double A1 = 1.0 / (dtau_mid * dtm1[r]), C1 = 1.0 / (dtau_mid * dtk);
-          F[r] = (1.0 + A1 * F[r] / (1.0 + F[r])) / C1;
-          z[r] = (SRC(k) + A1 * z[r]) / (C1 * (1.0 + F[r]));
-          SCR(NS_F + 2 * r, k) = F[r];
-          SCR(NS_Z + 2 * r, k) = z[r];
-          dtm1[r] = dtk;
-        }
-      }
-    }
-    // back substitution with the two-sided operator
-    double P[RF], Psi[RF], G[RF], dtk[RF];
-#pragma unroll
-    for (int r = 0; r < RF; r++) {
-      P[r] = Psi[r] = G[r] = 0.0;
-      dtk[r] = 1.0;
-      if (r < nrc) {
-        const double dtN = dtm1[r];   // dtau[N-2]
-        const double hN = B2_1 - (B2_0 - B2_1) / dtN;
-        const double abcN = 1.0 + 2.0 * 1.0 / dtN;
-        const double A1N = 2.0 / (dtN * dtN);
-        const double SN = SRC(N - 1) + 2.0 * hN / ((1.0 + 0.0) * dtN);
-        const double FN2 = SCR(NS_F + 2 * r, N - 2);
-        P[r] = (SN + A1N * SCR(NS_Z + 2 * r, N - 2)) / (abcN + A1N * (FN2 / (1.0 + FN2)));
-        Psi[r] = 1.0 / (abcN + A1N * FN2 / (1.0 + FN2));
-        G[r] = abcN / A1N;   // G[N-1]
-        dtk[r] = dtN;        // dtau[k] for k = N-2
-      }
-    }
-    emit(N - 1, P, Psi);
-    for (int k = N - 2; k >= 1; k--) {
-#pragma unroll
-      for (int r = 0; r < RF; r++) {
-        if (r < nrc) {
-          const double Fk = SCR(NS_F + 2 * r, k), Fm = SCR(NS_F + 2 * r, k - 1);
-          P[r] = P[r] / (1.0 + Fk) + SCR(NS_Z + 2 * r, k);
-          const double dtkm = dtau(r, k - 1);
-          const double dtau_mid = 0.5 * (dtk[r] + dtkm);
-          const double A1 = 1.0 / (dtau_mid * dtkm), C1 = 1.0 / (dtau_mid * dtk[r]);
-          Psi[r] = 1.0 / (1.0 + A1 * Fm / (1.0 + Fm) + C1 * G[r] / (1.0 + G[r]));
-          G[r] = (1.0 + C1 * G[r] / (1.0 + G[r])) / A1;
-          dtk[r] = dtkm;
-        }
-      }
-      emit(k, P, Psi);
-    }
-#pragma unroll
-    for (int r = 0; r < RF; r++) {
-      if (r < nrc) {
-        P[r] = P[r] / (1.0 + SCR(NS_F + 2 * r, 0)) + SCR(NS_Z + 2 * r, 0);
-        Psi[r] = 1.0 / (abc0[r] + C1_0[r] * G[r] / (1.0 + G[r]));
-      }
-    }
-    emit(0, P, Psi);
-  }
-  double dJmax = 0.0;
-  for (int k = 0; k < N; k++) {
-    const double dJ = fabs(1.0 - Jold[PK(k)] / Jnew[PK(k)]);
-    dJmax = dJmax > dJ ? dJmax : dJ;
-  }
-  B.dJ[(int64_t) (il_off + il) * ncol + ic] = dJmax;
-#undef HGT
-#undef CHI
-#undef SRC
-#undef SCR
-#undef STF
-#undef PK
 }
-#define RHG_INST_FE(MS)                                                                          \
-  template __global__ void k_nlte_feautrier<MS>(const DevModel *, const DevNlte *, NlteBufs,     \
-                                                const int32_t *, int, const int32_t *,           \
-                                                const int32_t *, int, int, int);
-RHG_INST_FE(2)
-RHG_INST_FE(4)
-RHG_INST_FE(6)
-RHG_INST_FE(8)
-#undef RHG_INST_FE
 
-// ---------------------------------------------------------------------------
 // The emergent spectrum after convergence, pyrh's final ray
-// (rh/rhf1d/pyrh_solveray.c:82-107): one ray at the caller's mu with the
-// converged populations, profiles for that ray (Armstrong, as the set-up's),
-// background scattering from the last J, no update of J.  One (column,
-// output wavelength) per thread: the opacity and source function into the
-// scratch rows, then the outward Bezier ray (wavelengths with a line) or
-// the Feautrier solution at mu (rh/rhf1d/formal.c:44-346).  I goes to
+// (rh/rhf1d/pyrh_solveray.c:82-107), at the wavelengths with a line: one ray
+// at the caller's mu with the converged populations, background scattering
+// from the last J, no update of J.  One (column, wavelength) per wavefront,
+// as k_nlte_bezier (every lane group carries the one outward ray).  I goes to
 // stokes[(column * 4) * nout + io]; Q, U, V are zero (field-free).
+template <int L, int P>
 __global__ void __launch_bounds__(64)
 k_nlte_emergent(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap, NlteBufs B,
                 const int32_t *__restrict__ out_ls, const int32_t *__restrict__ io_list, int nlist,
                 double mu, double *__restrict__ stokes) {
-  constexpr int MS = NLTE_MAXSET;
   const DevModel &M = *Mp;
   const DevNlte &A = *Ap;
-  const int ncol = B.ncol, Nmax = B.Nmax, ncb = (ncol + 63) / 64;
-  int cb, il;
-  xcd_tile(blockIdx.x, nlist, cb, il);
-  if (cb >= ncb) return;
-  const int ic = cb * 64 + threadIdx.x;
-  if (ic >= ncol) return;
+  int ic, il;
+  if (!nlte_tile(B.ncol, nlist, ic, il)) return;
   const int io = io_list[il], ls = out_ls[io], N = B.ndep[ic];
-  const int64_t fs = (int64_t) Nmax * ncol;
-  const int64_t nthr = (int64_t) nlist * ncb * 64;
-  double *scr = B.scr + (int64_t) il * ncb * 64 + ic;
-#define SCR(s, k) scr[((int64_t) (s) * Nmax + (k)) * nthr]
-#define STF(f, k) B.state[(int64_t) (f) * fs + (int64_t) (k) * ncol + ic]
-#define PK(k) ((int64_t) (k) * ncol + ic)
-  const int64_t wo = (int64_t) io * fs, jb = (int64_t) B.nout * fs;
-  const double *Jl = B.J + B.jpar[ic] * jb + wo;
-  const double *chic = B.cchi + wo, *etac = B.ceta + wo, *scac = B.csca + wo;
+  const int64_t fs = B.fs, col = (int64_t) ic * B.Kp, wo = (int64_t) io * fs + col;
+  const double *Jl = B.J + B.jpar[ic] * (int64_t) B.nout * fs + wo;
   const double lam = ldc(M.lamconst)[(int64_t) ls * RHG_LC_NCONST + RHG_LC_LAMBDA];
-  const double hc_k = HC / (KBOLTZMANN * NM_TO_M);
+  SetInfo<NLTE_MAXSET> si;
+  set_info<NLTE_MAXSET>(A, ls, lam, si);
+  const int t0 = (int) (threadIdx.x & (L - 1)) * P;
+  const double *Tc = B.geo + NG_T * fs + col;
+  const double B2_0 = planck_lam(Tc[N - 2], lam), B2_1 = planck_lam(Tc[N - 1], lam);
+  int k[P];
+  RayPath<P> g;
+  ray_points<P>(B, col, t0, N, true, k, g);
+  double C[P], S[P], I[P], Psi[P];
+#pragma unroll
+  for (int s = 0; s < P; s++) {
+    double chi, eta;
+    emergent_set(B, A, si, col + k[s], lam, mu, chi, eta);
+    C[s] = chi + B.cchi[wo + k[s]];
+    S[s] = fma(B.csca[wo + k[s]], Jl[k[s]], eta + B.ceta[wo + k[s]]) / C[s];
+  }
+  ray_sweep<L, P>(g, t0, N, true, 1.0 / mu, B2_0, B2_1, C, S, I, Psi);
+#pragma unroll
+  for (int s = 0; s < P; s++) {
+    if (threadIdx.x < L && t0 + s == N - 1) {
+      double *o = stokes + (int64_t) ic * 4 * B.nout + io;
+      o[0] = I[s];
+      o[B.nout] = 0.0;
+      o[2 * (int64_t) B.nout] = 0.0;
+      o[3 * (int64_t) B.nout] = 0.0;
+    }
+  }
+}
+#define RHG_INST_EM(L, P)                                                                       \
+  template __global__ void k_nlte_emergent<L, P>(const DevModel *, const DevNlte *, NlteBufs,   \
+                                                 const int32_t *, const int32_t *, int, double, \
+                                                 double *);
+RHG_INST_EM(32, 2)
+RHG_INST_EM(32, 3)
+RHG_INST_EM(64, 2)
+RHG_INST_EM(64, 3)
+RHG_INST_EM(64, 4)
+RHG_INST_EM(64, 8)
+#undef RHG_INST_EM
+
+// ---------------------------------------------------------------------------
+// Wavelengths with continua only: one opacity for all rays, and per ray the
+// Feautrier solution with its two-sided diagonal operator
+// (rh/rhf1d/feautrier.c:56-202, dark top, thermalised bottom, STANDARD order;
+// P is the mean of the two directions, weighted by the full ray weight).
+// One wavefront per wavelength and group of up to `per` active columns:
+//   1  depths on the lanes: opacity, source function and the rays' common
+//      path factor (chi_k + chi_{k+1}) (z_k - z_{k+1}) into LDS;
+//   2  (column, ray) on the lanes: elimination and back substitution, the
+//      only serial part, with F and z in LDS, overwritten by Psi and P;
+//   3  depths on the lanes: J and the rate terms summed over the rays.
+// More rays than NLTE_FE_RAYS run phases 2 and 3 in chunks.  MS is the
+// largest active set among the wavelengths of io_list (the member loops are
+// unrolled to it).  EM: the final ray at mu instead (k_nlte_emergent's
+// counterpart): one ray, its emergent intensity to stokes.
+// The elimination is written in F and q = F / (1 + F): with r = dtau_k /
+// dtau_{k-1} and d the mean of the two, F_k = d dtau_k + r q_{k-1} and
+// z_k = (d dtau_k S_k + r z_{k-1}) / (1 + F_k), one reciprocal in the chain.
+template <int MS, bool EM>
+__global__ void __launch_bounds__(64)
+k_nlte_feautrier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap, NlteBufs B,
+                 const int32_t *__restrict__ act, int nact, int per,
+                 const int32_t *__restrict__ out_ls, const int32_t *__restrict__ io_list, int nlist,
+                 int il_off, int nlist_all, int eval_op, double mu_em, double *__restrict__ stokes) {
+#pragma clang fp contract(fast)
+  extern __shared__ double lds[];
+  const DevModel &M = *Mp;
+  const DevNlte &A = *Ap;
+  int grp, il;
+  if (!nlte_tile((nact + per - 1) / per, nlist, grp, il)) return;
+  const int io = io_list[il], ls = out_ls[io], nrays = EM ? 1 : A.nrays;
+  const int first = grp * per, n_it = nact - first < per ? nact - first : per;
+  const int64_t fs = B.fs, jb = (int64_t) B.nout * fs;
+  const double lam = ldc(M.lamconst)[(int64_t) ls * RHG_LC_NCONST + RHG_LC_LAMBDA];
   SetInfo<MS> si;
   set_info<MS>(A, ls, lam, si);
-  const bool bez = si.n > 0 && A.as_bezier[ls];
-  for (int k = 0; k < N; k++) {
-    const double T = STF(RHG_CF_T, k), vb = B.vbroad[PK(k)], vz = STF(RHG_CF_VLOS, k);
-    double chi = 0.0, eta = 0.0;
-#pragma unroll
-    for (int n = 0; n < MS; n++) {
-      if (n < si.n) {
-        const double ni = B.pops[(int64_t) si.ti[n] * fs + PK(k)];
-        const double nj = B.pops[(int64_t) si.tj[n] * fs + PK(k)];
-        double V, gij;
-        if (si.line[n] >= 0) {
-          const int l = si.line[n];
-          const double lambda0 = A.ln_lambda0[l];
-          const double v = (lam - lambda0 - 0.0) * CLIGHT / (vb * lambda0);
-          const double vlos = mu * vz / vb;
-          const double ph = voigt_armstrong(B.adamp[(int64_t) l * fs + PK(k)], v + 1.0 * vlos) *
-                            1.0 / (SQRTPI * vb);
-          gij = si.gline[n];
-          V = si.cV[n] * ph;
-        } else {
-          gij = B.nstar[(int64_t) si.ti[n] * fs + PK(k)] / B.nstar[(int64_t) si.tj[n] * fs + PK(k)] *
-                exp(-hc_k / (lam * T));
-          V = si.alpha[n];
-        }
-        chi += V * (ni - gij * nj);
-        eta += si.tw[n] * gij * V * nj;
-      }
-    }
-    const double chi_t = chi + chic[PK(k)];
-    double S = eta + etac[PK(k)];
-    S += scac[PK(k)] * Jl[PK(k)];
-    SCR(NS_CHI, k) = chi_t;
-    SCR(NS_S, k) = S / chi_t;
-  }
-  const double B2_0 = planck_lam(STF(RHG_CF_T, N - 2), lam);
-  const double B2_1 = planck_lam(STF(RHG_CF_T, N - 1), lam);
-#define CHI(k) SCR(NS_CHI, k)
-#define SRC(k) SCR(NS_S, k)
-  double Iout;
-  if (bez) {
-    // outward ray from the thermalised bottom, rh/rhf1d/bezier_1D.c:306-541
-    const double zmu = 1.0 / mu;
-    auto dzb = [&](int k) { return STF(RHG_CF_DZ, k); };   // |z[k-1] - z[k]|
-    double dtau_uw = 0.5 * zmu * (CHI(N - 1) + CHI(N - 2)) * dzb(N - 1);
-    double I_upw = B2_1 - (B2_0 - B2_1) / dtau_uw;
-    int k = N - 2;
-    double dsup = dzb(k + 1) * zmu, dsdn = dzb(k) * zmu;
-    double dchi_up = (CHI(k) - CHI(k + 1)) / dsup;
-    double dchi_c = cent_div(dsup, dsdn, CHI(k + 1), CHI(k), CHI(k - 1));
-    double c1 = max0(CHI(k) - (dsup * (1.0 / 3.0)) * dchi_c);
-    double c2 = max0(CHI(k + 1) + (dsup * (1.0 / 3.0)) * dchi_up);
-    dtau_uw = dsup * (CHI(k) + CHI(k + 1) + c1 + c2) * 0.25;
-    double dS_up = (SRC(k) - SRC(k + 1)) / dtau_uw;
-    for (k = N - 2; k >= 1; k--) {
-      dsdn = dzb(k) * zmu;
-      double dchi_dn;
-      if (k > 1) {
-        const double dsdn2 = dzb(k - 1) * zmu;
-        dchi_dn = cent_div(dsdn, dsdn2, CHI(k), CHI(k - 1), CHI(k - 2));
+  const int lane = threadIdx.x, Nmax = B.Nmax;
+  constexpr int RF = EM ? 1 : NLTE_FE_RAYS;
+  const int FS = per * RF;   // F and z: [Nmax][per * RF]
+  double *Xs = lds, *Ss = Xs + per * Nmax, *Cs = Ss + per * Nmax, *Fs = Cs + per * Nmax,
+         *Zs = Fs + Nmax * FS;
+  auto column = [&](int it) { return EM ? first + it : act[first + it]; };
+
+  for (int it = 0; it < n_it; it++) {
+    const int ic = column(it), N = B.ndep[ic];
+    const int64_t col = (int64_t) ic * B.Kp, wo = (int64_t) io * fs + col;
+    const double *Jo = B.J + B.jpar[ic] * jb + wo, *Tc = B.geo + NG_T * fs + col;
+    for (int k = lane; k < N; k += 64) {
+      double chi = 0.0, eta = 0.0;
+      if constexpr (EM) {
+        SetInfo<NLTE_MAXSET> s8;
+        set_info<NLTE_MAXSET>(A, ls, lam, s8);
+        emergent_set(B, A, s8, col + k, lam, mu_em, chi, eta);
       } else {
-        dchi_dn = (CHI(k - 1) - CHI(k)) / dsdn;
+        SetDepth<MS> sd;
+        set_depth<MS>(B, si, col + k, Tc[k], lam, sd);
+#pragma unroll
+        for (int n = 0; n < MS; n++) {
+          if (n < si.n) {
+            // a line at a Feautrier wavelength (not produced by the set-up):
+            // its profile of the first ray
+            const double V = si.line[n] >= 0
+                                 ? si.cV[n] * B.phi[((int64_t) si.prow[n] * 2) * fs + col + k]
+                                 : si.alpha[n];
+            chi += V * sd.x[n];
+            eta += V * sd.e[n];
+          }
+        }
       }
-      c1 = max0(CHI(k) + (dsdn * (1.0 / 3.0)) * dchi_c);
-      c2 = max0(CHI(k - 1) - (dsdn * (1.0 / 3.0)) * dchi_dn);
-      const double dtau_dw = dsdn * (CHI(k) + CHI(k - 1) + c1 + c2) * 0.25;
-      const double dt03 = dtau_uw / 3.0;
-      double alpha, beta, gamma, theta, eps;
-      bezier3_coeffs(dtau_uw, alpha, beta, gamma, theta, eps);
-      const double dS_c = cent_div(dtau_uw, dtau_dw, SRC(k + 1), SRC(k), SRC(k - 1));
-      c1 = max0(SRC(k) - dt03 * dS_c);
-      c2 = max0(SRC(k + 1) + dt03 * dS_up);
-      I_upw = I_upw * eps + alpha * SRC(k) + beta * SRC(k + 1) + gamma * c1 + theta * c2;
-      dchi_c = dchi_dn;
-      dtau_uw = dtau_dw;
-      dS_up = dS_c;
+      const double C = chi + B.cchi[wo + k];
+      Cs[it * Nmax + k] = C;
+      Ss[it * Nmax + k] = fma(B.csca[wo + k], Jo[k], eta + B.ceta[wo + k]) / C;
     }
-    {
-      const double dt = 0.5 * zmu * (CHI(0) + CHI(1)) * dzb(1);
-      const double dS_uw = -(SRC(0) - SRC(1)) / dt;
-      double w[3];
-      w3(dt, w);
-      Iout = (1.0 - w[0]) * I_upw + w[0] * SRC(0) + w[1] * dS_uw;
-    }
-    (void) dchi_up;
-  } else {
-    // Feautrier at mu, rh/rhf1d/feautrier.c:56-202; the emergent intensity
-    // is (1 + f0) P[0] - h0 / (1 + r0) with r0 = h0 = 0
-#define HGT(k) STF(RHG_CF_HEIGHT, k)
-    const double zmu = 0.5 / mu;
-    auto dtau = [&](int k) { return zmu * (CHI(k) + CHI(k + 1)) * (HGT(k) - HGT(k + 1)); };
-    const double dt0 = dtau(0);
-    const double abc0 = 1.0 + 2.0 * 1.0 / dt0;
-    const double C1_0 = 2.0 / (dt0 * dt0);
-    const double S0 = SRC(0) + 2.0 * 0.0 / ((1.0 + 0.0) * dt0);
-    double F = abc0 / C1_0, z = S0 / (abc0 + C1_0);
-    SCR(NS_F, 0) = F;
-    SCR(NS_Z, 0) = z;
-    double dtm1 = dt0;
-    for (int k = 1; k < N - 1; k++) {
-      const double dtk = dtau(k);
-      const double dtau_mid = 0.5 * (dtk + dtm1);
-      const double A1 = 1.0 / (dtau_mid * dtm1), C1 = 1.0 / (dtau_mid * dtk);
-      F = (1.0 + A1 * F / (1.0 + F)) / C1;
-      z = (SRC(k) + A1 * z) / (C1 * (1.0 + F));
-      SCR(NS_F, k) = F;
-      SCR(NS_Z, k) = z;
-      dtm1 = dtk;
-    }
-    const double dtN = dtm1;
-    const double hN = B2_1 - (B2_0 - B2_1) / dtN;
-    const double abcN = 1.0 + 2.0 * 1.0 / dtN;
-    const double A1N = 2.0 / (dtN * dtN);
-    const double SN = SRC(N - 1) + 2.0 * hN / ((1.0 + 0.0) * dtN);
-    const double FN2 = SCR(NS_F, N - 2);
-    double P = (SN + A1N * SCR(NS_Z, N - 2)) / (abcN + A1N * (FN2 / (1.0 + FN2)));
-    for (int k = N - 2; k >= 0; k--) P = P / (1.0 + SCR(NS_F, k)) + SCR(NS_Z, k);
-    Iout = (1.0 + 1.0) * P - 0.0 / (1.0 + 0.0);
-#undef HGT
+    wave_sync();
+    const double *z = B.geo + NG_HEIGHT * fs + col;
+    for (int k = lane; k < N - 1; k += 64)
+      Xs[it * Nmax + k] = (Cs[it * Nmax + k] + Cs[it * Nmax + k + 1]) * (z[k] - z[k + 1]);
   }
-  double *o = stokes + (int64_t) ic * 4 * B.nout + io;
-  o[0] = Iout;
-  o[B.nout] = 0.0;
-  o[2 * (int64_t) B.nout] = 0.0;
-  o[3 * (int64_t) B.nout] = 0.0;
-#undef CHI
-#undef SRC
-#undef SCR
-#undef STF
-#undef PK
+  wave_sync();
+
+  for (int c0 = 0; c0 < nrays; c0 += RF) {
+    const int nrc = nrays - c0 < RF ? nrays - c0 : RF;
+    const int it_s = lane / RF, r_s = lane % RF;
+    if (it_s < n_it && r_s < nrc) {
+      const int ic = column(it_s), N = B.ndep[ic];
+      const double *Tc = B.geo + NG_T * fs + (int64_t) ic * B.Kp;
+      const double B2_0 = planck_lam(Tc[N - 2], lam), B2_1 = planck_lam(Tc[N - 1], lam);
+      const double zmu = 0.5 / (EM ? mu_em : A.muz[c0 + r_s]);
+      const double *X = Xs + it_s * Nmax, *Sv = Ss + it_s * Nmax;
+      double *F = Fs + lane, *Z = Zs + lane;
+      const double dt0 = zmu * X[0], abc0 = 1.0 + 2.0 / dt0, C1_0 = 2.0 / (dt0 * dt0);
+      double Fk = abc0 / C1_0, zk = Sv[0] / (abc0 + C1_0), q = ndiv(Fk, 1.0 + Fk);
+      F[0] = Fk;
+      Z[0] = zk;
+      double dtm = dt0, idtm = nrcp(dt0);
+#pragma unroll 2
+      for (int k = 1; k < N - 1; k++) {
+        const double dt = zmu * X[k], d = 0.5 * (dt + dtm) * dt, r = dt * idtm;
+        Fk = fma(r, q, d);
+        const double i1 = nrcp(1.0 + Fk);
+        zk = fma(d, Sv[k], r * zk) * i1;
+        q = Fk * i1;
+        F[k * FS] = Fk;
+        Z[k * FS] = zk;
+        dtm = dt;
+        idtm = nrcp(dt);
+      }
+      // back substitution with the two-sided operator
+      const double hN = B2_1 - (B2_0 - B2_1) / dtm;
+      const double abcN = 1.0 + 2.0 / dtm, A1N = 2.0 / (dtm * dtm);
+      const double SN = Sv[N - 1] + 2.0 * hN / dtm;
+      double P = (SN + A1N * zk) / (abcN + A1N * q);
+      double h = abcN / (A1N + abcN);   // G / (1 + G), G = abcN / A1N
+      Z[(N - 1) * FS] = P;
+      F[(N - 1) * FS] = 1.0 / (abcN + A1N * q);
+      double dtk = dtm, idtk = idtm, Fc = Fk;
+#pragma unroll 2
+      for (int k = N - 2; k >= 1; k--) {
+        const double Fm = F[(k - 1) * FS], dm = zmu * X[k - 1], idm = nrcp(dm);
+        P = fma(P, nrcp(1.0 + Fc), Z[k * FS]);
+        const double id = nrcp(0.5 * (dtk + dm));
+        const double qm = ndiv(Fm, 1.0 + Fm);
+        const double Psi = nrcp(1.0 + id * (idm * qm + idtk * h));
+        const double G = fma(dm * idtk, h, 0.5 * (dtk + dm) * dm);
+        h = ndiv(G, 1.0 + G);
+        Z[k * FS] = P;
+        F[k * FS] = Psi;
+        dtk = dm;
+        idtk = idm;
+        Fc = Fm;
+      }
+      P = fma(P, nrcp(1.0 + Fc), Z[0]);
+      if constexpr (EM) {
+        // (1 + f0) P[0] - h0 / (1 + r0) with r0 = h0 = 0
+        double *o = stokes + (int64_t) ic * 4 * B.nout + io;
+        o[0] = (1.0 + 1.0) * P;
+        o[B.nout] = 0.0;
+        o[2 * (int64_t) B.nout] = 0.0;
+        o[3 * (int64_t) B.nout] = 0.0;
+      } else {
+        Z[0] = P;
+        F[0] = 1.0 / (abc0 + C1_0 * h);
+      }
+    }
+    if constexpr (EM) return;
+    wave_sync();
+    for (int it = 0; it < n_it; it++) {
+      const int ic = column(it), N = B.ndep[ic];
+      const int64_t col = (int64_t) ic * B.Kp, wo = (int64_t) io * fs + col;
+      const int par = B.jpar[ic];
+      const double *Jo = B.J + par * jb + wo, *Tc = B.geo + NG_T * fs + col;
+      double *Jn = B.J + (1 - par) * jb + wo;
+      double dJ_it = 0.0;
+      for (int k = lane; k < N; k += 64) {
+        const double *F = Fs + k * FS + it * RF, *Z = Zs + k * FS + it * RF;
+        double j = c0 ? Jn[k] : 0.0;
+        for (int r = 0; r < nrc; r++) j += Z[r] * A.wmu[c0 + r];
+        Jn[k] = j;
+        if (c0 + RF >= nrays) {
+          const double dJ = fabs(1.0 - Jo[k] / j);
+          dJ_it = dJ_it > dJ ? dJ_it : dJ;
+        }
+        if (!eval_op) continue;
+        SetDepth<MS> sd;
+        set_depth<MS>(B, si, col + k, Tc[k], lam, sd);
+        double V[MS], aIJ[MS], aJI[MS];
+#pragma unroll
+        for (int n = 0; n < MS; n++) {
+          V[n] = aIJ[n] = aJI[n] = 0.0;
+          if (n < si.n) {
+            V[n] = si.line[n] >= 0 ? si.cV[n] * B.phi[((int64_t) si.prow[n] * 2) * fs + col + k]
+                                   : si.alpha[n];
+            if (c0 > 0) {
+              const double *aij = B.acc + ((int64_t) si.ent[n] * 2) * fs + col + k;
+              aIJ[n] = aij[0];
+              aJI[n] = aij[fs];
+            }
+          }
+        }
+        const double iC = 1.0 / Cs[it * Nmax + k];
+        for (int r = 0; r < nrc; r++)
+          rate_terms<MS>(si, sd, V, Z[r], F[r] * iC, A.wmu[c0 + r], aIJ, aJI);
+#pragma unroll
+        for (int n = 0; n < MS; n++) {
+          if (n < si.n) {
+            double *aij = B.acc + ((int64_t) si.ent[n] * 2) * fs + col + k;
+            aij[0] = aIJ[n];
+            aij[fs] = aJI[n];
+          }
+        }
+      }
+      if (c0 + RF >= nrays) {
+        for (int o = 32; o >= 1; o >>= 1) {
+          const double x = __shfl_xor(dJ_it, o);
+          dJ_it = dJ_it > x ? dJ_it : x;
+        }
+        if (lane == 0) B.dJ[(int64_t) ic * nlist_all + il_off + il] = dJ_it;
+      }
+    }
+    wave_sync();
+  }
 }
+#define RHG_INST_FE(MS, EM)                                                                      \
+  template __global__ void k_nlte_feautrier<MS, EM>(const DevModel *, const DevNlte *, NlteBufs, \
+                                                    const int32_t *, int, int, const int32_t *,  \
+                                                    const int32_t *, int, int, int, int, double, \
+                                                    double *);
+RHG_INST_FE(2, false)
+RHG_INST_FE(4, false)
+RHG_INST_FE(6, false)
+RHG_INST_FE(8, false)
+RHG_INST_FE(2, true)
+#undef RHG_INST_FE
 
 // the new J becomes the previous one for the columns just solved
 __global__ void k_nlte_flip(NlteBufs B, const int32_t *__restrict__ act, int nact) {
@@ -1088,18 +1106,22 @@ __global__ void k_nlte_flip(NlteBufs B, const int32_t *__restrict__ act, int nac
   B.jpar[ic] = 1 - B.jpar[ic];
 }
 
-// max over the list wavelengths of the per-wavelength dJ, per column
-__global__ void k_nlte_djmax(NlteBufs B, const int32_t *__restrict__ act, int nact, int nlist,
-                             double *__restrict__ djmax) {
-  const int slot = blockIdx.x * blockDim.x + threadIdx.x;
-  if (slot >= nact) return;
-  const int ic = act[slot];
+// max over the list wavelengths of the per-wavelength dJ, a wavefront per
+// column
+__global__ void __launch_bounds__(64)
+k_nlte_djmax(NlteBufs B, const int32_t *__restrict__ act, int nact, int nlist,
+             double *__restrict__ djmax) {
+  const int ic = act[blockIdx.x];
   double d = 0.0;
-  for (int il = 0; il < nlist; il++) {
-    const double x = B.dJ[(int64_t) il * B.ncol + ic];
+  for (int il = threadIdx.x; il < nlist; il += 64) {
+    const double x = B.dJ[(int64_t) ic * nlist + il];
     d = d > x ? d : x;
   }
-  djmax[ic] = d;
+  for (int o = 32; o >= 1; o >>= 1) {
+    const double x = __shfl_xor(d, o);
+    d = d > x ? d : x;
+  }
+  if (threadIdx.x == 0) djmax[ic] = d;
 }
 
 // ---------------------------------------------------------------------------
@@ -1220,43 +1242,44 @@ __device__ __forceinline__ void solve_improve_r(double (&a)[NLP][NLP], double (&
   for (int i = 0; i < NLP; i++) b[i] += res[i];
 }
 
-// Rate matrix and statistical equilibrium at one (column, depth),
+// Rate matrix and statistical equilibrium at D depths of one column,
 // rh/statequil.c:36-216: Gamma = C + the rate terms of each transition
-// summed over its wavelengths in order; the diagonal is minus the column
-// sums; the equation of the most populated level (isum = -1, else level
-// isum) is replaced by particle conservation.
+// summed over its wavelengths; the diagonal is minus the column sums; the
+// equation of the most populated level (isum = -1, else level isum) is
+// replaced by particle conservation.  The workgroup's wavefronts share
+// the sums (a transition's two directions are a task, the depths on the
+// lanes), the first one solves.  Launch (columns, ceil(Nmax / D)) workgroups
+// with D nl^2 doubles of LDS, D = stateq_depths.
 template <int NLP>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(64 * stateq_waves(NLP))
 k_nlte_stateq(const DevNlte *__restrict__ Ap, NlteBufs B, const int32_t *__restrict__ act,
               int nact, int isum) {
+  constexpr int D = stateq_depths(NLP), NT = 64 * stateq_waves(NLP) / D;
   const DevNlte &A = *Ap;
-  const int64_t p = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-  const int Nmax = B.Nmax, ncol = B.ncol, nl = A.nl;
-  if (p >= (int64_t) nact * Nmax) return;
-  const int slot = (int) (p % nact), k = (int) (p / nact);
-  const int ic = act[slot];
-  if (k >= B.ndep[ic]) return;
-  const int64_t fs = (int64_t) Nmax * ncol, pk = (int64_t) k * ncol + ic;
-  for (int q = 0; q < nl * nl; q++) B.Gam[(int64_t) q * fs + pk] = B.Cmat[(int64_t) q * fs + pk];
-  for (int t = 0; t < A.ntrans; t++) {
-    const int i = A.tr_i[t], j = A.tr_j[t], e0 = A.tr_ptr[t], ne = A.tr_nlam[t];
-    double *gij = B.Gam + (int64_t) (i * nl + j) * fs + pk;
-    double *gji = B.Gam + (int64_t) (j * nl + i) * fs + pk;
-    double sij = *gij, sji = *gji;
-    for (int e = e0; e < e0 + ne; e++) {
-      sij += B.acc[((int64_t) e * 2) * fs + pk];
-      sji += B.acc[((int64_t) e * 2 + 1) * fs + pk];
-    }
-    *gij = sij;
-    *gji = sji;
+  extern __shared__ double gam[];   // [nl * nl][D]
+  const int nl = A.nl, lane = threadIdx.x % D, w = threadIdx.x / D;
+  const int ic = act[blockIdx.x], k = blockIdx.y * D + lane, N = B.ndep[ic];
+  if ((int) blockIdx.y * D >= N) return;
+  const int64_t fs = B.fs, pk = (int64_t) ic * B.Kp + (k < N ? k : N - 1);
+  for (int q = w; q < nl * nl; q += NT) gam[q * D + lane] = B.Cmat[(int64_t) q * fs + pk];
+  __syncthreads();
+  for (int t = w; t < 2 * A.ntrans; t += NT) {
+    const int tr = t >> 1, i = A.tr_i[tr], j = A.tr_j[tr], ne = A.tr_nlam[tr];
+    const double *x = B.acc + ((int64_t) A.tr_ptr[tr] * 2 + (t & 1)) * fs + pk;
+    double sum = 0.0;
+#pragma unroll 16
+    for (int e = 0; e < ne; e++) sum += x[(int64_t) (2 * e) * fs];
+    atomicAdd(&gam[((t & 1) ? j * nl + i : i * nl + j) * D + lane], sum);
   }
+  __syncthreads();
+  if (w != 0 || k >= N) return;
   double a[NLP][NLP], nk[NLP];
 #pragma unroll
   for (int i = 0; i < NLP; i++) {
     nk[i] = (i < nl) ? B.pops[(int64_t) i * fs + pk] : 0.0;
 #pragma unroll
     for (int j = 0; j < NLP; j++)
-      a[i][j] = (i < nl && j < nl) ? B.Gam[(int64_t) (i * nl + j) * fs + pk] : (i == j ? 1.0 : 0.0);
+      a[i][j] = (i < nl && j < nl) ? gam[(i * nl + j) * D + lane] : (i == j ? 1.0 : 0.0);
   }
   int ie = 0;
   if (isum == -1) {
@@ -1309,22 +1332,23 @@ template __global__ void k_nlte_stateq<16>(const DevNlte *, NlteBufs, const int3
 // populations flattened level by level (index i * N + k).  The history
 // holds norder + 2 solutions; ng_init stored the starting solution in slot
 // 0, so before iteration niter (1-based) the count is niter.
-__global__ void k_nlte_ng(const DevNlte *__restrict__ Ap, NlteBufs B,
-                          const int32_t *__restrict__ act, int nact, int niter, int norder,
-                          int ndelay, int nperiod, double *__restrict__ dpops) {
+// A workgroup per column, the flattened populations over its threads.
+__global__ void __launch_bounds__(NG_BLOCK)
+k_nlte_ng(const DevNlte *__restrict__ Ap, NlteBufs B, const int32_t *__restrict__ act, int nact,
+          int niter, int norder, int ndelay, int nperiod, double *__restrict__ dpops) {
   const DevNlte &A = *Ap;
-  const int slot = blockIdx.x * blockDim.x + threadIdx.x;
-  if (slot >= nact) return;
-  const int ic = act[slot], N = B.ndep[ic], nl = A.nl, Nmax = B.Nmax, ncol = B.ncol;
-  const int NS = norder + 2;
-  const int64_t fs = (int64_t) Nmax * ncol, hs = (int64_t) nl * fs;
-  auto H = [&](int s, int i, int k) -> double & {
-    return B.hist[(int64_t) s * hs + (int64_t) i * fs + (int64_t) k * ncol + ic];
-  };
-  auto POP = [&](int i, int k) -> double & { return B.pops[(int64_t) i * fs + (int64_t) k * ncol + ic]; };
+  constexpr int NSUM = NLTE_MAXNG * (NLTE_MAXNG + 1), NW = NG_BLOCK / 64;
+  __shared__ double part[NW][NSUM], coef[NLTE_MAXNG];
+  const int ic = act[blockIdx.x], N = B.ndep[ic], nl = A.nl, tid = threadIdx.x, w = tid >> 6;
+  const int NS = norder + 2, np = nl * N;
+  const int64_t fs = B.fs, hs = (int64_t) nl * fs, o = (int64_t) ic * B.Kp;
+  auto at = [&](int p) { return (int64_t) (p / N) * fs + o + p % N; };
+  auto H = [&](int s, int64_t q) -> double & { return B.hist[(int64_t) s * hs + q]; };
   const int cur = niter % NS;
-  for (int i = 0; i < nl; i++)
-    for (int k = 0; k < N; k++) H(cur, i, k) = POP(i, k);
+  for (int p = tid; p < np; p += NG_BLOCK) {
+    const int64_t q = at(p);
+    H(cur, q) = B.pops[q];
+  }
   const int count = niter + 1;
   if (norder > 0 && count >= ndelay && !((count - ndelay) % nperiod)) {
     double Am[NLTE_MAXNG][NLTE_MAXNG], bv[NLTE_MAXNG];
@@ -1332,54 +1356,91 @@ __global__ void k_nlte_ng(const DevNlte *__restrict__ Ap, NlteBufs B,
     for (int i = 0; i < NLTE_MAXNG; i++) {
       bv[i] = 0.0;
 #pragma unroll
-      for (int j = 0; j < NLTE_MAXNG; j++) Am[i][j] = (i < norder || j < norder) ? 0.0 : (i == j ? 1.0 : 0.0);
+      for (int j = 0; j < NLTE_MAXNG; j++) Am[i][j] = 0.0;
     }
-    for (int i = 0; i < nl; i++)
-      for (int k = 0; k < N; k++) {
-        double D[NLTE_MAXNG + 1];
+    // (each thread reads the history entries that it writes)
+    for (int p = tid; p < np; p += NG_BLOCK) {
+      const int64_t q = at(p);
+      double D[NLTE_MAXNG + 1];
 #pragma unroll
-        for (int q = 0; q <= NLTE_MAXNG; q++) {
-          D[q] = 0.0;
-          // count >= ndelay >= norder + 2, so both slots are >= 0
-          if (q <= norder) D[q] = H((count - 1 - q) % NS, i, k) - H((count - 2 - q) % NS, i, k);
+      for (int r = 0; r <= NLTE_MAXNG; r++) {
+        D[r] = 0.0;
+        // count >= ndelay >= norder + 2, so both slots are >= 0
+        if (r <= norder) D[r] = H((count - 1 - r) % NS, q) - H((count - 2 - r) % NS, q);
+      }
+      const double wt = 1.0 / fabs(B.pops[q]);
+#pragma unroll
+      for (int j = 0; j < NLTE_MAXNG; j++) {
+        if (j < norder) {
+          bv[j] += wt * D[0] * (D[0] - D[j + 1]);
+#pragma unroll
+          for (int ii = 0; ii < NLTE_MAXNG; ii++)
+            if (ii < norder) Am[ii][j] += wt * (D[j + 1] - D[0]) * (D[ii + 1] - D[0]);
         }
-        const double w = 1.0 / fabs(POP(i, k));
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NLTE_MAXNG; i++) {
+      for (int s = 32; s >= 1; s >>= 1) bv[i] += __shfl_xor(bv[i], s);
+      if ((tid & 63) == 0) part[w][i] = bv[i];
+#pragma unroll
+      for (int j = 0; j < NLTE_MAXNG; j++) {
+        for (int s = 32; s >= 1; s >>= 1) Am[i][j] += __shfl_xor(Am[i][j], s);
+        if ((tid & 63) == 0) part[w][NLTE_MAXNG * (i + 1) + j] = Am[i][j];
+      }
+    }
+    __syncthreads();
+    if (tid == 0) {
+#pragma unroll
+      for (int i = 0; i < NLTE_MAXNG; i++) {
+        bv[i] = 0.0;
+        for (int v = 0; v < NW; v++) bv[i] += part[v][i];
 #pragma unroll
         for (int j = 0; j < NLTE_MAXNG; j++) {
-          if (j < norder) {
-            bv[j] += w * D[0] * (D[0] - D[j + 1]);
-#pragma unroll
-            for (int ii = 0; ii < NLTE_MAXNG; ii++)
-              if (ii < norder) Am[ii][j] += w * (D[j + 1] - D[0]) * (D[ii + 1] - D[0]);
-          }
+          Am[i][j] = (i < norder && j < norder) ? 0.0 : (i == j ? 1.0 : 0.0);
+          for (int v = 0; v < NW; v++) Am[i][j] += part[v][NLTE_MAXNG * (i + 1) + j];
         }
       }
-    solve_improve_r<NLTE_MAXNG>(Am, bv);
-    const int i0 = (count - 1) % NS;
-    for (int i = 0; i < nl; i++)
-      for (int k = 0; k < N; k++) {
-        double s = POP(i, k);
-        const double h0 = H(i0, i, k);
+      solve_improve_r<NLTE_MAXNG>(Am, bv);
 #pragma unroll
-        for (int q = 0; q < NLTE_MAXNG; q++)
-          if (q < norder) s += bv[q] * (H((count - 2 - q) % NS, i, k) - h0);
-        POP(i, k) = s;
-        H(i0, i, k) = s;
-      }
+      for (int i = 0; i < NLTE_MAXNG; i++) coef[i] = bv[i];
+    }
+    __syncthreads();
+    const int i0 = (count - 1) % NS;
+    for (int p = tid; p < np; p += NG_BLOCK) {
+      const int64_t q = at(p);
+      double s = B.pops[q];
+      const double h0 = H(i0, q);
+#pragma unroll
+      for (int r = 0; r < NLTE_MAXNG; r++)
+        if (r < norder) s += coef[r] * (H((count - 2 - r) % NS, q) - h0);
+      B.pops[q] = s;
+      H(i0, q) = s;
+    }
   }
   double dmax = 0.0;
   {
     const int so = (count - 2) % NS, sc = (count - 1) % NS;
-    for (int i = 0; i < nl; i++)
-      for (int k = 0; k < N; k++) {
-        const double c = H(sc, i, k);
-        if (c) {
-          const double d = fabs((c - H(so, i, k)) / c);
-          dmax = dmax > d ? dmax : d;
-        }
+    for (int p = tid; p < np; p += NG_BLOCK) {
+      const int64_t q = at(p);
+      const double c = H(sc, q);
+      if (c) {
+        const double d = fabs((c - H(so, q)) / c);
+        dmax = dmax > d ? dmax : d;
       }
+    }
   }
-  dpops[ic] = dmax;
+  for (int s = 32; s >= 1; s >>= 1) {
+    const double x = __shfl_xor(dmax, s);
+    dmax = dmax > x ? dmax : x;
+  }
+  __syncthreads();
+  if ((tid & 63) == 0) part[w][0] = dmax;
+  __syncthreads();
+  if (tid == 0) {
+    for (int v = 1; v < NW; v++) dmax = dmax > part[v][0] ? dmax : part[v][0];
+    dpops[ic] = dmax;
+  }
 }
 
 // populations (src: current or LTE) to the caller's layout
@@ -1393,7 +1454,7 @@ __global__ void k_nlte_out(const DevNlte *__restrict__ Ap, NlteBufs B, const dou
   const int k = (int) (p % Nmax);
   const int64_t q = p / Nmax;
   const int i = (int) (q % nl), ic = (int) (q / nl);
-  out[p] = k < B.ndep[ic] ? src[((int64_t) i * Nmax + k) * ncol + ic] : 0.0;
+  out[p] = k < B.ndep[ic] ? src[(int64_t) i * B.fs + (int64_t) ic * B.Kp + k] : 0.0;
 }
 
 }  // namespace rhg

@@ -14,21 +14,18 @@ constexpr double E_RYDBERG = 2.1798741E-18;
 constexpr int NLTE_MAXSET = 8;
 constexpr int NLTE_MAXLEV = 16;
 constexpr int NLTE_MAXNG = 4;                  // Ng order
-// per-thread scratch rows of k_nlte_feautrier and k_nlte_emergent: total
-// opacity, source function and the elimination coefficients F and z (ray r
-// of a Feautrier chunk in rows NS_F + 2 r and NS_Z + 2 r)
-enum { NS_CHI = 0, NS_S, NS_F, NS_Z };
-// rays of k_nlte_feautrier solved together (more rays in chunks of this
-// many), and the scratch rows per thread of the two kernels
+// rays of k_nlte_feautrier solved together (more rays in chunks of this many)
 constexpr int NLTE_FE_RAYS = 5;
-constexpr int NLTE_NSLOT = 2 + 2 * NLTE_FE_RAYS;
-constexpr int NLTE_NSLOT_EM = 4;
-// rays swept together by a k_nlte_bezier thread (more rays are swept in
-// chunks of this many)
-#ifndef RHG_NLTE_RB
-#define RHG_NLTE_RB 3
-#endif
-constexpr int NLTE_RB = RHG_NLTE_RB;
+// LDS of a k_nlte_feautrier workgroup for `per` columns, in doubles
+constexpr int nlte_fe_lds(int Nmax, int per, int rays) { return per * Nmax * (3 + 2 * rays); }
+// threads of k_nlte_ng; wavefronts of k_nlte_stateq for up to nlp levels
+constexpr int NG_BLOCK = 256;
+constexpr int stateq_waves(int nlp) { return nlp <= 6 ? 8 : 4; }
+constexpr int stateq_depths(int nlp) { return nlp <= 8 ? 64 : 16; }   // of a workgroup: at most 32 KB of LDS
+// depth-fastest copies of column-state fields (rows of NlteBufs::geo)
+enum { NG_T = 0, NG_VLOS, NG_DZ, NG_HEIGHT, NG_N };
+// rows of depths are padded to whole 64-byte lines
+constexpr int nlte_pitch(int Nmax) { return (Nmax + 7) & ~7; }
 
 // Device mirror of rhg_nlte_t, plus two derived tables: the transition of
 // each line (ln_tr) and each line's first row in the profile array
@@ -50,41 +47,54 @@ struct DevNlte {
   const double *muz, *wmu, *ray_H, *ray_He, *ray_H2;
 };
 
-// Device arrays of one batch of ncol columns.  Every per-depth array is
-// column-fastest: x[(row * Nmax + k) * ncol + column], row being a level,
-// a line, a level pair (i * nl + j), an output wavelength, ...
+// Device arrays of one batch of ncol columns.  Except for the LTE inputs
+// (state, lte_chi, lte_eta: column-fastest) every per-depth array is
+// depth-fastest: x[row * fs + column * Kp + k], fs = ncol * Kp, row being a
+// level, a line, a level pair (i * nl + j), an output wavelength, ...
 struct NlteBufs {
-  int ncol, Nmax, nfield, nout;
+  int ncol, Nmax, Kp, nfield, nout;
+  int64_t fs;
   const int32_t *ndep;
   double *state;                  // LTE column state, fields RHG_CF_*
+  const double *lte_chi, *lte_eta;  // [nout]: LTE continuum
+  double *geo;                    // [NG_N]: T, vlos, path, height
   double *nstar, *pops;           // [nl]: LTE and current populations
   double *ntot, *vbroad, *nHe;    // [1]: atom total, Doppler width, He I ground
   double *adamp, *wphi;           // [nline]: damping, 1 / profile normalisation
-  double *Cmat, *Gam;             // [nl * nl]: collision and rate matrices
+  double *Cmat;                   // [nl * nl]: collision matrix
   double *phi;                    // [(nphi * nrays + mu) * 2 + to_obs]: profiles
   double *cchi, *ceta, *csca;     // [nout]: background opacity (with scattering),
                                   //         emissivity and scattering opacity
   double *J;                      // [2 * nout]: mean intensity, previous and new
   int32_t *jpar;                  // per column: which half of J is the previous
   double *acc;                    // [nentry * 2 + s]: rate terms per quadrature point
-  double *scr;                    // [NLTE_NSLOT] per k_nlte_feautrier thread
-  double *dJ;                     // [nlist] x ncol: max |1 - J_old / J| per wavelength
+  double *dJ;                     // column x [nlist]: max |1 - J_old / J| per wavelength
   double *hist;                   // [(ng_order + 2) * nl]: Ng history
 };
 
 __global__ void k_nlte_pre(const DevModel *Mp, const DevNlte *Ap, NlteBufs B);
+// (tiles of 32 columns x 32 depths) (nout + NG_N) workgroups of 256 threads
 __global__ void k_nlte_bg(const DevModel *Mp, const DevNlte *Ap, NlteBufs B,
                           const int32_t *out_ls);
+// nphi ceil(ncol Nmax / 64) workgroups of 64 threads
 __global__ void k_nlte_profile(const DevModel *Mp, const DevNlte *Ap, NlteBufs B);
-template <int RB, int MS>
+__global__ void k_nlte_wphi(const DevNlte *Ap, NlteBufs B);
+template <int L, int P, int MS>
 __global__ void k_nlte_bezier(const DevModel *Mp, const DevNlte *Ap, NlteBufs B,
                               const int32_t *act, int nact, const int32_t *out_ls,
-                              const int32_t *io_list, int nlist, int il_off, int eval_op);
-template <int MS>
+                              const int32_t *io_list, int nlist, int il_off, int nlist_all,
+                              int eval_op);
+template <int MS, bool EM>
 __global__ void k_nlte_feautrier(const DevModel *Mp, const DevNlte *Ap, NlteBufs B,
-                                 const int32_t *act, int nact, const int32_t *out_ls,
-                                 const int32_t *io_list, int nlist, int il_off, int eval_op);
+                                 const int32_t *act, int nact, int per, const int32_t *out_ls,
+                                 const int32_t *io_list, int nlist, int il_off, int nlist_all,
+                                 int eval_op, double mu_em, double *stokes);
+// workgroups of the two kernels above for nact columns (or column groups)
+inline int64_t nlte_grid(int nact, int nlist) {
+  return nact >= NXCD ? xcd_grid(nact, nlist) : (int64_t) nact * nlist;
+}
 __global__ void k_nlte_flip(NlteBufs B, const int32_t *act, int nact);
+template <int L, int P>
 __global__ void k_nlte_emergent(const DevModel *Mp, const DevNlte *Ap, NlteBufs B,
                                 const int32_t *out_ls, const int32_t *io_list, int nlist,
                                 double mu, double *stokes);

@@ -191,3 +191,30 @@ def test_nlte_barklem_matches_reference(eng_mg, nm_mg, mg_fix, name):
     assert eI < TOL_MG_POPS
     # the last change is a difference of populations: off by at most twice theirs
     np.testing.assert_allclose(dpops, mg_fix[name + "__dpops"], rtol=0, atol=2 * TOL_MG_POPS)
+
+
+@pytest.mark.parametrize("nd", [4, 33, 64, 65, 96, 97, 128, 129, 192, 193, 256, 257, 512])
+def test_nlte_depth_counts(eng, nm, nd):
+    """Depth counts at the edges of what the lanes of a ray hold (a lane's
+    points, half a wavefront, a wavefront, both with more points per lane),
+    the batch's other column shallower, against the oracle over a few
+    iterations: the sweep's scan and the sums over rays and wavelengths change
+    order only, so the differences stay those of the tests above."""
+    import copy
+
+    import pyoracle
+    from pyrh_amd import workloads
+    few = copy.copy(nm)
+    few.nmax_iter = 3
+    atm, ndep = workloads.mixed_batch(2, seed=workloads.SEED_BASE + 60 + nd, ndep_choices=(nd,))
+    if nd > 8:
+        ndep[1] = nd - 5
+        atm[1, :, ndep[1]:] = 0.0
+    pops, niter, dpops, st = eng.nlte_solve(few, atm, ndep=ndep, mu=0.7, stokes=True)
+    cp, cn, cd, cs = pyoracle.nlte_solve(few, atm, ndep=ndep, mu=0.7, stokes=True)
+    for c in range(2):
+        n = ndep[c]
+        assert np.all(pops[c, :, n:] == 0.0)
+        assert _relerr(pops[c, :, :n], cp[c, :, :n]) < TOL_POPS
+    assert _relerr(st[:, 0], cs[:, 0]) < TOL_I
+    np.testing.assert_array_equal(niter, cn)
