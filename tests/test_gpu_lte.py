@@ -367,3 +367,18 @@ def test_magneto_optical_matches_oracle_on_map():
     assert eI < 1e-10 and eP < 1e-10
     with pytest.raises(EngineError):
         e.rf_lte(atm[:2])
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("ncol", [1, 63, 64, 65, 513, 1025, 4159])
+def test_gpu_batch_sizes_agree(engines, ncol, prec):
+    """The split of a batch's blocks, wavelengths and continuum tiles over the
+    chip follows its size; a column's result does not: each equals, bit for
+    bit, the same column in a batch of 4200, which matches the oracle."""
+    eng = engines("lte", workloads.wavelengths_630())
+    atm = workloads.stokes_map(4200, seed=workloads.SEED_BASE + 71)
+    full = eng.synth_lte(atm, precision=prec)
+    np.testing.assert_array_equal(eng.synth_lte(atm[:ncol], precision=prec), full[:ncol])
+    if ncol == 65 and prec == 0:
+        eI, eP = _err(full[:ncol], pyoracle.synth_lte(eng.model, atm[:ncol]))
+        assert eI <= TOL_I and eP <= TOL_QUV
