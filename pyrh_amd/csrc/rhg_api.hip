@@ -373,6 +373,28 @@ int rhg_open(const rhg_model_t *m, int device, rhg_context_t **out) {
     if (!rc) rc = upload(c, talpha.empty() ? nullptr : talpha.data(), talpha.size(), &d.tile_alpha);
   }
   if (!rc) {
+    // ktab: bilinear() over (temperature, wavelength) with the wavelength's
+    // part done
+    std::vector<double> kt((size_t) ns * rhg::KT_N, 0.0);
+    auto row = [&](double *g, const double *f, int ncolumn, int nrow, double y) {
+      if (!(y >= 0.0)) return;
+      const int j = (int) y, j1 = (j == nrow - 1) ? j : j + 1;
+      const double fy = y - j;
+      for (int i = 0; i < ncolumn; i++)
+        g[i] = (1.0 - fy) * f[j * ncolumn + i] + fy * f[j1 * ncolumn + i];
+    };
+    for (int ls = 0; ls < ns; ls++) {
+      const double *lc = m->lamconst + (size_t) ls * RHG_LC_NCONST;
+      double *g = kt.data() + (size_t) ls * rhg::KT_N;
+      row(g + rhg::KT_HMFF, m->hminff_kappa, rhg::NTHETA, rhg::NFF, lc[RHG_LC_HMIN_FF_LIDX]);
+      row(g + rhg::KT_H2M, m->h2mff_kappa, rhg::NTHETA_H2, rhg::NFF_H2, lc[RHG_LC_H2M_LIDX]);
+      row(g + rhg::KT_H2P, m->h2pff_kappa, rhg::NTEMP_H2P, rhg::NFF_H2P, lc[RHG_LC_H2P_LIDX]);
+      row(g + rhg::KT_OH, m->oh_cross, rhg::NTOH, rhg::NEOH, lc[RHG_LC_OH_EIDX]);
+      row(g + rhg::KT_CH, m->ch_cross, rhg::NTCH, rhg::NECH, lc[RHG_LC_CH_EIDX]);
+    }
+    rc = upload(c, kt.data(), kt.size(), &d.ktab);
+  }
+  if (!rc) {
     std::vector<double> cnt((size_t) (m->nmol > 0 ? m->nmol : 1) * rhg::NNUC_MAX, 0.0);
     for (int im = 0; im < m->nmol; im++)
       for (int j = 0; j < m->mol_nel[im]; j++) {
@@ -475,6 +497,17 @@ static int launch_state(rhg_context_t *c, const double *d_atm, const int32_t *d_
   return 0;
 }
 
+// Grid of k_continuum over npts points, and the bound-free tiles tpp of a
+// workgroup: all of them where the points alone make 8 wavefronts per SIMD
+// (1024 SIMDs), else split.
+static dim3 cont_grid(int64_t npts, int ntile, int &tpp) {
+  const int64_t nb = (npts + rhg::CONT_BLOCK - 1) / rhg::CONT_BLOCK;
+  const int64_t waves = nb * (rhg::CONT_BLOCK / 64);
+  const int64_t want = std::max<int64_t>(1, std::min<int64_t>(ntile, 8192 / waves));
+  tpp = (int) ((ntile + want - 1) / want);
+  return dim3((unsigned) nb, (unsigned) std::max(1, (ntile + tpp - 1) / std::max(tpp, 1)));
+}
+
 // The wavelength grids of a synthesis launch: the batch's block -> grid
 // table (ncol / 64 entries, -1: a block without columns) and the context's
 // per-grid wavelength lists (rhg_set_grids).
@@ -513,13 +546,14 @@ static int launch_synth(rhg_context_t *c, const double *d_atm, const int32_t *d_
   }
   HIPCHECK(hipEventRecord(c->ev[2], c->stream));
   {
-    dim3 blk(rhg::CONT_BLOCK), grd((unsigned) ((npts + rhg::CONT_BLOCK - 1) / rhg::CONT_BLOCK));
+    int tpp;
+    const dim3 blk(rhg::CONT_BLOCK), grd = cont_grid(npts, c->dm.ntile, tpp);
     const int32_t *bg = gl ? gl->blk_grid : nullptr, *gt = gl ? gl->tile : nullptr;
     const int32_t *gm = gl ? gl->mask : nullptr;
     const int gw = gl ? gl->mask_words : 0;
 #define RHG_LAUNCH_CONT(R, G)                                                                    \
   hipLaunchKernelGGL((rhg::k_continuum<R, G>), grd, blk, 0, c->stream, c->d_model, d_ndep, ncol, Nmax, \
-                     state, nfield, c->d_out_ls, nout, (R *) cchi, (R *) ceta, bg, gt, gm, gw)
+                     state, nfield, c->d_out_ls, nout, (R *) cchi, (R *) ceta, bg, gt, gm, gw, tpp)
     if (precision == RHG_PREC_FP32) {
       if (gl) RHG_LAUNCH_CONT(float, true); else RHG_LAUNCH_CONT(float, false);
     } else {
@@ -1299,9 +1333,11 @@ int launch_base(rhg_context_t *c, const double *d_atm, const int32_t *d_ndep, in
     HIPCHECK(hipGetLastError());
   }
   if (cchi) {
-    dim3 blk(rhg::CONT_BLOCK), grd((unsigned) ((npts + rhg::CONT_BLOCK - 1) / rhg::CONT_BLOCK));
+    int tpp;
+    const dim3 blk(rhg::CONT_BLOCK), grd = cont_grid(npts, c->dm.ntile, tpp);
     hipLaunchKernelGGL((rhg::k_continuum<R, false>), grd, blk, 0, c->stream, c->d_model, d_ndep, ncol, Nmax,
-                       state, nfield, c->d_out_ls, c->nout, cchi, ceta, (const int32_t *) nullptr, (const int32_t *) nullptr, (const int32_t *) nullptr, 0);
+                       state, nfield, c->d_out_ls, c->nout, cchi, ceta, (const int32_t *) nullptr,
+                       (const int32_t *) nullptr, (const int32_t *) nullptr, 0, tpp);
     HIPCHECK(hipGetLastError());
   }
   return 0;
@@ -2029,12 +2065,12 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
                          c->d_model, d_ndep, ncol, Nmax, cols->atm_scale, cols->mu, B.state, nfield,
                          (int32_t *) c->moving.p, (double *) nullptr);
       HIPCHECK(hipGetLastError());
-      hipLaunchKernelGGL((rhg::k_continuum<double, false>),
-                         dim3((unsigned) ((npts + rhg::CONT_BLOCK - 1) / rhg::CONT_BLOCK)),
-                         dim3(rhg::CONT_BLOCK), 0, c->stream, c->d_model, d_ndep, ncol, Nmax,
-                         B.state, nfield, c->d_out_ls, nout, (double *) c->cchi.p,
-                         (double *) c->ceta.p, (const int32_t *) nullptr, (const int32_t *) nullptr,
-                         (const int32_t *) nullptr, 0);
+      int tpp;
+      const dim3 gcont = cont_grid(npts, c->dm.ntile, tpp);
+      hipLaunchKernelGGL((rhg::k_continuum<double, false>), gcont, dim3(rhg::CONT_BLOCK), 0, c->stream,
+                         c->d_model, d_ndep, ncol, Nmax, B.state, nfield, c->d_out_ls, nout,
+                         (double *) c->cchi.p, (double *) c->ceta.p, (const int32_t *) nullptr,
+                         (const int32_t *) nullptr, (const int32_t *) nullptr, 0, tpp);
       HIPCHECK(hipGetLastError());
       hipLaunchKernelGGL(rhg::k_nlte_bg,
                          dim3((unsigned) ((int64_t) ((ncol + 31) / 32) * ((Nmax + 31) / 32) *
@@ -2076,7 +2112,7 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
       const int nfe = nlist - h.nbez;
       int r = timed(slot, [&]() -> int {
         if (h.nbez > 0) {
-          const dim3 grd((unsigned) rhg::nlte_grid(nact, h.nbez));
+          const dim3 grd((unsigned) rhg::xcd_grid(nact, h.nbez));
 #define RHG_LAUNCH_BEZ(L, P, MS)                                                                 \
   hipLaunchKernelGGL((rhg::k_nlte_bezier<L, P, MS>), grd, dim3(2 * L),                            \
                      (size_t) Nmax * sizeof(double), c->stream, c->d_model, d_at, B, d_act, nact, \
@@ -2103,7 +2139,7 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
           // the member loops unrolled to the largest active set (one launch:
           // split by set size, the launches would not fill the GPU)
           const int per = fe_per(nact, rhg::NLTE_FE_RAYS);
-          const dim3 grd((unsigned) rhg::nlte_grid((nact + per - 1) / per, nfe));
+          const dim3 grd((unsigned) rhg::xcd_grid((nact + per - 1) / per, nfe));
           const size_t lds = rhg::nlte_fe_lds(Nmax, per, rhg::NLTE_FE_RAYS) * sizeof(double);
 #define RHG_LAUNCH_FE(MS)                                                                        \
   hipLaunchKernelGGL((rhg::k_nlte_feautrier<MS, false>), grd, b64, lds, c->stream, c->d_model, d_at, \
@@ -2217,7 +2253,7 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
       double *d_st = device_ptrs ? stokes_out + (size_t) c0 * 4 * nout : (double *) c->nl_st.p;
       const int nfe = nlist - h.nbez;
       if (h.nbez > 0) {
-        const dim3 grd((unsigned) rhg::nlte_grid(ncol, h.nbez));
+        const dim3 grd((unsigned) rhg::xcd_grid(ncol, h.nbez));
 #define RHG_LAUNCH_EM(L, P)                                                                      \
   hipLaunchKernelGGL((rhg::k_nlte_emergent<L, P>), grd, b64, 0, c->stream, c->d_model, d_at, B,       \
                      c->d_out_ls, d_iolist, h.nbez, cols->mu, d_st)
@@ -2227,7 +2263,7 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
       }
       if (nfe > 0) {
         const int per = fe_per(ncol, 1);
-        const dim3 grd((unsigned) rhg::nlte_grid((ncol + per - 1) / per, nfe));
+        const dim3 grd((unsigned) rhg::xcd_grid((ncol + per - 1) / per, nfe));
         hipLaunchKernelGGL((rhg::k_nlte_feautrier<2, true>), grd, b64,
                            rhg::nlte_fe_lds(Nmax, per, 1) * sizeof(double), c->stream, c->d_model,
                            d_at, B, (const int32_t *) nullptr, ncol, per, c->d_out_ls,

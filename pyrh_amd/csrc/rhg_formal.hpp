@@ -54,7 +54,7 @@ __device__ __forceinline__ void form_point(const DevModel &M, int ls, int has_li
 __device__ __forceinline__ int ray_io(const int32_t *io_list, int nlist, const int32_t *blk_grid,
                                       const int32_t *gptr, int ncol, int &cb) {
   int t;
-  xcd_tile(blockIdx.x, nlist, cb, t);
+  xcd_tile(blockIdx.x, (ncol + 63) / 64, nlist, cb, t);
   if (!blk_grid) return io_list[t];
   if (cb * 64 >= ncol) return -1;
   const int g = ldc(blk_grid)[cb];
@@ -66,7 +66,7 @@ __device__ __forceinline__ int ray_io(const int32_t *io_list, int nlist, const i
 // workgroup -> (column block, entry t of the wavelength list io_list)
 #define RAY_TILE()                                                                       \
   int cb, t;                                                                             \
-  xcd_tile(blockIdx.x, nlist, cb, t);                                                    \
+  xcd_tile(blockIdx.x, (ncol + 63) / 64, nlist, cb, t);                                  \
   const int io = io_list[t]
 // the same through ray_io (kernels that take wavelength grids)
 #define RAY_TILE_GRID()                                                                  \

@@ -164,7 +164,7 @@ k_state(const DevModel *__restrict__ Mp, const double *__restrict__ atmos, const
   // after another on one XCD, so the atmosphere's cache lines (16 depths of
   // one row of one column) are fetched into that XCD's L2 once
   int cb, k;
-  xcd_tile(blockIdx.x, Nmax, cb, k);
+  xcd_tile(blockIdx.x, (ncol + 63) / 64, Nmax, cb, k);
   const int ic = cb * 64 + (int) threadIdx.x;
   if (ic >= ncol) return;
   if (k >= ndep[ic]) return;
@@ -507,48 +507,46 @@ __global__ void k_scales(const DevModel *__restrict__ Mp, const int32_t *__restr
 }
 
 // ---------------------------------------------------------------------------
-// Stage 3: continuum opacity and emissivity for every output wavelength at
-// one (column, depth), the terms of continuum_point() with what depends on
-// T and ne alone evaluated once.  The bound-free sums
-// sum_c alpha_c(lambda) n_i,c are accumulated BF_TILE wavelengths at a time
-// in registers (one load of n_i,c per tile; the tile's cross-sections are
-// wave-uniform) and handed to the per-wavelength pass through LDS.  One
-// exponential per wavelength: exp(-hc/(k lambda T)) is the reciprocal of the
-// Planck function's exp(hc/(k lambda T)).
-// Output layout: cchi[(io * Nmax + k) * ncol + column].  With wavelength
-// grids (blk_grid != nullptr, ncol a multiple of 64) the columns of block
-// ic / 64 belong to grid g = blk_grid[ic / 64] (-1: none) and take the
-// bound-free tiles gtile[2 g] .. gtile[2 g + 1] - 1 only, the tiles that hold
-// the grid's wavelengths, and in them the wavelengths io whose bit is set in
-// the grid's mask, bit io % 32 of gmask[g * gwords + io / 32] (the GRID
-// instantiation; the other ignores the three grid arguments).
-template <typename R, bool GRID>
-__global__ void __launch_bounds__(CONT_BLOCK)
-k_continuum(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep, int ncol, int Nmax,
-            const double *__restrict__ state, int nfield, const int32_t *__restrict__ out_ls,
-            int nout, R *__restrict__ cchi, R *__restrict__ ceta,
-            const int32_t *__restrict__ blk_grid, const int32_t *__restrict__ gtile,
-            const int32_t *__restrict__ gmask, int gwords) {
-  const DevModel &M = *Mp;
-  __shared__ double bf_lds[BF_TILE][CONT_BLOCK];
-  const int64_t gid = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= (int64_t) ncol * Nmax) return;
-  const int k = (int) (gid / ncol), ic = (int) (gid % ncol);
-  if (k >= ndep[ic]) return;
-  int tile0 = 0, tile1 = M.ntile;
-  const int32_t *gm = nullptr;
-  if constexpr (GRID) {
-    // a wavefront is 64 consecutive slots of one depth (ncol is a multiple
-    // of 64), one block: its grid and tile range are wave-uniform, and kept
-    // in scalar registers so that the tile tables stay scalar loads
-    const int g = __builtin_amdgcn_readfirstlane(blk_grid[ic >> 6]);
-    if (g < 0) return;
-    tile0 = __builtin_amdgcn_readfirstlane(gtile[2 * g]);
-    tile1 = __builtin_amdgcn_readfirstlane(gtile[2 * g + 1]);
-    gm = gmask + (int64_t) g * gwords;
+// Stage 3
+
+// 1 / x by the hardware estimate refined by two Newton steps (relative error
+// ~1e-16)
+__device__ __forceinline__ double krcp(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  double e = fma(-x, r, 1.0);
+  r = fma(r, e, r);
+  e = fma(-x, r, 1.0);
+  return fma(r, e, r);
+}
+
+// Place of x in an ascending temperature table of n entries, clamped to its
+// ends (rh/hydrogen.c:509-523), and linear interpolation there.
+struct TabAt {
+  int i, i1;
+  double fx;
+  __device__ __forceinline__ TabAt(int n, const double *t, double x) {
+    const double f = clamp_index(n, t, x);
+    i = (int) f;
+    i1 = i == n - 1 ? i : i + 1;
+    fx = f - i;
   }
-  const int64_t fs = (int64_t) Nmax * ncol;
-  const double *st = state + (int64_t) k * ncol + ic;
+  struct Pair {
+    double a, b;
+  };
+  __device__ __forceinline__ Pair load(const double *g) const { return {g[i], g[i1]}; }
+  __device__ __forceinline__ double operator()(Pair g) const { return (1.0 - fx) * g.a + fx * g.b; }
+};
+
+// FP64: the terms of continuum_point() in its order.  One exponential per
+// wavelength: exp(-hc/(k lambda T)) is the reciprocal of the Planck
+// function's exp(hc/(k lambda T)).
+template <typename R, bool GRID>
+__device__ __forceinline__ void continuum_plain(const DevModel &M, const double *__restrict__ st, int64_t fs,
+                                                int64_t pt, int64_t npt,
+                                                const int32_t *__restrict__ out_ls, int nout,
+                                                int tile0, int tile1, const int32_t *gm,
+                                                double (*bf_lds)[CONT_BLOCK], R *__restrict__ cchi,
+                                                R *__restrict__ ceta) {
   const double T = st[RHG_CF_T * fs], ne = st[RHG_CF_NE * fs];
   const double nHmin = st[RHG_CF_NHMIN * fs], nH0 = st[RHG_CF_NH0 * fs], np = st[RHG_CF_NP * fs];
   const double nH2 = st[RHG_CF_NH2 * fs], nOH = st[RHG_CF_NOH * fs], nCH = st[RHG_CF_NCH * fs];
@@ -668,11 +666,199 @@ k_continuum(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep, i
         chi_ai += chi;
         eta_ai += chi * Bnu;
       }
-      const int64_t o = ((int64_t) io * Nmax + k) * ncol + ic;
+      const int64_t o = io * npt + pt;
       cchi[o] = (R) chi_ai;
       ceta[o] = (R) eta_ai;
     }
   }
+}
+
+// FP32 form (FP64 arithmetic, stored in float): contracted, with the
+// wavelength's part of the table look-ups done beforehand (ktab) and one
+// exponential and one reciprocal for the Planck function and exp(-x): 23900
+// vector instructions per 64 points and 112 wavelengths where
+// continuum_plain takes 42800.  Bound by the latency of its loads (level
+// populations again for every tile, table gathers), so BF_AHEAD populations
+// are loaded at a time (2.94 ms without, 2.43 with, for 16384 columns of 82
+// depths; 2.76 before); in continuum_plain that spills and is slower.
+template <typename R, bool GRID>
+__device__ __forceinline__ void continuum_fast(const DevModel &M, const double *__restrict__ st, int64_t fs,
+                                                int64_t pt, int64_t npt,
+                                                const int32_t *__restrict__ out_ls, int nout,
+                                                int tile0, int tile1, const int32_t *gm,
+                                                double (*bf_lds)[CONT_BLOCK], R *__restrict__ cchi,
+                                                R *__restrict__ ceta) {
+#pragma clang fp contract(fast)
+  const double T = st[RHG_CF_T * fs], ne = st[RHG_CF_NE * fs];
+  const double nHmin = st[RHG_CF_NHMIN * fs], nH0 = st[RHG_CF_NH0 * fs], np = st[RHG_CF_NP * fs];
+  const double nH2 = st[RHG_CF_NH2 * fs], nOH = st[RHG_CF_NOH * fs], nCH = st[RHG_CF_NCH * fs];
+  const double C0 = Q_ELECTRON * Q_ELECTRON / (4.0 * PI * EPSILON_0) / sqrt(M_ELECTRON);
+  const double sigma_ff = 4.0 / 3.0 * sqrt(2.0 * PI / (3.0 * KBOLTZMANN)) * (C0 * C0 * C0) /
+                          (HPLANCK * CLIGHT);
+  // T- and ne-only factors (rh/hydrogen.c:509-523 table indices)
+  const double iT = 1.0 / T;
+  const double pe = ne * KBOLTZMANN * T;
+  const TabAt at_hmin(NTHETA, M.hminff_theta, THETA0 * iT), at_h2m(NTHETA_H2, M.h2mff_theta, THETA0 * iT),
+      at_h2p(NTEMP_H2P, M.h2pff_temp, T), at_oh(NTOH, M.oh_T, T), at_ch(NTCH, M.ch_T, T);
+  const double sqrt_theta = sqrt(THETA0 * iT), sff_T = sigma_ff / sqrt(T) * (ne * np);
+  const double f_hmin = (nH0 * 1.0E-29) * pe, f_hff = nH0 * (ne * (KBOLTZMANN * THETA0 * 1.0E-32));
+  const double f_h2p = (nH0 * 1.0E-29) * (np * 1.0E-20);
+  const double f_h2m = nH2 > 0.0 ? (nH2 * 1.0E-29) * pe : 0.0;
+  const double y_fac = T * (1.0 / (HPLANCK * CLIGHT));
+  const double f_oh = (T < ldc(M.oh_T)[0] || T > ldc(M.oh_T)[NTOH - 1]) ? 0.0 : nOH * (CM_TO_M * CM_TO_M);
+  const double f_ch = (T < ldc(M.ch_T)[0] || T > ldc(M.ch_T)[NTCH - 1]) ? 0.0 : nCH * (CM_TO_M * CM_TO_M);
+
+  for (int t = tile0; t < tile1; t++) {
+    const int io0 = t * BF_TILE;
+    {
+      double bf[BF_TILE];
+#pragma unroll
+      for (int j = 0; j < BF_TILE; j++) bf[j] = 0.0;
+      const int e0 = ldc(M.tile_ptr)[t], e1 = ldc(M.tile_ptr)[t + 1];
+      for (int e = e0; e < e1; e += BF_AHEAD) {
+        double ni[BF_AHEAD];
+#pragma unroll
+        for (int q = 0; q < BF_AHEAD; q++)
+          ni[q] = st[cont_field(ldc(M.tile_cont)[e + q < e1 ? e + q : e]) * fs];
+#pragma unroll
+        for (int q = 0; q < BF_AHEAD; q++) {
+          if (e + q < e1) {
+            const CDouble *al = ldc(M.tile_alpha) + (int64_t) (e + q) * BF_TILE;
+#pragma unroll
+            for (int j = 0; j < BF_TILE; j++) bf[j] += al[j] * ni[q];
+          }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < BF_TILE; j++) bf_lds[j][threadIdx.x] = bf[j];
+    }
+    const int nj = (nout - io0 < BF_TILE) ? nout - io0 : BF_TILE;
+#pragma unroll 1
+    for (int j = 0; j < nj; j++) {
+      const int io = io0 + j;
+      if constexpr (GRID)
+        if (!(((uint32_t) ldc(gm)[io >> 5] >> (io & 31)) & 1u)) continue;
+      const double bfj = bf_lds[j][threadIdx.x];
+      const int ls = ldc(out_ls)[io];
+      const CDouble *lc = ldc(M.lamconst) + (int64_t) ls * RHG_LC_NCONST;
+      const double *kt = M.ktab + (int64_t) ls * KT_N;
+      const double hc_kla = lc[RHG_LC_HC_KLA], twohnu3 = lc[RHG_LC_TWOHNU3_C2];
+      const double x = hc_kla * iT;
+      // every table entry of the wavelength is loaded here, at once: loads
+      // inside the branches below would each be waited for
+      const TabAt::Pair g_hmin = at_hmin.load(kt + KT_HMFF), g_h2m = at_h2m.load(kt + KT_H2M),
+          g_h2p = at_h2p.load(kt + KT_H2P), g_oh = at_oh.load(kt + KT_OH), g_ch = at_ch.load(kt + KT_CH);
+      // the stimulated-emission factor exp(-x) and the Planck function,
+      // rh/planck.c:38-63; past MAX_EXPONENT both are 0
+      const double stim = x <= MAX_EXPONENT ? exp(-x) : 0.0;
+      const double Bnu = twohnu3 * stim * krcp(1.0 - stim);
+      // chi_ai, eta_ai: terms without a source of their own; chi_B: those
+      // that emit with the Planck function
+      double chi_ai = 0.0, eta_ai = 0.0, chi_B;
+      if (lc[RHG_LC_HMIN_BF_ON] != 0.0) {
+        const double a = nHmin * lc[RHG_LC_HMIN_BF_ALPHA];
+        chi_ai = a * (1.0 - stim);
+        eta_ai = a * (twohnu3 * stim);
+      }
+      if (lc[RHG_LC_HMIN_FF_LIDX] >= 0.0) {
+        chi_B = f_hmin * at_hmin(g_hmin);
+      } else {
+        double theta_n = 1.0;
+        chi_B = 0.0;
+        for (int n = 1; n < 6; n++) {
+          theta_n *= sqrt_theta;
+          chi_B += theta_n * lc[RHG_LC_HFF_LONG0 + n - 1];
+        }
+        chi_B *= f_hff;
+      }
+      chi_ai *= lc[RHG_LC_HMIN_FUDGE];
+      eta_ai *= lc[RHG_LC_HMIN_FUDGE];
+      chi_B *= lc[RHG_LC_HMIN_FUDGE];
+      if (lc[RHG_LC_OH_EIDX] >= 0.0 && f_oh != 0.0) {
+        const double a = f_oh * exp(LG10 * at_oh(g_oh));
+        chi_ai += a * (1.0 - stim);
+        eta_ai += a * (twohnu3 * stim);
+      }
+      if (lc[RHG_LC_CH_EIDX] >= 0.0 && f_ch != 0.0) {
+        const double a = f_ch * exp(LG10 * at_ch(g_ch));
+        chi_ai += a * (1.0 - stim);
+        eta_ai += a * (twohnu3 * stim);
+      }
+      // bound-free (hydrogen and metals), rh/hydrogen.c:300-330,
+      // rh/metal.c:120-140: their h c / k lambda is rounded in another order,
+      // usually to the same value, else a unit in the last place off
+      {
+        const double bf_kla = lc[RHG_LC_BF_HC_KLA];
+        const double expla = fabs(bf_kla - hc_kla) <= 4.0E-16 * hc_kla ? stim : exp(-bf_kla * iT);
+        chi_ai += (1.0 - expla) * bfj;
+        eta_ai += lc[RHG_LC_BF_TWOHNU3_C2] * expla * bfj;
+      }
+      {
+        const double y = lc[RHG_LC_GFF_CY] * y_fac, x3 = lc[RHG_LC_GFF_X3];
+        const double gIII = 1.0 + 0.1728 * x3 * (1.0 + y) - 0.0496 * (x3 * x3) * (1.0 + (1.0 + y) * 0.33333333 * y);
+        const double g_ff = (gIII > 1.0) ? gIII : 1.0;
+        chi_B += sff_T * lc[RHG_LC_HFF_NU3] * (1.0 - stim) * g_ff;
+      }
+      if (lc[RHG_LC_H2P_LIDX] >= 0.0) chi_B += f_h2p * at_h2p(g_h2p);
+      if (lc[RHG_LC_H2M_LIDX] >= 0.0) chi_B += f_h2m * at_h2m(g_h2m);
+      const int64_t o = io * npt + pt;
+      cchi[o] = (R) (chi_ai + chi_B);
+      ceta[o] = (R) (eta_ai + chi_B * Bnu);
+    }
+  }
+}
+
+// Stage 3: continuum opacity and emissivity for every output wavelength at
+// one (column, depth), the terms of continuum_point() with what depends on
+// T and ne alone evaluated once.  The bound-free sums
+// sum_c alpha_c(lambda) n_i,c are accumulated BF_TILE wavelengths at a time
+// in registers (one load of n_i,c per tile; the tile's cross-sections are
+// wave-uniform) and handed to the per-wavelength pass through LDS.
+// Output layout: cchi[(io * Nmax + k) * ncol + column].  With wavelength
+// grids (blk_grid != nullptr, ncol a multiple of 64) the columns of block
+// ic / 64 belong to grid g = blk_grid[ic / 64] (-1: none) and take the
+// bound-free tiles gtile[2 g] .. gtile[2 g + 1] - 1 only, the tiles that hold
+// the grid's wavelengths, and in them the wavelengths io whose bit is set in
+// the grid's mask, bit io % 32 of gmask[g * gwords + io / 32] (the GRID
+// instantiation; the other ignores the three grid arguments).
+// blockIdx.y takes tpp tiles: the tiles are split over workgroups where the
+// points alone leave SIMDs idle (cont_grid): one column 337 -> 60 us, 512
+// mixed columns at 2000 wavelengths 7.4 -> 4.3 ms (3.5 with continuum_fast).
+template <typename R, bool GRID>
+__global__ void __launch_bounds__(CONT_BLOCK, 4)
+k_continuum(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep, int ncol, int Nmax,
+            const double *__restrict__ state, int nfield, const int32_t *__restrict__ out_ls,
+            int nout, R *__restrict__ cchi, R *__restrict__ ceta,
+            const int32_t *__restrict__ blk_grid, const int32_t *__restrict__ gtile,
+            const int32_t *__restrict__ gmask, int gwords, int tpp) {
+  const DevModel &M = *Mp;
+  __shared__ double bf_lds[BF_TILE][CONT_BLOCK];
+  const int64_t gid = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+  if (gid >= (int64_t) ncol * Nmax) return;
+  const int k = (int) (gid / ncol), ic = (int) (gid % ncol);
+  if (k >= ndep[ic]) return;
+  int tile0 = 0, tile1 = M.ntile;
+  const int32_t *gm = nullptr;
+  if constexpr (GRID) {
+    // a wavefront is 64 consecutive slots of one depth (ncol is a multiple
+    // of 64), one block: its grid and tile range are wave-uniform, and kept
+    // in scalar registers so that the tile tables stay scalar loads
+    const int g = __builtin_amdgcn_readfirstlane(blk_grid[ic >> 6]);
+    if (g < 0) return;
+    tile0 = __builtin_amdgcn_readfirstlane(gtile[2 * g]);
+    tile1 = __builtin_amdgcn_readfirstlane(gtile[2 * g + 1]);
+    gm = gmask + (int64_t) g * gwords;
+  }
+  tile0 += (int) blockIdx.y * tpp;
+  if (tile0 >= tile1) return;
+  if (tile1 > tile0 + tpp) tile1 = tile0 + tpp;
+  const int64_t fs = (int64_t) Nmax * ncol;
+  const double *st = state + (int64_t) k * ncol + ic;
+  const int64_t pt = (int64_t) k * ncol + ic;
+  if constexpr (sizeof(R) == 4)
+    continuum_fast<R, GRID>(M, st, fs, pt, fs, out_ls, nout, tile0, tile1, gm, bf_lds, cchi, ceta);
+  else
+    continuum_plain<R, GRID>(M, st, fs, pt, fs, out_ls, nout, tile0, tile1, gm, bf_lds, cchi, ceta);
 }
 
 #define RHG_KSTATE(NN)                                                                       \
@@ -691,7 +877,8 @@ RHG_KSTATE(8)
 #define RHG_KCONT(R, G)                                                                       \
   template __global__ void k_continuum<R, G>(const DevModel *, const int32_t *, int, int,      \
                                              const double *, int, const int32_t *, int, R *, R *, \
-                                             const int32_t *, const int32_t *, const int32_t *, int);
+                                             const int32_t *, const int32_t *, const int32_t *, int, \
+                                             int);
 RHG_KCONT(double, false)
 RHG_KCONT(double, true)
 RHG_KCONT(float, false)

@@ -70,30 +70,54 @@ struct DevModel {
   int ntile;
   const int32_t *tile_ptr, *tile_cont;
   const double *tile_alpha;
+  // per wavelength, the temperature tables of its continuum terms with the
+  // wavelength already interpolated: KT_N doubles, tables at KT_*
+  const double *ktab;
   // molecule stoichiometry as a dense table [nmol][NNUC_MAX] of counts
   const double *mol_cnt;
 };
 
-// output wavelengths per bound-free tile of k_continuum, and its block size
-constexpr int BF_TILE = 16;
+// output wavelengths per bound-free tile of k_continuum, the level
+// populations it loads ahead of their use, and its block size
+constexpr int BF_TILE = 16, BF_AHEAD = 8;
 constexpr int CONT_BLOCK = 256;
+enum { KT_HMFF = 0, KT_H2M = KT_HMFF + NTHETA, KT_H2P = KT_H2M + NTHETA_H2,
+       KT_OH = KT_H2P + NTEMP_H2P, KT_CH = KT_OH + NTOH, KT_N = KT_CH + NTCH };
 
-// Workgroup -> (column block of 64, output wavelength) for the per-ray
-// kernels.  Workgroups are dispatched round-robin over the 8 XCDs (linear
-// id mod 8), each XCD with its own L2; the mapping sends all nout
-// wavelengths of a column block to one XCD, consecutively, so that the
-// block's column state is fetched into that L2 once and reused by every
-// wavelength.  Launch xcd_grid(ncb, nout) workgroups; ids that map past the
-// last column block return cb >= ncb.
-constexpr int NXCD = 8;
-__host__ __device__ __forceinline__ int64_t xcd_grid(int ncb, int nout) {
-  return (int64_t) ((ncb + NXCD - 1) / NXCD) * NXCD * nout;
+// Workgroup -> (column block cb, entry t < n of the block's list: output
+// wavelengths or depths).  Workgroups are dispatched round-robin over the 8
+// XCDs (linear id mod 8), each XCD with its own L2.  The mapping deals out
+// pieces of a block's list, the first block's first: a piece's entries run
+// one after another on one XCD, so that what the block's entries share is
+// fetched into that L2 once.  A list stays whole from XCD_PIECES blocks on;
+// fewer blocks are cut into about that many pieces in all, as otherwise a
+// batch of fewer than 8 blocks leaves XCDs idle and one of blocks of
+// different depth (sorted, deepest first) waits for the XCD of the deepest
+// (512 columns of 64 to 256 depths, 2000 wavelengths: formal solution 59 ms
+// with whole lists, 35 in pieces; response functions of 90 columns
+// 82 ms and 33).  Launch xcd_grid(ncb, n) workgroups; ids past the end of a
+// list or of the blocks return cb = ncb, t = 0.
+constexpr int NXCD = 8, XCD_PIECES = 64;
+__host__ __device__ __forceinline__ int xcd_pieces(int ncb, int n) {
+  const int p = (XCD_PIECES + ncb - 1) / ncb;
+  return p < n ? p : n;
 }
-__device__ __forceinline__ void xcd_tile(int64_t b, int nout, int &cb, int &io) {
-  const int64_t per_group = (int64_t) NXCD * nout;
-  const int64_t g = b / per_group, r = b % per_group;
-  cb = (int) (g * NXCD + r % NXCD);
-  io = (int) (r / NXCD);
+__host__ __device__ __forceinline__ int64_t xcd_grid(int ncb, int n) {
+  const int p = xcd_pieces(ncb, n), len = (n + p - 1) / p;
+  return (((int64_t) ncb * p + NXCD - 1) / NXCD) * NXCD * len;
+}
+__device__ __forceinline__ void xcd_tile(uint32_t b, int ncb, int n, int &cb, int &t) {
+  const uint32_t p = xcd_pieces(ncb, n), len = (n + p - 1) / p;
+  const uint32_t g = b / (NXCD * len), r = b % (NXCD * len), piece = g * NXCD + r % NXCD;
+  cb = (int) (piece / p);
+  // a block's pieces rotate from one round over the XCDs to the next, so that
+  // no XCD gets the same (perhaps costlier) part of every block
+  const uint32_t part = (piece % p + cb * p / NXCD) % p;
+  t = (int) (part * len + r / NXCD);
+  if (cb >= ncb || t >= n) {
+    cb = ncb;
+    t = 0;
+  }
 }
 
 // Column state layout: state[(field * Nmax + k) * ncol + column]; fields
@@ -478,7 +502,7 @@ template <typename R, bool GRID>
 __global__ void k_continuum(const DevModel *M, const int32_t *ndep, int ncol, int Nmax,
                             const double *state, int nfield, const int32_t *out_ls, int nout,
                             R *cchi, R *ceta, const int32_t *blk_grid, const int32_t *gtile,
-                            const int32_t *gmask, int gwords);
+                            const int32_t *gmask, int gwords, int tpp);
 template <typename R, bool MO, bool LT>
 __global__ void k_formal_stokes(const DevModel *M, const int32_t *ndep, const int32_t *moving,
                                 int ncol, int Nmax, const double *state, const int32_t *out_ls,

@@ -646,19 +646,6 @@ __device__ __forceinline__ void ray_points(const NlteBufs &B, int64_t col, int t
   }
 }
 
-// Workgroup -> (slot of the active columns, entry of the wavelength list): the
-// wavelengths of a column on one XCD (xcd_tile), or, with fewer columns than
-// XCDs, over all of them.
-__device__ __forceinline__ bool nlte_tile(int nact, int nlist, int &slot, int &il) {
-  if (nact >= NXCD) {
-    xcd_tile(blockIdx.x, nlist, slot, il);
-    return slot < nact;
-  }
-  slot = (int) (blockIdx.x / nlist);
-  il = (int) (blockIdx.x % nlist);
-  return slot < nact;
-}
-
 // Wavelengths with an active line, one (column, wavelength) per workgroup of
 // 2 L threads:
 // the rays in both directions, the new mean intensity and with eval_op the
@@ -684,7 +671,8 @@ k_nlte_bezier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap, N
   const DevModel &M = *Mp;
   const DevNlte &A = *Ap;
   int slot, il;
-  if (!nlte_tile(nact, nlist, slot, il)) return;
+  xcd_tile(blockIdx.x, nact, nlist, slot, il);
+  if (slot >= nact) return;
   const int ic = act[slot], io = io_list[il], ls = out_ls[io];
   const int N = B.ndep[ic], nrays = A.nrays;
   const int64_t fs = B.fs, col = (int64_t) ic * B.Kp;
@@ -839,7 +827,8 @@ k_nlte_emergent(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap,
   const DevModel &M = *Mp;
   const DevNlte &A = *Ap;
   int ic, il;
-  if (!nlte_tile(B.ncol, nlist, ic, il)) return;
+  xcd_tile(blockIdx.x, B.ncol, nlist, ic, il);
+  if (ic >= B.ncol) return;
   const int io = io_list[il], ls = out_ls[io], N = B.ndep[ic];
   const int64_t fs = B.fs, col = (int64_t) ic * B.Kp, wo = (int64_t) io * fs + col;
   const double *Jl = B.J + B.jpar[ic] * (int64_t) B.nout * fs + wo;
@@ -913,7 +902,8 @@ k_nlte_feautrier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap
   const DevModel &M = *Mp;
   const DevNlte &A = *Ap;
   int grp, il;
-  if (!nlte_tile((nact + per - 1) / per, nlist, grp, il)) return;
+  xcd_tile(blockIdx.x, (nact + per - 1) / per, nlist, grp, il);
+  if (grp >= (nact + per - 1) / per) return;
   const int io = io_list[il], ls = out_ls[io], nrays = EM ? 1 : A.nrays;
   const int first = grp * per, n_it = nact - first < per ? nact - first : per;
   const int64_t fs = B.fs, jb = (int64_t) B.nout * fs;

@@ -89,10 +89,6 @@ __global__ void k_nlte_feautrier(const DevModel *Mp, const DevNlte *Ap, NlteBufs
                                  const int32_t *act, int nact, int per, const int32_t *out_ls,
                                  const int32_t *io_list, int nlist, int il_off, int nlist_all,
                                  int eval_op, double mu_em, double *stokes);
-// workgroups of the two kernels above for nact columns (or column groups)
-inline int64_t nlte_grid(int nact, int nlist) {
-  return nact >= NXCD ? xcd_grid(nact, nlist) : (int64_t) nact * nlist;
-}
 __global__ void k_nlte_flip(NlteBufs B, const int32_t *act, int nact);
 template <int L, int P>
 __global__ void k_nlte_emergent(const DevModel *Mp, const DevNlte *Ap, NlteBufs B,

@@ -71,7 +71,7 @@ __device__ __forceinline__ T point_get(const Point<T> &p, int m) {
 #define RF_SETUP()                                                                       \
   const DevModel &M = *Mp;                                                               \
   int cb, t;                                                                             \
-  xcd_tile(blockIdx.x, nlist, cb, t);                                                    \
+  xcd_tile(blockIdx.x, (ncol + 63) / 64, nlist, cb, t);                                  \
   const int ic = cb * 64 + threadIdx.x;                                                  \
   if (ic >= ncol) return;                                                                \
   const int io = io_list[t];                                                             \
@@ -87,7 +87,7 @@ __device__ __forceinline__ T point_get(const Point<T> &p, int m) {
 // takes part in staging it)
 #define RF_LINE_TABLE()                                                                  \
   int cb0, t0;                                                                           \
-  xcd_tile(blockIdx.x, nlist, cb0, t0);                                                  \
+  xcd_tile(blockIdx.x, (ncol + 63) / 64, nlist, cb0, t0);                                \
   if (cb0 * 64 >= ncol) return;                                                          \
   auto tab = [&]() {                                                                     \
     const int ls0 = out_ls[io_list[t0]];                                                 \
