@@ -392,6 +392,18 @@ int rhg_rf_lte_params(rhg_context_t *ctx, const rhg_columns_t *cols, int32_t pre
                       int32_t device_ptrs, int32_t nparam, const int32_t *params,
                       double *stokes_out, void *rf_out);
 
+/* The response functions of rhg_rf_lte_params contracted with the gradient of
+ * a loss with respect to the Stokes vector, on device memory of GPU `device`:
+ *   atmos_grad[(c * 9 + row) * ndep + k] =
+ *       sum_{s, l} grad[(c * 4 + s) * nout + l] * rf[...]
+ * for the atmosphere row of each of the nparam parameters (other rows are
+ * left alone).  rf holds floats (precision RHG_PREC_FP32) or doubles; work
+ * holds 4 nout ncol doubles.  Asynchronous on the HIP stream `stream` (0: the
+ * default stream).  No counterpart in the reference. */
+int rhg_rf_contract(int32_t device, void *stream, int32_t precision, int32_t nparam,
+                    const int32_t *params, int32_t ncol, int32_t ndep, int32_t nout,
+                    const void *rf, const double *grad, double *work, double *atmos_grad);
+
 /* d I / d log gf of the emergent intensity, the reference's analytic atomic
  * response functions: compute1d(get_atomic_rfs=True) (pyrh.pyx:604-660;
  * rh/rhf1d/bezier_1D.c:416-536, rh/kurucz.c:224-260, 696-699,

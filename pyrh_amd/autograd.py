@@ -18,7 +18,7 @@ constants.
 """
 from __future__ import annotations
 
-from .engine import RF_PARAMS, RF_ROWS
+from .engine import RF_PARAMS, RF_ROWS, rf_contract
 
 try:
     import torch
@@ -29,6 +29,17 @@ except ImportError:  # pragma: no cover - the product path needs torch for this 
 def _require_torch():
     if torch is None:
         raise RuntimeError("pyrh_amd.autograd needs PyTorch")
+
+
+def _contract_here(rf, g, shape):
+    """Whether backward may run rhg_rf_contract: plain CUDA tensors of one
+    device, the saved response functions as forward laid them out (a
+    saved-tensor hook may return others), and no graph of the backward itself
+    (create_graph), which torch has to see the operations of."""
+    return (type(rf) is torch.Tensor and type(g) is torch.Tensor and g.is_cuda
+            and rf.device == g.device and rf.dtype in (torch.float32, torch.float64)
+            and tuple(rf.shape) == shape and rf.is_contiguous()
+            and not (torch.is_grad_enabled() and (g.requires_grad or rf.requires_grad)))
 
 
 class _StokesFn(torch.autograd.Function if torch is not None else object):
@@ -57,7 +68,7 @@ class _StokesFn(torch.autograd.Function if torch is not None else object):
         engine.rf_lte_device(atmos.data_ptr(), ndep.data_ptr(), ncol, nd, st.data_ptr(),
                              rf.data_ptr(), mu=mu, precision=precision, params=params)
         ctx.save_for_backward(rf)
-        ctx.rows = [RF_ROWS[i] for i in ids]
+        ctx.ids = ids
         ctx.shape = atmos.shape
         return st
 
@@ -65,11 +76,19 @@ class _StokesFn(torch.autograd.Function if torch is not None else object):
     def backward(ctx, grad):
         (rf,) = ctx.saved_tensors
         g = grad.to(torch.float64)                                  # [ncol, 4, nout]
+        ncol, _, nd = ctx.shape
+        out = torch.zeros(ctx.shape, dtype=torch.float64, device=grad.device)
+        if _contract_here(rf, g, (len(ctx.ids), nd, 4, g.shape[-1], ncol)):
+            g = g.contiguous()
+            work = torch.empty(g.numel(), dtype=torch.float64, device=g.device)
+            rf_contract(g.device.index, torch.cuda.current_stream(g.device).cuda_stream,
+                        1 if rf.dtype == torch.float32 else 0, ctx.ids, ncol, nd, g.shape[-1],
+                        rf.data_ptr(), g.data_ptr(), work.data_ptr(), out.data_ptr())
+            return out, None, None, None, None
         # d L / d p(k) = sum over (Stokes, wavelength) of grad * rf
         contr = torch.einsum("csl,pkslc->cpk", g, rf.to(torch.float64))
-        out = torch.zeros(ctx.shape, dtype=torch.float64, device=grad.device)
-        for i, row in enumerate(ctx.rows):
-            out[:, row, :] = contr[:, i, :]
+        for i, p in enumerate(ctx.ids):
+            out[:, RF_ROWS[p], :] = contr[:, i, :]
         return out, None, None, None, None
 
 

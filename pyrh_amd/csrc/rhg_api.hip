@@ -1693,6 +1693,40 @@ int rhg_rf_lte_params(rhg_context_t *c, const rhg_columns_t *cols, int32_t preci
   return 0;
 }
 
+int rhg_rf_contract(int32_t device, void *stream, int32_t precision, int32_t nparam,
+                    const int32_t *params, int32_t ncol, int32_t ndep, int32_t nout,
+                    const void *rf, const double *grad, double *work, double *atmos_grad) {
+  if (!params || !rf || !grad || !work || !atmos_grad) return fail(RHG_EINVAL, "null argument");
+  if (precision != RHG_PREC_FP64 && precision != RHG_PREC_FP32)
+    return fail(RHG_EINVAL, "precision must be RHG_PREC_FP64 or RHG_PREC_FP32");
+  if (nparam < 1 || nparam > RHG_RF_NPARAM || ncol < 1 || ndep < 1 || ndep > RHG_MAX_DEPTH ||
+      nout < 1 || nout > 65535)
+    return fail(RHG_EINVAL, "bad batch shape");
+  rhg::RfRowList rows{};
+  for (int i = 0; i < nparam; i++) {
+    if (params[i] < 0 || params[i] >= RHG_RF_NPARAM) return fail(RHG_EINVAL, "unknown parameter");
+    rows.row[i] = kRfParam[params[i]].row;
+  }
+  int before = 0;
+  HIPCHECK(hipGetDevice(&before));
+  HIPCHECK(hipSetDevice(device));
+  const int nm = 4 * nout;
+  hipStream_t st = (hipStream_t) stream;
+  hipLaunchKernelGGL(rhg::k_rf_turn, dim3((unsigned) ((ncol + 31) / 32), (unsigned) ((nm + 31) / 32)),
+                     dim3(256), 0, st, grad, ncol, nm, work);
+  const dim3 grd((unsigned) ((ncol + 63) / 64), (unsigned) ((ndep + 1) / 2), (unsigned) nparam), blk(64);
+  if (precision == RHG_PREC_FP32)
+    hipLaunchKernelGGL(rhg::k_rf_contract<float>, grd, blk, 0, st, (const float *) rf,
+                       (const double *) work, ncol, ndep, nm, rows, atmos_grad);
+  else
+    hipLaunchKernelGGL(rhg::k_rf_contract<double>, grd, blk, 0, st, (const double *) rf,
+                       (const double *) work, ncol, ndep, nm, rows, atmos_grad);
+  const hipError_t e = hipGetLastError();
+  HIPCHECK(hipSetDevice(before));
+  if (e != hipSuccess) return fail(RHG_EDEVICE, std::string("rhg_rf_contract: ") + hipGetErrorString(e));
+  return 0;
+}
+
 int rhg_rf_loggf(rhg_context_t *c, const rhg_columns_t *cols, int32_t npar,
                  const int32_t *par_line, int32_t device_ptrs, double *stokes_out,
                  double *rf_out) {

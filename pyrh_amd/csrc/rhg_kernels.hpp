@@ -530,6 +530,11 @@ struct RfShiftList {
 __global__ void k_rf_perturb(const double *atmos, double *out, int64_t n, int Nmax,
                              RfShiftList shift);
 __global__ void k_rf_rep_ndep(const int32_t *ndep, int ncol, int32_t *out);
+struct RfRowList { int row[RHG_RF_NPARAM]; };
+__global__ void k_rf_turn(const double *in, int ncol, int nm, double *out);
+template <typename R>
+__global__ void k_rf_contract(const R *rf, const double *gT, int ncol, int nd, int nm, RfRowList rows,
+                              double *out);
 template <typename O>
 __global__ void k_rf_diff(const double *S, int64_t W, int64_t off_p, int64_t off_m, int ncol,
                           int64_t nrows, double scale, O *out);

@@ -36,6 +36,16 @@ NLTE_TIMINGS = ("setup_ms", "scatter_bezier_ms", "iter_bezier_ms", "stateq_ms", 
 TUNE_KEYS = ("line_table", "column_sort", "wave_order")
 
 
+def rf_contract(device, stream, precision, params, ncol, ndep, nout, d_rf, d_grad, d_work,
+                d_atmos_grad):
+    """rhg_rf_contract on device pointers (ints), asynchronous on the HIP
+    stream handle `stream`; params are ids into RF_PARAMS."""
+    ids = np.ascontiguousarray(params, dtype=np.int32)
+    _check(lib().rhg_rf_contract(int(device), stream, int(precision), int(ids.size),
+                                 ids.ctypes.data_as(C.POINTER(C.c_int32)), int(ncol), int(ndep),
+                                 int(nout), d_rf, d_grad, d_work, d_atmos_grad))
+
+
 class EngineError(RuntimeError):
     pass
 
@@ -85,6 +95,9 @@ def lib():
                                  C.c_void_p]
         L.rhg_rf_lte_params.argtypes = [C.c_void_p, C.POINTER(RhgColumns), C.c_int32, C.c_int32,
                                         C.c_int32, C.POINTER(C.c_int32), PD, C.c_void_p]
+        L.rhg_rf_contract.argtypes = [C.c_int32, C.c_void_p, C.c_int32, C.c_int32,
+                                      C.POINTER(C.c_int32), C.c_int32, C.c_int32, C.c_int32,
+                                      C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
         L.rhg_rf_loggf.argtypes = [C.c_void_p, C.POINTER(RhgColumns), C.c_int32,
                                    C.POINTER(C.c_int32), C.c_int32, PD, PD]
         L.rhg_nlte_solve.argtypes = [C.c_void_p, C.c_void_p, C.POINTER(RhgColumns), C.c_int32,

@@ -75,3 +75,33 @@ def test_autograd_against_finite_differences(eng):
             print(f"row {row} depth {k}: adjoint {ad:.6e}  fd {fd:.6e}  "
                   f"diff/max {abs(ad - fd) / gmax:.2e}", flush=True)
             assert abs(ad - fd) <= 1e-3 * gmax
+
+
+@pytest.mark.parametrize("ncol,nd,params", [(1, 82, ("T",)), (33, 51, ("B", "T", "vmic")),
+                                            (64, 82, ("chi", "gamma")), (97, 37, None)])
+@pytest.mark.parametrize("precision", (0, 1))
+def test_autograd_contraction_forms(eng, ncol, nd, params, precision):
+    """The contraction kernel against torch's, over column and depth counts off
+    its tiles, parameter subsets, and gradients that are expanded, transposed
+    or float; with create_graph the backward stays differentiable.  The sums
+    run over 448 terms in FP64 in another order: 1e-12 of the largest."""
+    import torch
+    from pyrh_amd import autograd
+    from pyrh_amd.engine import RF_PARAMS
+    params = params or RF_PARAMS
+    atm, _ = W.mixed_batch(ncol, seed=W.SEED_BASE + 83, ndep_choices=(nd,))
+    x = torch.from_numpy(atm).cuda().requires_grad_(True)
+    st = autograd.stokes(eng, x, precision=precision, params=params)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    dense = torch.randn(st.shape, generator=g, dtype=torch.float64, device="cuda")
+    turned = torch.randn(st.shape[::-1], generator=g, dtype=torch.float64, device="cuda").permute(2, 1, 0)
+    one = torch.ones((), dtype=torch.float64, device="cuda").expand(st.shape)
+    for grad in (dense, turned, one):
+        (a,) = torch.autograd.grad(st, x, grad, retain_graph=True)
+        w = grad.clone().requires_grad_(True)
+        (b,) = torch.autograd.grad(st, x, w, retain_graph=True, create_graph=True)
+        assert b.requires_grad and not a.requires_grad
+        c = b.detach()
+        assert float((a - c).abs().max()) <= 1e-12 * float(c.abs().max())
+        (d,) = torch.autograd.grad(b.sum(), w)      # the Jacobian summed over the rows
+        assert d.shape == st.shape and bool(torch.isfinite(d).all()) and float(d.abs().max()) > 0
