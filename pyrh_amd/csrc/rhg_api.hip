@@ -63,6 +63,9 @@ static __device__ __align__(256) unsigned char scratch[RHG_NOALLOC_SCRATCH_BYTES
 namespace {
 
 constexpr int kMaxDevices = 64;
+// split_points: rays of a batch and bytes of its points, at most
+constexpr int64_t kSplitRays = 8192;
+constexpr size_t kSplitBytes = (size_t) 4 << 30;
 // the hydrostatic builder's records held at a time: 16384 columns of 82
 // depths and 99 elements
 constexpr size_t kHseRecBytes = (size_t) 4 << 30;
@@ -508,6 +511,32 @@ static dim3 cont_grid(int64_t npts, int ntile, int &tpp) {
   return dim3((unsigned) nb, (unsigned) std::max(1, (ntile + tpp - 1) / std::max(tpp, 1)));
 }
 
+// Depths per workgroup of a kernel that is independent over depth, for `rays`
+// wavefronts of 64 columns at one wavelength: split until about 16 wavefronts
+// per SIMD (1024 SIMDs) are queued.
+static int depth_split(int64_t rays, int Nmax) {
+  const int n = (int) std::min<int64_t>(Nmax, std::max<int64_t>(1, 16384 / rays));
+  return (Nmax + n - 1) / n;
+}
+
+// Bytes of the points of a synthesis that forms them in a pass of their own
+// (depths in parallel) before the sweeps, or 0 where k_formal_stokes does both
+// in one.  The latter keeps two wavefronts of rays per SIMD in flight (2048)
+// and waits at every depth for loads, line tables and quotients, so few rays
+// take as long as 2048.  FP64, 82 depths, 112 wavelengths: one column 1.15 ms
+// in one pass, 0.25 in two; 512 1.70 and 0.69; 1003 1.77 and 1.09; 2300 3.11
+// and 2.33; 4600 (8064 rays, 2.7 GB) 4.90 and 4.42, where the points' traffic
+// has nearly caught up.  Mixed columns, 200 wavelengths of the 400-line list:
+// 200 columns 19.0 and 3.8, 512 19.8 and 7.0.  FP64 only: the FP32 form
+// contracts multiply-adds, in two passes not to the same last place as in one.
+static size_t split_points(const rhg_context *c, int32_t precision, int ncol, int Nmax) {
+  if (precision != RHG_PREC_FP64) return 0;
+  const int64_t rays = (int64_t) ((ncol + 63) / 64) * c->n_pol;
+  const size_t bytes = (size_t) c->n_pol * Nmax * ncol *
+                       rhg::point_ncomp(c->dm.magneto_optical != 0) * sizeof(double);
+  return rays <= kSplitRays && bytes <= kSplitBytes ? bytes : 0;
+}
+
 // The wavelength grids of a synthesis launch: the batch's block -> grid
 // table (ncol / 64 entries, -1: a block without columns) and the context's
 // per-grid wavelength lists (rhg_set_grids).
@@ -523,12 +552,14 @@ struct GridLaunch {
 // i to the caller's column perm[i] of d_atm and d_out (-1 - c: a copy of
 // column c that writes nothing).  gl (or nullptr): the batch's columns
 // are grouped by wavelength grid in whole blocks of 64 slots, each block
-// solving its grid's wavelengths only.
+// solving its grid's wavelengths only.  pts (or nullptr): room for the
+// polarized rays' points, which then are formed with every depth at once
+// before the sweeps (split_points; FP64, no grids).
 static int launch_synth(rhg_context_t *c, const double *d_atm, const int32_t *d_ndep,
                         const int32_t *perm, int ncol, int Nmax, double mu, int atm_scale,
                         int32_t precision, int nfield, double *state, int32_t *moving,
                         double *chiref, void *cchi, void *ceta, double *d_out,
-                        const GridLaunch *gl = nullptr) {
+                        const GridLaunch *gl = nullptr, double *pts = nullptr) {
   const int64_t npts = (int64_t) ncol * Nmax;
   const int nout = c->nout;
 
@@ -588,6 +619,29 @@ static int launch_synth(rhg_context_t *c, const double *d_atm, const int32_t *d_
                     l_pol, p_pol, n_pol, LT ? (unsigned) c->tab_bytes : 0u, , c->tab_maxl,       \
                     c->tab_maxc)
     const bool lt = c->tab_bytes > 0 && c->tune_line_table;
+#define RHG_SPLIT(LT, MO)                                                                        \
+  do {                                                                                           \
+    hipLaunchKernelGGL((rhg::k_rf_points<double, LT, MO>), grdk, blk,                            \
+                       LT ? (unsigned) c->tab_bytes : 0u, c->stream, c->d_model, d_ndep, moving, \
+                       ncol, Nmax, state, c->d_out_ls, l_pol, n_pol, (const double *) cchi,      \
+                       (const double *) ceta, mu, kd, pts, c->tab_maxl, c->tab_maxc);            \
+    HIPCHECK(hipGetLastError());                                                                 \
+    hipLaunchKernelGGL((rhg::k_rf_forward<0, false, MO>), grd, blk, 0, c->stream, c->d_model,    \
+                       d_ndep, ncol, Nmax, state, c->d_out_ls, l_pol, n_pol, nout,               \
+                       (const double *) pts, mu, d_out, (double *) nullptr, perm);               \
+    HIPCHECK(hipGetLastError());                                                                 \
+  } while (0)
+    if (pts && n_pol > 0) {
+      const int kd = depth_split((int64_t) ncb * n_pol, Nmax);
+      const dim3 grd((unsigned) rhg::xcd_grid(ncb, n_pol)),
+          grdk(grd.x, (unsigned) ((Nmax + kd - 1) / kd));
+      if (c->dm.magneto_optical) {
+        if (lt) RHG_SPLIT(true, true); else RHG_SPLIT(false, true);
+      } else {
+        if (lt) RHG_SPLIT(true, false); else RHG_SPLIT(false, false);
+      }
+    } else
+#undef RHG_SPLIT
     if (c->dm.magneto_optical) {
       if (lt) { RHG_STOKES(true, true) } else { RHG_STOKES(true, false) }
     } else {
@@ -999,9 +1053,12 @@ int synth(rhg_context_t *c, const rhg_columns_t *cols, int32_t precision, int32_
   double *state = (double *) c->state.p;
   int32_t *moving = (int32_t *) c->moving.p;
   double *chiref = chiref_out ? (double *) c->chiref.p : nullptr;
+  // room for the points if the batch is one for it and there is the memory
+  const size_t pts_b = col_grid ? 0 : split_points(c, precision, ncol, Nmax);
+  double *pts = pts_b && !c->rf_pts.ensure(pts_b) ? (double *) c->rf_pts.p : nullptr;
   if (int rc = launch_synth(c, d_atm, sndep, perm, nslot, Nmax, cols->mu, cols->atm_scale,
                             precision, nfield, state, moving, chiref, c->cchi.p, c->ceta.p, d_out,
-                            col_grid ? &gl : nullptr))
+                            col_grid ? &gl : nullptr, pts))
     return rc;
   if (!device_ptrs)
     HIPCHECK(hipMemcpyAsync(stokes_out, d_out, out_b, hipMemcpyDeviceToHost, c->stream));
@@ -1448,23 +1505,21 @@ int rf_chunk(rhg_context_t *c, const double *d_atm, const int32_t *d_ndep, int n
     R *aP = (R *) c->rf_aP.p, *aZ = (R *) c->rf_aZ.p, *aB = (R *) c->rf_aB.p;
     double *pts = (double *) c->rf_pts.p;
     // The points and the chain are independent over depth: their depths are
-    // split over workgroups until about 16 waves per SIMD are queued (1024
-    // SIMDs), so that few rays fill the chip and ragged columns even out.
-    const int64_t rays = (int64_t) ncb * npol;
-    const int nsplit = (int) std::min<int64_t>(Nmax, std::max<int64_t>(1, 16384 / rays));
-    const int kd = (Nmax + nsplit - 1) / nsplit;
+    // split over workgroups, so that few rays fill the chip and ragged columns
+    // even out.
+    const int kd = depth_split((int64_t) ncb * npol, Nmax);
     const dim3 grdk(grd.x, (unsigned) ((Nmax + kd - 1) / kd));
 #define RHG_LAUNCH_PTS(LT)                                                                       \
-  hipLaunchKernelGGL((rhg::k_rf_points<R, LT>), grdk, blk, LT ? (unsigned) c->tab_bytes : 0u,    \
+  hipLaunchKernelGGL((rhg::k_rf_points<R, LT, false>), grdk, blk, LT ? (unsigned) c->tab_bytes : 0u,    \
                      c->stream, c->d_model, d_ndep, moving, ncol, Nmax, state, c->d_out_ls,      \
                      c->d_io_pol, npol, cchi, ceta, mu, kd, pts, c->tab_maxl, c->tab_maxc)
     const bool lt = c->tab_bytes > 0 && c->tune_line_table;
     if (lt) RHG_LAUNCH_PTS(true); else RHG_LAUNCH_PTS(false);
 #undef RHG_LAUNCH_PTS
     HIPCHECK(hipGetLastError());
-    hipLaunchKernelGGL((rhg::k_rf_forward<sizeof(R) == 4>), grd, blk, 0, c->stream, c->d_model, d_ndep,
+    hipLaunchKernelGGL((rhg::k_rf_forward<sizeof(R) == 4, true, false>), grd, blk, 0, c->stream, c->d_model, d_ndep,
                        ncol, Nmax, state, c->d_out_ls, c->d_io_pol, npol, nout,
-                       (const double *) pts, mu, d_out, car);
+                       (const double *) pts, mu, d_out, car, (const int32_t *) nullptr);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipEventRecord(c->ev[3], c->stream));
     hipLaunchKernelGGL(rhg::k_rf_reverse<R>, grd, blk, 0, c->stream, c->d_model, d_ndep, ncol,

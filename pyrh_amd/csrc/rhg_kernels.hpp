@@ -538,18 +538,20 @@ __global__ void k_rf_contract(const R *rf, const double *gT, int ncol, int nd, i
 template <typename O>
 __global__ void k_rf_diff(const double *S, int64_t W, int64_t off_p, int64_t off_m, int ncol,
                           int64_t nrows, double scale, O *out);
-template <typename R, bool LT>
+// doubles of a stored point: chi, S[4], q[3], with the magneto-optical terms r[3]
+__host__ __device__ constexpr int point_ncomp(bool mo) { return mo ? 11 : 8; }
+template <typename R, bool LT, bool MO>
 __global__ void k_rf_points(const DevModel *M, const int32_t *ndep, const int32_t *moving, int ncol,
                             int Nmax, const double *state, const int32_t *out_ls,
                             const int32_t *io_list, int nlist, const R *cchi, const R *ceta,
                             double mu, int kd, double *pts, int tab_maxl, int tab_maxc);
 // FP64 in both forms; FORM 0 keeps the reference's operation order, FORM 1 is
 // compiled with FMA contraction
-template <int FORM>
+template <int FORM, bool TAPE, bool MO>
 __global__ void k_rf_forward(const DevModel *M, const int32_t *ndep, int ncol, int Nmax,
                              const double *state, const int32_t *out_ls, const int32_t *io_list,
                              int nlist, int nout, const double *pts, double mu, double *stokes,
-                             double *car);
+                             double *car, const int32_t *perm);
 template <typename R>
 __global__ void k_rf_reverse(const DevModel *M, const int32_t *ndep, int ncol, int Nmax,
                              const double *state, const int32_t *out_ls, const int32_t *io_list,

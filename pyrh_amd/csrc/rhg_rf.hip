@@ -92,5 +92,10 @@ template __global__ void k_rf_contract<float>(const float *, const double *, int
                                               double *);
 
 RHG_RF_INST(double)
+// the synthesis of few rays
+RHG_RF_PTS(double, false, true)
+RHG_RF_PTS(double, true, true)
+RHG_RF_FWD(double, false, false)
+RHG_RF_FWD(double, false, true)
 
 }  // namespace rhg

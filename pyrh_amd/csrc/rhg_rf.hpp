@@ -57,7 +57,8 @@ __device__ __forceinline__ T point_get(const Point<T> &p, int m) {
     case 4: return p.S[3];
     case 5: return p.q[0];
     case 6: return p.q[1];
-    default: return p.q[2];
+    case 7: return p.q[2];
+    default: return p.r[m - 8];
   }
 }
 
@@ -120,7 +121,9 @@ __device__ __forceinline__ T point_get(const Point<T> &p, int m) {
 //   forward 23.0 -> 2.3 + 9.9 for the points, reverse 75.8 -> 25.3 ms; the
 //   512-column 112-wavelength batch (FP32 form) 0.85 -> 0.20 + 0.25 and
 //   1.87 -> 1.17 ms
-template <typename R, bool LT>
+// The synthesis of a batch of few rays takes the same two steps (MO: with the
+// magneto-optical terms, three more numbers per point).
+template <typename R, bool LT, bool MO>
 __global__ void __launch_bounds__(64)
 k_rf_points(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
             const int32_t *__restrict__ moving_arr, int ncol, int Nmax,
@@ -137,34 +140,57 @@ k_rf_points(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
   const int k0 = (int) blockIdx.y * kd, k1 = N < k0 + kd ? N : k0 + kd;
   for (int k = k0; k < k1; k++) {
     Point<double> P;
-    form_point_vt<R, R, false>(tab, M.ncont, has_line, st0 + (int64_t) k * ncol, fs, mu_d, moving,
-                               cc[(int64_t) k * ncol], ce[(int64_t) k * ncol], P);
-    double *pp = pts + ((int64_t) t * Nmax + k) * 8 * ncol + ic;
+    form_point_vt<R, R, MO>(tab, M.ncont, has_line, st0 + (int64_t) k * ncol, fs, mu_d, moving,
+                            cc[(int64_t) k * ncol], ce[(int64_t) k * ncol], P);
+    constexpr int NC = point_ncomp(MO);
+    double *pp = pts + ((int64_t) t * Nmax + k) * NC * ncol + ic;
 #pragma unroll
-    for (int m = 0; m < 8; m++) pp[m * (int64_t) ncol] = point_get(P, m);
+    for (int m = 0; m < NC; m++) pp[m * (int64_t) ncol] = point_get(P, m);
   }
 }
 
-template <int FORM>
+// TAPE: with the carried state for the reverse sweep; without, the synthesis
+// of few rays, to column perm[ic] of the caller where there is a permutation.
+template <int FORM, bool TAPE, bool MO>
 __global__ void __launch_bounds__(64)
 k_rf_forward(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
              int ncol, int Nmax,
              const double *__restrict__ state, const int32_t *__restrict__ out_ls,
              const int32_t *__restrict__ io_list, int nlist, int nout,
              const double *__restrict__ pts, double mu_d,
-             double *__restrict__ stokes, double *__restrict__ car) {
+             double *__restrict__ stokes, double *__restrict__ car,
+             const int32_t *__restrict__ perm) {
   RF_SETUP();
   const double imu = 1.0 / mu_d;
   const double B2a = planck(Tc[(int64_t) (N - 2) * ncol], lc[RHG_LC_HC_KLA], lc[RHG_LC_TWOHNU3_C2]);
   const double B2b = planck(Tc[(int64_t) (N - 1) * ncol], lc[RHG_LC_HC_KLA], lc[RHG_LC_TWOHNU3_C2]);
   DeloState<double> s;
   Point<double> Pn, Pa;
-  RF_POINT(N - 1, Pa);
-  double cv[NCARRY_STEP];
+  auto point = [&](int k, Point<double> &P) {
+    constexpr int NC = point_ncomp(MO);
+    const double *pp = pts + ((int64_t) t * Nmax + k) * NC * ncol + ic;
+    P.chi = pp[0];
+#pragma unroll
+    for (int n = 0; n < 4; n++) P.S[n] = pp[(1 + n) * (int64_t) ncol];
+#pragma unroll
+    for (int n = 0; n < 3; n++) {
+      P.q[n] = pp[(5 + n) * (int64_t) ncol];
+      P.r[n] = MO ? pp[(8 + n) % NC * (int64_t) ncol] : 0.0;
+    }
+  };
+  point(N - 1, Pa);
+  auto tape = [&](int k) {
+    if constexpr (TAPE) {
+      double cv[NCARRY_STEP];
+      carry_to_array(s, cv);
+#pragma unroll
+      for (int c = 0; c < NCARRY_STEP; c++) CAR(k, c) = cv[c];
+    }
+  };
   for (int j = N - 1; j >= -1; j--) {
     // the next point's loads are in flight while this step runs
     Pn = Pa;
-    if (j > 0) RF_POINT(j - 1, Pa);
+    if (j > 0) point(j - 1, Pa);
     if (j == N - 1) {
       s.Pu = Pn;
     } else if (j == N - 2) {
@@ -173,18 +199,17 @@ k_rf_forward(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
       delo_prologue<double>(s, Pn, DZ(N - 1), DZ(N - 2), imu, B2a, B2b);
     } else {
       const int k = j + 2;
-      carry_to_array(s, cv);
-#pragma unroll
-      for (int c = 0; c < NCARRY_STEP; c++) CAR(k, c) = cv[c];
-      delo_step<double>(s, Pn, j >= 0, DZ(k), j >= 0 ? DZ(k - 1) : 0.0, imu);
+      tape(k);
+      if constexpr (MO) delo_step_mo<double>(s, Pn, j >= 0, DZ(k), j >= 0 ? DZ(k - 1) : 0.0, imu);
+      else delo_step<double>(s, Pn, j >= 0, DZ(k), j >= 0 ? DZ(k - 1) : 0.0, imu);
     }
   }
-  carry_to_array(s, cv);
-#pragma unroll
-  for (int c = 0; c < NCARRY_STEP; c++) CAR(0, c) = cv[c];
+  tape(0);
   double x[4];
-  delo_final<double>(s, DZ(1), imu, x);
-  double *out = stokes + (int64_t) ic * 4 * nout + io;
+  if constexpr (MO) delo_final_mo<double>(s, DZ(1), imu, x);
+  else delo_final<double>(s, DZ(1), imu, x);
+  const int oc = perm ? perm[ic] : ic;
+  double *out = stokes + (int64_t) oc * 4 * nout + io;
 #pragma unroll
   for (int i = 0; i < 4; i++) out[(int64_t) i * nout] = x[i];
 }
@@ -602,21 +627,21 @@ k_rf_chain(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
 #undef AB
 
 #define RHG_RF_INST(R)                                                                          \
-  template __global__ void k_rf_points<R, false>(                                               \
-      const DevModel *, const int32_t *, const int32_t *, int, int, const double *,             \
-      const int32_t *, const int32_t *, int, const R *, const R *, double, int, double *, int, int); \
-  template __global__ void k_rf_points<R, true>(                                                \
-      const DevModel *, const int32_t *, const int32_t *, int, int, const double *,             \
-      const int32_t *, const int32_t *, int, const R *, const R *, double, int, double *, int, int); \
-  template __global__ void k_rf_forward<sizeof(R) == 4>(                                        \
-      const DevModel *, const int32_t *, int, int, const double *, const int32_t *,             \
-      const int32_t *, int, int, const double *, double, double *, double *);                   \
+  RHG_RF_PTS(R, false, false) RHG_RF_PTS(R, true, false) RHG_RF_FWD(R, true, false)             \
   template __global__ void k_rf_reverse<R>(const DevModel *, const int32_t *,                  \
                                            int, int, const double *, const int32_t *,          \
                                            const int32_t *, int, const double *, double,       \
                                            const double *, R *, R *, R *);                     \
   RHG_RF_CHAIN(R, false)                                                                        \
   RHG_RF_CHAIN(R, true)
+#define RHG_RF_PTS(R, LT, MO)                                                                   \
+  template __global__ void k_rf_points<R, LT, MO>(                                              \
+      const DevModel *, const int32_t *, const int32_t *, int, int, const double *,             \
+      const int32_t *, const int32_t *, int, const R *, const R *, double, int, double *, int, int);
+#define RHG_RF_FWD(R, TAPE, MO)                                                                 \
+  template __global__ void k_rf_forward<sizeof(R) == 4, TAPE, MO>(                              \
+      const DevModel *, const int32_t *, int, int, const double *, const int32_t *,             \
+      const int32_t *, int, int, const double *, double, double *, double *, const int32_t *);
 #define RHG_RF_CHAIN(R, LT)                                                                     \
   template __global__ void k_rf_chain<R, LT>(const DevModel *, const int32_t *, const int32_t *, \
                                              int, int, const double *, const double *,          \
