@@ -376,6 +376,13 @@ int rhg_open(const rhg_model_t *m, int device, rhg_context_t **out) {
     if (!rc) rc = upload(c, talpha.empty() ? nullptr : talpha.data(), talpha.size(), &d.tile_alpha);
   }
   if (!rc) {
+    std::vector<double> smax((size_t) std::max(m->nline, 1), 0.0);
+    for (int l = 0; l < m->nline; l++)
+      for (int q = m->line_comp_ptr[l]; q < m->line_comp_ptr[l + 1]; q++)
+        smax[l] = std::max(smax[l], fabs(m->comp_shift[q]));
+    rc = upload(c, smax.data(), smax.size(), &d.line_smax);
+  }
+  if (!rc) {
     // ktab: bilinear() over (temperature, wavelength) with the wavelength's
     // part done
     std::vector<double> kt((size_t) ns * rhg::KT_N, 0.0);

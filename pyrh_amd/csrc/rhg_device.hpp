@@ -157,6 +157,23 @@ __device__ __forceinline__ cpx<T> cdiv(cpx<T> a, cpx<T> b) {
   const T id = rrcp(b.r * b.r + b.i * b.i);
   return {(a.r * b.r + a.i * b.i) * id, (a.i * b.r - a.r * b.i) * id};
 }
+// in float with the fused operations written out, so that region I rounds
+// alike in the general function and where the region is known beforehand
+__device__ __forceinline__ cpx<float> cdiv(cpx<float> a, cpx<float> b) {
+  const float id = rrcp(fmaf(b.r, b.r, b.i * b.i));
+  return {fmaf(a.r, b.r, a.i * b.i) * id, fmaf(a.i, b.r, -(a.r * b.i)) * id};
+}
+
+// z^2 + 1/2
+template <typename T>
+__device__ __forceinline__ cpx<T> csqh(cpx<T> z) {
+  cpx<T> w = cmul(z, z);
+  w.r = w.r + T(0.5);
+  return w;
+}
+__device__ __forceinline__ cpx<float> csqh(cpx<float> z) {
+  return {fmaf(z.r, z.r, fmaf(-z.i, z.i, 0.5f)), 2.0f * z.r * z.i};
+}
 
 __device__ __forceinline__ double rexp(double x) { return exp(x); }
 __device__ __forceinline__ float rexp(float x) { return __expf(x); }
@@ -193,8 +210,7 @@ __device__ __forceinline__ R voigt_humlicek_r(R a, R v, int region, R *F) {
   cpx<R> z = {a, -v}, z1, z2, u, e = {R(0), R(0)};
   if (region == 0) {
     z1 = {R(0.5641896) * z.r, R(0.5641896) * z.i};
-    z2 = cmul(z, z);
-    z2.r = z2.r + R(0.5);
+    z2 = csqh(z);
   } else if (region == 1) {
     u = cmul(z, z);
     z1 = {R(0.5641896) * u.r, R(0.5641896) * u.i};

@@ -2,6 +2,8 @@
 // opacity shared by the stages.
 #pragma once
 
+#include <type_traits>
+
 #include "rhg_device.hpp"
 #include "rhg_dual.hpp"
 
@@ -70,6 +72,8 @@ struct DevModel {
   int ntile;
   const int32_t *tile_ptr, *tile_cont;
   const double *tile_alpha;
+  // per line, the largest |shift| of its Zeeman components
+  const double *line_smax;
   // per wavelength, the temperature tables of its continuum terms with the
   // wavelength already interpolated: KT_N doubles, tables at KT_*
   const double *ktab;
@@ -172,6 +176,7 @@ struct LineTabG {
   __device__ __forceinline__ bool damped(int i) const { return ldc(M.line_Grad)[line(i)] != 0.0; }
   __device__ __forceinline__ bool polar(int i) const { return ldc(M.line_polar)[line(i)] != 0; }
   __device__ __forceinline__ double larmor(int i) const { return ldc(M.line_larmor)[line(i)]; }
+  __device__ __forceinline__ double smax(int i) const { return ldc(M.line_smax)[line(i)]; }
   __device__ __forceinline__ int c0(int i) const { return ldc(M.line_comp_ptr)[line(i)]; }
   __device__ __forceinline__ int c1(int i) const { return ldc(M.line_comp_ptr)[line(i) + 1]; }
   __device__ __forceinline__ double shift(int c) const { return ldc(M.comp_shift)[c]; }
@@ -188,7 +193,7 @@ struct LineTabG {
 // order as from the ungrouped list, and the component loop needs no
 // per-component branch.
 struct LineRecL {
-  double dv, larmor;
+  double dv, larmor, smax;
   int line, flags, c0, c1;   // flags: 1 damped, 2 polarizable
   int cpi, csp;              // first pi and first sigma+ component
 };
@@ -210,6 +215,7 @@ struct LineTabL {
     return __builtin_amdgcn_readfirstlane(rec[i].flags) & 2;
   }
   __device__ __forceinline__ double larmor(int i) const { return rec[i].larmor; }
+  __device__ __forceinline__ double smax(int i) const { return rec[i].smax; }
   __device__ __forceinline__ int c0(int i) const { return __builtin_amdgcn_readfirstlane(rec[i].c0); }
   __device__ __forceinline__ int c1(int i) const { return __builtin_amdgcn_readfirstlane(rec[i].c1); }
   __device__ __forceinline__ int cpi(int i) const { return __builtin_amdgcn_readfirstlane(rec[i].cpi); }
@@ -241,6 +247,7 @@ __device__ __forceinline__ LineTabL stage_lines(const DevModel &M, int ls, char 
     const bool damped = ldc(M.line_Grad)[l] != 0.0, polar = ldc(M.line_polar)[l] != 0;
     rec[i].dv = ldc(M.lam_line_dv)[p0 + i];
     rec[i].larmor = ldc(M.line_larmor)[l];
+    rec[i].smax = ldc(M.line_smax)[l];
     rec[i].line = l;
     rec[i].flags = (damped ? 1 : 0) | (polar ? 2 : 0);
     // only a damped polarizable line uses its components
@@ -332,42 +339,55 @@ __device__ __forceinline__ T line_profile_t(const Tab &tab, int i, int lb, const
       T phi_sm = T(0), phi_pi = T(0), phi_sp = T(0);
       T psi_sm = T(0), psi_pi = T(0), psi_sp = T(0);
       const int c0 = tab.c0(i), c1 = tab.c1(i);
-      if constexpr (Tab::grouped) {
-        // one Delta M group [a, b) into its sums; the next component's
-        // shift and strength are read while this one's profile is formed
-        auto group = [&](int a, int b, T &phi_g, T &psi_g) {
-          double sh = a < b ? tab.shift(a) : 0.0, sg = a < b ? tab.strength(a) : 0.0;
-          for (int nz = a; nz < b; nz++) {
-            const double shc = sh, sgc = sg;
-            if (nz + 1 < b) {
-              sh = tab.shift(nz + 1);
-              sg = tab.strength(nz + 1);
+      // the region of component nz's argument u; FAR: region 0 (I) for every
+      // component and lane, without the test
+      auto component = [&](auto FAR, double shift, TV &Fw) -> T {
+        const T u = v - T(shift) * vB;
+        const int reg = decltype(FAR)::value ? 0 : humlicek_region(val(adamp), val(u));
+        return (T) VoigtEval<TV>::eval((TV) adamp, (TV) u, reg, &Fw);
+      };
+      auto components = [&](auto FAR) {
+        if constexpr (Tab::grouped) {
+          // one Delta M group [a, b) into its sums; the next component's
+          // shift and strength are read while this one's profile is formed
+          auto group = [&](int a, int b, T &phi_g, T &psi_g) {
+            double sh = a < b ? tab.shift(a) : 0.0, sg = a < b ? tab.strength(a) : 0.0;
+            for (int nz = a; nz < b; nz++) {
+              const double shc = sh, sgc = sg;
+              if (nz + 1 < b) {
+                sh = tab.shift(nz + 1);
+                sg = tab.strength(nz + 1);
+              }
+              TV Fw;
+              const T Hc = component(FAR, shc, Fw);
+              acc_prod(phi_g, T(sgc), Hc);
+              if constexpr (MO) acc_prod(psi_g, T(sgc), (T) Fw);
             }
+          };
+          group(c0, tab.cpi(i), phi_sm, psi_sm);
+          group(tab.cpi(i), tab.csp(i), phi_pi, psi_pi);
+          group(tab.csp(i), c1, phi_sp, psi_sp);
+        } else {
+          for (int nz = c0; nz < c1; nz++) {
             TV Fw;
-            const T u = v - T(shc) * vB;
-            const int reg = humlicek_region(val(adamp), val(u));
-            const T Hc = (T) VoigtEval<TV>::eval((TV) adamp, (TV) u, reg, &Fw);
-            acc_prod(phi_g, T(sgc), Hc);
-            if constexpr (MO) acc_prod(psi_g, T(sgc), (T) Fw);
+            const T H = component(FAR, tab.shift(nz), Fw);
+            const T Fv = (T) Fw;
+            (void) Fv;
+            const int q = tab.q(nz);
+            const T sg = T(tab.strength(nz));
+            acc_prod(q == -1 ? phi_sm : (q == 0 ? phi_pi : phi_sp), sg, H);
+            if constexpr (MO) acc_prod(q == -1 ? psi_sm : (q == 0 ? psi_pi : psi_sp), sg, Fv);
           }
-        };
-        group(c0, tab.cpi(i), phi_sm, psi_sm);
-        group(tab.cpi(i), tab.csp(i), phi_pi, psi_pi);
-        group(tab.csp(i), c1, phi_sp, psi_sp);
-      } else {
-        for (int nz = c0; nz < c1; nz++) {
-          TV Fw;
-          const T u = v - T(tab.shift(nz)) * vB;
-          const int reg = humlicek_region(val(adamp), val(u));
-          const T H = (T) VoigtEval<TV>::eval((TV) adamp, (TV) u, reg, &Fw);
-          const T Fv = (T) Fw;
-          (void) Fv;
-          const int q = tab.q(nz);
-          const T sg = T(tab.strength(nz));
-          acc_prod(q == -1 ? phi_sm : (q == 0 ? phi_pi : phi_sp), sg, H);
-          if constexpr (MO) acc_prod(q == -1 ? psi_sm : (q == 0 ? psi_pi : psi_sp), sg, Fv);
         }
-      }
+      };
+      // A line far from the wavelength in every lane: all its components are
+      // in region 0 (|u| + a >= 15 with |u| >= |v| - max|shift| |vB|, with
+      // room for rounding), whose function is a third of the instructions of
+      // the general one with its test and branches; most of a blended list.
+      if (__all(fabs(val(v)) - tab.smax(i) * fabs(val(vB)) + val(adamp) >= 15.01))
+        components(std::true_type{});
+      else
+        components(std::false_type{});
       const T phi_sigma = phi_sp + phi_sm;
       const T phi_delta = T(0.5) * phi_pi - T(0.25) * phi_sigma;
       phi = (phi_delta * sin2_gamma + T(0.5) * phi_sigma) * sv;

@@ -124,7 +124,7 @@ __device__ __forceinline__ T point_get(const Point<T> &p, int m) {
 // The synthesis of a batch of few rays takes the same two steps (MO: with the
 // magneto-optical terms, three more numbers per point).
 template <typename R, bool LT, bool MO>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(64, 3)
 k_rf_points(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
             const int32_t *__restrict__ moving_arr, int ncol, int Nmax,
             const double *__restrict__ state, const int32_t *__restrict__ out_ls,
