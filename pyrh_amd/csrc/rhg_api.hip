@@ -65,7 +65,7 @@ namespace {
 constexpr int kMaxDevices = 64;
 // split_points: rays of a batch and bytes of its points, at most
 constexpr int64_t kSplitRays = 8192;
-constexpr size_t kSplitBytes = (size_t) 4 << 30;
+constexpr size_t kSplitBytes = (size_t) 3 << 30;
 // the hydrostatic builder's records held at a time: 16384 columns of 82
 // depths and 99 elements
 constexpr size_t kHseRecBytes = (size_t) 4 << 30;
@@ -532,8 +532,9 @@ static int depth_split(int64_t rays, int Nmax) {
 // and waits at every depth for loads, line tables and quotients, so few rays
 // take as long as 2048.  FP64, 82 depths, 112 wavelengths: one column 1.15 ms
 // in one pass, 0.25 in two; 512 1.70 and 0.69; 1003 1.77 and 1.09; 2300 3.11
-// and 2.33; 4600 (8064 rays, 2.7 GB) 4.90 and 4.42, where the points' traffic
-// has nearly caught up.  Mixed columns, 200 wavelengths of the 400-line list:
+// and 2.33; 4600 (8064 rays, 2.7 GB) 4.90 and 4.42, 9000 8.7 and 9.3: the
+// points' traffic has caught up (with the magneto-optical terms at 3.7 GB, 4600
+// columns 6.02 and 6.13).  Mixed columns, 200 wavelengths of the 400-line list:
 // 200 columns 19.0 and 3.8, 512 19.8 and 7.0.  FP64 only: the FP32 form
 // contracts multiply-adds, in two passes not to the same last place as in one.
 static size_t split_points(const rhg_context *c, int32_t precision, int ncol, int Nmax) {
