@@ -2212,7 +2212,8 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
           const dim3 grd((unsigned) rhg::xcd_grid(nact, h.nbez));
 #define RHG_LAUNCH_BEZ(L, P, MS)                                                                 \
   hipLaunchKernelGGL((rhg::k_nlte_bezier<L, P, MS>), grd, dim3(2 * L),                            \
-                     (size_t) Nmax * sizeof(double), c->stream, c->d_model, d_at, B, d_act, nact, \
+                     rhg::nlte_bez_lds(L, P, MS, Nmax) * sizeof(double), c->stream, c->d_model,   \
+                     d_at, B, d_act, nact,                                                       \
                      c->d_out_ls, d_iolist, h.nbez, 0, nlist, eval)
 #define RHG_LAUNCH_BEZ_P(L, P)                                                                   \
   do {                                                                                           \

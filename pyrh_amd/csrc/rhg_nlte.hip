@@ -651,15 +651,16 @@ __device__ __forceinline__ void ray_points(const NlteBufs &B, int64_t col, int t
 // the rays in both directions, the new mean intensity and with eval_op the
 // radiative rate terms (rh/rhf1d/formal.c:44-346, rh/fillgamma.c:82-332),
 // summed over the rays in registers; the outward lanes' sums are turned to
-// the inward lanes' depths through LDS at the end (N doubles).  J is
+// the inward lanes' depths through LDS at the end.  J is
 // double-buffered per column (jpar): the previous J enters the source
 // function, the new one is built.
 // Measured on a pass over 465 such wavelengths: one column 26 us (5.3 ms with
 // a lane per column: all its wavefronts on one XCD, one lane of each), 1500
-// columns of 82 depths 9.9 ms (16.5): 3.76e9 vector instructions, 65% of the
-// SIMDs' cycles, the rest waits of the two wavefronts that the registers
-// allow.  P = 3 at 32 lanes per direction covers 82 depths with 85% of the
-// lanes.
+// columns of 82 depths 8.0 ms (16.5), bound by the issue of 3.8e9 vector
+// instructions and the waits of the two wavefronts per SIMD that the registers
+// allow: 9.9 ms with the member data in registers and a ray's profiles loaded
+// as it begins.  P = 3 at 32 lanes per direction covers 82 depths with 85% of
+// the lanes.
 template <int L, int P, int MS>
 __global__ void __launch_bounds__(2 * L, (P <= 3 && MS <= 2 ? 2 : 1))
 k_nlte_bezier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap, NlteBufs B,
@@ -690,11 +691,47 @@ k_nlte_bezier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap, N
   int k[P];
   RayPath<P> g;
   ray_points<P>(B, col, t0, N, outward, k, g);
-  SetDepth<MS> sd[P];
+  // member data of the lane's points: in LDS, column threadIdx.x of each row,
+  // where it fits (the registers then hold the next ray's profiles)
+  constexpr bool STASH = nlte_stash(P, MS);
+  double *stash = turn + B.Nmax + threadIdx.x;
+  SetDepth<MS> sd_r[STASH ? 1 : P];
+  auto put_depth = [&](int s, const SetDepth<MS> &d) {
+    if constexpr (STASH) {
+#pragma unroll
+      for (int n = 0; n < MS; n++) {
+        double *q = stash + (s * MS + n) * 4 * 2 * L;
+        q[0] = d.x[n];
+        q[2 * L] = d.e[n];
+        q[4 * L] = d.gij[n];
+        q[6 * L] = d.wla[n];
+      }
+    } else {
+      sd_r[s] = d;
+    }
+  };
+  auto get_depth = [&](int s) -> SetDepth<MS> {
+    if constexpr (STASH) {
+      SetDepth<MS> d;
+#pragma unroll
+      for (int n = 0; n < MS; n++) {
+        const double *q = stash + (s * MS + n) * 4 * 2 * L;
+        d.x[n] = q[0];
+        d.e[n] = q[2 * L];
+        d.gij[n] = q[4 * L];
+        d.wla[n] = q[6 * L];
+      }
+      return d;
+    } else {
+      return sd_r[s];
+    }
+  };
   double cc[P], s0[P], js[P], sIJ[P][MS], sJI[P][MS];
 #pragma unroll
   for (int s = 0; s < P; s++) {
-    set_depth<MS>(B, si, col + k[s], Tc[k[s]], lam, sd[s]);
+    SetDepth<MS> d;
+    set_depth<MS>(B, si, col + k[s], Tc[k[s]], lam, d);
+    put_depth(s, d);
     cc[s] = B.cchi[wo + k[s]];
     s0[s] = fma(B.csca[wo + k[s]], Jold[k[s]], B.ceta[wo + k[s]]);
     js[s] = 0.0;
@@ -702,32 +739,44 @@ k_nlte_bezier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap, N
     for (int n = 0; n < MS; n++) sIJ[s][n] = sJI[s][n] = 0.0;
   }
   const int dir = outward ? 1 : 0;
+  // a ray's profiles are loaded one ray ahead
+  double ph[P][MS];
+  auto fetch = [&](int mu) {
+#pragma unroll
+    for (int s = 0; s < P; s++)
+#pragma unroll
+      for (int n = 0; n < MS; n++)
+        ph[s][n] = n < si.n && si.line[n] >= 0
+                       ? B.phi[((int64_t) (si.prow[n] + mu) * 2 + dir) * fs + col + k[s]] : 0.0;
+  };
+  fetch(0);
   for (int mu = 0; mu < nrays; mu++) {
     const double zmu = 1.0 / A.muz[mu], wmu = 0.5 * A.wmu[mu];
     double V[P][MS], C[P], S[P], iC[P], I[P], Psi[P];
 #pragma unroll
     for (int s = 0; s < P; s++) {
+      const SetDepth<MS> d = get_depth(s);
       double chi = 0.0, eta = 0.0;
 #pragma unroll
       for (int n = 0; n < MS; n++) {
         V[s][n] = 0.0;
         if (n < si.n) {
-          V[s][n] = si.line[n] >= 0
-                        ? si.cV[n] * B.phi[((int64_t) (si.prow[n] + mu) * 2 + dir) * fs + col + k[s]]
-                        : si.alpha[n];
-          chi += V[s][n] * sd[s].x[n];
-          eta += V[s][n] * sd[s].e[n];
+          V[s][n] = si.line[n] >= 0 ? si.cV[n] * ph[s][n] : si.alpha[n];
+          chi += V[s][n] * d.x[n];
+          eta += V[s][n] * d.e[n];
         }
       }
       C[s] = chi + cc[s];
       iC[s] = nrcp(C[s]);
       S[s] = (eta + s0[s]) * iC[s];
     }
+    if (mu + 1 < nrays) fetch(mu + 1);
     ray_sweep<L, P>(g, t0, N, outward, zmu, B2_0, B2_1, C, S, I, Psi);
 #pragma unroll
     for (int s = 0; s < P; s++) {
       js[s] += wmu * I[s];
-      if (eval_op) rate_terms<MS>(si, sd[s], V[s], I[s], Psi[s] * iC[s], wmu, sIJ[s], sJI[s]);
+      if (eval_op)
+        rate_terms<MS>(si, get_depth(s), V[s], I[s], Psi[s] * iC[s], wmu, sIJ[s], sJI[s]);
     }
   }
   // the inward lanes add the outward lanes' sum at each of their depths
