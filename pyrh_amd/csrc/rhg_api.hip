@@ -2197,10 +2197,12 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
       return 0;
     };
     // columns a k_nlte_feautrier workgroup shares its lanes between: as many
-    // as 24 KB of LDS hold, fewer while they would leave SIMDs idle
+    // as 36 KB of LDS hold (four workgroups per CU: 1500 columns of 82 depths
+    // 0.90 ms a pass; 9 KB 1.66, 24 KB 1.14, 52 KB 1.08), fewer while they
+    // would leave SIMDs idle
     auto fe_per = [&](int nact, int rays) {
       int per = 12;
-      while (per > 1 && rhg::nlte_fe_lds(Nmax, per, rays) * sizeof(double) > 24576) per--;
+      while (per > 1 && rhg::nlte_fe_lds(Nmax, per, rays) * sizeof(double) > 36864) per--;
       while (per > 1 && (int64_t) nact * (nlist - h.nbez) / per < 1024) per--;
       return per;
     };
