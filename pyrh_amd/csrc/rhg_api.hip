@@ -38,7 +38,12 @@ struct DevBuf {
     if (p) (void) hipFree(p);
     p = nullptr;
     bytes = 0;
-    if (hipMalloc(&p, n) != hipSuccess) return -1;
+    if (hipMalloc(&p, n) != hipSuccess) {
+      // callers may go on with less memory: the failure is not the next launch's
+      (void) hipGetLastError();
+      p = nullptr;
+      return -1;
+    }
     bytes = n;
     return 0;
   }

@@ -8,7 +8,7 @@
 //
 // The layers are a serial chain, so what bounds the builder is the length of
 // that chain, not the chip's rate.  Everything that a layer's temperature
-// alone fixes (about 350 numbers: every exponential, power and table look-up)
+// alone fixes (about 320 numbers: every exponential, power and table look-up)
 // is formed first by k_hse_tables, in parallel over columns and depths;
 // k_hse then runs the chain with a group of lanes per column that share the
 // elements of the electron-density step and the molecules of the chemical
