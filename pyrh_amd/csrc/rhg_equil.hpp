@@ -1,6 +1,5 @@
-// Chemical equilibrium at one depth, shared by the column-state kernel of
-// the synthesis and the hydrostatic-equilibrium builder: molecular
-// equilibrium constants (rh/chemequil.c:452-533) and the Newton solution of
+// Chemical equilibrium at one depth: molecular equilibrium constants (also
+// the hydrostatic builder's) (rh/chemequil.c:452-533) and the Newton solution of
 // the nuclei and molecule densities (rh/chemequil.c:107-393).
 #pragma once
 
@@ -101,30 +100,24 @@ __device__ __forceinline__ void small_solve(double (&a)[NN][NN], double (&b)[NN]
 // nuclei block by the Schur complement S = D - B C, solved, and corrected
 // once with the residual of the reduced system, as the reference refines
 // its LU solution once (rh/ludcmp.c:55-84).  Molecule stoichiometry is the
-// dense table M.mol_cnt[m][nucleus]; the per-molecule equilibrium constant,
-// density and Saha product live in LDS (lds_phi, lds_nmol, lds_saha, stride
-// blockDim.x), everything per nucleus in registers.  With lds_saha nullptr
-// the Saha products are formed again where they are reused, by the same
-// operations (so the same values), which saves a third of the LDS.
+// dense table M.mol_cnt[m][nucleus]; the per-molecule equilibrium constant
+// and density live in LDS (lds_phi, lds_nmol, stride blockDim.x), everything
+// per nucleus in registers.  The Saha products are formed again where they
+// are reused, by the same operations (so the same values), which saves a
+// third of the LDS.
 template <int NN>
 __device__ void chem_eq(const DevModel &M, double T, double ne, double nHtot,
                         const double (&fn0)[NN], double (&nnuc)[NN], double *lds_phi,
-                        double *lds_nmol, double *lds_saha, int ls_stride, double &PhiHmin_out,
-                        bool phi_ready = false, const double *tcache = nullptr) {
+                        double *lds_nmol, int ls_stride, double &PhiHmin_out) {
   const int Nm = M.nmol;
   const double CI = (HPLANCK / (2.0 * PI * M_ELECTRON)) * (HPLANCK / KBOLTZMANN);
   double a[NN];
 #pragma unroll
   for (int i = 0; i < NN; i++) a[i] = ldc(M.nucl_abund)[i] * nHtot;
-  // tcache: pow(CI/T, 1.5) and exp(E_ION_HMIN/kT) formed by a caller that
-  // solves this temperature again
-  double PhiHmin = tcache ? 0.25 * tcache[0] * tcache[1]
-                          : 0.25 * pow(CI / T, 1.5) * exp(0.754 * EV / (KBOLTZMANN * T));
+  double PhiHmin = 0.25 * pow(CI / T, 1.5) * exp(0.754 * EV / (KBOLTZMANN * T));
   double fHmin = ne * fn0[0] * PhiHmin;
-  // phi_ready: lds_phi already holds the constants at this T (a caller
-  // that solves the same temperature again)
   for (int m = 0; m < Nm; m++) {
-    if (!phi_ready) lds_phi[m * ls_stride] = equilconstant(M, m, T);
+    lds_phi[m * ls_stride] = equilconstant(M, m, T);
     lds_nmol[m * ls_stride] = 0.0;
   }
 #pragma unroll
@@ -154,14 +147,12 @@ __device__ void chem_eq(const DevModel &M, double T, double ne, double nHtot,
       sv /= ipow(ne, ldc(M.mol_charge)[m]);
       return sv;
     };
-    auto saha_of = [&](int m) { return lds_saha ? lds_saha[m * ls_stride] : saha(m); };
     for (int m = 0; m < Nm; m++) {
       CDouble *cnt = ldc(M.mol_cnt) + m * NNUC_MAX;
       const double nm = lds_nmol[m * ls_stride];
 #pragma unroll
       for (int i = 0; i < NN; i++)
         if (cnt[i] != 0.0) f1[i] += cnt[i] * nm;
-      if (lds_saha) lds_saha[m * ls_stride] = saha(m);
     }
     // S = D - B C, rhs = f1 - B f2  (C[m][nu] = -saha_m count_nu / n_nu,
     // f2[m] = n_m - saha_m)
@@ -174,7 +165,7 @@ __device__ void chem_eq(const DevModel &M, double T, double ne, double nHtot,
     S[0][0] += fHmin;
     for (int m = 0; m < Nm; m++) {
       CDouble *cnt = ldc(M.mol_cnt) + m * NNUC_MAX;
-      const double sv = saha_of(m);
+      const double sv = saha(m);
       const double f2 = lds_nmol[m * ls_stride] - sv;
       double C[NN];
 #pragma unroll
@@ -213,7 +204,7 @@ __device__ void chem_eq(const DevModel &M, double T, double ne, double nHtot,
     double dnmax = 0.0;
     for (int m = 0; m < Nm; m++) {
       CDouble *cnt = ldc(M.mol_cnt) + m * NNUC_MAX;
-      const double sv = saha_of(m);
+      const double sv = saha(m);
       const double nold = lds_nmol[m * ls_stride];
       double x2 = nold - sv;
 #pragma unroll

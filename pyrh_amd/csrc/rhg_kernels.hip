@@ -232,7 +232,7 @@ k_state(const DevModel *__restrict__ Mp, const double *__restrict__ atmos, const
   const int lstride = blockDim.x;
   double *lds_phi = lds_mol + threadIdx.x;
   double *lds_nmol = lds_phi + M.nmol * lstride;
-  chem_eq<NN>(M, T, ne, nHtot, fn0, nnuc, lds_phi, lds_nmol, nullptr, lstride, PhiHmin);
+  chem_eq<NN>(M, T, ne, nHtot, fn0, nnuc, lds_phi, lds_nmol, lstride, PhiHmin);
   double fracn[NN];
 #pragma unroll
   for (int i = 0; i < NN; i++) fracn[i] = nnuc[i] / (ldc(M.atom_abund)[ldc(M.nucl_atom)[i]] * nHtot);
