@@ -42,8 +42,10 @@ __device__ __forceinline__ HseT hse_tcache(const DevHse &H, double T, double Uk0
 }
 
 // 1 / x and a / b by the hardware reciprocal estimate refined by two Newton
-// steps (relative error ~1e-16, not correctly rounded): the quotients of the
-// layer chain, where the IEEE division sequence is a long dependent chain
+// steps (relative error ~1e-16, not correctly rounded): the quotients inside
+// the sums over elements and molecules, where the IEEE division sequence is a
+// long dependent chain.  The few of a pressure iteration itself are IEEE: a
+// rounded reciprocal would bias every layer alike
 __device__ __forceinline__ double hrcp(double x) {
   double r = __builtin_amdgcn_rcp(x);
   double e = fma(-x, r, 1.0);
@@ -301,7 +303,7 @@ __device__ __forceinline__ bool group_any(bool x, const HseGroup &G) {
 __device__ __forceinline__ double hse_group_ne(const DevHse &H, const HseGroup &G, double nHtot) {
   const double p15 = G.rec[HSE_T_P15];
   const double PhiH = 0.5 * p15 * G.rec[HSE_T_EH];
-  double ne_old = hdiv(sqrt(1.0 + 4.0 * nHtot * PhiH) - 1.0, 2.0 * PhiH), ne = ne_old;
+  double ne_old = (sqrt(1.0 + 4.0 * nHtot * PhiH) - 1.0) / (2.0 * PhiH), ne = ne_old;
   const double PhiHmin = 0.25 * p15 * G.rec[HSE_T_EHMIN];
   const double CT2 = 2.0 * G.rec[HSE_T_PM15], inv_nH = hrcp(nHtot);
   for (int niter = 0; niter < HSE_N_MAX_ELECTRON_ITER; niter++) {
@@ -338,7 +340,7 @@ __device__ __forceinline__ double hse_group_ne(const DevHse &H, const HseGroup &
       }
     }
     group_sum(acc, G.lpc);
-    ne = ne_old - hdiv(nHtot * acc[0], 1.0 - nHtot * acc[1]);
+    ne = ne_old - nHtot * acc[0] / (1.0 - nHtot * acc[1]);
     const bool done = fabs(ne - ne_old) <= HSE_MAX_ELECTRON_ERROR * fabs(ne_old);
     ne_old = ne;
     if (done) break;
@@ -510,7 +512,7 @@ __device__ __forceinline__ void hse_layer(const DevModel &M, const DevHse &H, co
   const double PhiHmin = 0.25 * p15 * rec[HSE_T_EHMIN];
   hse_group_chem<NN>(M, G, ne, nHtot, fn0, phi, ne * fn0[0] * PhiHmin, nnuc);
 #pragma unroll
-  for (int i = 0; i < NN; i++) fracn[i] = hdiv(nnuc[i], ldc(M.atom_abund)[ldc(M.nucl_atom)[i]] * nHtot);
+  for (int i = 0; i < NN; i++) fracn[i] = nnuc[i] / (ldc(M.atom_abund)[ldc(M.nucl_atom)[i]] * nHtot);
   const double nH0 = nstar0n[0] * fracn[0];
   double np = rec[HSE_T_NP];
   for (int m = 0; m < H.np_dz; m++) np *= ci;
@@ -648,7 +650,7 @@ k_hse(const DevModel *__restrict__ Mp, DevHse H, int lpc, int cpb, int ncol, int
   const bool store = (sub == 0);
   const bool tau = (atm_scale == 0);
   const double g = M.gravity, LOG10 = log(10.0), wH = AMU * M.wght_per_H;
-  const double inv_tA = 1.0 / M.totalAbund;
+  const double tA = M.totalAbund;
   auto load = [&](int k) {
     wave_sync();
     const double *r = rc + (int64_t) k * H.nrec;
@@ -662,31 +664,31 @@ k_hse(const DevModel *__restrict__ Mp, DevHse H, int lpc, int cpb, int ncol, int
   double pg = pg_top[ic], ne = 0.0, opac = 0.0, rho = 0.0, z_prev = 0.0;
   for (int k = 0; k < N; k++) {
     const double z = tau ? pow10d(sc[k]) : sc[k] * KM_TO_M;
-    const double ikT = 1.0 / (KBOLTZMANN * Tc[k]);
+    const double T = Tc[k];
     load(k);
     const double pg_prev = pg, rho_prev = rho, ne_prev = ne;
     double dlogtau = 0.0, beta1 = 0.0;
     if (k > 0) {
       if (tau) {
         const double q = rho / opac;
-        pg += g * q * (z - z_prev);
+        pg += g * rho / opac * (z - z_prev);
         beta1 = q * z_prev;
         dlogtau = log10(z) - log10(z_prev);
       } else {
         pg += g * rho * (z_prev - z);
       }
     }
-    double nH = (pg * ikT - ne_prev) * inv_tA;
+    double nH = (pg / KBOLTZMANN / T - ne_prev) / tA;
     int iter = 0;
     while (iter < H.nmax_iter) {
       rho = wH * nH;
       hse_layer<NN>(M, H, G, nH, tau, ne, opac);
       if (k > 0) {
-        if (tau) pg = pg_prev + LOG10 * g * (hdiv(rho, opac) * z + beta1) / 2 * dlogtau;
+        if (tau) pg = pg_prev + LOG10 * g * (rho / opac * z + beta1) / 2 * dlogtau;
         else pg = pg_prev + g * (z_prev - z) * sqrt(rho * rho_prev);
       }
       const double old = nH;
-      nH = (pg * ikT - ne) * inv_tA;
+      nH = (pg / KBOLTZMANN / T - ne) / tA;
       iter++;
       if (fabs(hdiv(nH - old, nH)) <= H.iter_limit) break;
     }
