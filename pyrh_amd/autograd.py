@@ -22,6 +22,7 @@ from .engine import RF_PARAMS, RF_ROWS, rf_contract
 
 try:
     import torch
+    from torch.autograd import forward_ad
 except ImportError:  # pragma: no cover - the product path needs torch for this module
     torch = None
 
@@ -31,12 +32,21 @@ def _require_torch():
         raise RuntimeError("pyrh_amd.autograd needs PyTorch")
 
 
+def _bare(t):
+    """Whether a tensor's memory is all there is to it: no subclass, no
+    wrapper of a function transform, no forward-mode tangent, no pending
+    negation."""
+    return (type(t) is torch.Tensor and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+            and forward_ad.unpack_dual(t).tangent is None and not t.is_neg())
+
+
 def _contract_here(rf, g, shape):
     """Whether backward may run rhg_rf_contract: plain CUDA tensors of one
-    device, the saved response functions as forward laid them out (a
-    saved-tensor hook may return others), and no graph of the backward itself
-    (create_graph), which torch has to see the operations of."""
-    return (type(rf) is torch.Tensor and type(g) is torch.Tensor and g.is_cuda
+    device (_bare: the kernel reads their memory and nothing else), the saved
+    response functions as forward laid them out (a saved-tensor hook may
+    return others), and no graph of the backward itself (create_graph), which
+    torch has to see the operations of."""
+    return (_bare(rf) and _bare(g) and g.is_cuda
             and rf.device == g.device and rf.dtype in (torch.float32, torch.float64)
             and tuple(rf.shape) == shape and rf.is_contiguous()
             and not (torch.is_grad_enabled() and (g.requires_grad or rf.requires_grad)))

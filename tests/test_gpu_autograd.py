@@ -105,3 +105,30 @@ def test_autograd_contraction_forms(eng, ncol, nd, params, precision):
         assert float((a - c).abs().max()) <= 1e-12 * float(c.abs().max())
         (d,) = torch.autograd.grad(b.sum(), w)      # the Jacobian summed over the rows
         assert d.shape == st.shape and bool(torch.isfinite(d).all()) and float(d.abs().max()) > 0
+
+
+def _small_graph(eng, ncol=3, precision=0):
+    import torch
+    from pyrh_amd import autograd
+    x = torch.from_numpy(W.stokes_map(ncol, seed=W.SEED_BASE + 84)).cuda().requires_grad_(True)
+    st = autograd.stokes(eng, x, precision=precision, params=("T", "B"))
+    w = torch.linspace(-1.0, 1.0, 2 * st.numel(), dtype=torch.float64, device="cuda").view(2, *st.shape)
+    return x, st, w
+
+
+@pytest.mark.parametrize("precision", (0, 1))
+def test_autograd_carries_forward_tangents(eng, precision):
+    """The backward is linear in the incoming gradient, so under forward-mode
+    the tangent of a dual gradient goes through the same contraction: to the
+    gradient of the tangent (sums in another order, 1e-12 of the largest)."""
+    import torch
+    import torch.autograd.forward_ad as fad
+    x, st, (w, t) = _small_graph(eng, precision=precision)
+    (gw,) = torch.autograd.grad(st, x, w, retain_graph=True)
+    (gt,) = torch.autograd.grad(st, x, t, retain_graph=True)
+    with fad.dual_level():
+        (g,) = torch.autograd.grad(st, x, fad.make_dual(w, t), retain_graph=True)
+        primal, tangent = fad.unpack_dual(g)
+        assert tangent is not None
+        for a, b in ((primal, gw), (tangent, gt)):
+            assert float((a - b).abs().max()) <= 1e-12 * float(b.abs().max())

@@ -240,3 +240,21 @@ def test_grid_positions_and_table():
     np.testing.assert_array_equal(flat[ptr[1]:ptr[2]], pos[1])
     with pytest.raises(ValueError, match="not on the merged grid"):
         api.grid_positions(m, [np.array([wl[0] + 1e-4])])
+
+
+def test_contraction_takes_bare_tensors_only():
+    """The autograd backward hands raw memory to its kernel for tensors that
+    are nothing but memory."""
+    torch = pytest.importorskip("torch")
+    import torch.autograd.forward_ad as fad
+    from pyrh_amd.autograd import _bare
+    t = torch.ones(2, 4, 3, dtype=torch.float64)
+    assert _bare(t) and _bare(t.permute(2, 1, 0)) and _bare(t.clone().requires_grad_(True))
+    assert not _bare(torch.nn.Parameter(t))
+    assert not _bare(torch.conj(torch.complex(t, t)).imag)
+    with fad.dual_level():
+        assert not _bare(fad.make_dual(t, torch.ones_like(t))) and _bare(t)
+    seen = []
+    torch.func.vmap(lambda v: (seen.append(_bare(v)), v)[1])(t)
+    torch.func.jvp(lambda v: (seen.append(_bare(v)), v)[1], (t,), (t,))
+    assert seen == [False, False]
