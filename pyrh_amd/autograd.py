@@ -40,13 +40,19 @@ def _bare(t):
             and forward_ad.unpack_dual(t).tangent is None and not t.is_neg())
 
 
+def _watched():
+    """Whether a mode sees the operations run now (make_fx and other
+    dispatch modes, torch-function modes): it would not see a kernel."""
+    return torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0
+
+
 def _contract_here(rf, g, shape):
     """Whether backward may run rhg_rf_contract: plain CUDA tensors of one
     device (_bare: the kernel reads their memory and nothing else), the saved
     response functions as forward laid them out (a saved-tensor hook may
-    return others), and no graph of the backward itself (create_graph), which
-    torch has to see the operations of."""
-    return (_bare(rf) and _bare(g) and g.is_cuda
+    return others), and nobody who has to see the operations: a graph of the
+    backward itself (create_graph), a tracer or another mode (_watched)."""
+    return (_bare(rf) and _bare(g) and not _watched() and g.is_cuda
             and rf.device == g.device and rf.dtype in (torch.float32, torch.float64)
             and tuple(rf.shape) == shape and rf.is_contiguous()
             and not (torch.is_grad_enabled() and (g.requires_grad or rf.requires_grad)))

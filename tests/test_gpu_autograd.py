@@ -132,3 +132,16 @@ def test_autograd_carries_forward_tangents(eng, precision):
         assert tangent is not None
         for a, b in ((primal, gw), (tangent, gt)):
             assert float((a - b).abs().max()) <= 1e-12 * float(b.abs().max())
+
+
+def test_autograd_backward_can_be_traced(eng):
+    """make_fx records the backward's operations: the graph replays the
+    gradient of other incoming gradients too."""
+    import torch
+    from torch.fx.experimental.proxy_tensor import make_fx
+    x, st, (w, t) = _small_graph(eng)
+    backward = lambda g: torch.autograd.grad(st, x, g, retain_graph=True)[0]
+    graph = make_fx(backward)(w)
+    for g in (w, t):
+        a, b = graph(g), backward(g)
+        assert float((a - b).abs().max()) <= 1e-12 * float(b.abs().max())

@@ -258,3 +258,24 @@ def test_contraction_takes_bare_tensors_only():
     torch.func.vmap(lambda v: (seen.append(_bare(v)), v)[1])(t)
     torch.func.jvp(lambda v: (seen.append(_bare(v)), v)[1], (t,), (t,))
     assert seen == [False, False]
+
+
+def test_contraction_steps_aside_for_modes():
+    torch = pytest.importorskip("torch")
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from pyrh_amd.autograd import _watched
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    assert not _watched()
+    for mode in (Functions, Dispatch):
+        with mode():
+            assert _watched()
+    assert not _watched()
