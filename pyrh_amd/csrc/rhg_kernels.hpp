@@ -368,15 +368,31 @@ __device__ __forceinline__ T line_profile_t(const Tab &tab, int i, int lb, const
           group(tab.cpi(i), tab.csp(i), phi_pi, psi_pi);
           group(tab.csp(i), c1, phi_sp, psi_sp);
         } else {
+          // a component's sum is selected by value: selected by address, the
+          // sums would live in scratch memory
+          T phis[3] = {T(0), T(0), T(0)}, psis[3] = {T(0), T(0), T(0)};
+          auto add = [](T (&sum)[3], int q, const T &a, const T &b) {
+            T s = q == -1 ? sum[0] : (q == 0 ? sum[1] : sum[2]);
+            acc_prod(s, a, b);
+            sum[0] = q == -1 ? s : sum[0];
+            sum[1] = q == 0 ? s : sum[1];
+            sum[2] = q == -1 || q == 0 ? sum[2] : s;
+          };
           for (int nz = c0; nz < c1; nz++) {
             TV Fw;
             const T H = component(FAR, tab.shift(nz), Fw);
-            const T Fv = (T) Fw;
-            (void) Fv;
             const int q = tab.q(nz);
             const T sg = T(tab.strength(nz));
-            acc_prod(q == -1 ? phi_sm : (q == 0 ? phi_pi : phi_sp), sg, H);
-            if constexpr (MO) acc_prod(q == -1 ? psi_sm : (q == 0 ? psi_pi : psi_sp), sg, Fv);
+            add(phis, q, sg, H);
+            if constexpr (MO) add(psis, q, sg, (T) Fw);
+          }
+          phi_sm = phis[0];
+          phi_pi = phis[1];
+          phi_sp = phis[2];
+          if constexpr (MO) {
+            psi_sm = psis[0];
+            psi_pi = psis[1];
+            psi_sp = psis[2];
           }
         }
       };

@@ -279,3 +279,47 @@ def test_contraction_steps_aside_for_modes():
         with mode():
             assert _watched()
     assert not _watched()
+
+
+def _kernels():
+    """The compiler's resource figures {mangled name: metadata} of the
+    library's gfx950 kernels, from its code objects' metadata notes."""
+    import struct
+    msgpack = pytest.importorskip("msgpack")
+    from pyrh_amd.build import LIB
+    d, out, pos = LIB.read_bytes(), {}, 0
+    magic = b"__CLANG_OFFLOAD_BUNDLE__"
+    while (pos := d.find(magic, pos)) >= 0:
+        (n,), q = struct.unpack_from("<Q", d, pos + 24), pos + 32
+        for _ in range(n):
+            off, size, tl = struct.unpack_from("<QQQ", d, q)
+            if b"gfx950" in d[q + 24:q + 24 + tl] and size:
+                elf = d[pos + off:pos + off + size]
+                phoff, = struct.unpack_from("<Q", elf, 32)
+                phsz, phn = struct.unpack_from("<HH", elf, 54)
+                for h in range(phoff, phoff + phn * phsz, phsz):
+                    kind, _, o = struct.unpack_from("<IIQ", elf, h)
+                    if kind != 4:                       # PT_NOTE
+                        continue
+                    nlen, dlen, ntype = struct.unpack_from("<III", elf, o)
+                    if ntype == 32:                     # NT_AMDGPU_METADATA
+                        a = o + 12 + (nlen + 3) // 4 * 4
+                        for k in msgpack.unpackb(elf[a:a + dlen])["amdhsa.kernels"]:
+                            out[k[".name"]] = k
+            q += 24 + tl
+        pos += len(magic)
+    assert out
+    return out
+
+
+def test_component_sums_stay_in_registers():
+    """The kernels that read line lists from the model select a Zeeman
+    component's sum by value: selected by address, the sums lie in scratch
+    memory (32 bytes a lane and more) or in LDS."""
+    ks = _kernels()
+    small = [k for n, k in ks.items() if re.search(
+        r"k_formal_stokesI[df]Lb0ELb0EE|k_formal_scalarI|k_rf_loggf|k_rf_pointsI[df]Lb0E", n)]
+    assert len(small) == 8
+    assert all(k[".private_segment_fixed_size"] <= 8 for k in small)
+    mo = [k for n, k in ks.items() if re.search(r"k_formal_stokesI[df]Lb1ELb0EE", n)]
+    assert len(mo) == 2 and all(k[".group_segment_fixed_size"] == 0 for k in mo)
