@@ -19,9 +19,11 @@ namespace rhg {
 // instead of a vector memory access per lane.  Only for data no kernel
 // writes while it runs.
 typedef __attribute__((address_space(4))) const double CDouble;
+typedef __attribute__((address_space(4))) const float CFloat;
 typedef __attribute__((address_space(4))) const int32_t CInt;
 __device__ __forceinline__ CDouble *ldc(const double *p) { return (CDouble *) p; }
 __device__ __forceinline__ CInt *ldc(const int32_t *p) { return (CInt *) p; }
+__device__ __forceinline__ CFloat *ldc(const float *p) { return (CFloat *) p; }
 
 struct DevModel {
   int stokes_mode, magneto_optical;
@@ -72,8 +74,8 @@ struct DevModel {
   int ntile;
   const int32_t *tile_ptr, *tile_cont;
   const double *tile_alpha;
-  // per line, the largest |shift| of its Zeeman components
-  const double *line_smax;
+  // per line, the largest |shift| of its Zeeman components, rounded up
+  const float *line_smax;
   // per wavelength, the temperature tables of its continuum terms with the
   // wavelength already interpolated: KT_N doubles, tables at KT_*
   const double *ktab;
@@ -176,7 +178,7 @@ struct LineTabG {
   __device__ __forceinline__ bool damped(int i) const { return ldc(M.line_Grad)[line(i)] != 0.0; }
   __device__ __forceinline__ bool polar(int i) const { return ldc(M.line_polar)[line(i)] != 0; }
   __device__ __forceinline__ double larmor(int i) const { return ldc(M.line_larmor)[line(i)]; }
-  __device__ __forceinline__ double smax(int i) const { return ldc(M.line_smax)[line(i)]; }
+  __device__ __forceinline__ double smax(int i) const { return (double) ldc(M.line_smax)[line(i)]; }
   __device__ __forceinline__ int c0(int i) const { return ldc(M.line_comp_ptr)[line(i)]; }
   __device__ __forceinline__ int c1(int i) const { return ldc(M.line_comp_ptr)[line(i) + 1]; }
   __device__ __forceinline__ double shift(int c) const { return ldc(M.comp_shift)[c]; }
@@ -192,11 +194,16 @@ struct LineTabG {
 // each group feeds its own sum, so the sums see the same terms in the same
 // order as from the ungrouped list, and the component loop needs no
 // per-component branch.
+// (40 bytes: a list of up to 16 KB is staged)
 struct LineRecL {
-  double dv, larmor, smax;
-  int line, flags, c0, c1;   // flags: 1 damped, 2 polarizable
+  static constexpr uint32_t DAMPED = 1u << 31, POLAR = 1u << 30, LINE = POLAR - 1;
+  double dv, larmor;
+  float smax;
+  uint32_t line;             // with DAMPED and POLAR
+  int c0, c1;
   int cpi, csp;              // first pi and first sigma+ component
 };
+static_assert(sizeof(LineRecL) == 40, "LineRecL");
 
 struct LineTabL {
   static constexpr bool grouped = true;
@@ -204,18 +211,15 @@ struct LineTabL {
   const double *shift_, *strength_;
   const int *q_;
   int n;
-  __device__ __forceinline__ int line(int i) const {
-    return __builtin_amdgcn_readfirstlane(rec[i].line);
+  __device__ __forceinline__ uint32_t word(int i) const {
+    return (uint32_t) __builtin_amdgcn_readfirstlane((int) rec[i].line);
   }
+  __device__ __forceinline__ int line(int i) const { return (int) (word(i) & LineRecL::LINE); }
   __device__ __forceinline__ double dv(int i) const { return rec[i].dv; }
-  __device__ __forceinline__ bool damped(int i) const {
-    return __builtin_amdgcn_readfirstlane(rec[i].flags) & 1;
-  }
-  __device__ __forceinline__ bool polar(int i) const {
-    return __builtin_amdgcn_readfirstlane(rec[i].flags) & 2;
-  }
+  __device__ __forceinline__ bool damped(int i) const { return word(i) & LineRecL::DAMPED; }
+  __device__ __forceinline__ bool polar(int i) const { return word(i) & LineRecL::POLAR; }
   __device__ __forceinline__ double larmor(int i) const { return rec[i].larmor; }
-  __device__ __forceinline__ double smax(int i) const { return rec[i].smax; }
+  __device__ __forceinline__ double smax(int i) const { return (double) rec[i].smax; }
   __device__ __forceinline__ int c0(int i) const { return __builtin_amdgcn_readfirstlane(rec[i].c0); }
   __device__ __forceinline__ int c1(int i) const { return __builtin_amdgcn_readfirstlane(rec[i].c1); }
   __device__ __forceinline__ int cpi(int i) const { return __builtin_amdgcn_readfirstlane(rec[i].cpi); }
@@ -248,8 +252,7 @@ __device__ __forceinline__ LineTabL stage_lines(const DevModel &M, int ls, char 
     rec[i].dv = ldc(M.lam_line_dv)[p0 + i];
     rec[i].larmor = ldc(M.line_larmor)[l];
     rec[i].smax = ldc(M.line_smax)[l];
-    rec[i].line = l;
-    rec[i].flags = (damped ? 1 : 0) | (polar ? 2 : 0);
+    rec[i].line = (uint32_t) l | (damped ? LineRecL::DAMPED : 0u) | (polar ? LineRecL::POLAR : 0u);
     // only a damped polarizable line uses its components
     rec[i].c1 = (damped && polar) ? ldc(M.line_comp_ptr)[l + 1] - ldc(M.line_comp_ptr)[l] : 0;
   }
@@ -266,7 +269,7 @@ __device__ __forceinline__ LineTabL stage_lines(const DevModel &M, int ls, char 
   // components grouped by Delta M = -1, 0, +1, each in the model's order
   for (int i = 0; i < n; i++) {
     const int a = rec[i].c0, cnt = rec[i].c1 - a;
-    const int g0 = ldc(M.line_comp_ptr)[rec[i].line];
+    const int g0 = ldc(M.line_comp_ptr)[rec[i].line & LineRecL::LINE];
     int nsm = 0, npi = 0;
     for (int c = 0; c < cnt; c++) {
       const int qc = ldc(M.comp_q)[g0 + c];

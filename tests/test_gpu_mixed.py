@@ -184,3 +184,27 @@ def test_mixed_rf_sorted(eng):
         err = np.max(np.abs(ad[0] - fd[0])) / scale
         print(f"dI/dT depth {k}: max err {err:.2e} of max |dI/dT|", flush=True)
         assert err < 1e-3
+
+
+@pytest.mark.parametrize("nline,staged", ((74, 1), (75, 0)))
+def test_line_list_at_the_lds_limit(tmp_path, nline, staged):
+    """A line of nine components takes 40 + 9 * 20 bytes of the staged list's
+    16384: 74 such lines at one wavelength are staged, 75 are read from the
+    model; a staged list gives the bits of the other."""
+    from pyrh_amd.engine import Engine
+    run = W.mixed_run_dir(str(tmp_path / "run"), str(RUN))
+    recs = [f"{630.0 + 1e-4 * i:10.4f}" + r[10:] for i, r in enumerate(W.mixed_line_records(nline))]
+    (tmp_path / "run" / "fe_synthetic400").write_text("\n".join(recs) + "\n")
+    m = model.build_model(model.open_run(run), W.mixed_wavelengths()[995:1005])
+    a = m.arrays
+    assert int(np.diff(a["lam_line_ptr"]).max()) == nline
+    assert np.all(np.diff(a["line_comp_ptr"]) == 9)
+    e = Engine(m)
+    assert e.tuning()["line_table"] == staged
+    atm, nd = W.mixed_batch(66, seed=W.SEED_BASE + 85, ndep_choices=(64, 70))
+    for prec in (0, 1):
+        e.set_tuning("line_table", 1)
+        st = e.synth_lte(atm, ndep=nd, precision=prec)
+        e.set_tuning("line_table", 0)
+        np.testing.assert_array_equal(st, e.synth_lte(atm, ndep=nd, precision=prec))
+    e.close()
