@@ -381,14 +381,10 @@ int rhg_open(const rhg_model_t *m, int device, rhg_context_t **out) {
     if (!rc) rc = upload(c, talpha.empty() ? nullptr : talpha.data(), talpha.size(), &d.tile_alpha);
   }
   if (!rc) {
-    std::vector<float> smax((size_t) std::max(m->nline, 1), 0.0f);
+    std::vector<double> smax((size_t) std::max(m->nline, 1), 0.0);
     for (int l = 0; l < m->nline; l++)
-      for (int q = m->line_comp_ptr[l]; q < m->line_comp_ptr[l + 1]; q++) {
-        const double x = fabs(m->comp_shift[q]);
-        float f = (float) x;
-        if ((double) f < x) f = nextafterf(f, INFINITY);
-        smax[l] = std::max(smax[l], f);
-      }
+      for (int q = m->line_comp_ptr[l]; q < m->line_comp_ptr[l + 1]; q++)
+        smax[l] = std::max(smax[l], fabs(m->comp_shift[q]));
     rc = upload(c, smax.data(), smax.size(), &d.line_smax);
   }
   if (!rc) {

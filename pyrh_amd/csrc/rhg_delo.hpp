@@ -56,8 +56,8 @@ __device__ __forceinline__ void form_point_f(const DevModel &M, int ls, int has_
                                              const Field &F, T mu, int moving, T cchi, T ceta,
                                              Point<T> &p) {
   const int p0 = ldc(M.lam_line_ptr)[ls];
-  form_point_t<T, TV, MO>(LineTabG(M, p0, ldc(M.lam_line_ptr)[ls + 1] - p0), M.ncont, has_line, F, mu,
-                          moving, cchi, ceta, p);
+  form_point_t<T, TV, MO>(LineTabGDirect(M, p0, ldc(M.lam_line_ptr)[ls + 1] - p0), M.ncont, has_line,
+                          F, mu, moving, cchi, ceta, p);
 }
 
 // FP64 point over the column state at st (stride fs) with the Humlicek
@@ -69,16 +69,6 @@ __device__ __forceinline__ void form_point_vt(const Tab &tab, int ncont, int has
   auto F = [st, fs](int f) { return st[f * fs]; };
   form_point_t<double, TV, MO>(tab, ncont, has_line, F, mu, moving, (double) cchi, (double) ceta,
                                p);
-}
-
-// the same over wavelength ls's line list in the model
-template <typename TV, typename R, bool MO = false>
-__device__ __forceinline__ void form_point_v(const DevModel &M, int ls, int has_line,
-                                             const double *st, int64_t fs, double mu, int moving,
-                                             R cchi, R ceta, Point<double> &p) {
-  const int p0 = ldc(M.lam_line_ptr)[ls];
-  form_point_vt<TV, R, MO>(LineTabG(M, p0, ldc(M.lam_line_ptr)[ls + 1] - p0), M.ncont, has_line, st,
-                           fs, mu, moving, cchi, ceta, p);
 }
 
 // y = K(q) x for K(q) = [[0, q^T], [q, 0]]

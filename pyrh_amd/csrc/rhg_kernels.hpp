@@ -19,11 +19,9 @@ namespace rhg {
 // instead of a vector memory access per lane.  Only for data no kernel
 // writes while it runs.
 typedef __attribute__((address_space(4))) const double CDouble;
-typedef __attribute__((address_space(4))) const float CFloat;
 typedef __attribute__((address_space(4))) const int32_t CInt;
 __device__ __forceinline__ CDouble *ldc(const double *p) { return (CDouble *) p; }
 __device__ __forceinline__ CInt *ldc(const int32_t *p) { return (CInt *) p; }
-__device__ __forceinline__ CFloat *ldc(const float *p) { return (CFloat *) p; }
 
 struct DevModel {
   int stokes_mode, magneto_optical;
@@ -74,8 +72,8 @@ struct DevModel {
   int ntile;
   const int32_t *tile_ptr, *tile_cont;
   const double *tile_alpha;
-  // per line, the largest |shift| of its Zeeman components, rounded up
-  const float *line_smax;
+  // per line, the largest |shift| of its Zeeman components
+  const double *line_smax;
   // per wavelength, the temperature tables of its continuum terms with the
   // wavelength already interpolated: KT_N doubles, tables at KT_*
   const double *ktab;
@@ -167,24 +165,31 @@ __device__ __forceinline__ double atom_sum(const DevModel &M, int l0, int nl, do
 // (lambda/lambda0 - 1) c, and its Zeeman components are c0(i) .. c1(i)-1.
 // LineTabG reads the model in global memory; LineTabL (below) reads a copy
 // staged in LDS by the kernel.
-struct LineTabG {
-  static constexpr bool grouped = false;
+// AHEAD: whether the component loop reads a component's constants ahead.
+template <bool AHEAD>
+struct LineTabGlobal {
+  static constexpr bool grouped = false, ahead = AHEAD;
   const DevModel &M;
   int p0, n;
   // entries p0 .. p0 + n - 1 of the model's wavelength line lists
-  __device__ __forceinline__ LineTabG(const DevModel &M_, int p0_, int n_) : M(M_), p0(p0_), n(n_) {}
+  __device__ __forceinline__ LineTabGlobal(const DevModel &M_, int p0_, int n_) : M(M_), p0(p0_), n(n_) {}
   __device__ __forceinline__ int line(int i) const { return ldc(M.lam_line_idx)[p0 + i]; }
   __device__ __forceinline__ double dv(int i) const { return ldc(M.lam_line_dv)[p0 + i]; }
   __device__ __forceinline__ bool damped(int i) const { return ldc(M.line_Grad)[line(i)] != 0.0; }
   __device__ __forceinline__ bool polar(int i) const { return ldc(M.line_polar)[line(i)] != 0; }
   __device__ __forceinline__ double larmor(int i) const { return ldc(M.line_larmor)[line(i)]; }
-  __device__ __forceinline__ double smax(int i) const { return (double) ldc(M.line_smax)[line(i)]; }
+  __device__ __forceinline__ double smax(int i) const { return ldc(M.line_smax)[line(i)]; }
   __device__ __forceinline__ int c0(int i) const { return ldc(M.line_comp_ptr)[line(i)]; }
   __device__ __forceinline__ int c1(int i) const { return ldc(M.line_comp_ptr)[line(i) + 1]; }
   __device__ __forceinline__ double shift(int c) const { return ldc(M.comp_shift)[c]; }
   __device__ __forceinline__ double strength(int c) const { return ldc(M.comp_strength)[c]; }
   __device__ __forceinline__ int q(int c) const { return ldc(M.comp_q)[c]; }
 };
+using LineTabG = LineTabGlobal<true>;
+// for kernels of three and more waves per SIMD, which hide those reads: the
+// scalar Stokes modes, 6000 map columns in FP32, take 2.69 ms without, 2.79
+// with
+using LineTabGDirect = LineTabGlobal<false>;
 
 // A wavelength's line list staged in LDS (one copy per wavefront; every
 // lane reads the same address, so the reads are broadcasts).  Counts and
@@ -198,7 +203,7 @@ struct LineTabG {
 struct LineRecL {
   static constexpr uint32_t DAMPED = 1u << 31, POLAR = 1u << 30, LINE = POLAR - 1;
   double dv, larmor;
-  float smax;
+  float smax;                // rounded up
   uint32_t line;             // with DAMPED and POLAR
   int c0, c1;
   int cpi, csp;              // first pi and first sigma+ component
@@ -251,7 +256,7 @@ __device__ __forceinline__ LineTabL stage_lines(const DevModel &M, int ls, char 
     const bool damped = ldc(M.line_Grad)[l] != 0.0, polar = ldc(M.line_polar)[l] != 0;
     rec[i].dv = ldc(M.lam_line_dv)[p0 + i];
     rec[i].larmor = ldc(M.line_larmor)[l];
-    rec[i].smax = ldc(M.line_smax)[l];
+    rec[i].smax = __double2float_ru(ldc(M.line_smax)[l]);
     rec[i].line = (uint32_t) l | (damped ? LineRecL::DAMPED : 0u) | (polar ? LineRecL::POLAR : 0u);
     // only a damped polarizable line uses its components
     rec[i].c1 = (damped && polar) ? ldc(M.line_comp_ptr)[l + 1] - ldc(M.line_comp_ptr)[l] : 0;
@@ -388,17 +393,19 @@ __device__ __forceinline__ T line_profile_t(const Tab &tab, int i, int lb, const
           double sh = c0 < c1 ? tab.shift(c0) : 0.0, sg = c0 < c1 ? tab.strength(c0) : 0.0;
           int q = c0 < c1 ? tab.q(c0) : 0;
           for (int nz = c0; nz < c1; nz++) {
-            const double shc = sh, sgc = sg;
-            const int qc = q;
-            if (nz + 1 < c1) {
+            const double shc = Tab::ahead ? sh : tab.shift(nz), sga = sg;
+            const int qa = q;
+            if (Tab::ahead && nz + 1 < c1) {
               sh = tab.shift(nz + 1);
               sg = tab.strength(nz + 1);
               q = tab.q(nz + 1);
             }
             TV Fw;
             const T H = component(FAR, shc, Fw);
-            add(phis, qc, T(sgc), H);
-            if constexpr (MO) add(psis, qc, T(sgc), (T) Fw);
+            const int qc = Tab::ahead ? qa : tab.q(nz);
+            const T sgc = T(Tab::ahead ? sga : tab.strength(nz));
+            add(phis, qc, sgc, H);
+            if constexpr (MO) add(psis, qc, sgc, (T) Fw);
           }
           phi_sm = phis[0];
           phi_pi = phis[1];
@@ -448,7 +455,7 @@ __device__ __forceinline__ T line_profile_f(const DevModel &M, int e, int l, con
                                             T vz, int moving, T &phi_Q, T &phi_U, T &phi_V,
                                             T *psi = nullptr) {
   (void) l;
-  return line_profile_t<T, TV, MO>(LineTabG(M, e, 1), 0, line_field_base(M.ncont), F, mu, vz,
+  return line_profile_t<T, TV, MO>(LineTabGDirect(M, e, 1), 0, line_field_base(M.ncont), F, mu, vz,
                                    moving, phi_Q, phi_U, phi_V, psi);
 }
 
@@ -498,7 +505,7 @@ __device__ __forceinline__ void line_point_f(const DevModel &M, int ls, const Fi
                                              T &chiI, T *chiQ, T &etaI, T *etaQ, int moving,
                                              T *chip = nullptr) {
   const int p0 = ldc(M.lam_line_ptr)[ls];
-  line_point_t<T, TV, MO>(LineTabG(M, p0, ldc(M.lam_line_ptr)[ls + 1] - p0), M.ncont, F, mu, chiI, chiQ,
+  line_point_t<T, TV, MO>(LineTabGDirect(M, p0, ldc(M.lam_line_ptr)[ls + 1] - p0), M.ncont, F, mu, chiI, chiQ,
                           etaI, etaQ, moving, chip);
 }
 
