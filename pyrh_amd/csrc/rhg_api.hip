@@ -2000,18 +2000,33 @@ struct NlteTimer {
 }  // namespace
 
 // run LAUNCH(L, P) with the lanes per ray direction L and the points per lane
-// P for Nmax depths (L P >= Nmax): two or three points per lane hide the
-// latency of a point's arithmetic, more spill
-#define RHG_RAY_POINTS(Nmax, LAUNCH)        \
-  do {                                      \
-    if ((Nmax) <= 64) LAUNCH(32, 2);        \
-    else if ((Nmax) <= 96) LAUNCH(32, 3);   \
-    else if ((Nmax) <= 128) LAUNCH(64, 2);  \
-    else if ((Nmax) <= 192) LAUNCH(64, 3);  \
-    else if ((Nmax) <= 256) LAUNCH(64, 4);  \
-    else LAUNCH(64, 8);                     \
+// P for columns of up to Nd depths (L P >= Nd): two or three points per lane hide
+// the latency of a point's arithmetic, more spill
+#define RHG_RAY_POINTS(Nd, LAUNCH)        \
+  do {                                    \
+    if ((Nd) <= 32) LAUNCH(32, 1);        \
+    else if ((Nd) <= 64) LAUNCH(32, 2);   \
+    else if ((Nd) <= 96) LAUNCH(32, 3);   \
+    else if ((Nd) <= 128) LAUNCH(64, 2);  \
+    else if ((Nd) <= 192) LAUNCH(64, 3);  \
+    else if ((Nd) <= 256) LAUNCH(64, 4);  \
+    else if ((Nd) <= 384) LAUNCH(128, 3); \
+    else LAUNCH(128, 4);                  \
   } while (0)
-static_assert(64 * 8 >= RHG_MAX_DEPTH, "RHG_RAY_POINTS covers every depth count");
+// the same where up to eight transitions are active at a wavelength, whose
+// member data fills the registers of two points: the 16-level Na I atom, two
+// passes, 2000 columns of 96 depths 47 ms (three points, 315 registers spilled:
+// 60), 800 of 256 42 ms (four, 736 spilled: 107)
+#define RHG_RAY_POINTS_WIDE(Nd, LAUNCH)   \
+  do {                                    \
+    if ((Nd) <= 32) LAUNCH(32, 1);        \
+    else if ((Nd) <= 64) LAUNCH(32, 2);   \
+    else if ((Nd) <= 128) LAUNCH(64, 2);  \
+    else if ((Nd) <= 256) LAUNCH(128, 2); \
+    else if ((Nd) <= 384) LAUNCH(128, 3); \
+    else LAUNCH(128, 4);                  \
+  } while (0)
+static_assert(128 * 4 >= RHG_MAX_DEPTH, "RHG_RAY_POINTS covers every depth count");
 
 extern "C" {
 
@@ -2219,17 +2234,18 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
           const dim3 grd((unsigned) rhg::xcd_grid(nact, h.nbez));
 #define RHG_LAUNCH_BEZ(L, P, MS)                                                                 \
   hipLaunchKernelGGL((rhg::k_nlte_bezier<L, P, MS>), grd, dim3(2 * L),                            \
-                     rhg::nlte_bez_lds(L, P, MS, Nmax) * sizeof(double), c->stream, c->d_model,   \
+                     rhg::nlte_bez_lds(L, P, MS) * sizeof(double), c->stream, c->d_model,   \
                      d_at, B, d_act, nact,                                                       \
                      c->d_out_ls, d_iolist, h.nbez, 0, nlist, eval)
-#define RHG_LAUNCH_BEZ_P(L, P)                                                                   \
-  do {                                                                                           \
-    if (h.maxset_bez <= 2) RHG_LAUNCH_BEZ(L, P, 2);                                              \
-    else if (h.maxset_bez <= 4) RHG_LAUNCH_BEZ(L, P, 4);                                         \
-    else RHG_LAUNCH_BEZ(L, P, 8);                                                                \
-  } while (0)
-          RHG_RAY_POINTS(Nmax, RHG_LAUNCH_BEZ_P);
-#undef RHG_LAUNCH_BEZ_P
+#define RHG_LAUNCH_BEZ_2(L, P) RHG_LAUNCH_BEZ(L, P, 2)
+#define RHG_LAUNCH_BEZ_4(L, P) RHG_LAUNCH_BEZ(L, P, 4)
+#define RHG_LAUNCH_BEZ_8(L, P) RHG_LAUNCH_BEZ(L, P, 8)
+          if (h.maxset_bez <= 2) RHG_RAY_POINTS(Nmax, RHG_LAUNCH_BEZ_2);
+          else if (h.maxset_bez <= 4) RHG_RAY_POINTS(Nmax, RHG_LAUNCH_BEZ_4);
+          else RHG_RAY_POINTS_WIDE(Nmax, RHG_LAUNCH_BEZ_8);
+#undef RHG_LAUNCH_BEZ_2
+#undef RHG_LAUNCH_BEZ_4
+#undef RHG_LAUNCH_BEZ_8
 #undef RHG_LAUNCH_BEZ
           HIPCHECK(hipGetLastError());
         }
@@ -2359,9 +2375,11 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
       const int nfe = nlist - h.nbez;
       if (h.nbez > 0) {
         const dim3 grd((unsigned) rhg::xcd_grid(ncol, h.nbez));
+        // (one ray: a direction's lanes in one wavefront)
 #define RHG_LAUNCH_EM(L, P)                                                                      \
-  hipLaunchKernelGGL((rhg::k_nlte_emergent<L, P>), grd, b64, 0, c->stream, c->d_model, d_at, B,       \
-                     c->d_out_ls, d_iolist, h.nbez, cols->mu, d_st)
+  hipLaunchKernelGGL((rhg::k_nlte_emergent<std::min(L, 64), (P * L / std::min(L, 64))>), grd,     \
+                     b64, 0, c->stream, c->d_model, d_at, B, c->d_out_ls, d_iolist, h.nbez,      \
+                     cols->mu, d_st)
         RHG_RAY_POINTS(Nmax, RHG_LAUNCH_EM);
 #undef RHG_LAUNCH_EM
         HIPCHECK(hipGetLastError());

@@ -503,21 +503,77 @@ struct RayPath {
   double dz[P], idz[P], al[P];
 };
 
+// The neighbouring lanes of a ray direction.  With L = 128 a direction's lanes
+// are two wavefronts (first half and second half), which meet in `edge`
+// (RAY_EDGE doubles of LDS per direction, one slot per exchange of a sweep):
+// a slot is written again only after the barriers of the exchanges that
+// follow its reading.
+constexpr int RAY_EDGE = 15;
+template <int L>
+struct RayLanes {
+  double *edge;   // of this direction (L > 64)
+  bool second;    // the lane is in the direction's second wavefront
+
+  // up: replaced by the previous lane's values, dn: by the next lane's (the
+  // first and the last lane of a direction get values that are never used)
+  template <int SLOT, int NU, int ND>
+  __device__ __forceinline__ void exchange(double (&up)[NU], double (&dn)[ND]) const {
+    if constexpr (L > 64) {
+      const int lane = threadIdx.x & 63;
+      if (!second && lane == 63)
+#pragma unroll
+        for (int i = 0; i < NU; i++) edge[SLOT + i] = up[i];
+      if (second && lane == 0)
+#pragma unroll
+        for (int i = 0; i < ND; i++) edge[SLOT + NU + i] = dn[i];
+    }
+#pragma unroll
+    for (int i = 0; i < NU; i++) up[i] = from_prev(up[i]);
+#pragma unroll
+    for (int i = 0; i < ND; i++) dn[i] = from_next(dn[i]);
+    if constexpr (L > 64) {
+      __syncthreads();
+      const int lane = threadIdx.x & 63;
+      if (second && lane == 0)
+#pragma unroll
+        for (int i = 0; i < NU; i++) up[i] = edge[SLOT + i];
+      if (!second && lane == 63)
+#pragma unroll
+        for (int i = 0; i < ND; i++) dn[i] = edge[SLOT + NU + i];
+    }
+  }
+  template <int SLOT>
+  __device__ __forceinline__ double prev(double x) const {
+    double up[1] = {x}, dn[1] = {0.0};
+    if constexpr (L > 64) exchange<SLOT>(up, dn);
+    else up[0] = from_prev(x);
+    return up[0];
+  }
+  template <int SLOT>
+  __device__ __forceinline__ double next(double x) const {
+    double up[1] = {0.0}, dn[1] = {x};
+    if constexpr (L > 64) exchange<SLOT>(up, dn);
+    else dn[0] = from_next(x);
+    return dn[0];
+  }
+};
+
 // one ray's intensity and operator at the points from the opacities C (with
 // reciprocals iC), source functions S, 1 / mu and the boundary's Planck
 // function (outward: B at the two deepest points)
 template <int L, int P>
-__device__ __forceinline__ void ray_sweep(const RayPath<P> &g, int t0, int N, bool outward,
-                                          double zmu, double B2_0, double B2_1,
+__device__ __forceinline__ void ray_sweep(const RayLanes<L> &lanes, const RayPath<P> &g, int t0,
+                                          int N, bool outward, double zmu, double B2_0, double B2_1,
                                           const double (&C)[P], const double (&S)[P],
                                           double (&I)[P], double (&Psi)[P]) {
 #pragma clang fp contract(fast)
   double f[P], dchi[P], dtau[P], idt[P], sl[P], dS[P], E[P], b[P];
-  const double C_prev = from_prev(C[P - 1]), C_next = from_next(C[0]);
-  const double S_prev = from_prev(S[P - 1]);
+  double CS_prev[2] = {C[P - 1], S[P - 1]}, C0_next[1] = {C[0]};
+  lanes.template exchange<0>(CS_prev, C0_next);
+  const double C_prev = CS_prev[0], S_prev = CS_prev[1], C_next = C0_next[0];
 #pragma unroll
   for (int s = 0; s < P; s++) f[s] = (C[s] - (s ? C[s > 0 ? s - 1 : 0] : C_prev)) * g.idz[s];
-  const double f_next = from_next(f[0]);
+  const double f_next = lanes.template next<3>(f[0]);
 #pragma unroll
   for (int s = 0; s < P; s++) {
     const int t = t0 + s;
@@ -526,7 +582,7 @@ __device__ __forceinline__ void ray_sweep(const RayPath<P> &g, int t0, int N, bo
     if (t == 0) dchi[s] = fn;
     if (t == N - 1) dchi[s] = f[s];
   }
-  const double dchi_prev = from_prev(dchi[P - 1]);
+  const double dchi_prev = lanes.template prev<5>(dchi[P - 1]);
 #pragma unroll
   for (int s = 0; s < P; s++) {
     const double Cm = s ? C[s > 0 ? s - 1 : 0] : C_prev, dm = s ? dchi[s > 0 ? s - 1 : 0] : dchi_prev;
@@ -536,7 +592,9 @@ __device__ __forceinline__ void ray_sweep(const RayPath<P> &g, int t0, int N, bo
     idt[s] = nrcp(dtau[s]);
     sl[s] = (S[s] - (s ? S[s > 0 ? s - 1 : 0] : S_prev)) * idt[s];
   }
-  const double dtau_next = from_next(dtau[0]), sl_next = from_next(sl[0]);
+  double none[1] = {0.0}, ts_next[2] = {dtau[0], sl[0]};
+  lanes.template exchange<7>(none, ts_next);
+  const double dtau_next = ts_next[0], sl_next = ts_next[1];
 #pragma unroll
   for (int s = 0; s < P; s++) {
     const double tn = s < P - 1 ? dtau[s < P - 1 ? s + 1 : s] : dtau_next;
@@ -546,7 +604,7 @@ __device__ __forceinline__ void ray_sweep(const RayPath<P> &g, int t0, int N, bo
     dS[s] = p > 0.0 ? 3.0 * p * ts * nrcp((ts + dtau[s]) * sl[s] + (ts + tn) * sn) : 0.0;
     if (t0 + s == 0) dS[s] = sn;
   }
-  const double dS_prev = from_prev(dS[P - 1]);
+  const double dS_prev = lanes.template prev<10>(dS[P - 1]);
 #pragma unroll
   for (int s = 0; s < P; s++) {
     const int t = t0 + s;
@@ -614,9 +672,18 @@ __device__ __forceinline__ void ray_sweep(const RayPath<P> &g, int t0, int N, bo
   RAY_SCAN(0x114, 0xf)   // row_shr:4
   RAY_SCAN(0x118, 0xf)   // row_shr:8
   RAY_SCAN(0x142, 0xa)   // row_bcast:15 into rows 1 and 3
-  if constexpr (L == 64) RAY_SCAN(0x143, 0xc)   // row_bcast:31 into rows 2 and 3
+  if constexpr (L >= 64) RAY_SCAN(0x143, 0xc)   // row_bcast:31 into rows 2 and 3
 #undef RAY_SCAN
   double Iu = from_prev(Lb);
+  if constexpr (L > 64) {
+    // the first wavefront's last intensity enters the second (moves between
+    // lanes stay outside of the branches: every lane has to take part)
+    const double Eu = from_prev(LE);
+    if (!lanes.second && (threadIdx.x & 63) == 63) lanes.edge[12] = Lb;
+    __syncthreads();
+    const double I1 = lanes.edge[12];
+    if (lanes.second) Iu = (threadIdx.x & 63) == 0 ? I1 : fma(Eu, I1, Iu);
+  }
 #pragma unroll
   for (int s = 0; s < P; s++) {
     Iu = t0 + s == 0 ? b[s] : fma(E[s], Iu, b[s]);
@@ -626,9 +693,10 @@ __device__ __forceinline__ void ray_sweep(const RayPath<P> &g, int t0, int N, bo
 
 // the lane's points: depths, paths and interval weights (points
 // past the last stand at the last depth and are never read)
-template <int P>
-__device__ __forceinline__ void ray_points(const NlteBufs &B, int64_t col, int t0, int N,
-                                           bool outward, int (&k)[P], RayPath<P> &g) {
+template <int L, int P>
+__device__ __forceinline__ void ray_points(const RayLanes<L> &lanes, const NlteBufs &B, int64_t col,
+                                           int t0, int N, bool outward, int (&k)[P],
+                                           RayPath<P> &g) {
 #pragma clang fp contract(fast)
 #pragma unroll
   for (int s = 0; s < P; s++) {
@@ -638,7 +706,7 @@ __device__ __forceinline__ void ray_points(const NlteBufs &B, int64_t col, int t
     g.dz[s] = B.geo[NG_DZ * B.fs + col + (outward ? N - tu : tu)];
     g.idz[s] = nrcp(g.dz[s]);
   }
-  const double dz_next = from_next(g.dz[0]);
+  const double dz_next = lanes.template next<13>(g.dz[0]);
 #pragma unroll
   for (int s = 0; s < P; s++) {
     const double dn = s < P - 1 ? g.dz[s < P - 1 ? s + 1 : s] : dz_next;
@@ -660,7 +728,12 @@ __device__ __forceinline__ void ray_points(const NlteBufs &B, int64_t col, int t
 // instructions and the waits of the two wavefronts per SIMD that the registers
 // allow: 9.9 ms with the member data in registers and a ray's profiles loaded
 // as it begins.  P = 3 at 32 lanes per direction covers 82 depths with 85% of
-// the lanes.
+// the lanes.  Deeper columns take more lanes, not more points: above 256 depths
+// two wavefronts per direction with three or four points (up to 10 registers
+// spilled), where one with eight spilled 167 to 813 and fell behind a lane per
+// column.  Solves of three Ca II iterations, a lane per column / one wavefront /
+// these: 2000 columns of 256 depths 501 / 310 / 310 ms, 1500 of 384
+// 620 / 673 / 283, 1200 of 512 804 / 587 / 428.
 template <int L, int P, int MS>
 __global__ void __launch_bounds__(2 * L, (P <= 3 && MS <= 2 ? 2 : 1))
 k_nlte_bezier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap, NlteBufs B,
@@ -690,11 +763,13 @@ k_nlte_bezier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap, N
   const double B2_0 = planck_lam(Tc[N - 2], lam), B2_1 = planck_lam(Tc[N - 1], lam);
   int k[P];
   RayPath<P> g;
-  ray_points<P>(B, col, t0, N, outward, k, g);
+  __shared__ double edge[L > 64 ? 2 * RAY_EDGE : 1];
+  const RayLanes<L> lanes{L > 64 && outward ? edge + RAY_EDGE : edge, L > 64 && (threadIdx.x & 64)};
+  ray_points<L, P>(lanes, B, col, t0, N, outward, k, g);
   // member data of the lane's points: in LDS, column threadIdx.x of each row,
   // where it fits (the registers then hold the next ray's profiles)
-  constexpr bool STASH = nlte_stash(P, MS);
-  double *stash = turn + B.Nmax + threadIdx.x;
+  constexpr bool STASH = nlte_stash(L, P, MS);
+  double *stash = turn + L * P + threadIdx.x;
   SetDepth<MS> sd_r[STASH ? 1 : P];
   auto put_depth = [&](int s, const SetDepth<MS> &d) {
     if constexpr (STASH) {
@@ -771,7 +846,7 @@ k_nlte_bezier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap, N
       S[s] = (eta + s0[s]) * iC[s];
     }
     if (mu + 1 < nrays) fetch(mu + 1);
-    ray_sweep<L, P>(g, t0, N, outward, zmu, B2_0, B2_1, C, S, I, Psi);
+    ray_sweep<L, P>(lanes, g, t0, N, outward, zmu, B2_0, B2_1, C, S, I, Psi);
 #pragma unroll
     for (int s = 0; s < P; s++) {
       js[s] += wmu * I[s];
@@ -798,9 +873,14 @@ k_nlte_bezier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap, N
       dJmax = dJmax > dJ ? dJmax : dJ;
     }
   }
-  for (int o = L / 2; o >= 1; o >>= 1) {
+  for (int o = L < 64 ? L / 2 : 32; o >= 1; o >>= 1) {
     const double x = __shfl_xor(dJmax, o);
     dJmax = dJmax > x ? dJmax : x;
+  }
+  if constexpr (L > 64) {
+    if (threadIdx.x == 64) edge[0] = dJmax;
+    __syncthreads();
+    if (threadIdx.x == 0) dJmax = dJmax > edge[0] ? dJmax : edge[0];
   }
   if (threadIdx.x == 0) B.dJ[(int64_t) ic * nlist_all + il_off + il] = dJmax;
   if (!eval_op) return;
@@ -824,13 +904,21 @@ k_nlte_bezier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap, N
   template __global__ void k_nlte_bezier<L, P, MS>(const DevModel *, const DevNlte *, NlteBufs,  \
                                                    const int32_t *, int, const int32_t *,        \
                                                    const int32_t *, int, int, int, int);
-#define RHG_INST_BEZ_MS(L, P) RHG_INST_BEZ(L, P, 2) RHG_INST_BEZ(L, P, 4) RHG_INST_BEZ(L, P, 8)
+#define RHG_INST_BEZ_MS(L, P) RHG_INST_BEZ(L, P, 2) RHG_INST_BEZ(L, P, 4)
+RHG_INST_BEZ_MS(32, 1)
 RHG_INST_BEZ_MS(32, 2)
 RHG_INST_BEZ_MS(32, 3)
 RHG_INST_BEZ_MS(64, 2)
 RHG_INST_BEZ_MS(64, 3)
 RHG_INST_BEZ_MS(64, 4)
-RHG_INST_BEZ_MS(64, 8)
+RHG_INST_BEZ_MS(128, 3)
+RHG_INST_BEZ_MS(128, 4)
+RHG_INST_BEZ(32, 1, 8)
+RHG_INST_BEZ(32, 2, 8)
+RHG_INST_BEZ(64, 2, 8)
+RHG_INST_BEZ(128, 2, 8)
+RHG_INST_BEZ(128, 3, 8)
+RHG_INST_BEZ(128, 4, 8)
 #undef RHG_INST_BEZ_MS
 #undef RHG_INST_BEZ
 
@@ -889,7 +977,8 @@ k_nlte_emergent(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap,
   const double B2_0 = planck_lam(Tc[N - 2], lam), B2_1 = planck_lam(Tc[N - 1], lam);
   int k[P];
   RayPath<P> g;
-  ray_points<P>(B, col, t0, N, true, k, g);
+  const RayLanes<L> lanes{nullptr, false};
+  ray_points<L, P>(lanes, B, col, t0, N, true, k, g);
   double C[P], S[P], I[P], Psi[P];
 #pragma unroll
   for (int s = 0; s < P; s++) {
@@ -898,7 +987,7 @@ k_nlte_emergent(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap,
     C[s] = chi + B.cchi[wo + k[s]];
     S[s] = fma(B.csca[wo + k[s]], Jl[k[s]], eta + B.ceta[wo + k[s]]) / C[s];
   }
-  ray_sweep<L, P>(g, t0, N, true, 1.0 / mu, B2_0, B2_1, C, S, I, Psi);
+  ray_sweep<L, P>(lanes, g, t0, N, true, 1.0 / mu, B2_0, B2_1, C, S, I, Psi);
 #pragma unroll
   for (int s = 0; s < P; s++) {
     if (threadIdx.x < L && t0 + s == N - 1) {
@@ -914,11 +1003,13 @@ k_nlte_emergent(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap,
   template __global__ void k_nlte_emergent<L, P>(const DevModel *, const DevNlte *, NlteBufs,   \
                                                  const int32_t *, const int32_t *, int, double, \
                                                  double *);
+RHG_INST_EM(32, 1)
 RHG_INST_EM(32, 2)
 RHG_INST_EM(32, 3)
 RHG_INST_EM(64, 2)
 RHG_INST_EM(64, 3)
 RHG_INST_EM(64, 4)
+RHG_INST_EM(64, 6)
 RHG_INST_EM(64, 8)
 #undef RHG_INST_EM
 

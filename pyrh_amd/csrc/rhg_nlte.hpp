@@ -24,11 +24,11 @@ constexpr int stateq_waves(int nlp) { return nlp <= 6 ? 8 : 4; }
 constexpr int stateq_depths(int nlp) { return nlp <= 8 ? 64 : 16; }   // of a workgroup: at most 32 KB of LDS
 // depth-fastest copies of column-state fields (rows of NlteBufs::geo)
 enum { NG_T = 0, NG_VLOS, NG_DZ, NG_HEIGHT, NG_N };
-// k_nlte_bezier: whether the member data of a thread's P points lies in LDS,
-// and a workgroup's LDS in doubles
-constexpr bool nlte_stash(int P, int MS) { return MS <= 2 && P <= 4; }
-constexpr int nlte_bez_lds(int L, int P, int MS, int Nmax) {
-  return Nmax + (nlte_stash(P, MS) ? P * MS * 4 * 2 * L : 0);
+// k_nlte_bezier: whether the member data of a thread's P points lies in LDS
+// (48 KB at most), and a workgroup's LDS in doubles
+constexpr bool nlte_stash(int L, int P, int MS) { return MS <= 2 && L * P <= 384; }
+constexpr int nlte_bez_lds(int L, int P, int MS) {
+  return L * P + (nlte_stash(L, P, MS) ? P * MS * 4 * 2 * L : 0);
 }
 // rows of depths are padded to whole 64-byte lines
 constexpr int nlte_pitch(int Nmax) { return (Nmax + 7) & ~7; }

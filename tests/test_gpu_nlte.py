@@ -193,10 +193,11 @@ def test_nlte_barklem_matches_reference(eng_mg, nm_mg, mg_fix, name):
     np.testing.assert_allclose(dpops, mg_fix[name + "__dpops"], rtol=0, atol=2 * TOL_MG_POPS)
 
 
-@pytest.mark.parametrize("nd", [4, 33, 64, 65, 96, 97, 128, 129, 192, 193, 256, 257, 512])
+@pytest.mark.parametrize("nd", [4, 32, 33, 64, 65, 96, 97, 128, 129, 192, 193, 256, 257, 384, 385,
+                                512])
 def test_nlte_depth_counts(eng, nm, nd):
     """Depth counts at the edges of what the lanes of a ray hold (a lane's
-    points, half a wavefront, a wavefront, both with more points per lane),
+    points, half a wavefront, a wavefront, two, with more points per lane),
     the batch's other column shallower, against the oracle over a few
     iterations: the sweep's scan and the sums over rays and wavelengths change
     order only, so the differences stay those of the tests above."""
@@ -218,3 +219,52 @@ def test_nlte_depth_counts(eng, nm, nd):
         assert _relerr(pops[c, :, :n], cp[c, :, :n]) < TOL_POPS
     assert _relerr(st[:, 0], cs[:, 0]) < TOL_I
     np.testing.assert_array_equal(niter, cn)
+
+
+@pytest.fixture(scope="module")
+def wide(tmp_path_factory):
+    """Na I with all 16 levels active: wavelengths with up to eight active
+    transitions, with a line and without (the reference wavelength where none
+    is).  The model atom lists no collisions; neighbouring levels get a
+    collision strength of 1."""
+    import shutil
+    from pyrh_amd import model, nlte, workloads
+    from pyrh_amd.engine import Engine
+    run = tmp_path_factory.mktemp("na") / "run"
+    shutil.copytree(GOLDEN / "run_nlte_mg", run)
+    atoms = [ln.replace("PASSIVE", "ACTIVE ") if "Na.atom" in ln else
+             ln.replace("ACTIVE ", "PASSIVE") if "MgI_6level" in ln else ln
+             for ln in (run / "atoms.input").read_text().splitlines()]
+    (run / "atoms.input").write_text("\n".join(atoms) + "\n")
+    kw = (run / "keyword.input").read_text()
+    (run / "keyword.input").write_text(kw.rstrip() + "\n  LAMBDA_REF = 2000.0\n")
+    nm = nlte.build_nlte(model.open_run(str(run)), workloads.wavelengths_630())
+    n, bez = np.diff(nm.as_ptr), np.asarray(nm.as_bezier) > 0
+    assert nm.nlevel == 16 and n[bez].max() == 8 and n[~bez].max() == 8
+    i32 = np.int32
+    nm.coll_type, nm.coll_i, nm.coll_j = np.zeros(15, i32), np.arange(15, dtype=i32), np.arange(1, 16, dtype=i32)
+    nm.coll_ptr = np.arange(0, 32, 2, dtype=i32)
+    nm.coll_T, nm.coll_c, nm.coll_M = np.tile([1e3, 1e5], 15), np.ones(30), np.zeros(30)
+    e = Engine(nm.lte)
+    yield e, nm
+    e.close()
+
+
+@pytest.mark.parametrize("nd", [32, 64, 65, 128, 129, 256, 257, 384, 385])
+def test_nlte_wide_sets(wide, nd):
+    """The forms for up to eight active transitions, at the edges of their
+    lanes, against the oracle after one iteration (a minority stage as Mg I:
+    the same tolerance)."""
+    import copy
+
+    import pyoracle
+    from pyrh_amd import workloads
+    e, nm = wide
+    m = copy.copy(nm)
+    m.nmax_iter, m.nmax_scatter = 1, 0
+    atm, ndep = workloads.mixed_batch(2, seed=workloads.SEED_BASE + 90 + nd, ndep_choices=(nd,))
+    pops = e.nlte_solve(m, atm, ndep=ndep)[0]
+    ref = pyoracle.nlte_solve(m, atm, ndep=ndep)[0]
+    err = _relerr(pops, ref)
+    print(f"Na I, {nd} depths: max rel err {err:.2e}", flush=True)
+    assert err < TOL_MG_ONE_ITER

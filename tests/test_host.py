@@ -323,3 +323,10 @@ def test_component_sums_stay_in_registers():
     # 24: the spill count leaves out a few bytes of the slots it takes
     assert len(sums) == 10 and all(own(k) <= 24 for k in sums)
     assert all(k[".group_segment_fixed_size"] == 0 for k in sums)
+
+
+def test_deep_nlte_rays_stay_in_registers():
+    """Every depth count's k_nlte_bezier up to four active transitions keeps
+    a column's points in registers (a few spills at most)."""
+    ks = [k for n, k in _kernels().items() if re.search(r"k_nlte_bezierILi\d+ELi\dELi[24]E", n)]
+    assert len(ks) == 16 and all(k[".vgpr_spill_count"] <= 16 for k in ks)
