@@ -2000,8 +2000,8 @@ struct NlteTimer {
 }  // namespace
 
 // run LAUNCH(L, P) with the lanes per ray direction L and the points per lane
-// P for columns of up to Nd depths (L P >= Nd): two or three points per lane hide
-// the latency of a point's arithmetic, more spill
+// P for columns of up to Nd depths, a value of kRayDepths (L P >= Nd): two or
+// three points per lane hide the latency of a point's arithmetic, more spill
 #define RHG_RAY_POINTS(Nd, LAUNCH)        \
   do {                                    \
     if ((Nd) <= 32) LAUNCH(32, 1);        \
@@ -2026,7 +2026,67 @@ struct NlteTimer {
     else if ((Nd) <= 384) LAUNCH(128, 3); \
     else LAUNCH(128, 4);                  \
   } while (0)
-static_assert(128 * 4 >= RHG_MAX_DEPTH, "RHG_RAY_POINTS covers every depth count");
+static constexpr int kRayDepths[] = {32, 64, 96, 128, 192, 256, 384, 512};
+static constexpr int kRayClasses = sizeof(kRayDepths) / sizeof(int);
+static_assert(kRayDepths[kRayClasses - 1] >= RHG_MAX_DEPTH, "kRayDepths covers every depth count");
+// depths (columns times the difference of two classes) below which a launch of
+// its own costs more than it saves, about 0.1 ms a pass: six Ca II iterations
+// over 2 columns each of 64, 128 and 256 depths 3.8 ms together, 4.1 apart; 20
+// of 82 and 300 of 128 32.6 and 33.0; 8 of 64 and 8 of 256 5.8 and 4.8; 30 of
+// 82 and 300 of 256 81.9 and 77.8
+static constexpr int64_t kRayClassMin = 1024;
+
+namespace {
+
+// The columns of a batch by depth class, so that a column's rays take the
+// lanes of its own depth count and not of the batch's deepest column.
+struct RayClasses {
+  std::vector<int32_t> order;          // columns by class, in the batch's order within one
+  std::vector<int8_t> of;              // class of a column
+  int deepest[kRayClasses]{};          // depths of a class's deepest column
+
+  // A class joins the next deeper one where that adds less than kRayClassMin
+  // depths.
+  RayClasses(const int32_t *ndep, int ncol) : order(ncol), of(ncol) {
+    int count[kRayClasses]{}, to[kRayClasses], start[kRayClasses + 1]{};
+    for (int i = 0; i < ncol; i++) {
+      int q = 0;
+      while (kRayDepths[q] < ndep[i]) q++;
+      of[i] = (int8_t) q;
+      count[q]++;
+      deepest[q] = std::max(deepest[q], (int) ndep[i]);
+    }
+    for (int q = 0; q < kRayClasses; q++) to[q] = q;
+    for (int q = 0; q < kRayClasses; q++) {
+      if (!count[q]) continue;
+      int d = q + 1;
+      while (d < kRayClasses && !count[d]) d++;
+      if (d == kRayClasses) break;
+      if (count[q] * (int64_t) (kRayDepths[d] - kRayDepths[q]) >= kRayClassMin) continue;
+      for (int &t : to)
+        if (t == q) t = d;
+      count[d] += count[q];
+      count[q] = 0;
+    }
+    for (int q = 0; q < kRayClasses; q++) start[q + 1] = start[q] + count[q];
+    for (int i = 0; i < ncol; i++) {
+      of[i] = (int8_t) to[of[i]];
+      order[start[of[i]]++] = i;
+    }
+  }
+  // f(class, offset, columns) for the runs of one class in a list of columns,
+  // at most `most` columns at a time
+  template <typename F>
+  void runs(const std::vector<int32_t> &list, int most, F &&f) const {
+    const int n = (int) list.size();
+    for (int i = 0, j; i < n; i = j) {
+      for (j = i + 1; j < n && j - i < most && of[list[j]] == of[list[i]]; j++) {}
+      f((int) of[list[i]], i, j - i);
+    }
+  }
+};
+
+}  // namespace
 
 extern "C" {
 
@@ -2208,9 +2268,9 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
     });
     if (rc) return rc;
 
-    std::vector<int32_t> act(ncol), keep;
+    const RayClasses classes(hndep.data() + c0, ncol);
+    std::vector<int32_t> act = classes.order, keep;
     std::vector<double> red(ncol);
-    for (int i = 0; i < ncol; i++) act[i] = i;
     auto upload_act = [&]() -> int {
       HIPCHECK(hipMemcpyAsync(d_act, act.data(), act.size() * sizeof(int32_t), hipMemcpyHostToDevice,
                               c->stream));
@@ -2220,29 +2280,31 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
     // as 36 KB of LDS hold (four workgroups per CU: 1500 columns of 82 depths
     // 0.90 ms a pass; 9 KB 1.66, 24 KB 1.14, 52 KB 1.08), fewer while they
     // would leave SIMDs idle
-    auto fe_per = [&](int nact, int rays) {
+    const int nfe = nlist - h.nbez;
+    auto fe_per = [&](int nact, int rays, int Nd) {
       int per = 12;
-      while (per > 1 && rhg::nlte_fe_lds(Nmax, per, rays) * sizeof(double) > 36864) per--;
-      while (per > 1 && (int64_t) nact * (nlist - h.nbez) / per < 1024) per--;
+      while (per > 1 && rhg::nlte_fe_lds(Nd, per, rays) * sizeof(double) > 36864) per--;
+      while (per > 1 && (int64_t) nact * nfe / per < 1024) per--;
       return per;
     };
+    const int most = ncol;
     auto rt = [&](int slot, int eval) -> int {
       const int nact = (int) act.size();
-      const int nfe = nlist - h.nbez;
       int r = timed(slot, [&]() -> int {
         if (h.nbez > 0) {
-          const dim3 grd((unsigned) rhg::xcd_grid(nact, h.nbez));
 #define RHG_LAUNCH_BEZ(L, P, MS)                                                                 \
   hipLaunchKernelGGL((rhg::k_nlte_bezier<L, P, MS>), grd, dim3(2 * L),                            \
-                     rhg::nlte_bez_lds(L, P, MS) * sizeof(double), c->stream, c->d_model,   \
-                     d_at, B, d_act, nact,                                                       \
-                     c->d_out_ls, d_iolist, h.nbez, 0, nlist, eval)
+                     rhg::nlte_bez_lds(L, P, MS) * sizeof(double), c->stream, c->d_model, d_at, B, \
+                     d_act + off, n, c->d_out_ls, d_iolist, h.nbez, 0, nlist, eval)
 #define RHG_LAUNCH_BEZ_2(L, P) RHG_LAUNCH_BEZ(L, P, 2)
 #define RHG_LAUNCH_BEZ_4(L, P) RHG_LAUNCH_BEZ(L, P, 4)
 #define RHG_LAUNCH_BEZ_8(L, P) RHG_LAUNCH_BEZ(L, P, 8)
-          if (h.maxset_bez <= 2) RHG_RAY_POINTS(Nmax, RHG_LAUNCH_BEZ_2);
-          else if (h.maxset_bez <= 4) RHG_RAY_POINTS(Nmax, RHG_LAUNCH_BEZ_4);
-          else RHG_RAY_POINTS_WIDE(Nmax, RHG_LAUNCH_BEZ_8);
+          classes.runs(act, most, [&](int q, int off, int n) {
+            const dim3 grd((unsigned) rhg::xcd_grid(n, h.nbez));
+            if (h.maxset_bez <= 2) RHG_RAY_POINTS(kRayDepths[q], RHG_LAUNCH_BEZ_2);
+            else if (h.maxset_bez <= 4) RHG_RAY_POINTS(kRayDepths[q], RHG_LAUNCH_BEZ_4);
+            else RHG_RAY_POINTS_WIDE(kRayDepths[q], RHG_LAUNCH_BEZ_8);
+          });
 #undef RHG_LAUNCH_BEZ_2
 #undef RHG_LAUNCH_BEZ_4
 #undef RHG_LAUNCH_BEZ_8
@@ -2257,19 +2319,22 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
       if (r) return r;
       r = timed(8 + (slot == 2), [&]() -> int {
         if (nfe > 0) {
-          // the member loops unrolled to the largest active set (one launch:
-          // split by set size, the launches would not fill the GPU)
-          const int per = fe_per(nact, rhg::NLTE_FE_RAYS);
-          const dim3 grd((unsigned) rhg::xcd_grid((nact + per - 1) / per, nfe));
-          const size_t lds = rhg::nlte_fe_lds(Nmax, per, rhg::NLTE_FE_RAYS) * sizeof(double);
+          // the member loops unrolled to the largest active set (one launch
+          // per depth class: split by set size, the launches would not fill
+          // the GPU)
 #define RHG_LAUNCH_FE(MS)                                                                        \
   hipLaunchKernelGGL((rhg::k_nlte_feautrier<MS, false>), grd, b64, lds, c->stream, c->d_model, d_at, \
-                     B, d_act, nact, per, c->d_out_ls, d_iolist + h.nbez, nfe, h.nbez, nlist, eval, \
-                     0.0, (double *) nullptr)
-          if (h.maxset_fe <= 2) RHG_LAUNCH_FE(2);
-          else if (h.maxset_fe <= 4) RHG_LAUNCH_FE(4);
-          else if (h.maxset_fe <= 6) RHG_LAUNCH_FE(6);
-          else RHG_LAUNCH_FE(8);
+                     B, d_act + off, n, per, Nd, c->d_out_ls, d_iolist + h.nbez, nfe, h.nbez, nlist, \
+                     eval, 0.0, (double *) nullptr)
+          classes.runs(act, most, [&](int q, int off, int n) {
+            const int Nd = classes.deepest[q], per = fe_per(n, rhg::NLTE_FE_RAYS, Nd);
+            const dim3 grd((unsigned) rhg::xcd_grid((n + per - 1) / per, nfe));
+            const size_t lds = rhg::nlte_fe_lds(Nd, per, rhg::NLTE_FE_RAYS) * sizeof(double);
+            if (h.maxset_fe <= 2) RHG_LAUNCH_FE(2);
+            else if (h.maxset_fe <= 4) RHG_LAUNCH_FE(4);
+            else if (h.maxset_fe <= 6) RHG_LAUNCH_FE(6);
+            else RHG_LAUNCH_FE(8);
+          });
 #undef RHG_LAUNCH_FE
           HIPCHECK(hipGetLastError());
         }
@@ -2309,8 +2374,7 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
     // accelerated lambda iterations
     std::vector<int32_t> niter(ncol, 0);
     std::vector<double> dpops(ncol, 0.0);
-    act.resize(ncol);
-    for (int i = 0; i < ncol; i++) act[i] = i;
+    act = classes.order;
     if ((rc = upload_act())) return rc;
     HIPCHECK(hipMemcpyAsync(B.hist, B.pops, row * nl, hipMemcpyDeviceToDevice, c->stream));
     const int ndelay = std::max(a->ng_delay, a->ng_order + 2);
@@ -2355,8 +2419,7 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
     // N_MAX_SCATTER passes, each column stopping at max dJ <= ITER_LIMIT,
     // rh/rhf1d/pyrh_compute1dray.c:332-337), then the final ray
     if (stokes_out) {
-      act.resize(ncol);
-      for (int i = 0; i < ncol; i++) act[i] = i;
+      act = classes.order;
       if ((rc = upload_act())) return rc;
       for (int it = 0; it < a->nmax_scatter && !act.empty(); it++) {
         if ((rc = rt(1, 0))) return rc;
@@ -2372,25 +2435,30 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
         if (!act.empty() && (rc = upload_act())) return rc;
       }
       double *d_st = device_ptrs ? stokes_out + (size_t) c0 * 4 * nout : (double *) c->nl_st.p;
-      const int nfe = nlist - h.nbez;
+      act = classes.order;
+      if ((rc = upload_act())) return rc;
       if (h.nbez > 0) {
-        const dim3 grd((unsigned) rhg::xcd_grid(ncol, h.nbez));
         // (one ray: a direction's lanes in one wavefront)
 #define RHG_LAUNCH_EM(L, P)                                                                      \
   hipLaunchKernelGGL((rhg::k_nlte_emergent<std::min(L, 64), (P * L / std::min(L, 64))>), grd,     \
-                     b64, 0, c->stream, c->d_model, d_at, B, c->d_out_ls, d_iolist, h.nbez,      \
-                     cols->mu, d_st)
-        RHG_RAY_POINTS(Nmax, RHG_LAUNCH_EM);
+                     b64, 0, c->stream, c->d_model, d_at, B, d_act + off, n, c->d_out_ls, d_iolist,    \
+                     h.nbez, cols->mu, d_st)
+        classes.runs(act, most, [&](int q, int off, int n) {
+          const dim3 grd((unsigned) rhg::xcd_grid(n, h.nbez));
+          RHG_RAY_POINTS(kRayDepths[q], RHG_LAUNCH_EM);
+        });
 #undef RHG_LAUNCH_EM
         HIPCHECK(hipGetLastError());
       }
       if (nfe > 0) {
-        const int per = fe_per(ncol, 1);
-        const dim3 grd((unsigned) rhg::xcd_grid((ncol + per - 1) / per, nfe));
-        hipLaunchKernelGGL((rhg::k_nlte_feautrier<2, true>), grd, b64,
-                           rhg::nlte_fe_lds(Nmax, per, 1) * sizeof(double), c->stream, c->d_model,
-                           d_at, B, (const int32_t *) nullptr, ncol, per, c->d_out_ls,
-                           d_iolist + h.nbez, nfe, h.nbez, nlist, 0, cols->mu, d_st);
+        classes.runs(act, most, [&](int q, int off, int n) {
+          const int Nd = classes.deepest[q], per = fe_per(n, 1, Nd);
+          const dim3 grd((unsigned) rhg::xcd_grid((n + per - 1) / per, nfe));
+          hipLaunchKernelGGL((rhg::k_nlte_feautrier<2, true>), grd, b64,
+                             rhg::nlte_fe_lds(Nd, per, 1) * sizeof(double), c->stream, c->d_model,
+                             d_at, B, d_act + off, n, per, Nd, c->d_out_ls, d_iolist + h.nbez, nfe,
+                             h.nbez, nlist, 0, cols->mu, d_st);
+        });
         HIPCHECK(hipGetLastError());
       }
       if (!device_ptrs)

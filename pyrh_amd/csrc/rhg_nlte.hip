@@ -959,13 +959,15 @@ __device__ __forceinline__ void emergent_set(const NlteBufs &B, const DevNlte &A
 template <int L, int P>
 __global__ void __launch_bounds__(64)
 k_nlte_emergent(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap, NlteBufs B,
-                const int32_t *__restrict__ out_ls, const int32_t *__restrict__ io_list, int nlist,
-                double mu, double *__restrict__ stokes) {
+                const int32_t *__restrict__ act, int nact, const int32_t *__restrict__ out_ls,
+                const int32_t *__restrict__ io_list, int nlist, double mu,
+                double *__restrict__ stokes) {
   const DevModel &M = *Mp;
   const DevNlte &A = *Ap;
-  int ic, il;
-  xcd_tile(blockIdx.x, B.ncol, nlist, ic, il);
-  if (ic >= B.ncol) return;
+  int slot, il;
+  xcd_tile(blockIdx.x, nact, nlist, slot, il);
+  if (slot >= nact) return;
+  const int ic = act[slot];
   const int io = io_list[il], ls = out_ls[io], N = B.ndep[ic];
   const int64_t fs = B.fs, col = (int64_t) ic * B.Kp, wo = (int64_t) io * fs + col;
   const double *Jl = B.J + B.jpar[ic] * (int64_t) B.nout * fs + wo;
@@ -1001,8 +1003,8 @@ k_nlte_emergent(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap,
 }
 #define RHG_INST_EM(L, P)                                                                       \
   template __global__ void k_nlte_emergent<L, P>(const DevModel *, const DevNlte *, NlteBufs,   \
-                                                 const int32_t *, const int32_t *, int, double, \
-                                                 double *);
+                                                 const int32_t *, int, const int32_t *,         \
+                                                 const int32_t *, int, double, double *);
 RHG_INST_EM(32, 1)
 RHG_INST_EM(32, 2)
 RHG_INST_EM(32, 3)
@@ -1034,7 +1036,7 @@ RHG_INST_EM(64, 8)
 template <int MS, bool EM>
 __global__ void __launch_bounds__(64)
 k_nlte_feautrier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap, NlteBufs B,
-                 const int32_t *__restrict__ act, int nact, int per,
+                 const int32_t *__restrict__ act, int nact, int per, int Nd,
                  const int32_t *__restrict__ out_ls, const int32_t *__restrict__ io_list, int nlist,
                  int il_off, int nlist_all, int eval_op, double mu_em, double *__restrict__ stokes) {
 #pragma clang fp contract(fast)
@@ -1050,12 +1052,12 @@ k_nlte_feautrier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap
   const double lam = ldc(M.lamconst)[(int64_t) ls * RHG_LC_NCONST + RHG_LC_LAMBDA];
   SetInfo<MS> si;
   set_info<MS>(A, ls, lam, si);
-  const int lane = threadIdx.x, Nmax = B.Nmax;
+  const int lane = threadIdx.x;
   constexpr int RF = EM ? 1 : NLTE_FE_RAYS;
-  const int FS = per * RF;   // F and z: [Nmax][per * RF]
-  double *Xs = lds, *Ss = Xs + per * Nmax, *Cs = Ss + per * Nmax, *Fs = Cs + per * Nmax,
-         *Zs = Fs + Nmax * FS;
-  auto column = [&](int it) { return EM ? first + it : act[first + it]; };
+  const int FS = per * RF;   // F and z: [Nd][per * RF]
+  double *Xs = lds, *Ss = Xs + per * Nd, *Cs = Ss + per * Nd, *Fs = Cs + per * Nd,
+         *Zs = Fs + Nd * FS;
+  auto column = [&](int it) { return act[first + it]; };
 
   for (int it = 0; it < n_it; it++) {
     const int ic = column(it), N = B.ndep[ic];
@@ -1084,13 +1086,13 @@ k_nlte_feautrier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap
         }
       }
       const double C = chi + B.cchi[wo + k];
-      Cs[it * Nmax + k] = C;
-      Ss[it * Nmax + k] = fma(B.csca[wo + k], Jo[k], eta + B.ceta[wo + k]) / C;
+      Cs[it * Nd + k] = C;
+      Ss[it * Nd + k] = fma(B.csca[wo + k], Jo[k], eta + B.ceta[wo + k]) / C;
     }
     wave_sync();
     const double *z = B.geo + NG_HEIGHT * fs + col;
     for (int k = lane; k < N - 1; k += 64)
-      Xs[it * Nmax + k] = (Cs[it * Nmax + k] + Cs[it * Nmax + k + 1]) * (z[k] - z[k + 1]);
+      Xs[it * Nd + k] = (Cs[it * Nd + k] + Cs[it * Nd + k + 1]) * (z[k] - z[k + 1]);
   }
   wave_sync();
 
@@ -1102,7 +1104,7 @@ k_nlte_feautrier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap
       const double *Tc = B.geo + NG_T * fs + (int64_t) ic * B.Kp;
       const double B2_0 = planck_lam(Tc[N - 2], lam), B2_1 = planck_lam(Tc[N - 1], lam);
       const double zmu = 0.5 / (EM ? mu_em : A.muz[c0 + r_s]);
-      const double *X = Xs + it_s * Nmax, *Sv = Ss + it_s * Nmax;
+      const double *X = Xs + it_s * Nd, *Sv = Ss + it_s * Nd;
       double *F = Fs + lane, *Z = Zs + lane;
       const double dt0 = zmu * X[0], abc0 = 1.0 + 2.0 / dt0, C1_0 = 2.0 / (dt0 * dt0);
       double Fk = abc0 / C1_0, zk = Sv[0] / (abc0 + C1_0), q = ndiv(Fk, 1.0 + Fk);
@@ -1193,7 +1195,7 @@ k_nlte_feautrier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap
             }
           }
         }
-        const double iC = 1.0 / Cs[it * Nmax + k];
+        const double iC = 1.0 / Cs[it * Nd + k];
         for (int r = 0; r < nrc; r++)
           rate_terms<MS>(si, sd, V, Z[r], F[r] * iC, A.wmu[c0 + r], aIJ, aJI);
 #pragma unroll
@@ -1218,8 +1220,9 @@ k_nlte_feautrier(const DevModel *__restrict__ Mp, const DevNlte *__restrict__ Ap
 }
 #define RHG_INST_FE(MS, EM)                                                                      \
   template __global__ void k_nlte_feautrier<MS, EM>(const DevModel *, const DevNlte *, NlteBufs, \
-                                                    const int32_t *, int, int, const int32_t *,  \
-                                                    const int32_t *, int, int, int, int, double, \
+                                                    const int32_t *, int, int, int,              \
+                                                    const int32_t *, const int32_t *, int, int,  \
+                                                    int, int, double,                            \
                                                     double *);
 RHG_INST_FE(2, false)
 RHG_INST_FE(4, false)

@@ -16,8 +16,9 @@ constexpr int NLTE_MAXLEV = 16;
 constexpr int NLTE_MAXNG = 4;                  // Ng order
 // rays of k_nlte_feautrier solved together (more rays in chunks of this many)
 constexpr int NLTE_FE_RAYS = 5;
-// LDS of a k_nlte_feautrier workgroup for `per` columns, in doubles
-constexpr int nlte_fe_lds(int Nmax, int per, int rays) { return per * Nmax * (3 + 2 * rays); }
+// LDS of a k_nlte_feautrier workgroup for `per` columns of at most Nd depths,
+// in doubles
+constexpr int nlte_fe_lds(int Nd, int per, int rays) { return per * Nd * (3 + 2 * rays); }
 // threads of k_nlte_ng; wavefronts of k_nlte_stateq for up to nlp levels
 constexpr int NG_BLOCK = 256;
 constexpr int stateq_waves(int nlp) { return nlp <= 6 ? 8 : 4; }
@@ -92,14 +93,15 @@ __global__ void k_nlte_bezier(const DevModel *Mp, const DevNlte *Ap, NlteBufs B,
                               int eval_op);
 template <int MS, bool EM>
 __global__ void k_nlte_feautrier(const DevModel *Mp, const DevNlte *Ap, NlteBufs B,
-                                 const int32_t *act, int nact, int per, const int32_t *out_ls,
-                                 const int32_t *io_list, int nlist, int il_off, int nlist_all,
-                                 int eval_op, double mu_em, double *stokes);
+                                 const int32_t *act, int nact, int per, int Nd,
+                                 const int32_t *out_ls, const int32_t *io_list, int nlist,
+                                 int il_off, int nlist_all, int eval_op, double mu_em,
+                                 double *stokes);
 __global__ void k_nlte_flip(NlteBufs B, const int32_t *act, int nact);
 template <int L, int P>
 __global__ void k_nlte_emergent(const DevModel *Mp, const DevNlte *Ap, NlteBufs B,
-                                const int32_t *out_ls, const int32_t *io_list, int nlist,
-                                double mu, double *stokes);
+                                const int32_t *act, int nact, const int32_t *out_ls,
+                                const int32_t *io_list, int nlist, double mu, double *stokes);
 __global__ void k_nlte_djmax(NlteBufs B, const int32_t *act, int nact, int nlist,
                              double *djmax);
 template <int NLP>

@@ -268,3 +268,69 @@ def test_nlte_wide_sets(wide, nd):
     err = _relerr(pops, ref)
     print(f"Na I, {nd} depths: max rel err {err:.2e}", flush=True)
     assert err < TOL_MG_ONE_ITER
+
+
+def _depth_mix(spec, seed):
+    """Map-like columns of the depth counts {depths: columns}, shuffled."""
+    from pyrh_amd import workloads
+    atm, nd = np.zeros((sum(spec.values()), 9, max(spec))), []
+    for n, c in spec.items():
+        a, d = workloads.mixed_batch(c, seed=workloads.SEED_BASE + seed + n, ndep_choices=(n,))
+        atm[len(nd):len(nd) + c, :, :n] = a
+        nd += d.tolist()
+    perm = np.random.default_rng(seed).permutation(len(nd))
+    return np.ascontiguousarray(atm[perm]), np.array(nd, np.int32)[perm]
+
+
+def test_nlte_ragged_batch_by_depth(eng, nm):
+    """Columns of a ragged batch are solved by depth class: with every class
+    large enough for a launch of its own, each column's populations and
+    spectrum are, bit for bit, those of a batch of its own depth count."""
+    import copy
+    few = copy.copy(nm)
+    few.nmax_iter = 3
+    atm, nd = _depth_mix({30: 41, 82: 37, 130: 21, 300: 9}, 400)
+    pops, niter, _, st = eng.nlte_solve(few, atm, ndep=nd, stokes=True)
+    for n in np.unique(nd):
+        c = np.flatnonzero(nd == n)
+        p, i, _, s = eng.nlte_solve(few, np.ascontiguousarray(atm[c, :, :n]), stokes=True)
+        np.testing.assert_array_equal(pops[c, :, :n], p)
+        assert not pops[c, :, n:].any()
+        np.testing.assert_array_equal(st[c], s)
+        np.testing.assert_array_equal(niter[c], i)
+
+
+def test_nlte_small_classes_join(eng, nm):
+    """A few columns of several depth counts share the lanes of the deepest:
+    against the oracle."""
+    import copy
+    import pyoracle
+    few = copy.copy(nm)
+    few.nmax_iter = 3
+    atm, nd = _depth_mix({4: 1, 30: 2, 60: 1, 90: 1, 200: 1}, 410)
+    pops, niter, _, st = eng.nlte_solve(few, atm, ndep=nd, stokes=True)
+    cp, cn, _, cs = pyoracle.nlte_solve(few, atm, ndep=nd, stokes=True)
+    for c, n in enumerate(nd):
+        assert _relerr(pops[c, :, :n], cp[c, :, :n]) < TOL_POPS
+    assert _relerr(st[:, 0], cs[:, 0]) < TOL_I
+    np.testing.assert_array_equal(niter, cn)
+
+
+def test_nlte_few_deep_columns_cost_their_own(eng, nm):
+    """Four columns of 512 depths among 600 of 82: about what the two batches
+    take apart (six times that, when every column took the lanes of the
+    deepest)."""
+    import copy
+    few = copy.copy(nm)
+    few.nmax_iter = 3
+
+    def ms(spec):
+        atm, nd = _depth_mix(spec, 420)
+        out = []
+        for _ in range(3):
+            eng.nlte_solve(few, atm, ndep=nd)
+            out.append(eng.nlte_timings()["total_ms"])
+        return min(out)
+    apart, both = ms({82: 600}) + ms({512: 4}), ms({82: 600, 512: 4})
+    print(f"apart {apart:.1f} ms, together {both:.1f} ms", flush=True)
+    assert both < 2.5 * apart
