@@ -2129,7 +2129,11 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
   size_t freeb = 0, totb = 0;
   HIPCHECK(hipMemGetInfo(&freeb, &totb));
   const size_t budget = freeb / 4 * 3;
-  int chunk = (int) std::min<size_t>((size_t) ncol_all, budget / per_col);
+  // (the grids of k_nlte_profile and k_nlte_bg stay below 2^32 threads)
+  const int64_t thr_col = std::max((int64_t) Nmax * h.nphi,
+                                   (int64_t) 8 * ((Nmax + 31) / 32) * (nout + rhg::NG_N));
+  int chunk = (int) std::min<size_t>({(size_t) ncol_all, budget / per_col,
+                                      (size_t) std::max<int64_t>(1, 0xffffffffll / thr_col - 64)});
   // whole blocks of 64 columns where the batch is split; a batch that fits is
   // one chunk whatever its size (1500 columns of the Ca II atom as 1472 + 28
   // ran a second solve for the 28: 694 ms, in one chunk 521 ms)
@@ -2287,7 +2291,9 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
       while (per > 1 && (int64_t) nact * nfe / per < 1024) per--;
       return per;
     };
-    const int most = ncol;
+    // columns of a launch: with up to 256 threads per (column, wavelength) a
+    // grid stays below 2^32 threads
+    const int most = std::max(64, (int) std::min<int64_t>(ncol, 0xffffffffll / (256ll * nlist) / 64 * 64));
     auto rt = [&](int slot, int eval) -> int {
       const int nact = (int) act.size();
       int r = timed(slot, [&]() -> int {

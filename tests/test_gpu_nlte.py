@@ -334,3 +334,20 @@ def test_nlte_few_deep_columns_cost_their_own(eng, nm):
     apart, both = ms({82: 600}) + ms({512: 4}), ms({82: 600, 512: 4})
     print(f"apart {apart:.1f} ms, together {both:.1f} ms", flush=True)
     assert both < 2.5 * apart
+
+
+def test_nlte_more_columns_than_a_launch_takes(eng, nm):
+    """A grid holds less than 2^32 threads, 64 per (column, wavelength) for
+    shallow columns: 140000 columns of four depths take several launches.  A
+    column's result does not depend on its launch."""
+    import copy
+    from pyrh_amd import workloads
+    one = copy.copy(nm)
+    one.nmax_iter, one.nmax_scatter = 1, 0
+    n = 140000
+    nbez = int(np.count_nonzero((np.diff(nm.as_ptr) > 0) & (np.asarray(nm.as_bezier) > 0)))
+    assert n * nbez * 64 > 2 ** 32
+    atm, _ = workloads.mixed_batch(50, seed=workloads.SEED_BASE + 430, ndep_choices=(4,))
+    small = eng.nlte_solve(one, atm)[0]
+    big = eng.nlte_solve(one, np.tile(atm, (n // 50, 1, 1)))[0]
+    np.testing.assert_array_equal(big.reshape(n // 50, *small.shape), np.broadcast_to(small, (n // 50, *small.shape)))
