@@ -547,7 +547,12 @@ static size_t split_points(const rhg_context *c, int32_t precision, int ncol, in
   const int64_t rays = (int64_t) ((ncol + 63) / 64) * c->n_pol;
   const size_t bytes = (size_t) c->n_pol * Nmax * ncol *
                        rhg::point_ncomp(c->dm.magneto_optical != 0) * sizeof(double);
-  return rays <= kSplitRays && bytes <= kSplitBytes ? bytes : 0;
+  size_t most = kSplitBytes;
+  // PYRH_AMD_POINT_BYTES caps the memory of the points, which the context keeps
+  // (0: always one pass)
+  if (const char *cap = getenv("PYRH_AMD_POINT_BYTES"))
+    most = (size_t) std::min<unsigned long long>(most, strtoull(cap, nullptr, 10));
+  return rays <= kSplitRays && bytes <= most ? bytes : 0;
 }
 
 // The wavelength grids of a synthesis launch: the batch's block -> grid
@@ -2710,9 +2715,14 @@ int rhg_hse(rhg_context_t *c, const rhg_hse_t *h, int32_t ncol, int32_t Nmax, co
                                       "above its ground level");
   }
   // The records of all depths are formed before the chain runs, for as many
-  // columns at a time as HSE_REC_BYTES hold (or as can be allocated).
+  // columns at a time as kHseRecBytes hold (or as can be allocated).
   const size_t rec_col = (size_t) Nmax * H.nrec * sizeof(double);
   int chunk = (int) std::min<size_t>(ncol, std::max<size_t>(kHseRecBytes / rec_col, 1));
+  // PYRH_AMD_HSE_CHUNK caps the chunk (a caller that needs the memory; tests)
+  if (const char *cap = getenv("PYRH_AMD_HSE_CHUNK")) {
+    const long v = strtol(cap, nullptr, 10);
+    if (v > 0) chunk = (int) std::min<long>(chunk, v);
+  }
   while (c->hs_rec.ensure((size_t) chunk * rec_col)) {
     if (chunk <= 64) return fail(RHG_ENOMEM, "device allocation for the layer tables failed");
     chunk = (chunk + 1) / 2;

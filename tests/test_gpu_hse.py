@@ -94,7 +94,7 @@ def test_hse_batch_matches_oracle(fix):
     np.testing.assert_array_equal(p2[0], ne[perm])
 
 
-@pytest.mark.parametrize("lanes", [2, 4, 8, 16, 32, 64])
+@pytest.mark.parametrize("lanes", [1, 2, 4, 8, 16, 32, 64])
 @pytest.mark.parametrize("scale", [0, 2])
 def test_hse_lane_groups(fix, lanes, scale, monkeypatch):
     """Every lane-group width, on a column count that leaves the last
@@ -114,6 +114,32 @@ def test_hse_lane_groups(fix, lanes, scale, monkeypatch):
     for a, b in zip(out[:4], (ref[0], ref[1], ref[2], ref[3])):
         assert max(relerr(a[c, :nd[c]], b[c, :nd[c]]) for c in range(19)) < TOL
     np.testing.assert_array_equal(out[4], ref[4])
+
+
+@pytest.mark.parametrize("chunk", [1, 7, 20])
+def test_hse_in_chunks(fix, chunk, monkeypatch):
+    """A batch whose records are formed some columns at a time, ragged, from
+    host and from device memory: bit for bit the batch in one piece."""
+    import torch
+    from pyrh_amd import workloads as W
+    e, hm = engine(fix, "single")
+    n = 20
+    T = W.stokes_map(n, seed=W.SEED_BASE + 45)[:, 1]
+    nd = np.full(n, W.NDEP, np.int32)
+    nd[[0, 6, 7, 19]] = 1, 40, 81, 3
+    sc = np.ascontiguousarray(np.broadcast_to(W.LOGTAU, T.shape))
+    pg = np.linspace(0.08, 0.12, n)
+    monkeypatch.setenv("RHG_HSE_LANES", "16")
+    ref = e.hse(hm, sc, T, pg, 0, nd)
+    monkeypatch.setenv("PYRH_AMD_HSE_CHUNK", str(chunk))
+    for a, b in zip(e.hse(hm, sc, T, pg, 0, nd), ref):
+        np.testing.assert_array_equal(a, b)
+    dev = [torch.from_numpy(np.ascontiguousarray(x)).cuda() for x in (sc, T, pg, nd)]
+    out = [torch.zeros(T.shape, dtype=torch.float64, device="cuda") for _ in range(4)]
+    e.hse_device(hm, *(x.data_ptr() for x in dev), n, W.NDEP, *(o.data_ptr() for o in out))
+    torch.cuda.synchronize()
+    for a, b in zip(out, ref):
+        np.testing.assert_array_equal(a.cpu().numpy(), b)
 
 
 def test_hse_device_pointers(fix):
