@@ -96,7 +96,7 @@ def test_autograd_contraction_forms(eng, ncol, nd, params, precision):
     dense = torch.randn(st.shape, generator=g, dtype=torch.float64, device="cuda")
     turned = torch.randn(st.shape[::-1], generator=g, dtype=torch.float64, device="cuda").permute(2, 1, 0)
     one = torch.ones((), dtype=torch.float64, device="cuda").expand(st.shape)
-    for grad in (dense, turned, one):
+    for grad in (dense, turned, one, dense.float()):
         (a,) = torch.autograd.grad(st, x, grad, retain_graph=True)
         w = grad.clone().requires_grad_(True)
         (b,) = torch.autograd.grad(st, x, w, retain_graph=True, create_graph=True)

@@ -370,15 +370,56 @@ def test_magneto_optical_matches_oracle_on_map():
 
 
 @pytest.mark.parametrize("prec", [0, 1])
-@pytest.mark.parametrize("ncol", [1, 63, 64, 65, 513, 1025, 4159])
+@pytest.mark.parametrize("ncol", [1, 63, 64, 65, 513, 1025, 4159, 4672, 4673])
 def test_gpu_batch_sizes_agree(engines, ncol, prec):
     """The split of a batch's blocks, wavelengths and continuum tiles over the
-    chip follows its size; a column's result does not: each equals, bit for
-    bit, the same column in a batch of 4200, which matches the oracle."""
+    chip follows its size, and in FP64 whether the points are formed before
+    the sweeps (up to 73 blocks of 64 columns here, 4672 columns); a column's
+    result does not: each equals, bit for bit, the same column in a batch of
+    4800, which matches the oracle."""
     eng = engines("lte", workloads.wavelengths_630())
-    atm = workloads.stokes_map(4200, seed=workloads.SEED_BASE + 71)
+    atm = workloads.stokes_map(4800, seed=workloads.SEED_BASE + 71)
     full = eng.synth_lte(atm, precision=prec)
     np.testing.assert_array_equal(eng.synth_lte(atm[:ncol], precision=prec), full[:ncol])
     if ncol == 65 and prec == 0:
         eI, eP = _err(full[:ncol], pyoracle.synth_lte(eng.model, atm[:ncol]))
         assert eI <= TOL_I and eP <= TOL_QUV
+
+
+@pytest.mark.parametrize("ncol", [65, 3985, 3986])
+def test_gpu_magneto_optical_batch_sizes_agree(ncol):
+    """The same with the magneto-optical terms, whose points reach their 3 GB
+    at 3985 columns."""
+    from conftest import GOLDEN
+    from pyrh_amd import api
+    e = api.engine_for(str(GOLDEN / "run_lte_mo"), workloads.wavelengths_630())
+    atm = workloads.stokes_map(4100, seed=workloads.SEED_BASE + 72)
+    full = e.synth_lte(atm, 0.8)
+    np.testing.assert_array_equal(e.synth_lte(atm[:ncol], 0.8), full[:ncol])
+
+
+@pytest.mark.parametrize("run", ["run_lte", "run_lte_mo"])
+def test_gpu_points_memory_cap(run, monkeypatch):
+    """PYRH_AMD_POINT_BYTES = 0 keeps the FP64 synthesis of few rays in one
+    pass, without memory for the points: the same bits."""
+    from conftest import GOLDEN
+    from pyrh_amd import model
+    from pyrh_amd.engine import Engine
+    import torch
+    m = model.build_model(model.open_run(str(GOLDEN / run)), workloads.wavelengths_630())
+    atm = workloads.stokes_map(300, seed=workloads.SEED_BASE + 73)
+
+    def synth():
+        e = Engine(m)
+        e.synth_lte(atm[:1], precision=1)       # the context's fixed memory
+        free = torch.cuda.mem_get_info()[0]
+        st = e.synth_lte(atm)
+        used = free - torch.cuda.mem_get_info()[0]
+        e.close()
+        return st, used
+    two, held = synth()
+    monkeypatch.setenv("PYRH_AMD_POINT_BYTES", "0")
+    one, less = synth()
+    np.testing.assert_array_equal(one, two)
+    points = 300 * 82 * 112 * 8 * (11 if run == "run_lte_mo" else 8)
+    assert held - less >= points

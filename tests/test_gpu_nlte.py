@@ -351,3 +351,55 @@ def test_nlte_more_columns_than_a_launch_takes(eng, nm):
     small = eng.nlte_solve(one, atm)[0]
     big = eng.nlte_solve(one, np.tile(atm, (n // 50, 1, 1)))[0]
     np.testing.assert_array_equal(big.reshape(n // 50, *small.shape), np.broadcast_to(small, (n // 50, *small.shape)))
+
+
+def test_nlte_columns_that_share_a_feautrier_workgroup(eng, nm):
+    """At 150 columns a continuum wavelength's workgroup holds several columns
+    (as many as keep every SIMD busy; the last group is part empty, the
+    columns differ in depth and retire one by one): bit for bit the columns in
+    batches of 6, each alone in its workgroup, and the oracle's."""
+    import copy
+    import pyoracle
+    from pyrh_amd import workloads
+    few = copy.copy(nm)
+    few.nmax_iter = 20     # some columns converge before, some do not
+    n = 150
+    atm = workloads.stokes_map(n, seed=workloads.SEED_BASE + 440)
+    nd = np.full(n, workloads.NDEP, np.int32)
+    nd[::7], nd[3::11] = 70, 66
+    for c in range(n):
+        atm[c, :, nd[c]:] = 0.0
+    nfe = len(nm.as_bezier) - 1 - int(np.count_nonzero((np.diff(nm.as_ptr) > 0) & (np.asarray(nm.as_bezier) > 0)))
+    assert n * nfe // 4 >= 1024 and n % 4 and 6 * nfe < 1024
+    pops, niter, dpops, st = eng.nlte_solve(few, atm, ndep=nd, mu=0.8, stokes=True)
+    assert niter.min() < niter.max()
+    for c in range(0, n, 6):
+        p, i, d, s = eng.nlte_solve(few, atm[c:c + 6], ndep=nd[c:c + 6], mu=0.8, stokes=True)
+        np.testing.assert_array_equal(pops[c:c + 6], p)
+        np.testing.assert_array_equal(niter[c:c + 6], i)
+        np.testing.assert_array_equal(dpops[c:c + 6], d)
+        np.testing.assert_array_equal(st[c:c + 6], s)
+    pick = [0, 3, 77, 149]
+    cp, cn, _, cs = pyoracle.nlte_solve(few, np.ascontiguousarray(atm[pick]), ndep=nd[pick], mu=0.8, stokes=True)
+    for q, c in enumerate(pick):
+        assert _relerr(pops[c, :, :nd[c]], cp[q, :, :nd[c]]) < TOL_POPS
+    assert _relerr(st[pick, 0], cs[:, 0]) < TOL_I
+    np.testing.assert_array_equal(niter[pick], cn)
+
+
+@pytest.mark.parametrize("nrays", [1, 4, 6, 11])
+def test_nlte_ray_counts(eng, nm, nrays):
+    """Ray counts off the chunks of five that the continuum wavelengths are
+    solved in, against the oracle."""
+    import copy
+    import pyoracle
+    from pyrh_amd import nlte, workloads
+    few = copy.copy(nm)
+    few.nmax_iter = 3
+    few.muz, few.wmu = nlte.gauss_legendre(nrays)
+    atm = workloads.stokes_map(3, seed=workloads.SEED_BASE + 450)
+    pops, niter, _, st = eng.nlte_solve(few, atm, mu=0.9, stokes=True)
+    cp, cn, _, cs = pyoracle.nlte_solve(few, atm, mu=0.9, stokes=True)
+    assert _relerr(pops, cp) < TOL_POPS
+    assert _relerr(st[:, 0], cs[:, 0]) < TOL_I
+    np.testing.assert_array_equal(niter, cn)
