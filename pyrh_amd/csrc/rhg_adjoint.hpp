@@ -129,7 +129,7 @@ __device__ __forceinline__ void delo_step_vjp(const StepCarry &C, const Point<do
   const double a1 = Pd.chi - (dsdn * (1.0 / 3.0)) * dchi_dn;
   const double c2 = a2 > 0.0 ? a2 : 0.0, c1 = a1 > 0.0 ? a1 : 0.0;
   const double dtau_dw = 0.25 * dsdn * (P0.chi + Pd.chi + c1 + c2);
-  const Bezier3<Dual<double>> bzd = bezier3(Dual<double>(C.dtau_uw, 1.0));
+  const Bezier3<Dual> bzd = bezier3_d(C.dtau_uw);
   const double al = bzd.alpha.v, be = bzd.beta.v, ga = bzd.gamma.v, th = bzd.theta.v,
                ep = bzd.eps.v;
   const double dt03 = C.dtau_uw * (1.0 / 3.0);

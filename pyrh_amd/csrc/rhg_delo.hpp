@@ -1,9 +1,9 @@
 // The polarized cubic DELO-Bezier recursion of one emergent ray
 // (rh/rhf1d/bezier_1D.c:52-300, to_obs: depth N-1 up to 0) split into its
 // prologue, one depth step and the last (linear) interval, on an explicit
-// state, for any number type T (double, float, or a dual number of either).
-// The synthesis kernels run it on plain numbers; the response-function
-// kernels run the same code on dual numbers to differentiate each step.
+// state, in the number type T.  The synthesis and the response functions'
+// forward sweep run it; the reverse sweep has each step's hand-written
+// vector-Jacobian product (rhg_adjoint.hpp).
 #pragma once
 
 #include "rhg_kernels.hpp"
@@ -159,20 +159,11 @@ __device__ __forceinline__ void delo_prologue(DeloState<T> &s, const Point<T> &P
 // in FP64; the FP64 form keeps the reference's eps = exp(-dtau).
 template <typename T> struct Wide { using type = T; static constexpr bool widened = false; };
 template <> struct Wide<float> { using type = double; static constexpr bool widened = true; };
-template <> struct Wide<Dual<float>> { using type = Dual<double>; static constexpr bool widened = true; };
 
 __device__ __forceinline__ double widen(double x) { return x; }
 __device__ __forceinline__ double widen(float x) { return (double) x; }
-__device__ __forceinline__ Dual<double> widen(Dual<double> x) { return x; }
-__device__ __forceinline__ Dual<double> widen(Dual<float> x) {
-  return Dual<double>((double) x.v, (double) x.d);
-}
 __device__ __forceinline__ void narrow(double x, double &y) { y = x; }
 __device__ __forceinline__ void narrow(double x, float &y) { y = (float) x; }
-__device__ __forceinline__ void narrow(Dual<double> x, Dual<double> &y) { y = x; }
-__device__ __forceinline__ void narrow(Dual<double> x, Dual<float> &y) {
-  y = Dual<float>((float) x.v, (float) x.d);
-}
 
 template <typename T>
 __device__ __forceinline__ void delo_rhs_solve(DeloState<T> &s, T alpha_, T beta_, T gamma_,
@@ -262,21 +253,12 @@ __device__ __forceinline__ void delo_step(DeloState<T> &s, const Point<T> &Pn, b
   s.dchi_c = dchi_dn;
 }
 
-// w3 weights of the last interval in double with their derivative in dtau
-// carried by dual numbers
+// w3 weights of the last interval in double
 __device__ __forceinline__ void w3_t(double dt, double *w) { w3(dt, w); }
 __device__ __forceinline__ void w3_t(float dt, float *w) {
   double wd[3];
   w3((double) dt, wd);
   w[0] = (float) wd[0]; w[1] = (float) wd[1]; w[2] = (float) wd[2];
-}
-template <typename R>
-__device__ __forceinline__ void w3_t(Dual<R> dt, Dual<R> *w) {
-  double wd[3], dw[2];
-  w3d((double) dt.v, wd, dw);
-  w[0] = {(R) wd[0], (R) dw[0] * dt.d};
-  w[1] = {(R) wd[1], (R) dw[1] * dt.d};
-  w[2] = {(R) wd[2], R(0)};
 }
 
 // The last (linear) interval, bezier_1D.c:264-299, from the state after the

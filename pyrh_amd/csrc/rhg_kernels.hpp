@@ -321,8 +321,7 @@ __device__ __forceinline__ void acc_prod(double &acc, const double &a, const dou
 
 // Profile of slot i of a wavelength's line list (line l) at one depth,
 // RLKProfile rh/kurucz.c:729-827 for the emergent ray (to_obs = 1), in the
-// number type T (double, float, or a dual number of either).  F(field)
-// returns a column-state field at that depth as a T; the Doppler offset
+// number type T.  F(field) returns a column-state field at that depth as a T; the Doppler offset
 // (lambda/lambda0 - 1) c comes from the line table in FP64.  Returns phi;
 // phi_Q,U,V are set for a polarizable line with damping, and with MO (the
 // magneto-optical terms) the Faraday-Voigt profiles psi[3] = psi_Q,U,V
@@ -351,8 +350,8 @@ __device__ __forceinline__ T line_profile_t(const Tab &tab, int i, int lb, const
       // component and lane, without the test
       auto component = [&](auto FAR, double shift, TV &Fw) -> T {
         const T u = v - T(shift) * vB;
-        const int reg = decltype(FAR)::value ? 0 : humlicek_region(val(adamp), val(u));
-        return (T) VoigtEval<TV>::eval((TV) adamp, (TV) u, reg, &Fw);
+        const int reg = decltype(FAR)::value ? 0 : humlicek_region(adamp, u);
+        return (T) voigt_humlicek_r<TV>((TV) adamp, (TV) u, reg, &Fw);
       };
       auto components = [&](auto FAR) {
         if constexpr (Tab::grouped) {
@@ -421,7 +420,7 @@ __device__ __forceinline__ T line_profile_t(const Tab &tab, int i, int lb, const
       // in region 0 (|u| + a >= 15 with |u| >= |v| - max|shift| |vB|, with
       // room for rounding), whose function is a third of the instructions of
       // the general one with its test and branches; most of a blended list.
-      if (__all(fabs(val(v)) - tab.smax(i) * fabs(val(vB)) + val(adamp) >= 15.01))
+      if (__all(fabs(v) - tab.smax(i) * fabs(vB) + adamp >= 15.01))
         components(std::true_type{});
       else
         components(std::false_type{});
@@ -439,7 +438,7 @@ __device__ __forceinline__ T line_profile_t(const Tab &tab, int i, int lb, const
         psi[2] = T(0.5) * (psi_sp - psi_sm) * cosg * sv;
       }
     } else {
-      phi = voigt_armstrong_t(adamp, v) * sv;
+      phi = (T) voigt_armstrong((double) adamp, (double) v) * sv;
     }
   } else {
     phi = (fabs(v) <= T(MAX_GAUSS_DOPPLER)) ? rexp(-v * v) : T(0);

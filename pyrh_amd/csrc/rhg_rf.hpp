@@ -118,8 +118,9 @@ __device__ __forceinline__ T point_get(const Point<T> &p, int m) {
 // and again in every wave's chain) left the chip idle: the points are formed
 // here with every depth at once and read back, 64 bytes each.
 //   90 columns of 64-256 depths, 350 wavelengths of the 400-line list, FP64:
-//   forward 23.0 -> 2.3 + 9.9 for the points, reverse 75.8 -> 25.3 ms; the
-//   512-column 112-wavelength batch (FP32 form) 0.85 -> 0.20 + 0.25 and
+//   forward 23.0 -> 2.3 + 9.9 for the points, reverse 75.8 -> 25.3 ms (5.0 for
+//   points and forward and 9.0 since lists are dealt out in pieces, xcd_tile);
+//   the 512-column 112-wavelength batch (FP32 form) 0.85 -> 0.20 + 0.25 and
 //   1.87 -> 1.17 ms
 // The synthesis of a batch of few rays takes the same two steps (MO: with the
 // magneto-optical terms, three more numbers per point).
@@ -396,7 +397,8 @@ k_rf_reverse(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
 // registers of those tangents: 1 wave per SIMD, 53.1 ms for 90 columns of
 // 64-256 depths x 350 wavelengths of the 400-line list, FP64, T, v_LOS and
 // B, and 2.49 ms for 512 columns x 112 wavelengths, FP32 form, all six.  This
-// form: 33.4 and 1.59 ms at two waves per SIMD.)
+// form: 33.4 and 1.59 ms at two waves per SIMD; 10.2 and 1.56 since lists are
+// dealt out in pieces, xcd_tile.)
 template <typename R, bool LT>
 __global__ void __launch_bounds__(64, 2)
 k_rf_chain(const DevModel *__restrict__ Mp, const int32_t *__restrict__ ndep,
