@@ -74,9 +74,13 @@ constexpr size_t kSplitBytes = (size_t) 3 << 30;
 // the hydrostatic builder's records held at a time: 16384 columns of 82
 // depths and 99 elements
 constexpr size_t kHseRecBytes = (size_t) 4 << 30;
-// LDS for a staged line list, at most: 16 KB keeps 8 one-wavefront
-// workgroups per CU (the register limit of the polarized kernels)
-constexpr size_t kLineTabMaxBytes = 16384;
+// LDS for a staged line list, at most: with 20 KB a CU's 160 KB keep 8
+// one-wavefront workgroups (the register limit of the polarized kernels)
+constexpr size_t kLineTabMaxBytes = 20480;
+// the same for k_rf_points, whose registers allow 12: 11 workgroups.  4096
+// columns under 60 lines (13.7 KB) take 31.8 ms staged and 33.2 from the model,
+// 73 lines (16.6 KB) 42.0 and 39.7, 85 lines 52.0 and 46.4
+constexpr size_t kLineTabPointsBytes = 160 * 1024 / 11;
 std::atomic<void *> g_scratch_ptr[kMaxDevices];
 std::mutex g_scratch_mutex;
 
@@ -653,10 +657,11 @@ static int launch_synth(rhg_context_t *c, const double *d_atm, const int32_t *d_
       const int kd = depth_split((int64_t) ncb * n_pol, Nmax);
       const dim3 grd((unsigned) rhg::xcd_grid(ncb, n_pol)),
           grdk(grd.x, (unsigned) ((Nmax + kd - 1) / kd));
+      const bool ltp = lt && c->tab_bytes <= kLineTabPointsBytes;
       if (c->dm.magneto_optical) {
-        if (lt) RHG_SPLIT(true, true); else RHG_SPLIT(false, true);
+        if (ltp) RHG_SPLIT(true, true); else RHG_SPLIT(false, true);
       } else {
-        if (lt) RHG_SPLIT(true, false); else RHG_SPLIT(false, false);
+        if (ltp) RHG_SPLIT(true, false); else RHG_SPLIT(false, false);
       }
     } else
 #undef RHG_SPLIT
@@ -1532,7 +1537,7 @@ int rf_chunk(rhg_context_t *c, const double *d_atm, const int32_t *d_ndep, int n
                      c->stream, c->d_model, d_ndep, moving, ncol, Nmax, state, c->d_out_ls,      \
                      c->d_io_pol, npol, cchi, ceta, mu, kd, pts, c->tab_maxl, c->tab_maxc)
     const bool lt = c->tab_bytes > 0 && c->tune_line_table;
-    if (lt) RHG_LAUNCH_PTS(true); else RHG_LAUNCH_PTS(false);
+    if (lt && c->tab_bytes <= kLineTabPointsBytes) RHG_LAUNCH_PTS(true); else RHG_LAUNCH_PTS(false);
 #undef RHG_LAUNCH_PTS
     HIPCHECK(hipGetLastError());
     hipLaunchKernelGGL((rhg::k_rf_forward<sizeof(R) == 4, true, false>), grd, blk, 0, c->stream, c->d_model, d_ndep,

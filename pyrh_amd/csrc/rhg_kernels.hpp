@@ -199,16 +199,11 @@ using LineTabGDirect = LineTabGlobal<false>;
 // each group feeds its own sum, so the sums see the same terms in the same
 // order as from the ungrouped list, and the component loop needs no
 // per-component branch.
-// (40 bytes: a list of up to 16 KB is staged)
 struct LineRecL {
-  static constexpr uint32_t DAMPED = 1u << 31, POLAR = 1u << 30, LINE = POLAR - 1;
-  double dv, larmor;
-  float smax;                // rounded up
-  uint32_t line;             // with DAMPED and POLAR
-  int c0, c1;
+  double dv, larmor, smax;
+  int line, flags, c0, c1;   // flags: 1 damped, 2 polarizable
   int cpi, csp;              // first pi and first sigma+ component
 };
-static_assert(sizeof(LineRecL) == 40, "LineRecL");
 
 struct LineTabL {
   static constexpr bool grouped = true;
@@ -216,15 +211,18 @@ struct LineTabL {
   const double *shift_, *strength_;
   const int *q_;
   int n;
-  __device__ __forceinline__ uint32_t word(int i) const {
-    return (uint32_t) __builtin_amdgcn_readfirstlane((int) rec[i].line);
+  __device__ __forceinline__ int line(int i) const {
+    return __builtin_amdgcn_readfirstlane(rec[i].line);
   }
-  __device__ __forceinline__ int line(int i) const { return (int) (word(i) & LineRecL::LINE); }
   __device__ __forceinline__ double dv(int i) const { return rec[i].dv; }
-  __device__ __forceinline__ bool damped(int i) const { return word(i) & LineRecL::DAMPED; }
-  __device__ __forceinline__ bool polar(int i) const { return word(i) & LineRecL::POLAR; }
+  __device__ __forceinline__ bool damped(int i) const {
+    return __builtin_amdgcn_readfirstlane(rec[i].flags) & 1;
+  }
+  __device__ __forceinline__ bool polar(int i) const {
+    return __builtin_amdgcn_readfirstlane(rec[i].flags) & 2;
+  }
   __device__ __forceinline__ double larmor(int i) const { return rec[i].larmor; }
-  __device__ __forceinline__ double smax(int i) const { return (double) rec[i].smax; }
+  __device__ __forceinline__ double smax(int i) const { return rec[i].smax; }
   __device__ __forceinline__ int c0(int i) const { return __builtin_amdgcn_readfirstlane(rec[i].c0); }
   __device__ __forceinline__ int c1(int i) const { return __builtin_amdgcn_readfirstlane(rec[i].c1); }
   __device__ __forceinline__ int cpi(int i) const { return __builtin_amdgcn_readfirstlane(rec[i].cpi); }
@@ -256,8 +254,9 @@ __device__ __forceinline__ LineTabL stage_lines(const DevModel &M, int ls, char 
     const bool damped = ldc(M.line_Grad)[l] != 0.0, polar = ldc(M.line_polar)[l] != 0;
     rec[i].dv = ldc(M.lam_line_dv)[p0 + i];
     rec[i].larmor = ldc(M.line_larmor)[l];
-    rec[i].smax = __double2float_ru(ldc(M.line_smax)[l]);
-    rec[i].line = (uint32_t) l | (damped ? LineRecL::DAMPED : 0u) | (polar ? LineRecL::POLAR : 0u);
+    rec[i].smax = ldc(M.line_smax)[l];
+    rec[i].line = l;
+    rec[i].flags = (damped ? 1 : 0) | (polar ? 2 : 0);
     // only a damped polarizable line uses its components
     rec[i].c1 = (damped && polar) ? ldc(M.line_comp_ptr)[l + 1] - ldc(M.line_comp_ptr)[l] : 0;
   }
@@ -274,7 +273,7 @@ __device__ __forceinline__ LineTabL stage_lines(const DevModel &M, int ls, char 
   // components grouped by Delta M = -1, 0, +1, each in the model's order
   for (int i = 0; i < n; i++) {
     const int a = rec[i].c0, cnt = rec[i].c1 - a;
-    const int g0 = ldc(M.line_comp_ptr)[rec[i].line & LineRecL::LINE];
+    const int g0 = ldc(M.line_comp_ptr)[rec[i].line];
     int nsm = 0, npi = 0;
     for (int c = 0; c < cnt; c++) {
       const int qc = ldc(M.comp_q)[g0 + c];
@@ -321,10 +320,10 @@ __device__ __forceinline__ void acc_prod(double &acc, const double &a, const dou
 
 // Profile of slot i of a wavelength's line list (line l) at one depth,
 // RLKProfile rh/kurucz.c:729-827 for the emergent ray (to_obs = 1), in the
-// number type T.  F(field) returns a column-state field at that depth as a T; the Doppler offset
-// (lambda/lambda0 - 1) c comes from the line table in FP64.  Returns phi;
-// phi_Q,U,V are set for a polarizable line with damping, and with MO (the
-// magneto-optical terms) the Faraday-Voigt profiles psi[3] = psi_Q,U,V
+// number type T.  F(field) returns a column-state field at that depth as a T;
+// the Doppler offset (lambda/lambda0 - 1) c comes from the line table in FP64.
+// Returns phi; phi_Q,U,V are set for a polarizable line with damping, and with
+// MO (the magneto-optical terms) the Faraday-Voigt profiles psi[3] = psi_Q,U,V
 // (rh/kurucz.c:811-819).  The Humlicek functions of the Zeeman components
 // are evaluated in TV (T, or float in the FP32 form), their sums and
 // combinations in T.
@@ -454,7 +453,7 @@ __device__ __forceinline__ T line_profile_f(const DevModel &M, int e, int l, con
                                             T vz, int moving, T &phi_Q, T &phi_U, T &phi_V,
                                             T *psi = nullptr) {
   (void) l;
-  return line_profile_t<T, TV, MO>(LineTabGDirect(M, e, 1), 0, line_field_base(M.ncont), F, mu, vz,
+  return line_profile_t<T, TV, MO>(LineTabG(M, e, 1), 0, line_field_base(M.ncont), F, mu, vz,
                                    moving, phi_Q, phi_U, phi_V, psi);
 }
 
@@ -504,8 +503,8 @@ __device__ __forceinline__ void line_point_f(const DevModel &M, int ls, const Fi
                                              T &chiI, T *chiQ, T &etaI, T *etaQ, int moving,
                                              T *chip = nullptr) {
   const int p0 = ldc(M.lam_line_ptr)[ls];
-  line_point_t<T, TV, MO>(LineTabGDirect(M, p0, ldc(M.lam_line_ptr)[ls + 1] - p0), M.ncont, F, mu, chiI, chiQ,
-                          etaI, etaQ, moving, chip);
+  line_point_t<T, TV, MO>(LineTabGDirect(M, p0, ldc(M.lam_line_ptr)[ls + 1] - p0), M.ncont, F, mu,
+                          chiI, chiQ, etaI, etaQ, moving, chip);
 }
 
 // the same with the fields read from the column state at st (stride fs)

@@ -186,10 +186,10 @@ def test_mixed_rf_sorted(eng):
         assert err < 1e-3
 
 
-@pytest.mark.parametrize("nline,staged", ((74, 1), (75, 0)))
+@pytest.mark.parametrize("nline,staged", ((74, 1), (89, 1), (90, 0)))
 def test_line_list_at_the_lds_limit(tmp_path, nline, staged):
-    """A line of nine components takes 40 + 9 * 20 bytes of the staged list's
-    16384: 74 such lines at one wavelength are staged, 75 are read from the
+    """A line of nine components takes 48 + 9 * 20 bytes of the staged list's
+    20480: 89 such lines at one wavelength are staged, 90 are read from the
     model; a staged list gives the bits of the other."""
     from pyrh_amd.engine import Engine
     run = W.mixed_run_dir(str(tmp_path / "run"), str(RUN))
