@@ -1858,6 +1858,7 @@ struct NlteHost {
   // (Bezier rays) first, then the continuum-only ones (Feautrier)
   std::vector<int32_t> ln_tr, ln_phi, io_list;
   int nbez = 0, nentry = 0, nphi = 0, maxset_bez = 0, maxset_fe = 0;
+  bool joined = false;   // two transitions join the same levels
 };
 
 int nlte_check(const rhg_context_t *c, const rhg_nlte_t *a, NlteHost &h) {
@@ -1882,6 +1883,7 @@ int nlte_check(const rhg_context_t *c, const rhg_nlte_t *a, NlteHost &h) {
   for (int t = 0; t < a->ntrans; t++) {
     const int i = a->tr_i[t], j = a->tr_j[t];
     if (i < 0 || j <= i || j >= nl) return fail(RHG_EINVAL, "transition levels out of range");
+    for (int u = 0; u < t; u++) h.joined |= a->tr_i[u] == i && a->tr_j[u] == j;
     if (a->tr_nblue[t] < 0 || a->tr_nlam[t] < 1 || a->tr_nblue[t] + a->tr_nlam[t] > ns)
       return fail(RHG_EINVAL, "transition span outside the grid");
     if (a->tr_ptr[t + 1] - a->tr_ptr[t] != a->tr_nlam[t]) return fail(RHG_EINVAL, "tr_ptr inconsistent");
@@ -2403,7 +2405,7 @@ int rhg_nlte_solve(rhg_context_t *c, const rhg_nlte_t *a, const rhg_columns_t *c
                      dim3((unsigned) nact, (unsigned) ((Nmax - 1) / rhg::stateq_depths(NLP) + 1)),  \
                      dim3(64 * rhg::stateq_waves(NLP)),                                             \
                      (size_t) rhg::stateq_depths(NLP) * nl * nl * sizeof(double), c->stream, d_at,  \
-                     B, d_act, nact, a->isum)
+                     B, d_act, nact, a->isum, h.joined ? 0 : 1)
         if (nl <= 4) RHG_LAUNCH_SE(4);
         else if (nl <= 6) RHG_LAUNCH_SE(6);
         else if (nl <= 8) RHG_LAUNCH_SE(8);

@@ -1381,12 +1381,15 @@ __device__ __forceinline__ void solve_improve_r(double (&a)[NLP][NLP], double (&
 // equation of the most populated level (isum = -1, else level isum) is
 // replaced by particle conservation.  The workgroup's wavefronts share
 // the sums (a transition's two directions are a task, the depths on the
-// lanes), the first one solves.  Launch (columns, ceil(Nmax / D)) workgroups
-// with D nl^2 doubles of LDS, D = stateq_depths.
+// lanes), the first one solves.  A task alone adds to its matrix element, as
+// long as no two transitions join the same levels; where some do (share = 0),
+// the first wavefront takes all tasks, in the transitions' order.  Launch
+// (columns, ceil(Nmax / D)) workgroups with D nl^2 doubles of LDS, D =
+// stateq_depths.
 template <int NLP>
 __global__ void __launch_bounds__(64 * stateq_waves(NLP))
 k_nlte_stateq(const DevNlte *__restrict__ Ap, NlteBufs B, const int32_t *__restrict__ act,
-              int nact, int isum) {
+              int nact, int isum, int share) {
   constexpr int D = stateq_depths(NLP), NT = 64 * stateq_waves(NLP) / D;
   const DevNlte &A = *Ap;
   extern __shared__ double gam[];   // [nl * nl][D]
@@ -1396,13 +1399,14 @@ k_nlte_stateq(const DevNlte *__restrict__ Ap, NlteBufs B, const int32_t *__restr
   const int64_t fs = B.fs, pk = (int64_t) ic * B.Kp + (k < N ? k : N - 1);
   for (int q = w; q < nl * nl; q += NT) gam[q * D + lane] = B.Cmat[(int64_t) q * fs + pk];
   __syncthreads();
-  for (int t = w; t < 2 * A.ntrans; t += NT) {
+  const int nt = share ? 2 * A.ntrans : (w ? 0 : 2 * A.ntrans);
+  for (int t = w; t < nt; t += share ? NT : 1) {
     const int tr = t >> 1, i = A.tr_i[tr], j = A.tr_j[tr], ne = A.tr_nlam[tr];
     const double *x = B.acc + ((int64_t) A.tr_ptr[tr] * 2 + (t & 1)) * fs + pk;
     double sum = 0.0;
 #pragma unroll 16
     for (int e = 0; e < ne; e++) sum += x[(int64_t) (2 * e) * fs];
-    atomicAdd(&gam[((t & 1) ? j * nl + i : i * nl + j) * D + lane], sum);
+    gam[((t & 1) ? j * nl + i : i * nl + j) * D + lane] += sum;
   }
   __syncthreads();
   if (w != 0 || k >= N) return;
@@ -1454,10 +1458,10 @@ k_nlte_stateq(const DevNlte *__restrict__ Ap, NlteBufs B, const int32_t *__restr
     if (i < nl) B.pops[(int64_t) i * fs + pk] = nk[i];
 }
 
-template __global__ void k_nlte_stateq<4>(const DevNlte *, NlteBufs, const int32_t *, int, int);
-template __global__ void k_nlte_stateq<6>(const DevNlte *, NlteBufs, const int32_t *, int, int);
-template __global__ void k_nlte_stateq<8>(const DevNlte *, NlteBufs, const int32_t *, int, int);
-template __global__ void k_nlte_stateq<16>(const DevNlte *, NlteBufs, const int32_t *, int, int);
+template __global__ void k_nlte_stateq<4>(const DevNlte *, NlteBufs, const int32_t *, int, int, int);
+template __global__ void k_nlte_stateq<6>(const DevNlte *, NlteBufs, const int32_t *, int, int, int);
+template __global__ void k_nlte_stateq<8>(const DevNlte *, NlteBufs, const int32_t *, int, int, int);
+template __global__ void k_nlte_stateq<16>(const DevNlte *, NlteBufs, const int32_t *, int, int, int);
 
 // ---------------------------------------------------------------------------
 // Ng acceleration of one column's populations and the maximum relative

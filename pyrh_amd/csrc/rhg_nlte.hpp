@@ -106,7 +106,7 @@ __global__ void k_nlte_djmax(NlteBufs B, const int32_t *act, int nact, int nlist
                              double *djmax);
 template <int NLP>
 __global__ void k_nlte_stateq(const DevNlte *Ap, NlteBufs B, const int32_t *act, int nact,
-                              int isum);
+                              int isum, int share);
 __global__ void k_nlte_ng(const DevNlte *Ap, NlteBufs B, const int32_t *act, int nact,
                           int niter, int norder, int ndelay, int nperiod, double *dpops);
 __global__ void k_nlte_out(const DevNlte *Ap, NlteBufs B, const double *src, double *out);

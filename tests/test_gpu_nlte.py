@@ -403,3 +403,36 @@ def test_nlte_ray_counts(eng, nm, nrays):
     assert _relerr(pops, cp) < TOL_POPS
     assert _relerr(st[:, 0], cs[:, 0]) < TOL_I
     np.testing.assert_array_equal(niter, cn)
+
+
+def test_nlte_transitions_that_join_the_same_levels(eng, nm):
+    """A continuum given as two of half its cross-section: against the oracle,
+    and the same bits in every run (the two transitions' rates add to one
+    matrix element, in the transitions' order)."""
+    import copy
+    import pyoracle
+    from pyrh_amd import workloads
+    two = copy.copy(nm)
+    two.nmax_iter = 4
+    t = int(np.flatnonzero(nm.tr_type == 1)[0])
+    n, p = nm.tr_type.size, int(nm.tr_ptr[t])
+    span = int(nm.tr_nlam[t])
+    add = lambda x, v: np.concatenate([x, np.atleast_1d(v)]).astype(x.dtype)
+    alpha = nm.tr_alpha.copy()
+    alpha[p:p + span] *= 0.5
+    for name in ("tr_type", "tr_i", "tr_j", "tr_nblue", "tr_nlam", "tr_line"):
+        setattr(two, name, add(getattr(nm, name), getattr(nm, name)[t]))
+    two.tr_ptr = add(nm.tr_ptr, nm.tr_ptr[-1] + span)
+    two.tr_alpha = add(alpha, alpha[p:p + span])
+    two.tr_wlam = add(nm.tr_wlam, nm.tr_wlam[p:p + span])
+    sets = [list(nm.as_tr[nm.as_ptr[k]:nm.as_ptr[k + 1]]) for k in range(nm.as_ptr.size - 1)]
+    for k in range(int(nm.tr_nblue[t]), int(nm.tr_nblue[t]) + span):
+        sets[k].append(n)
+    two.as_ptr = np.concatenate([[0], np.cumsum([len(x) for x in sets])]).astype(nm.as_ptr.dtype)
+    two.as_tr = np.concatenate([np.asarray(x, nm.as_tr.dtype) for x in sets])
+    atm = workloads.stokes_map(5, seed=workloads.SEED_BASE + 460)
+    ref = pyoracle.nlte_solve(two, atm)[0]
+    runs = [eng.nlte_solve(two, atm)[0] for _ in range(3)]
+    assert _relerr(runs[0], ref) < TOL_POPS
+    for r in runs[1:]:
+        np.testing.assert_array_equal(r, runs[0])
